@@ -405,16 +405,17 @@ VX_API vx_status vx_norm_mul_mat_swiglu(const vx_tensor * x, const vx_tensor * n
                                         const vx_tensor * up, const vx_tensor * dst, int act_mode, vx_stream stream);
 VX_API int vx_supports_norm_mul_mat_swiglu(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate,
                                            const vx_tensor * up, const vx_tensor * dst);
-/* the same call at prefill sizes (vx_supports_mul_mat_swiglu_tiled's shapes on the pre-tiled Q8_0 kernel, 1024 tokens or
- * more): the norm and its weight are applied by the pass that lays the activations out in tiles, x is read once and the
+/* the same call at prompt and prefill sizes (vx_supports_mul_mat_swiglu_tiled's shapes where the activations are laid out in
+ * tiles beforehand: up to 1024 tokens, and on the pre-tiled Q8_0 kernel beyond): the norm and its weight are applied by the pass that lays the activations out in tiles, x is read once and the
  * normalised tensor is never stored.  Same bits as RMS_NORM, MUL, then vx_mul_mat_swiglu. */
 VX_API int vx_supports_norm_mul_mat_swiglu_tiled(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate,
                                                  const vx_tensor * up, const vx_tensor * dst, int act_mode);
-/* mlp_forward and the residual update behind it at prefill sizes (src/minicpm.cpp:718-747, 775-786):
+/* mlp_forward and the residual update behind it at prompt and prefill sizes (17 tokens on; src/minicpm.cpp:718-747, 775-786):
  *   dst = residual + scale * (down . (silu(gate . n) * (up . n))),  n = RMS_NORM(x) * norm_w
  * for the node chain RMS_NORM, MUL, MUL_MAT, MUL_MAT, GLU(SWIGLU), MUL_MAT, SCALE, ADD.  The pair's results go to the down
  * projection as f16 tiles; the [tokens x ffn] tensor between them is not stored.  Same bits as the separate calls
- * (vx_norm_mul_mat_swiglu, vx_mul_mat_scale_add).  Q8_0 weights, VX_ACT_FLOAT, shapes that the pre-tiled kernel takes. */
+ * (vx_norm_mul_mat_swiglu, vx_mul_mat_scale_add).  VX_ACT_FLOAT, Q8_0 weights and shapes that the pre-tiled kernel takes, or
+ * Q8_0 / F16 weights at prompt sizes. */
 VX_API int vx_supports_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate, const vx_tensor * up,
                                  const vx_tensor * down, const vx_tensor * residual, const vx_tensor * dst, int act_mode);
 VX_API vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate,
@@ -425,8 +426,8 @@ VX_API vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, flo
 VX_API vx_status vx_mul_mat_swiglu(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * dst,
                                    int act_mode, vx_stream stream);
 VX_API int vx_supports_mul_mat_swiglu(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * dst);
-/* The same group at prefill sizes (64 tokens or more, f16 activations): both products on the LDS-tiled kernel, whose
- * work-groups hold a tile of gate rows and the same rows of up and apply the GLU as they store -- the two F32 products
+/* The same group at prompt and prefill sizes (what the streaming kernel no longer takes, f16 activations): both products on
+ * a tiled kernel, whose work-groups hold a tile of gate rows and the same rows of up and apply the GLU as they store -- the two F32 products
  * (tokens x 2 x rows x 4 bytes written and read again) never reach memory.  vx_mul_mat_swiglu takes these shapes too;
  * this predicate needs the activation mode because under VX_ACT_Q8 the tiled products run on kernels without that epilogue. */
 VX_API int vx_supports_mul_mat_swiglu_tiled(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * dst,

@@ -1,0 +1,101 @@
+"""GPU: the product kernel for 17 to 1024 tokens (csrc/gemm_mid.hip) at the edges of its tiles -- ragged token and row tiles,
+the shortest and longest K it takes, a batch, both weight types -- and the groups built on it against their separate calls."""
+import numpy as np
+import pytest
+
+from reflib import rng
+from test_gpu_fused import dev, ok, q8_dev, same_bits, say
+
+pytestmark = pytest.mark.gpu
+
+
+def dequant(q, K):
+    b = q.reshape(q.shape[0], K // 32, 34)
+    d = np.ascontiguousarray(b[:, :, :2]).view(np.float16).astype(np.float64)
+    return (np.ascontiguousarray(b[:, :, 2:]).view(np.int8).astype(np.float64) * d).reshape(q.shape[0], K)
+
+
+@pytest.mark.parametrize("M,K,N,nb", [(16, 1024, 17, 1), (1000, 1024, 33, 1), (128, 768, 64, 2), (1024, 1024, 203, 1), (40, 2304, 31, 3),
+                                      (1024, 4096, 129, 1), (520, 4096, 17, 1), (4096, 1024, 65, 1), (1024, 1024, 1024, 1), (72, 16384, 100, 1)])
+@pytest.mark.parametrize("wtype", ["q8", "f16"])
+def test_products(pkg, gpu, monkeypatch, M, K, N, nb, wtype):
+    import torch
+    say(f"product of some tens of tokens M={M} K={K} N={N} batch={nb} weights={wtype}")
+    L, d = pkg.lib(), pkg.desc
+    g = rng("mid", M, K, N, nb)
+    w = (0.05 * g.standard_normal((M, K))).astype(np.float32)
+    if wtype == "q8":
+        wg, _ = q8_dev(w)
+        wd, w64 = pkg.desc_q8(wg, K), dequant(wg.cpu().numpy(), K)
+    else:
+        wg = dev(w.astype(np.float16))
+        wd, w64 = d(wg), w.astype(np.float16).astype(np.float64)
+    x = g.standard_normal((nb, N, K)).astype(np.float32)
+    xd = dev(x)
+    out = torch.full((nb, N + 2, M), 7.0, dtype=torch.float32, device="cuda")   # a strided destination: rows past N must stay
+    dst = out[:, :N].unsqueeze(1) if nb > 1 else out[0, :N]
+    ok(pkg, L.vx_mul_mat(wd, d(xd.unsqueeze(1) if nb > 1 else xd[0]), d(dst), pkg.ACT_FLOAT, None), "mul_mat")
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert (got[:, N:] == 7.0).all()
+    x16 = x.astype(np.float16).astype(np.float64)
+    # fp32 sums of exact products: 32 terms inside an instruction, K / 128 scaled additions per group of blocks, four groups
+    bound = (32 + K // 128 + 4) * 2.0 ** -24 * np.einsum("bnk,mk->bnm", np.abs(x16), np.abs(w64), optimize=True)
+    assert (np.abs(got[:, :N] - np.einsum("bnk,mk->bnm", x16, w64, optimize=True)) <= bound + 1e-30).all()
+    # the residual update is the product's value, scaled and added with a rounding each
+    res = dev(g.standard_normal((nb, N, M)).astype(np.float32))
+    upd = torch.empty_like(res)
+    v = (lambda t: t.unsqueeze(1)) if nb > 1 else (lambda t: t[0])
+    ok(pkg, L.vx_mul_mat_scale_add(wd, d(v(xd)), d(v(res)), d(v(upd)), 0.7, pkg.ACT_FLOAT, None), "mul_mat_scale_add")
+    torch.cuda.synchronize()
+    prod = torch.from_numpy(got[:, :N]).cuda()
+    assert same_bits(upd, (res + prod * np.float32(0.7)).contiguous())
+    if K in (768, 1024) and M <= 1024 and N <= 448:   # the streaming kernel's shapes: the same order of every sum
+        monkeypatch.setenv("VX_GEMM_MID", "0")
+        old = torch.empty((nb, N, M), dtype=torch.float32, device="cuda")
+        ok(pkg, L.vx_mul_mat(wd, d(v(xd)), d(v(old)), pkg.ACT_FLOAT, None), "mul_mat")
+        torch.cuda.synchronize()
+        assert same_bits(old, prod.contiguous())
+
+
+@pytest.mark.parametrize("T,B", [(17, 1), (45, 1), (64, 1), (203, 1), (300, 3), (1024, 1)])
+@pytest.mark.parametrize("wtype", ["q8", "f16"])
+def test_groups_equal_their_separate_calls(pkg, gpu, T, B, wtype):
+    """norm + q/k/v + rope and the MLP with its residual update, sequences flattened into one token dimension."""
+    import torch
+    say(f"layer groups of some tens of tokens T={T} B={B} weights={wtype}")
+    L, d = pkg.lib(), pkg.desc
+    K, H, Hkv, F, N = 1024, 16, 2, 4096, T * B
+    g = rng("mid-groups", T, B)
+    keep = []
+
+    def weight(m, k):
+        w = (0.05 * g.standard_normal((m, k))).astype(np.float32)
+        t = q8_dev(w)[0] if wtype == "q8" else dev(w.astype(np.float16))
+        keep.append(t)
+        return pkg.desc_q8(t, k) if wtype == "q8" else d(t)
+
+    wq, wk, wv, wg, wu, wd = weight(K, K), weight(128, K), weight(128, K), weight(F, K), weight(F, K), weight(K, F)
+    x, nw = dev((2 * g.standard_normal((N, K))).astype(np.float32)), dev((1 + 0.1 * g.standard_normal(K)).astype(np.float32))
+    pos, ff = dev((np.arange(T) + 5).astype(np.int32)), dev((1 + g.random(32)).astype(np.float32))
+    new = lambda *s: torch.full(s, float("nan"), dtype=torch.float32, device="cuda")
+    rope = (64, 2, 32768, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+    n, q1, k1, v1, q2, k2, v2 = new(N, K), new(B, T, H, 64), new(B, T, Hkv, 64), new(N, 128), new(B, T, H, 64), new(B, T, Hkv, 64), new(N, 128)
+    ok(pkg, L.vx_rms_norm_mul(d(x), d(nw), d(n), 1e-5, None), "norm")
+    for w, t, rot in ((wq, q1, True), (wk, k1, True), (wv, v1, False)):
+        ok(pkg, L.vx_mul_mat(w, d(n), d(t.view(N, -1)), pkg.ACT_FLOAT, None), "mul_mat")
+        if rot:
+            ok(pkg, L.vx_rope(d(t), pos.data_ptr(), ff.data_ptr(), d(t), *rope, None), "rope")
+    assert L.vx_supports_norm_qkv_proj_rope_tiled(d(x), d(nw), wq, wk, wv, d(q2), d(k2), d(v2), 64, 2, pkg.ACT_FLOAT) == 1
+    ok(pkg, L.vx_norm_qkv_proj_rope(d(x), d(nw), 1e-5, wq, wk, wv, pos.data_ptr(), ff.data_ptr(), d(q2), d(k2), d(v2), *rope, pkg.ACT_FLOAT, None), "qkv")
+    torch.cuda.synchronize()
+    assert same_bits(q1, q2) and same_bits(k1, k2) and same_bits(v1, v2)
+    gate, up, act, o1, o2 = new(N, F), new(N, F), new(N, F), new(N, K), new(N, K)
+    ok(pkg, L.vx_mul_mat(wg, d(n), d(gate), pkg.ACT_FLOAT, None), "gate")
+    ok(pkg, L.vx_mul_mat(wu, d(n), d(up), pkg.ACT_FLOAT, None), "up")
+    ok(pkg, L.vx_glu(pkg.GLU_SWIGLU, d(gate), d(up), d(act), 0, None), "glu")
+    ok(pkg, L.vx_mul_mat_scale_add(wd, d(act), d(x), d(o1), 0.3, pkg.ACT_FLOAT, None), "down")
+    assert L.vx_supports_mlp_tiled(d(x), d(nw), wg, wu, wd, d(x), d(o2), pkg.ACT_FLOAT) == 1
+    ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, wg, wu, wd, d(x), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp_tiled")
+    torch.cuda.synchronize()
+    assert same_bits(o1, o2)

@@ -1,0 +1,572 @@
+// gemm_mid.hip -- MUL_MAT for some tens to a thousand tokens (a prompt, concurrent LocDiT requests): Q8_0 / F16 weights.
+//
+// What bounds these products is neither the matrix cores nor HBM (a 203-token layer is 6 GFLOP and 16 MB of weights) but
+// what each of the chip's 256 compute units has to bring in and issue for its small tile, and the time until its first
+// bytes arrive.  Hence:
+//   * the activations are rounded to f16 once, by a pass of their own that also applies a fused norm and fills the
+//     rotation's angle table (gm_acts_kernel), and laid out as 1 KB operand tiles: a work-group brings in half the bytes
+//     and converts nothing;
+//   * weights come as raw Q8_0 rows (1.06 bytes a weight), both by direct loads into LDS issued by two waves that do
+//     nothing else -- with every wave loading and multiplying, two fifths of a step's 218 instructions were address,
+//     branch and M0 bookkeeping in front of the products (64 x 64 tile: 0.54 us per 128 of K, 0.36 now);
+//   * four waves of a row group share the k blocks (block kb: group kb mod 4), so that small tiles keep a compute unit's
+//     four SIMDs busy; their sums are added in group order at the end -- the order of the streaming kernel's four waves
+//     (mul_mat.hip), whose products of more than 16 tokens come out with the same bits here;
+//   * a step's products are interleaved with their scaled additions and with the next step's conversion: a SIMD issues one
+//     vector instruction every four cycles, so an exactly scaled 16 x 16 x 32 product costs its own slot and four
+//     additions, 20 cycles against the matrix core's 16, plus the conversions -- 7 slots in all at two row tiles x eight
+//     token tiles a wave.
+// Measured on cold weights (microseconds a launch, without the 3 us of the activation pass, which the norm's launch was
+// before; in brackets the streaming / LDS-tiled kernels of mul_mat.hip): 203 tokens: 1024 x 1024 4.7 [10.7], 1024 x 4096 8.8
+// [16.6 + 4.4 for the K cut's second launch], gate/up pair 10.9 [20.7]; 45 tokens: 3.7 [5.8], 6.7 [9.9 + 6.0], 6.0 [7.3 +
+// 7.3 + 3.4]; 1024 tokens: 7.5 [10], 17.7 [26 + 5.5], 38 [46].
+#include "gemm_mid.hpp"
+#include "mm_common.hpp"
+
+#include <cstdlib>
+#include <type_traits>
+
+namespace {
+
+struct gm_args {
+    vx_gm_mat     mat[3];
+    int           nmat;
+    const char *  w2;
+    const half8_t * xt;            // [batch][k block][n_tt][64] operand tiles
+    int           n_tt, n_kb;
+    int           N, ne12;
+    const char *  res;
+    uint64_t      rnb1, rnb2, rnb3;
+    float         res_scale;
+    _Float16 *    tile_out;
+    int           out_tt;
+    const float2 * rope_tab;       // [token][32] cos, sin
+};
+
+enum { GM_PLAIN = 0, GM_SWIGLU = 1, GM_SEGS = 2 };
+
+template <int N> __device__ __forceinline__ void gm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
+
+template <int WT, int MT, int NT, int RW, int KG, int CH, int S>
+struct gm_shape {
+    static constexpr int NC = KG * RW, NWAVES = NC + 2;       // compute waves; one wave brings the weights, one the activations
+    static constexpr int ROWS = 16 * MT * RW, TOKS = 16 * NT;
+    static constexpr int PIECES = WT == VX_GM_Q8 ? (CH == 1 ? 9 : 17) : 16 * CH; // 16-byte pieces of a row per stage
+    static constexpr int PITCH = PIECES * 16;
+    static constexpr int WINST = (ROWS * PIECES + 63) / 64, XINST = 4 * CH * NT;
+    static constexpr int WBYTES = WINST * 1024, XBYTES = XINST * 1024, STAGE = WBYTES + XBYTES;
+    static constexpr int STEPS = 4 * CH / KG;                 // k blocks of a stage per compute wave
+    static constexpr int NP = NT < 4 ? NT : 4;                // token tiles per pass of the final sum
+    static constexpr int RED = KG * RW * MT * NP * 1024;
+    static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
+};
+
+template <int WT, int MT, int NT, int RW, int KG, int CH, int S, int EPI>
+__global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a) {
+    using sh = gm_shape<WT, MT, NT, RW, KG, CH, S>;
+    static_assert((CH == 1 || CH == 2) && 4 * CH % KG == 0, "stages of 128 or 256 k, whole steps");
+    static_assert(EPI == GM_PLAIN || MT % 2 == 0, "pairs of row tiles inside a wave");
+    extern __shared__ __align__(1024) char gm_smem[];
+    typedef __attribute__((address_space(3))) char lds_char;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
+    const int j = lane >> 4, c = lane & 15;
+    const int g = wid % KG, rw = wid / KG; // k group (block kb belongs to group kb mod KG), row group
+
+    int mi = 0, tx = blockIdx.x;
+    if constexpr (EPI == GM_SEGS) {
+        if (a.nmat > 1 && tx >= a.mat[1].wg0) mi = 1;
+        if (a.nmat > 2 && tx >= a.mat[2].wg0) mi = 2;
+        tx -= a.mat[mi].wg0;
+    }
+    const vx_gm_mat & mt = a.mat[mi];
+    const int M = mt.M;
+    if (tx * sh::ROWS >= (EPI == GM_SWIGLU ? 2 * M : M)) return; // padding of the grid
+    const int tt0 = blockIdx.y * NT;
+    const int batch = blockIdx.z;
+    const int nst = a.n_kb / (4 * CH);
+
+    // first row of local row tile lt (wave row rw holds lt = rw * MT + m)
+    auto row_of = [&](int lt) {
+        if constexpr (EPI == GM_SWIGLU) return tx * (sh::ROWS / 2) + 16 * (lt >> 1);      // even tiles W, odd tiles the same rows of W2
+        if constexpr (EPI == GM_SEGS && MT == 2) { // 32 rows a wave: (d .. d + 15, d + 32 .. d + 47) of one head
+            const int q = tx * RW + lt / MT;
+            return (q >> 1) * 64 + 16 * (q & 1) + 32 * (lt % MT);
+        }
+        return tx * sh::ROWS + 16 * lt;
+    };
+
+    const uint32_t smem0 = (uint32_t) (uintptr_t) (lds_char *) gm_smem;
+    float4_t acc[MT][NT];
+    if (wid >= sh::NC) {
+        // ---- the two waves that fill the stages.  Stage st is announced by barrier st; the stage that takes its buffer
+        // again is requested after barrier st + 1, when every compute wave holds stage st's operands in registers.
+        if (wid == sh::NC) {
+            const char * wptr[sh::WINST];
+#pragma unroll
+            for (int i = 0; i < sh::WINST; ++i) {
+                const int P = i * 64 + lane, row = min(P / sh::PIECES, sh::ROWS - 1); // (the last load's spare lanes: into the stage's padding)
+                int piece = P % sh::PIECES;
+                const int lt = row >> 4, cc = row & 15;
+                if constexpr (WT == VX_GM_F16) piece ^= cc; // the sixteen rows' pieces over the banks
+                const char * wsel = EPI == GM_SWIGLU && (lt & 1) ? a.w2 : mt.w;
+                wptr[i] = wsel + (uint64_t) (uint32_t) min(row_of(lt) + cc, M - 1) * mt.nb01 + piece * 16;
+            }
+            auto issue = [&](int st, int buf) {
+                const uint32_t base = smem0 + (uint32_t) buf * sh::STAGE;
+                const int woff = WT == VX_GM_F16 ? 256 * CH * st : CH == 2 ? 272 * st : 136 * st - 8 * (st & 1);
+#pragma unroll
+                for (int i = 0; i < sh::WINST; ++i)
+                    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(wptr[i] + woff), "s"(base + (uint32_t) i * 1024) : "memory");
+            };
+            constexpr int L = sh::WINST;
+            static_assert(L * (S - 2) <= 63, "loads in flight are counted in six bits");
+#pragma unroll
+            for (int s = 0; s < S; ++s) if (s < nst) issue(s, s);
+            int buf = S - 1; // where the stage before last lies (st = 0: unused)
+            for (int st = 0; st < nst; ++st) {
+                const int younger = min(st == 0 ? S - 1 : S - 2, nst - 1 - st);
+                if (younger >= S - 2) gm_wait<L * (S - 2)>();
+                else if (S > 3 && younger == 1) gm_wait<L>();
+                else gm_wait<0>();
+                __builtin_amdgcn_s_barrier();
+                if (st > 0 && st - 1 + S < nst) issue(st - 1 + S, buf);
+                buf = buf + 1 == S ? 0 : buf + 1;
+            }
+        } else {
+            const char * xsrc = (const char *) (a.xt + ((int64_t) batch * a.n_kb * a.n_tt + tt0) * 64);
+            const uint32_t loff = (uint32_t) lane * 16;
+            auto issue = [&](int st, int buf) {
+                const uint32_t base = smem0 + (uint32_t) buf * sh::STAGE + sh::WBYTES;
+#pragma unroll
+                for (int kb = 0; kb < 4 * CH; ++kb) { // NT consecutive tiles of a k block (past the last token tile: the next block's, dropped at the store)
+                    const char * p = xsrc + (int64_t) (st * 4 * CH + kb) * a.n_tt * 1024;
+#pragma unroll
+                    for (int t0 = 0; t0 < NT; t0 += 4) {
+                        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(loff), "s"(p + t0 * 1024), "s"(base + (uint32_t) (kb * NT + t0) * 1024) : "memory");
+                        if (t0 + 1 < NT) asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(loff), "s"(p + t0 * 1024) : "memory");
+                        if (t0 + 2 < NT) asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(loff), "s"(p + t0 * 1024) : "memory");
+                        if (t0 + 3 < NT) asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(loff), "s"(p + t0 * 1024) : "memory");
+                    }
+                }
+            };
+            constexpr int L = sh::XINST;
+            static_assert(L * (S - 2) <= 63, "loads in flight are counted in six bits");
+#pragma unroll
+            for (int s = 0; s < S; ++s) if (s < nst) issue(s, s);
+            int buf = S - 1;
+            for (int st = 0; st < nst; ++st) {
+                const int younger = min(st == 0 ? S - 1 : S - 2, nst - 1 - st);
+                if (younger >= S - 2) gm_wait<L * (S - 2)>();
+                else if (S > 3 && younger == 1) gm_wait<L>();
+                else gm_wait<0>();
+                __builtin_amdgcn_s_barrier();
+                if (st > 0 && st - 1 + S < nst) issue(st - 1 + S, buf);
+                buf = buf + 1 == S ? 0 : buf + 1;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[m][n] = float4_t{0, 0, 0, 0};
+        // this lane's operand addresses inside a stage: its row of row tile 0, its slot of token tile 0
+        const uint32_t wl = (uint32_t) ((rw * MT * 16 + c) * sh::PITCH + (WT == VX_GM_Q8 ? VX_Q8_BLOCK * g : 0));
+        const uint32_t xl = (uint32_t) (sh::WBYTES + g * NT * 1024 + lane * 16);
+        const uint32_t sh16 = g & 1 ? 0u : 16u;                       // an even block's quants sit 2 bytes into their dwords
+        const uint32_t qoff = 8u * (uint32_t) j + (g & 1 ? 2u : 0u);
+        typedef const __attribute__((address_space(3))) uint32_t lds_u32;
+        typedef const __attribute__((address_space(3))) half8_t  lds_half8;
+        // The operands of a step are in registers before it begins: the weights' as f16 (bop, with the block scales d), the
+        // activations' (x).  While it is multiplied the next step's bytes are read, x[n] as soon as its last product has
+        // been issued, and the weights' are turned into f16 between the second half of the products.
+        struct wops { half8_t bop[MT]; float d[MT]; } A, B;
+        half8_t  x[NT];
+        uint32_t wq[MT][3]; _Float16 wd[MT];
+        auto read_w = [&](wops & o, int st, int sp, int buf) {
+            const lds_char * base = (const lds_char *) gm_smem + buf * sh::STAGE;
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                if constexpr (WT == VX_GM_Q8) {
+                    const lds_char * p = base + wl + (CH == 1 ? 8 * (st & 1) : 0) + sp * (KG * VX_Q8_BLOCK) + m * 16 * sh::PITCH;
+                    lds_u32 * qp = (lds_u32 *) (p + qoff);
+                    wq[m][0] = qp[0]; wq[m][1] = qp[1]; wq[m][2] = qp[2];
+                    wd[m] = *(const __attribute__((address_space(3))) _Float16 *) p;
+                } else {
+                    const uint32_t piece = (uint32_t) (4 * (KG * sp + g) + j) ^ (uint32_t) c;
+                    o.bop[m] = *(lds_half8 *) (base + (rw * MT * 16 + m * 16 + c) * sh::PITCH + piece * 16);
+                }
+            }
+        };
+        auto convert = [&](wops & o, int m) {
+            o.bop[m] = q8_to_half8(__builtin_amdgcn_alignbit(wq[m][1], wq[m][0], sh16), __builtin_amdgcn_alignbit(wq[m][2], wq[m][1], sh16));
+            o.d[m] = (float) wd[m];
+            asm volatile("" : "+v"(o.d[m]));
+        };
+        auto read_x = [&](int n, int sp, int buf) { x[n] = *(lds_half8 *) ((const lds_char *) gm_smem + buf * sh::STAGE + xl + (sp * KG * NT + n) * 1024); };
+        auto step = [&](auto MORE, const wops & o, wops & nx, int st1, int sp1, int buf1) {
+            constexpr bool more = decltype(MORE)::value;
+            if constexpr (more) read_w(nx, st1, sp1, buf1);
+            constexpr int T = MT * NT, LAG = T < 2 ? T : 2; // the scaled additions of a product follow the MFMA LAG further on
+            float4_t blk[LAG];
+#pragma unroll
+            for (int i = 0; i < T + (WT == VX_GM_Q8 ? LAG : 0); ++i) {
+                if constexpr (WT == VX_GM_Q8) {
+                    if (i >= LAG) {
+                        const int q = i - LAG;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[q % MT][q / MT][r] = __builtin_fmaf(blk[q % LAG][r], o.d[q % MT], acc[q % MT][q / MT][r]);
+                    }
+                    if (i < T) blk[i % LAG] = mfma16(x[i / MT], o.bop[i % MT], float4_t{0, 0, 0, 0});
+                } else if (i < T) {
+                    acc[i % MT][i / MT] = mfma16(x[i / MT], o.bop[i % MT], acc[i % MT][i / MT]);
+                }
+                if constexpr (more) {
+                    if (i < T && i % MT == MT - 1) read_x(i / MT, sp1, buf1);
+                    if constexpr (WT == VX_GM_Q8) {
+                        constexpr int H = T / 2, E = (T - H) / MT > 0 ? (T - H) / MT : 1; // convert tile m behind product H + E m
+                        if constexpr (T >= 2 * MT) { if (i >= H && (i - H) % E == 0 && (i - H) / E < MT) convert(nx, (i - H) / E); }
+                        else if (i == T - 1) { _Pragma("unroll") for (int m = 0; m < MT; ++m) convert(nx, m); }
+                    }
+                }
+            }
+        };
+        auto barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+        barrier();
+        read_w(A, 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) read_x(n, 0, 0);
+        if constexpr (WT == VX_GM_Q8) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) convert(A, m);
+        }
+        int buf = 0;
+        using more = std::true_type;
+        using last = std::false_type;
+        auto advance = [&]() { buf = buf + 1 == S ? 0 : buf + 1; barrier(); };
+        // (two steps a turn and no branch inside a turn: across one the compiler would sink a step's additions)
+        if constexpr (sh::STEPS == 1) {
+            for (int st = 0; st + 2 < nst; st += 2) {
+                advance();
+                step(more{}, A, B, st + 1, 0, buf);
+                advance();
+                step(more{}, B, A, st + 2, 0, buf);
+            }
+            advance();
+            step(more{}, A, B, nst - 1, 0, buf);
+        } else {
+            for (int st = 0; st + 1 < nst; ++st) {
+                step(more{}, A, B, st, 1, buf);
+                advance();
+                step(more{}, B, A, st + 1, 0, buf);
+            }
+            step(more{}, A, B, nst - 1, 1, buf);
+        }
+        step(last{}, B, A, 0, 0, 0);
+    }
+
+    // ---- the k groups' sums, in group order; wave (rw, g) finishes token tiles n = g mod 4 of its row group
+    const int  i12 = batch % a.ne12, i13 = batch / a.ne12;
+    float4_t * red = (float4_t *) gm_smem; // [group][row group][m][n - 4 p][lane]
+#pragma unroll
+    for (int p = 0; p < (NT + 3) / 4; ++p) {
+        constexpr int NP = sh::NP;
+        __syncthreads();
+        if (wid < sh::NC) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NP; ++n)
+                    if (4 * p + n < NT) red[(((g * RW + rw) * MT + m) * NP + n) * 64 + lane] = acc[m][4 * p + n];
+        }
+        __syncthreads();
+        const int n = g;
+        if (wid >= sh::NC || n >= NP || 4 * p + n >= NT) continue; // (uniform; nothing below synchronises)
+        const int tok0 = 16 * (tt0 + 4 * p + n);
+        if (tok0 >= a.N) continue;
+        float4_t v[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            v[m] = red[((rw * MT + m) * NP + n) * 64 + lane];
+#pragma unroll
+            for (int gg = 1; gg < KG; ++gg) v[m] += red[(((gg * RW + rw) * MT + m) * NP + n) * 64 + lane];
+        }
+        char * db = mt.dst + (uint64_t) i12 * mt.nb2 + (uint64_t) i13 * mt.nb3;
+        if constexpr (EPI == GM_SWIGLU) {
+#pragma unroll
+            for (int m = 0; m < MT; m += 2) {
+                const int row = row_of(rw * MT + m) + c;
+                if (row >= M) continue;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int   tok = tok0 + 4 * j + r;
+                    const float gt = v[m][r], u = v[m + 1][r];
+                    float h = (gt / (1.0f + expf(-gt))) * u;
+                    if (a.tile_out) { // (uniform) rounded to f16 as the next product's activation pass would round it; whole tiles are written
+                        asm volatile("" : "+v"(h)); // the fp32 value the GLU node holds, formed as such
+                        const uint64_t tile = ((uint64_t) batch * (uint32_t) (M >> 5) + (uint32_t) (row >> 5)) * (uint32_t) a.out_tt + (uint32_t) (tok >> 4);
+                        a.tile_out[(tile * 64 + ((row >> 3) & 3) * 16 + (tok & 15)) * 8 + (row & 7)] = (_Float16) h;
+                    } else if (tok < a.N) {
+                        *(float *) (db + (uint64_t) tok * mt.nb1 + (uint64_t) row * 4) = h;
+                    }
+                }
+            }
+        } else {
+            if constexpr (EPI == GM_SEGS) {
+                if (mt.rope) { // (uniform) tile m holds d = row mod 64 < 32, tile m + MT / 2 the partners d + 32
+#pragma unroll
+                    for (int m = 0; m < MT / 2; ++m) {
+                        const int d = (row_of(rw * MT + m) + c) & 31;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int    tok = min(tok0 + 4 * j + r, a.N - 1);
+                            const float2 cs = a.rope_tab[tok * 32 + d];
+                            float y0, y1;
+                            rope_rotate(v[m][r], v[m + MT / 2][r], cs.x, cs.y, y0, y1);
+                            v[m][r] = y0; v[m + MT / 2][r] = y1;
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const int row = row_of(rw * MT + m) + c;
+                if (row >= M) continue;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int tok = tok0 + 4 * j + r;
+                    if (tok >= a.N) continue;
+                    float val = v[m][r];
+                    if (EPI == GM_PLAIN && a.res)
+                        val = scaled_residual(val, a.res_scale, *(const float *) (a.res + (uint64_t) i12 * a.rnb2 + (uint64_t) i13 * a.rnb3 + (uint64_t) tok * a.rnb1 + (uint64_t) row * 4));
+                    *(float *) (db + (uint64_t) tok * mt.nb1 + (uint64_t) row * 4) = val;
+                }
+            }
+        }
+    }
+}
+
+// ---- activations -> operand tiles ------------------------------------------------------------------------------------
+struct gm_acts {
+    const char *  x;
+    uint64_t      nb11, nb12, nb13;
+    int           ne12, N, K, n_tt, n_kb, row_blocks;
+    const float * norm_w;
+    float         eps;
+    half8_t *     xt;
+    // rotation angles of the launch behind (blocks from row_blocks on)
+    const int32_t * pos; const float * ff;
+    rope_params   rp;
+    int           rope_T;
+    float2 *      tab;
+};
+
+// One wave = one token: its row rounded to f16 (normalised first: RMS_NORM in the RMS_NORM kernel's wave-per-row order, then
+// the MUL node, each rounded as the separate kernels round) and stored as its sixteen-byte pieces of the tiles.  Four tokens
+// a work-group and no LDS: with some tens to a thousand tokens the pass is one trip to memory and its latency, and a tile's
+// sixteen rows in one work-group of 1024 threads (as qt_acts_norm_kernel has it for prefill sizes) leave most of the chip idle.
+template <bool NORM>
+__global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
+    if ((int) blockIdx.x >= a.row_blocks) { // the angle table: (cos, sin) of (token, pair), a chain of multiplications and two trigonometric evaluations each
+        const int idx = ((int) blockIdx.x - a.row_blocks) * 256 + (int) threadIdx.x;
+        if (idx >= a.N * 32 || blockIdx.y) return;
+        const int tok = idx >> 5, ip = idx & 31;
+        float c, sn;
+        rope_cos_sin(a.rp, (float) a.pos[tok % a.rope_T], ip, a.ff ? a.ff[ip] : 1.0f, c, sn);
+        a.tab[idx] = make_float2(c, sn);
+        return;
+    }
+    const int tok = (int) blockIdx.x * 4 + wid, batch = blockIdx.y;
+    if (tok >= 16 * a.n_tt) return;
+    const int i12 = batch % a.ne12, i13 = batch / a.ne12;
+    const int nvec = a.K / 4;
+    char * out = (char *) (a.xt + ((int64_t) batch * a.n_kb * a.n_tt + (tok >> 4)) * 64) + (tok & 15) * 16;
+    auto put = [&](int iv, half4_t h) { // columns 4 iv .. + 3: half a piece of k block iv / 8
+        *(half4_t *) (out + (int64_t) (iv >> 3) * a.n_tt * 1024 + ((iv >> 1) & 3) * 256 + (iv & 1) * 8) = h;
+    };
+    if (tok >= a.N) { // (uniform) the last tile's missing tokens
+        for (int iv = lane; iv < nvec; iv += 64) put(iv, half4_t{0, 0, 0, 0});
+        return;
+    }
+    const float * row = (const float *) (a.x + (uint64_t) i12 * a.nb12 + (uint64_t) i13 * a.nb13 + (uint64_t) tok * a.nb11);
+    if constexpr (NORM) {
+        vx_rms_row r;
+        float4     gn[4];
+        vx_rms_row_load(r, row, a.K, lane);
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc)
+            if (lane + 64 * cc < nvec) gn[cc] = ((const float4 *) a.norm_w)[lane + 64 * cc];
+        const float sc = vx_rms_row_scale(r, a.K, lane, a.eps);
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+            if (lane + 64 * cc >= nvec) break;
+            float       v[4]  = { r.v[cc].x, r.v[cc].y, r.v[cc].z, r.v[cc].w };
+            const float gg[4] = { gn[cc].x, gn[cc].y, gn[cc].z, gn[cc].w };
+            half4_t h;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { v[i] *= sc; v[i] *= gg[i]; h[i] = (_Float16) v[i]; }
+            put(lane + 64 * cc, h);
+        }
+    } else {
+        for (int iv0 = lane; iv0 < nvec; iv0 += 64 * 4) {
+            float4_t v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = ((const float4_t *) row)[min(iv0 + 64 * u, nvec - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (iv0 + 64 * u >= nvec) break;
+                half4_t h;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) h[i] = (_Float16) v[u][i];
+                put(iv0 + 64 * u, h);
+            }
+        }
+    }
+}
+
+// ---- tile choice -----------------------------------------------------------------------------------------------------
+// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages); what a work-group costs, measured: microseconds
+// per 128 of K and fixed, and how many of them a compute unit holds
+#define GM_TILES(X) \
+    X(0, 1, 1, 1, 2, 3, 0.127f, 0.95f, 4) \
+    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f, 2) \
+    X(2, 2, 2, 1, 2, 3, 0.190f, 1.40f, 2) \
+    X(3, 2, 4, 1, 1, 3, 0.276f, 1.30f, 2) \
+    X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f, 2) \
+    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f, 1)
+constexpr int GM_N_TILES = 6;
+struct gm_tile { int rows, toks, mt; float per_step, fixed; int per_cu; };
+const gm_tile gm_tiles[GM_N_TILES] = {
+#define X(I, MT, NT, RW, CH, S, A_, B_, OCC) { 16 * MT * RW, 16 * NT, MT, A_, B_, OCC },
+    GM_TILES(X)
+#undef X
+};
+
+template <int WT, int MT, int NT, int RW, int CH, int S, int EPI>
+bool gm_launch(const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
+    using sh = gm_shape<WT, MT, NT, RW, 4, CH, S>;
+    auto kern = gm_kernel<WT, MT, NT, RW, 4, CH, S, EPI>;
+    static bool raised = false;
+    if (!raised && sh::LDS > 64 * 1024) {
+        if (hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, sh::LDS) != hipSuccess) { (void) hipGetLastError(); return false; }
+        raised = true;
+    }
+    vx_launch(kern, dim3((unsigned) gx, (unsigned) gy, (unsigned) nbatch), dim3(64 * sh::NWAVES), (size_t) sh::LDS, st, a);
+    return true;
+}
+
+template <int WT>
+bool gm_go(int tile, int epi, const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
+    switch (tile) {
+#define X(I, MT, NT, RW, CH, S, A_, B_, OCC)                                                                              \
+        case I:                                                                                                         \
+            if (epi == GM_PLAIN) return gm_launch<WT, MT, NT, RW, CH, S, GM_PLAIN>(a, gx, gy, nbatch, st);              \
+            if constexpr (MT % 2 == 0) {                                                                                \
+                if (epi == GM_SWIGLU) return gm_launch<WT, MT, NT, RW, CH, S, GM_SWIGLU>(a, gx, gy, nbatch, st);        \
+                return gm_launch<WT, MT, NT, RW, CH, S, GM_SEGS>(a, gx, gy, nbatch, st);                                \
+            }                                                                                                           \
+            return false;
+        GM_TILES(X)
+#undef X
+    }
+    return false;
+}
+
+} // namespace
+
+bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch) {
+    const char * e = getenv("VX_GEMM_MID"); // 0: the kernels of mul_mat.hip for these shapes (read on every call: a test compares the two)
+    if (e && atoi(e) == 0) return false;
+    (void) wtype;
+    // (VX_GEMM_Q8T, when it is set, decides between the two prefill kernels for every product of 1024 tokens or more)
+    if (N >= 1024 && getenv("VX_GEMM_Q8T")) return false;
+    if (N <= 16 || N * nbatch > 1024 || nbatch > 65535) return false;
+    // K of whole 256s (the stages).  Up to 16 tokens are the streaming kernel's; what it takes beyond them with K of 513 to
+    // 1024 it sums in this kernel's order, and with K above 2048 it takes nothing beyond them: elsewhere a call that one of
+    // the two had to decline (alignment, VX_ACT_Q8's groups) would differ from its neighbours in the last bit.
+    return K % 256 == 0 && ((K > 512 && K <= 1024) || (K > 2048 && K <= 16384));
+}
+
+bool vx_gm_takes(const vx_gm_call & c) {
+    if (!vx_gm_region(c.wtype, c.K, c.N, (int64_t) c.ne12 * c.ne13)) return false;
+    auto al16 = [](const void * p, uint64_t s) { return (uintptr_t) p % 16 == 0 && s % 16 == 0; };
+    for (int i = 0; i < c.nmat; ++i) {
+        if (!al16(c.mat[i].w, c.mat[i].nb01) || c.mat[i].M < 1) return false;
+        if (c.nmat > 1 && c.mat[i].M % 64) return false;
+    }
+    if (c.w2 && !al16(c.w2, 0)) return false;
+    if (!c.tile_in && !(al16(c.x, c.nb11) && c.nb12 % 16 == 0 && c.nb13 % 16 == 0)) return false;
+    if (c.norm_w && (c.K > 1024 || (uintptr_t) c.norm_w % 16)) return false;
+    return true;
+}
+
+size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch) {
+    // (a work-group's last stage may read up to 7 tiles past the last token tile: their products are dropped)
+    return (size_t) nbatch * (size_t) (K / 32) * (size_t) ((N + 15) / 16) * 1024 + 8192;
+}
+
+vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
+    const int nbatch = c.ne12 * c.ne13;
+    gm_args a = {};
+    for (int i = 0; i < c.nmat; ++i) a.mat[i] = c.mat[i];
+    a.nmat = c.nmat; a.w2 = c.w2;
+    a.n_kb = (int) (c.K / 32); a.N = (int) c.N; a.ne12 = c.ne12;
+    a.n_tt = c.tile_in ? c.tile_tt : (int) ((c.N + 15) / 16);
+    a.res = c.res; a.rnb1 = c.rnb1; a.rnb2 = c.rnb2; a.rnb3 = c.rnb3; a.res_scale = c.res_scale;
+    a.tile_out = (_Float16 *) c.tile_out; a.out_tt = c.tile_tt;
+    bool rotate = false;
+    for (int i = 0; i < c.nmat; ++i) rotate = rotate || c.mat[i].rope;
+    const size_t xt_bytes = c.tile_in ? 0 : vx_gm_tile_bytes(c.K, c.N, nbatch), tab_bytes = rotate ? (size_t) c.N * 32 * sizeof(float2) : 0;
+    void * ws = nullptr;
+    if (xt_bytes + tab_bytes) {
+        const vx_status rc = vx_workspace(st, c.ws_offset + xt_bytes + tab_bytes, &ws);
+        if (rc != VX_OK) return rc;
+    }
+    char * base = (char *) ws + c.ws_offset;
+    a.xt = c.tile_in ? (const half8_t *) c.tile_in : (const half8_t *) base;
+    if (!c.tile_in) {
+        gm_acts p = {};
+        p.x = c.x; p.nb11 = c.nb11; p.nb12 = c.nb12; p.nb13 = c.nb13; p.ne12 = c.ne12;
+        p.N = a.N; p.K = (int) c.K; p.n_tt = a.n_tt; p.n_kb = a.n_kb;
+        p.row_blocks = 4 * a.n_tt;
+        p.norm_w = c.norm_w; p.eps = c.norm_eps;
+        p.xt = (half8_t *) base;
+        int blocks = p.row_blocks;
+        if (rotate) {
+            p.pos = c.pos; p.ff = c.ff; p.rp = c.rp; p.rope_T = c.rope_T;
+            p.tab = (float2 *) (base + xt_bytes);
+            a.rope_tab = p.tab;
+            blocks += (a.N * 32 + 255) / 256;
+        }
+        if (c.norm_w) vx_launch(gm_acts_kernel<true>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p);
+        else          vx_launch(gm_acts_kernel<false>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p);
+    }
+    // the tile whose work-groups finish first by the measured costs
+    const int epi = c.w2 ? GM_SWIGLU : c.nmat > 1 ? GM_SEGS : GM_PLAIN;
+    int best = -1;
+    float best_us = 0.0f;
+    for (int t = 0; t < GM_N_TILES; ++t) {
+        const gm_tile & g = gm_tiles[t];
+        if (epi != GM_PLAIN && g.mt % 2) continue;
+        int64_t wx = 0;
+        if (epi == GM_SWIGLU) wx = (2 * (int64_t) c.mat[0].M + g.rows - 1) / g.rows;
+        else for (int i = 0; i < c.nmat; ++i) wx += (c.mat[i].M + g.rows - 1) / g.rows;
+        const int64_t wgs = wx * ((c.N + g.toks - 1) / g.toks) * nbatch;
+        const float one = g.fixed + g.per_step * (float) (c.K / 128);
+        // (work-groups that share a compute unit share its vector units: the fixed part of one hides behind the other's products)
+        const float per_cu = (float) ((wgs + 255) / 256);
+        const float us = per_cu <= 1.0f ? one : g.per_cu == 1 ? per_cu * one : one + (per_cu - 1.0f) * (g.per_step * (float) (c.K / 128) + 0.3f * g.fixed);
+        if (best < 0 || us < best_us) { best = t; best_us = us; }
+    }
+    const gm_tile & g = gm_tiles[best];
+    int64_t gx = 0;
+    if (epi == GM_SWIGLU) gx = (2 * (int64_t) c.mat[0].M + g.rows - 1) / g.rows;
+    else for (int i = 0; i < c.nmat; ++i) { a.mat[i].wg0 = (int) gx; gx += (c.mat[i].M + g.rows - 1) / g.rows; }
+    const int64_t gy = (c.N + g.toks - 1) / g.toks;
+    // Row tile x of every token tile goes to XCD x mod 8 (work-groups are dealt round-robin, the grid's width a multiple of
+    // 8): its weights come into one L2.
+    if (gx > 8 && epi != GM_SEGS) gx = (gx + 7) / 8 * 8;
+    if (gx > 0x7fffffff || gy > 65535) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
+    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) gx, (int) gy, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) gx, (int) gy, nbatch, st);
+    return ok ? VX_OK : vx_fail(VX_ERR_HIP, "mul_mat: the kernel could not be given its LDS");
+}

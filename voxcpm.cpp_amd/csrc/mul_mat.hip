@@ -24,7 +24,8 @@
 // staged K-split variant of the GEMM kernel remains for F32 weights and ragged K.
 //
 // Algorithmic HBM bytes: weights once (34 bytes per 32 weights) + activations + output.
-#include "vx_common.hpp"
+#include "mm_common.hpp"
+#include "gemm_mid.hpp"
 #include "rope_common.hpp"
 
 #include <cstdlib>
@@ -85,37 +86,8 @@ struct mm_args {
     int   w_slot;     // bytes between the images of consecutive MFMA columns: the row's bytes plus padding
 };
 
-// a + x * s with the product rounded before the sum, as a SCALE node followed by an ADD node rounds
-__device__ __forceinline__ float scaled_residual(float x, float s, float a) {
-#pragma clang fp contract(off)
-    const float t = x * s;
-    return a + t;
-}
-
 constexpr int WT_Q8 = 0, WT_F16 = 1, WT_F32 = 2;
 constexpr int KC_BLOCKS = 4; // 32-wide k blocks staged per round
-
-__device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-// 8 int8 (two dwords) -> 8 f16, exactly
-__device__ __forceinline__ half8_t q8_to_half8(uint32_t lo, uint32_t hi) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const uint32_t bias = 0x64646464u;
-    lo ^= 0x80808080u;
-    hi ^= 0x80808080u;
-    u32x4 r;
-    r[0] = __builtin_amdgcn_perm(bias, lo, 0x04010400u);
-    r[1] = __builtin_amdgcn_perm(bias, lo, 0x04030402u);
-    r[2] = __builtin_amdgcn_perm(bias, hi, 0x04010400u);
-    r[3] = __builtin_amdgcn_perm(bias, hi, 0x04030402u);
-    half8_t h = __builtin_bit_cast(half8_t, r);
-    const _Float16 off = (_Float16) 1152.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) h[i] -= off;
-    return h;
-}
 
 // The 8 quants lane-group j needs from Q8_0 block kb of a row: bytes 34*kb + 2 + 8j .. +8, which are
 // only 2-byte aligned.  Vector loads that are not dword-aligned are served lane by lane and run
@@ -2518,8 +2490,43 @@ bool launch_mm_cut(const mm_args & a, int nbatch, hipStream_t st) {
     return true;
 }
 
+// The product as gemm_mid.hip's kernel sees it; false where it is not one of its shapes (there one weight matrix serves every
+// batch entry).
+bool mid_fill(vx_gm_call & c, const mm_args & a, int nbatch, int wt) {
+    if (wt == WT_F32 || !(nbatch == 1 || (a.r2 == a.ne12 && a.r3 * a.ne12 == nbatch)) || a.M >= ((int64_t) 1 << 30)) return false;
+    c = vx_gm_call{};
+    c.wtype = wt == WT_Q8 ? VX_GM_Q8 : VX_GM_F16;
+    c.nmat = a.nseg > 0 ? a.nseg : 1;
+    if (a.nseg > 0) {
+        for (int i = 0; i < a.nseg; ++i) {
+            const gv_seg & sg = a.seg[i];
+            c.mat[i] = vx_gm_mat{ sg.w, sg.dst, (int) sg.M, 0, sg.nb01, sg.nb1, sg.nb2, sg.nb3, sg.rope };
+        }
+        if (a.head_dim != 64 || a.rp.n_dims != 64 || a.rp.mode != 2 || a.rope_T <= 0) return false;
+    } else {
+        c.mat[0] = vx_gm_mat{ a.w, a.dst, (int) a.M, 0, a.nb01, a.nb1, a.nb2, a.nb3, 0 };
+    }
+    c.w2 = a.w2;
+    c.K = a.K; c.N = a.N; c.ne12 = a.ne12; c.ne13 = nbatch / a.ne12;
+    c.x = a.x; c.nb11 = a.nb11; c.nb12 = a.nb12; c.nb13 = a.nb13;
+    c.norm_w = a.norm_w; c.norm_eps = a.norm_eps;
+    c.tile_in = a.tile_in; c.tile_tt = a.tile_tt; c.tile_out = a.tile_out;
+    c.res = a.res; c.rnb1 = a.rnb1; c.rnb2 = a.rnb2; c.rnb3 = a.rnb3; c.res_scale = a.res_scale;
+    c.pos = a.pos; c.ff = a.ff; c.rp = a.rp; c.rope_T = a.rope_T;
+    c.ws_offset = a.ws_offset;
+    return vx_gm_takes(c);
+}
+// true: the product was that kernel's (a failure, of the workspace for instance, is left as the call's status)
+bool launch_mid(const mm_args & a, int nbatch, int wt, hipStream_t st) {
+    vx_gm_call c;
+    if (!mid_fill(c, a, nbatch, wt)) return false;
+    t_ws_status = vx_gm_run(c, st);
+    return true;
+}
+
 template <int WT, bool ACT_Q8>
 void launch(const mm_args & a, int nbatch, hipStream_t st) {
+    if constexpr (WT != WT_F32 && !ACT_Q8) { if (launch_mid(a, nbatch, WT, st)) return; }
     if constexpr (WT != WT_F32) { if (launch_gemv<WT, ACT_Q8>(a, nbatch, st)) return; }
     if constexpr (WT != WT_F32 && !ACT_Q8) { if (launch_gemm_lds<WT>(a, nbatch, st) || ws_failed()) return; }
     if constexpr (WT != WT_F32) { if (launch_gemm128<WT, ACT_Q8>(a, nbatch, st)) return; }
@@ -2603,12 +2610,30 @@ extern "C" vx_status vx_mul_mat(const vx_tensor * src0, const vx_tensor * src1, 
 // MUL_MAT(gate) , MUL_MAT(up) , GLU(SWIGLU split) as one launch for decode-sized token counts
 // (MiniCPMModel::mlp_forward, src/minicpm.cpp:718-747).  Both products are formed exactly as vx_mul_mat
 // forms them (same block order, same reduction order), so the result equals the three separate nodes'.
+// gemm_mid.hip's kernel serves gate and up alone as well as the pair, but each only on 16-byte boundaries: a pair of which one
+// matrix is on such a boundary and the other is not would be summed in another order than the two products by themselves.
+static bool mid_split(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1) {
+    return vx_gm_region(gate->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, gate->ne[0], src1->ne[1], src1->ne[2] * src1->ne[3]) &&
+           ((uintptr_t) gate->data % 16 == 0) != ((uintptr_t) up->data % 16 == 0);
+}
+
 extern "C" int vx_supports_mul_mat_swiglu(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * dst) {
     if (!vx_supports_mul_mat(gate, src1, dst) || !up) return 0;
     if (gate->type != VX_TYPE_Q8_0 && gate->type != VX_TYPE_F16) return 0;
     if (up->type != gate->type) return 0;
     for (int i = 0; i < 4; ++i) if (up->ne[i] != gate->ne[i] || up->nb[i] != gate->nb[i]) return 0;
+    if (mid_split(gate, up, src1)) return 0;
     return gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]);
+}
+
+static void swiglu_fill(mm_args & a, const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * norm_w, float eps,
+                        const vx_tensor * dst);
+// the pair on gemm_mid.hip's kernel
+static bool swiglu_mid_ok(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * norm_w, const vx_tensor * dst) {
+    mm_args a = {};
+    swiglu_fill(a, gate, up, src1, norm_w, 0.0f, dst);
+    vx_gm_call c;
+    return mid_fill(c, a, (int) (src1->ne[2] * src1->ne[3]), gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16);
 }
 
 // Prefill sizes: both products on the LDS-tiled kernel, the GLU in its epilogue (f16 activations only: under VX_ACT_Q8
@@ -2631,6 +2656,8 @@ extern "C" int vx_supports_mul_mat_swiglu_tiled(const vx_tensor * gate, const vx
     if (gate->type != VX_TYPE_Q8_0 && gate->type != VX_TYPE_F16) return 0;
     if (up->type != gate->type) return 0;
     for (int i = 0; i < 4; ++i) if (up->ne[i] != gate->ne[i] || up->nb[i] != gate->nb[i]) return 0;
+    if (mid_split(gate, up, src1)) return 0;
+    if (src1->ne[1] <= 64 && !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0])) return act_mode == VX_ACT_FLOAT && swiglu_mid_ok(gate, up, src1, nullptr, dst);
     // (neither the pair nor one product on its own may be a shape of the streaming kernel: it sums the K blocks in another order)
     return !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]) && !gemv_shape_ok(src1->ne[1], gate->ne[1], gate->ne[0]) &&
            gemm_lds_swiglu_ok(gate, up, src1, dst, act_mode);
@@ -2676,9 +2703,11 @@ static void swiglu_fill(mm_args & a, const vx_tensor * gate, const vx_tensor * u
 // kernel takes), the norm in its activation pass.
 static bool norm_swiglu_tiled_ok(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate, const vx_tensor * up, const vx_tensor * dst,
                                  int act_mode) {
-    if (!gate || gate->type != VX_TYPE_Q8_0 || !norm_prologue_ok(x, norm_w) || !norm_w->data || (uintptr_t) norm_w->data % 16 || !x->data ||
-        (uintptr_t) x->data % 16) return false;
+    if (!gate || (gate->type != VX_TYPE_Q8_0 && gate->type != VX_TYPE_F16) || !norm_prologue_ok(x, norm_w) || !norm_w->data || (uintptr_t) norm_w->data % 16 ||
+        !x->data || (uintptr_t) x->data % 16) return false;
     if (!vx_supports_mul_mat_swiglu_tiled(gate, up, x, dst, act_mode)) return false;
+    if (swiglu_mid_ok(gate, up, x, norm_w, dst)) return true;
+    if (gate->type != VX_TYPE_Q8_0) return false;
     mm_args a = {};
     swiglu_fill(a, gate, up, x, norm_w, 0.0f, dst);
     return gemm_q8t_takes(a, (int) (x->ne[2] * x->ne[3]), true);
@@ -2720,7 +2749,8 @@ static vx_status swiglu_run(const vx_tensor * gate, const vx_tensor * up, const 
     hipStream_t st = (hipStream_t) stream;
     bool ok;
     (void) take_ws_status();
-    if (tiled)                           ok = gate->type == VX_TYPE_Q8_0 ? launch_gemm_lds_swiglu<WT_Q8>(a, nbatch, st) : launch_gemm_lds_swiglu<WT_F16>(a, nbatch, st);
+    if ((act_mode == VX_ACT_FLOAT || gate->type == VX_TYPE_F16) && launch_mid(a, nbatch, gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16, st)) ok = true;
+    else if (tiled)                      ok = gate->type == VX_TYPE_Q8_0 ? launch_gemm_lds_swiglu<WT_Q8>(a, nbatch, st) : launch_gemm_lds_swiglu<WT_F16>(a, nbatch, st);
     else if (gate->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
     else                                 ok = launch_gemv<WT_F16, false>(a, nbatch, st);
     if (ws_failed()) return take_ws_status(); // (the pre-tiled kernel's workspace: never answered by another kernel)
@@ -2779,10 +2809,15 @@ extern "C" vx_status vx_mul_mat_scale_add(const vx_tensor * src0, const vx_tenso
     a.x_aligned = ((uintptr_t) src1->data % 16 == 0) && src1->nb[1] % 16 == 0 && src1->nb[2] % 16 == 0 && src1->nb[3] % 16 == 0;
     const int nbatch = (int) (src1->ne[2] * src1->ne[3]);
     hipStream_t st = (hipStream_t) stream;
-    bool ok;
+    bool ok = false;
     (void) take_ws_status();
-    if (src0->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
-    else                            ok = launch_gemv<WT_F16, false>(a, nbatch, st);
+    if (src0->type == VX_TYPE_F16 || act_mode == VX_ACT_FLOAT) {
+        ok = launch_mid(a, nbatch, src0->type == VX_TYPE_F16 ? WT_F16 : WT_Q8, st);
+        if (ws_failed()) return take_ws_status();
+    }
+    if (ok) {}
+    else if (src0->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
+    else                                 ok = launch_gemv<WT_F16, false>(a, nbatch, st);
     if (!ok) { // not the streaming kernel's shape: the tiled kernels with K cut (see vx_supports_mul_mat_scale_add)
         if (src0->type == VX_TYPE_Q8_0) {
             if (act_mode == VX_ACT_Q8) ok = launch_mm_cut<WT_Q8, true>(a, nbatch, st);
@@ -2826,10 +2861,10 @@ extern "C" vx_status vx_mul_mat_scale_add(const vx_tensor * src0, const vx_tenso
 // whose epilogue writes silu(g) * u as f16 tiles, and the down projection that takes those tiles as they are, with the
 // update in its epilogue.  The intermediate [tokens x ffn] tensor is neither stored in fp32 nor read back and re-laid-out
 // (at 65536 tokens x 4096: a gigabyte each way).  Every value is rounded where the separate calls round it: same bits.
-static bool mlp_fill(mm_args & a, mm_args & b, const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
+static bool mlp_fill(mm_args & a, mm_args & b, bool & mid, const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
                      const vx_tensor * down, const vx_tensor * residual, float scale, const vx_tensor * dst, int act_mode) {
     if (!x || !norm_w || !gate || !up || !down || !residual || !dst) return false;
-    if (down->type != VX_TYPE_Q8_0 || down->ne[2] != 1 || down->ne[3] != 1 || gate->ne[2] != 1 || gate->ne[3] != 1) return false;
+    if (down->type != gate->type || (down->type != VX_TYPE_Q8_0 && down->type != VX_TYPE_F16) || down->ne[2] != 1 || down->ne[3] != 1 || gate->ne[2] != 1 || gate->ne[3] != 1) return false;
     if (down->ne[0] != gate->ne[1] || gate->ne[1] % 32 || dst->ne[0] != down->ne[1] || dst->ne[1] != x->ne[1] || dst->ne[2] != x->ne[2] || dst->ne[3] != x->ne[3]) return false;
     if (dst->type != VX_TYPE_F32 || dst->nb[0] != 4 || residual->type != VX_TYPE_F32 || residual->nb[0] != 4 || !vx_same_shape(residual, dst)) return false;
     // the intermediate as the separate calls would see it: dense [ffn, tokens, batch]
@@ -2837,7 +2872,9 @@ static bool mlp_fill(mm_args & a, mm_args & b, const vx_tensor * x, const vx_ten
     act.ne[0] = gate->ne[1];
     act.nb[1] = (uint64_t) act.ne[0] * 4; act.nb[2] = act.nb[1] * (uint64_t) act.ne[1]; act.nb[3] = act.nb[2] * (uint64_t) act.ne[2];
     act.data = x->data; // (only its alignment is looked at)
-    if (!norm_swiglu_tiled_ok(x, norm_w, gate, up, &act, act_mode)) return false;
+    // (17 to 32 tokens: the pair is announced as the streaming kernel's shape and runs on gemm_mid.hip's kernel all the same)
+    if (!norm_swiglu_tiled_ok(x, norm_w, gate, up, &act, act_mode) &&
+        !(act_mode == VX_ACT_FLOAT && vx_supports_norm_mul_mat_swiglu(x, norm_w, gate, up, &act) && swiglu_mid_ok(gate, up, x, norm_w, &act))) return false;
     if (!vx_supports_mul_mat_scale_add(down, &act, residual, dst)) return false;
     swiglu_fill(a, gate, up, x, norm_w, eps, &act);
     b = mm_args{};
@@ -2855,6 +2892,15 @@ static bool mlp_fill(mm_args & a, mm_args & b, const vx_tensor * x, const vx_ten
     b.w_aligned = ((uintptr_t) down->data % 4 == 0) && down->nb[1] % 4 == 0;
     b.x_aligned = 1;
     const int nbatch = (int) (x->ne[2] * x->ne[3]);
+    {   // both products on gemm_mid.hip's kernel, as the separate calls would run them
+        const int wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
+        vx_gm_call c;
+        mm_args d = b;
+        d.tile_in = x->data; // (taken over as tiles: the activations' own alignment does not matter)
+        mid = (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 && mid_fill(c, a, nbatch, wt) && mid_fill(c, d, nbatch, wt);
+        if (mid) return true;
+        if (wt != WT_Q8) return false;
+    }
     // both products on the pre-tiled kernel, as the separate calls would run them
     return gemm_lds_mode() != 0 && b.w_aligned && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 &&
            gemm_q8t_takes(a, nbatch, true) && gemm_q8t_takes(b, nbatch, false) && (uint64_t) 256 * b.rnb1 + 1024 < (1ull << 32);
@@ -2863,13 +2909,15 @@ static bool mlp_fill(mm_args & a, mm_args & b, const vx_tensor * x, const vx_ten
 extern "C" int vx_supports_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate, const vx_tensor * up, const vx_tensor * down,
                                      const vx_tensor * residual, const vx_tensor * dst, int act_mode) {
     mm_args a = {}, b = {};
-    return mlp_fill(a, b, x, norm_w, 0.0f, gate, up, down, residual, 0.0f, dst, act_mode);
+    bool mid = false;
+    return mlp_fill(a, b, mid, x, norm_w, 0.0f, gate, up, down, residual, 0.0f, dst, act_mode);
 }
 
 extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
                                   const vx_tensor * down, const vx_tensor * residual, float scale, const vx_tensor * dst, int act_mode, vx_stream stream) {
     mm_args a = {}, b = {};
-    if (!mlp_fill(a, b, x, norm_w, eps, gate, up, down, residual, scale, dst, act_mode))
+    bool mid = false;
+    if (!mlp_fill(a, b, mid, x, norm_w, eps, gate, up, down, residual, scale, dst, act_mode))
         return vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the shapes of vx_supports_norm_mul_mat_swiglu_tiled, a Q8_0 down projection that the pre-tiled kernel takes, "
                        "an F32 residual of dst's shape");
     if (!x->data || !norm_w->data || !gate->data || !up->data || !down->data || !residual->data || !dst->data) return vx_fail(VX_ERR_INVALID, "mlp_tiled: null data");
@@ -2878,10 +2926,22 @@ extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w,
     hipStream_t st = (hipStream_t) stream;
     // the tiles between the two products: whole 128-token tiles of the pair (it writes every token of its tiles), at the front of
     // the workspace; both products put what they need behind them (a block that a later, larger request replaces stays valid)
-    const int    tile_tt = (int) ((a.N + QT_TOKS - 1) / QT_TOKS) * (QT_TOKS / 16);
-    const size_t tiles   = ((size_t) nbatch * (size_t) (a.M / 32) * (size_t) tile_tt * 1024 + 255) & ~(size_t) 255;
+    // (gemm_mid.hip's kernel: the tiles of the tokens that exist)
+    const int    tile_tt = mid ? (int) ((a.N + 15) / 16) : (int) ((a.N + QT_TOKS - 1) / QT_TOKS) * (QT_TOKS / 16);
+    const size_t tiles   = ((mid ? vx_gm_tile_bytes(a.M, a.N, nbatch) : (size_t) nbatch * (size_t) (a.M / 32) * (size_t) tile_tt * 1024) + 255) & ~(size_t) 255;
     void * ws = nullptr;
     (void) take_ws_status();
+    if (mid) { // one request for all the group needs: its pieces lie in one block, also when it grows
+        const vx_status rc = vx_workspace(st, tiles + vx_gm_tile_bytes(a.K, a.N, nbatch), &ws);
+        if (rc != VX_OK) return rc;
+        const int wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
+        a.ws_offset = tiles; a.tile_out = ws; a.tile_tt = tile_tt;
+        b.tile_in = ws; b.tile_tt = tile_tt;
+        if (!launch_mid(a, nbatch, wt, st) || ws_failed()) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the gate/up product could not be launched");
+        if (!launch_mid(b, nbatch, wt, st) || ws_failed()) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the down projection could not be launched");
+        VX_LAUNCH_CHECK();
+        return VX_OK;
+    }
     const vx_status rc = vx_workspace(st, tiles, &ws);
     if (rc != VX_OK) return rc;
     a.ws_offset = tiles; a.tile_out = ws; a.tile_tt = tile_tt;
@@ -2896,7 +2956,7 @@ extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w,
 // A projection with its residual update whose activations a kernel in front of it (the prefill attention's epilogue) has
 // left as this kernel's f16 tiles: vx_mul_mat_scale_add without its activation pass.  Taken where the separate call runs
 // on the pre-tiled kernel, so the bits are the same.
-static bool proj_tiles_fill(mm_args & b, const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale, int act_mode) {
+static bool proj_tiles_fill(mm_args & b, bool & mid, const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale, int act_mode) {
     if (!w || !x || !residual || !dst || act_mode != VX_ACT_FLOAT || gemm_lds_mode() == 0) return false;
     if (w->type != VX_TYPE_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1 || x->type != VX_TYPE_F32 || !vx_is_contiguous(x)) return false;
     if (!vx_supports_mul_mat_scale_add(w, x, residual, dst) || !vx_same_shape(residual, dst) || residual->nb[0] != 4 || dst->nb[0] != 4) return false;
@@ -2915,6 +2975,11 @@ static bool proj_tiles_fill(mm_args & b, const vx_tensor * w, const vx_tensor * 
     b.w_aligned = ((uintptr_t) w->data % 4 == 0) && w->nb[1] % 4 == 0;
     b.x_aligned = ((uintptr_t) x->data % 16 == 0) && x->nb[1] % 16 == 0 && x->nb[2] % 16 == 0 && x->nb[3] % 16 == 0;
     const int64_t nbatch = x->ne[2] * x->ne[3];
+    {   // gemm_mid.hip's kernel, as the separate call would run it (sequences flattened into one token dimension, as the graphs have them)
+        vx_gm_call c;
+        mid = b.x_aligned && nbatch == 1 && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 && mid_fill(c, b, (int) nbatch, WT_Q8);
+        if (mid) return true;
+    }
     // (what launch_gemm_lds asks for before it hands a product to the pre-tiled kernel)
     if ((uint64_t) b.M * b.nb01 >= (1ull << 32) || (uint64_t) 256 * b.nb11 + 256 >= (1ull << 32) || (uint64_t) 256 * b.nb1 + 1024 >= (1ull << 32) ||
         b.K >= (1ll << 28) || b.N <= 16) return false;
@@ -2926,7 +2991,13 @@ static bool proj_tiles_fill(mm_args & b, const vx_tensor * w, const vx_tensor * 
 bool vx_proj_tiles_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, int act_mode,
                       uint32_t * tile_tt, uint32_t * n_kb, size_t * tile_bytes, size_t * own_bytes) {
     mm_args b;
-    if (!proj_tiles_fill(b, w, x, residual, dst, 0.0f, act_mode)) return false;
+    bool mid = false;
+    if (!proj_tiles_fill(b, mid, w, x, residual, dst, 0.0f, act_mode)) return false;
+    if (mid) {
+        *tile_tt = (uint32_t) ((b.N + 15) / 16); *n_kb = (uint32_t) (b.K / 32); *own_bytes = 0;
+        *tile_bytes = (vx_gm_tile_bytes(b.K, b.N, x->ne[2] * x->ne[3]) + 255) & ~(size_t) 255;
+        return true;
+    }
     {   // what the product itself puts behind the tiles when the weights' tiles are not kept: as launch_gemm_q8t sizes them
         const size_t kb = (size_t) (b.K / 32), rt = (size_t) ((b.M + 15) / 16);
         *own_bytes = kb * rt * 1024 + (kb * ((rt + 3) & ~(size_t) 3) * 16 * 4 + 1023) / 1024 * 1024 + 1024;
@@ -2941,10 +3012,17 @@ bool vx_proj_tiles_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor 
 vx_status vx_proj_tiles_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale,
                             int act_mode, const void * tiles, size_t ws_offset, hipStream_t st) {
     mm_args b;
-    if (!proj_tiles_fill(b, w, x, residual, dst, scale, act_mode)) return vx_fail(VX_ERR_UNSUPPORTED, "projection over tiles: a shape outside the pre-tiled kernel");
+    bool mid = false;
+    if (!proj_tiles_fill(b, mid, w, x, residual, dst, scale, act_mode)) return vx_fail(VX_ERR_UNSUPPORTED, "projection over tiles: a shape outside the pre-tiled kernel");
     if (!w->data || !residual->data || !dst->data || !tiles) return vx_fail(VX_ERR_INVALID, "projection over tiles: null data");
-    b.ws_offset = ws_offset; b.tile_in = tiles; b.tile_tt = (int) ((b.N + QT_TOKS - 1) / QT_TOKS * (QT_TOKS / 16));
+    b.ws_offset = ws_offset; b.tile_in = tiles; b.tile_tt = mid ? (int) ((b.N + 15) / 16) : (int) ((b.N + QT_TOKS - 1) / QT_TOKS * (QT_TOKS / 16));
     (void) take_ws_status();
+    if (mid) {
+        if (!launch_mid(b, (int) (x->ne[2] * x->ne[3]), WT_Q8, st) || ws_failed())
+            return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "projection over tiles: the product could not be launched");
+        VX_LAUNCH_CHECK();
+        return VX_OK;
+    }
     if (!launch_gemm_q8t<false>(b, (int) (x->ne[2] * x->ne[3]), st, gemm_lds_mode() == 2))
         return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "projection over tiles: the product could not be launched");
     VX_LAUNCH_CHECK();
@@ -3012,7 +3090,7 @@ static vx_status qkv_run(const vx_tensor * norm_w, float eps, const vx_tensor * 
 // destination; the two rotations in the product's epilogue (heads of 64 rows) or as launches of their own, in place.  Taken when every piece is what the separate
 // nodes would run -- each product on a tiled kernel with its K whole (the pre-tiled kernel and the LDS-operand kernel form
 // and add a block's products identically) -- so the bits are those of RMS_NORM, MUL, three MUL_MATs and two ROPEs.
-static bool qkv_tiled_fill(mm_args & a, const vx_tensor * norm_w, float eps, const vx_tensor * wq, const vx_tensor * wk, const vx_tensor * wv,
+static bool qkv_tiled_fill(mm_args & a, bool & mid, const vx_tensor * norm_w, float eps, const vx_tensor * wq, const vx_tensor * wk, const vx_tensor * wv,
                            const vx_tensor * x, const vx_tensor * q_dst, const vx_tensor * k_dst, const vx_tensor * v_dst, int n_dims, int mode, int act_mode) {
     if (!wq || !wk || !wv || !x || !norm_w || !q_dst || !k_dst || !v_dst || act_mode != VX_ACT_FLOAT || gemm_lds_mode() == 0) return false;
     const vx_tensor * ws[3] = { wq, wk, wv };
@@ -3030,10 +3108,12 @@ static bool qkv_tiled_fill(mm_args & a, const vx_tensor * norm_w, float eps, con
     a.w_aligned = 1;
     a.nseg = 3;
     const int nbatch = (int) x->ne[3];
+    const bool mid_ok = vx_gm_region(wq->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, a.K, a.N, nbatch);
     for (int i = 0; i < 3; ++i) {
         const vx_tensor * w = ws[i];
-        if (w->type != VX_TYPE_Q8_0 || w->ne[0] != wq->ne[0] || w->ne[2] != 1 || w->ne[3] != 1 || !vx_positive(w) || w->ne[1] % 64) return false;
-        if (w->nb[0] != VX_Q8_BLOCK || w->nb[1] < vx_row_size(w->type, w->ne[0])) return false;
+        if ((wq->type != VX_TYPE_Q8_0 && wq->type != VX_TYPE_F16) || w->type != wq->type || w->ne[0] != wq->ne[0] || w->ne[2] != 1 || w->ne[3] != 1 || !vx_positive(w) ||
+            w->ne[1] % 64) return false;
+        if (w->nb[0] != vx_type_size(w->type) || w->nb[1] < vx_row_size(w->type, w->ne[0])) return false;
         gv_seg & sg = a.seg[i];
         sg.w = (const char *) w->data; sg.dst = (char *) ds[i]->data;
         sg.M = w->ne[1]; sg.nb01 = w->nb[1];
@@ -3041,6 +3121,7 @@ static bool qkv_tiled_fill(mm_args & a, const vx_tensor * norm_w, float eps, con
         if (i == 2) { sg.nb1 = v_dst->nb[1]; sg.nb3 = v_dst->nb[3]; }
         a.w_aligned = a.w_aligned && ((uintptr_t) w->data % 4 == 0) && w->nb[1] % 4 == 0;
         a.M += sg.M;
+        if (mid_ok) continue;
         // the product on its own: a tiled kernel with its K whole (not the streaming kernel, no cut K, not the older kernels)
         const int64_t t64 = ((sg.M + 63) / 64) * ((a.N + 63) / 64) * nbatch;
         const bool    big = ((sg.M + 127) / 128) * ((a.N + 127) / 128) * nbatch >= 192;
@@ -3049,6 +3130,14 @@ static bool qkv_tiled_fill(mm_args & a, const vx_tensor * norm_w, float eps, con
     a.w = a.seg[0].w; a.dst = a.seg[0].dst; a.nb01 = a.seg[0].nb01; a.nb1 = a.seg[0].nb1; a.nb3 = a.seg[0].nb3;
     a.x_aligned = ((uintptr_t) x->data % 16 == 0) && x->nb[1] % 16 == 0 && x->nb[3] % 16 == 0;
     a.norm_w = (const float *) norm_w->data; a.norm_eps = eps;
+    if (mid_ok) { // gemm_mid.hip's kernel, with each matrix alone as well
+        a.seg[0].rope = a.seg[1].rope = 1;
+        a.head_dim = n_dims; a.rp.n_dims = n_dims; a.rp.mode = mode; a.rope_T = (int) q_dst->ne[2]; // (what the rotation's shape check looks at)
+        vx_gm_call c;
+        mid = norm_w->data && n_dims == 64 && q_dst->ne[0] == 64 && k_dst->ne[0] == 64 && q_dst->ne[2] == k_dst->ne[2] && mid_fill(c, a, nbatch, wq->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16);
+        return mid;
+    }
+    if (wq->type != VX_TYPE_Q8_0) return false;
     return a.w_aligned && a.x_aligned && norm_w->data && (uintptr_t) norm_w->data % 16 == 0 && gemm_q8t_takes(a, nbatch, false);
 }
 
@@ -3056,7 +3145,8 @@ extern "C" int vx_supports_norm_qkv_proj_rope_tiled(const vx_tensor * x, const v
                                                     const vx_tensor * wv, const vx_tensor * q_dst, const vx_tensor * k_dst, const vx_tensor * v_dst,
                                                     int n_dims, int mode, int act_mode) {
     mm_args a;
-    return qkv_tiled_fill(a, norm_w, 0.0f, wq, wk, wv, x, q_dst, k_dst, v_dst, n_dims, mode, act_mode) &&
+    bool mid = false;
+    return qkv_tiled_fill(a, mid, norm_w, 0.0f, wq, wk, wv, x, q_dst, k_dst, v_dst, n_dims, mode, act_mode) &&
            vx_supports_rope(q_dst, q_dst, n_dims, mode) && vx_supports_rope(k_dst, k_dst, n_dims, mode);
 }
 
@@ -3111,7 +3201,7 @@ extern "C" vx_status vx_kv_proj_rope(const vx_tensor * wk, const vx_tensor * wv,
     a.K = wk->ne[0]; a.N = x->ne[1];
     a.M = 0;
     a.nb11 = x->nb[1]; a.nb12 = x->nb[2]; a.nb13 = x->nb[3];
-    a.ne12 = 1; a.r2 = 1; a.r3 = 1;
+    a.ne12 = 1; a.r2 = 1; a.r3 = (int) x->ne[3];
     a.rows_wg = 16;
     a.w_aligned = 1;
     a.nseg = 2;
@@ -3136,8 +3226,11 @@ extern "C" vx_status vx_kv_proj_rope(const vx_tensor * wk, const vx_tensor * wv,
     const int nbatch = (int) x->ne[3];
     hipStream_t st = (hipStream_t) stream;
     bool ok;
-    if (wk->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
+    (void) take_ws_status();
+    if ((act_mode == VX_ACT_FLOAT || wk->type == VX_TYPE_F16) && launch_mid(a, nbatch, wk->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16, st)) ok = true;
+    else if (wk->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
     else                          ok = launch_gemv<WT_F16, false>(a, nbatch, st);
+    if (ws_failed()) return take_ws_status();
     if (!ok) return vx_fail(VX_ERR_UNSUPPORTED, "kv_proj_rope: shape outside the streaming kernel");
     VX_LAUNCH_CHECK();
     return VX_OK;
@@ -3157,14 +3250,29 @@ extern "C" vx_status vx_norm_qkv_proj_rope(const vx_tensor * x, const vx_tensor 
                                            int n_ctx_orig, float freq_base, float freq_scale, float ext_factor, float attn_factor,
                                            float beta_fast, float beta_slow, int act_mode, vx_stream stream) {
     if (!x || !norm_w || !norm_w->data) return vx_fail(VX_ERR_INVALID, "norm_qkv_proj_rope: null tensor");
+    mm_args a;
+    bool mid = false;
+    if (qkv_tiled_fill(a, mid, norm_w, eps, wq, wk, wv, x, q_dst, k_dst, v_dst, n_dims, mode, act_mode) && mid) {
+        // gemm_mid.hip's kernel: the norm (and the rotation's angles) in its activation pass, the three products one launch
+        if (!pos || !x->data || !q_dst->data || !k_dst->data || !v_dst->data || !wq->data || !wk->data || !wv->data)
+            return vx_fail(VX_ERR_INVALID, "norm_qkv_proj_rope: null data");
+        if (!(eps >= 0.0f)) return vx_fail(VX_ERR_INVALID, "norm_qkv_proj_rope: eps must be >= 0");
+        if ((uintptr_t) q_dst->data % 4 || (uintptr_t) k_dst->data % 4 || (uintptr_t) v_dst->data % 4) return vx_fail(VX_ERR_UNSUPPORTED, "norm_qkv_proj_rope: misaligned tensor data");
+        a.pos = pos; a.ff = freq_factors;
+        a.rp = rope_make_params(n_dims, mode, n_ctx_orig, freq_base, freq_scale, ext_factor, attn_factor, beta_fast, beta_slow);
+        (void) take_ws_status();
+        if (!launch_mid(a, (int) x->ne[3], wq->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16, (hipStream_t) stream) || ws_failed())
+            return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "norm_qkv_proj_rope: the product could not be launched");
+        VX_LAUNCH_CHECK();
+        return VX_OK;
+    }
     if (!vx_supports_norm_qkv_proj_rope(x, norm_w, wq, wk, wv, q_dst, k_dst, v_dst, n_dims, mode) &&
         vx_supports_norm_qkv_proj_rope_tiled(x, norm_w, wq, wk, wv, q_dst, k_dst, v_dst, n_dims, mode, act_mode)) {
         // prefill sizes: the norm in the activation pass, one product launch for the three matrices, the rotations in place
         if (!pos || !x->data || !q_dst->data || !k_dst->data || !v_dst->data || !wq->data || !wk->data || !wv->data)
             return vx_fail(VX_ERR_INVALID, "norm_qkv_proj_rope: null data");
         if (!(eps >= 0.0f)) return vx_fail(VX_ERR_INVALID, "norm_qkv_proj_rope: eps must be >= 0");
-        mm_args a;
-        if (!qkv_tiled_fill(a, norm_w, eps, wq, wk, wv, x, q_dst, k_dst, v_dst, n_dims, mode, act_mode))
+        if (!qkv_tiled_fill(a, mid, norm_w, eps, wq, wk, wv, x, q_dst, k_dst, v_dst, n_dims, mode, act_mode))
             return vx_fail(VX_ERR_UNSUPPORTED, "norm_qkv_proj_rope: shape outside the pre-tiled kernel");
         (void) take_ws_status();
         // heads of 64 rows: the rotations in the product's epilogue, from an angle table (VX_QKV_ROPE_EPILOGUE=0: as launches of their own)
@@ -3209,7 +3317,7 @@ static vx_status qkv_run(const vx_tensor * norm_w, float eps, const vx_tensor * 
     a.K = wq->ne[0]; a.N = x->ne[1];
     a.M = 0;
     a.nb11 = x->nb[1]; a.nb12 = x->nb[2]; a.nb13 = x->nb[3];
-    a.ne12 = 1; a.r2 = 1; a.r3 = 1;
+    a.ne12 = 1; a.r2 = 1; a.r3 = (int) x->ne[3];
     a.rows_wg = 16;
     a.w_aligned = 1;
     a.nseg = 3;
@@ -3236,8 +3344,11 @@ static vx_status qkv_run(const vx_tensor * norm_w, float eps, const vx_tensor * 
     const int nbatch = (int) x->ne[3];
     hipStream_t st = (hipStream_t) stream;
     bool ok;
-    if (wq->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
+    (void) take_ws_status();
+    if ((act_mode == VX_ACT_FLOAT || wq->type == VX_TYPE_F16) && launch_mid(a, nbatch, wq->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16, st)) ok = true;
+    else if (wq->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
     else                          ok = launch_gemv<WT_F16, false>(a, nbatch, st);
+    if (ws_failed()) return take_ws_status();
     if (!ok) return vx_fail(VX_ERR_UNSUPPORTED, "qkv_proj_rope: shape outside the streaming kernel");
     VX_LAUNCH_CHECK();
     return VX_OK;
