@@ -1114,17 +1114,19 @@ extern "C" vx_status vx_flash_attn_ext_kv2_store(const vx_tensor * q, const vx_t
 }
 
 // attention_forward at prefill size (src/minicpm.cpp:682-713): FLASH_ATTN_EXT over the projections' own K/V, then the
-// cache write, its two sums, the ordering scalar and the ADD1 on the attention's result.  The write and the scalar are
-// launched first and the scalar joins the attention's epilogue, so the result is stored once.
-struct pf_store_ctx {
-    const vx_tensor * k_src, * k_slot, * v_src, * v_slot;
-    float scale, bias;
-};
-constexpr size_t PF_STORE_FRONT = 4096, PF_STORE_ADDEND_AT = 2048; // 256 block totals, then the scalar
+// cache write, its two sums, the ordering scalar and the ADD1 on the attention's result.  The write is part of the launch
+// that prepares the attention's operands and the scalar joins the attention's epilogue, so the result is stored once.
+struct pf_store_sides { kvs_side k, v; };
+constexpr size_t PF_STORE_FRONT = VX_PF_FRONT;
 
-static vx_status pf_store_launch(void * front, void * ctx, hipStream_t st) {
-    const pf_store_ctx * c = (const pf_store_ctx *) ctx;
-    return vx_kv_store_scalar(c->k_src, c->k_slot, c->v_src, c->v_slot, c->scale, c->bias, front, (float *) ((char *) front + PF_STORE_ADDEND_AT), st);
+static void pf_store_front(vx_pf_front & f, pf_store_sides & s, const vx_tensor * k_src, const vx_tensor * k_slot, const vx_tensor * v_src,
+                           const vx_tensor * v_slot, float scale, float bias) {
+    kvs_side_fill(s.k, k_src, k_slot);
+    kvs_side_fill(s.v, v_src, v_slot);
+    f.bytes = PF_STORE_FRONT;
+    f.ks = &s.k; f.vs = &s.v;
+    (void) vx_kv_store_scalar_ok(k_src, k_slot, v_src, v_slot, &f.store_large);
+    f.scale = scale; f.bias = bias;
 }
 
 extern "C" int vx_supports_flash_attn_ext_store(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
@@ -1152,25 +1154,15 @@ extern "C" vx_status vx_flash_attn_ext_store(const vx_tensor * q, const vx_tenso
         const vx_status rc = vx_flash_attn_ext(q, k, v, mask, sinks, dst, scale, max_bias, logit_softcap, stream);
         return rc != VX_OK ? rc : vx_kv_store_sync(k_src, k_slot, v_src, v_slot, dst, dst, sync_scale, sync_bias, stream);
     }
-    pf_store_ctx c{ k_src, k_slot, v_src, v_slot, sync_scale, sync_bias };
-    const vx_pf_front front{ PF_STORE_FRONT, PF_STORE_ADDEND_AT, pf_store_launch, &c };
+    pf_store_sides sides;
+    vx_pf_front front{};
+    pf_store_front(front, sides, k_src, k_slot, v_src, v_slot, sync_scale, sync_bias);
     return vx_fattn_prefill(q, k, v, mask, sinks, nullptr, dst, scale, max_bias, logit_softcap, (hipStream_t) stream, &front);
 }
 
 // The same block with the o projection and its residual update behind it (src/minicpm.cpp:708-715, 762-768): the
 // attention's epilogue rounds its result to f16 straight into the projection's activation tiles, so the tokens x hidden
 // attention output is neither stored in fp32 nor read back and laid out again.
-struct pf_store_proj_ctx {
-    pf_store_ctx store;
-    void *       front;
-};
-
-static vx_status pf_store_proj_launch(void * front, void * ctx, hipStream_t st) {
-    pf_store_proj_ctx * c = (pf_store_proj_ctx *) ctx;
-    c->front = front;
-    return pf_store_launch(front, &c->store, st);
-}
-
 // the tensor attn describes, in the attention's own shape [head_dim, heads, tokens, batch] (the same dense memory order)
 static vx_tensor pf_attn_shape(const vx_tensor * q, const vx_tensor * attn) {
     vx_tensor ad = *attn;
@@ -1237,8 +1229,11 @@ extern "C" vx_status vx_flash_attn_ext_store_proj(const vx_tensor * q, const vx_
                                                      sync_bias, stream);
         return rc != VX_OK ? rc : vx_mul_mat_scale_add(w_o, attn, residual, dst, res_scale, act_mode, stream);
     }
-    pf_store_proj_ctx c{ { k_src, k_slot, v_src, v_slot, sync_scale, sync_bias }, nullptr };
-    vx_pf_front front{ PF_STORE_FRONT, PF_STORE_ADDEND_AT, pf_store_proj_launch, &c };
+    pf_store_sides sides;
+    vx_pf_front front{};
+    pf_store_front(front, sides, k_src, k_slot, v_src, v_slot, sync_scale, sync_bias);
+    void * block = nullptr;
+    front.base = &block;
     size_t proj_bytes = 0;
     if (!pf_proj_geometry(q, attn, w_o, residual, dst, act_mode, &front, &proj_bytes)) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext_store_proj: tile geometry");
     hipStream_t st = (hipStream_t) stream;
@@ -1252,7 +1247,7 @@ extern "C" vx_status vx_flash_attn_ext_store_proj(const vx_tensor * q, const vx_
     vx_status rc = vx_fattn_prefill(q, k, v, mask, sinks, nullptr, &ad, scale, max_bias, logit_softcap, st, &front);
     if (rc != VX_OK) return rc == VX_ERR_UNSUPPORTED ? vx_fail(rc, "flash_attn_ext_store_proj: the LDS-tiled kernel declined") : rc;
     // the projection: its own needs go behind the front (a block that a larger request replaces stays valid)
-    return vx_proj_tiles_run(w_o, attn, residual, dst, res_scale, act_mode, (const char *) c.front + PF_STORE_FRONT, front.bytes, st);
+    return vx_proj_tiles_run(w_o, attn, residual, dst, res_scale, act_mode, (const char *) block + PF_STORE_FRONT, front.bytes, st);
 }
 
 // ---- the entry point that allocates nothing ------------------------------------------------------------

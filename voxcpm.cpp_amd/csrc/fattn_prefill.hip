@@ -14,8 +14,10 @@
 // Roofline: MFMA-bound in principle (4 * D flops per score); at D = 64 the exp, the rounding
 // and the row sums of a score (VALU) need about as many issue cycles as its share of the
 // matrix instructions, so the two pipes have to run side by side to come near the peak.
+#include "kvs_common.hpp"
 #include "vx_common.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace {
@@ -24,11 +26,17 @@ constexpr int PF_WAVES = 4;
 constexpr int PF_COLS  = 256; // columns per work-group
 constexpr int PF_KT    = 64;  // keys per tile
 constexpr int PF_MAX_TILES = 1024;
+constexpr int PF_TOTALS = 128;       // block totals of one sum of a cache write, at most
+constexpr int PF_TOTALS_INLINE = 64; // up to here a wave of every attention work-group adds them (two sequences of 512 tokens: 32 a side; beside
+                                     // the tile list that takes less than the 4.5 us of a launch for one number), beyond pf_scalar_kernel does
 
 struct pf_args {
     const char * q; const char * k; const char * v; const char * vl; const char * mask;
     const float * sinks;
     const float * add1; // optional scalar added to every output element (a fused GGML_OP_ADD1)
+    const double * totals; // or the block totals of a cache write's two sums (n_tk of k at 0, n_tv of v at PF_TOTALS), which give that scalar
+    int n_tk, n_tv;
+    float sync_scale, sync_bias;
     _Float16 * tile_out; // optional: the result as f16 activation tiles of the product that follows, instead of dst
     uint32_t tile_tt, tile_bs, tile_ts;
     float * dst;
@@ -43,22 +51,36 @@ struct pf_args {
     int kv_f32;
 };
 
+// What the launch in front of the attention kernel prepares, each by work-groups of its own: the cache write of the same
+// attention block (n_store work-groups), the mask's tile flags (n_mask), the f16 images of F32 K / V (the rest).
+struct pf_prep_args {
+    kvs_side ks, vs;
+    double * totals;
+    int store_large, n_tk, n_store; // the SUMs' form (below); work-groups (large) or totals of the k side; work-groups of both
+    const char * mask;
+    uint64_t nbm1, nbm2, nbm3;
+    int nem2, n_q, n_kv, RB, n_rb, n_tiles, vec_ok, n_units, n_mask;
+    uint8_t * flags; uint8_t * bits;
+    const char * k; const char * v;
+    uint64_t nbk1, nbk2, nbk3, nbv1, nbv2, nbv3;
+    int Hkv, key_blocks;
+    _Float16 * k16; _Float16 * vhi; _Float16 * vlo;
+};
+
 // classifies mask tiles: one wave per (key tile, row block, mask batch).  A lane reads 8 keys
 // (16 bytes) of a row, so the wave covers 8 rows of the 64-key tile per step.  Flags: 0 no key of the tile is visible to
 // any row of the block; 1 every entry is zero; 2 some entry is a finite non-zero value; 3 zeros and -inf only.  For the
 // last kind the rows' visibility is also left as one bit per key (bits[mask batch][row][tile], keys past n_kv cleared),
 // so that the attention kernel applies such a tile -- a causal mask's diagonal -- from 8 bytes per row.
-__global__ __launch_bounds__(64) void pf_mask_flags_kernel(const char * mask, uint64_t nbm1, uint64_t nbm2, uint64_t nbm3,
-                                                           int nem2, int n_q, int n_kv, int RB, int n_rb, int n_tiles,
-                                                           int vec_ok, uint8_t * flags, uint8_t * bits) {
-    const int tile = blockIdx.x, rb = blockIdx.y, mb = blockIdx.z;
-    const char * mp = mask + (uint64_t) (mb % nem2) * nbm2 + (uint64_t) (mb / nem2) * nbm3;
-    const int r0 = rb * RB, r1 = min(n_q, (rb + 1) * RB);
+__device__ __forceinline__ void pf_mask_unit(const pf_prep_args & a, int unit, int lane) {
+    const int tile = unit % a.n_tiles, rb = (unit / a.n_tiles) % a.n_rb, mb = unit / a.n_tiles / a.n_rb;
+    const char * mp = a.mask + (uint64_t) (mb % a.nem2) * a.nbm2 + (uint64_t) (mb / a.nem2) * a.nbm3;
+    const int r0 = rb * a.RB, r1 = min(a.n_q, (rb + 1) * a.RB);
     bool any_visible = false, any_nonzero = false, any_hidden = false;
-    if (vec_ok && (tile + 1) * PF_KT <= n_kv) {
-        const int sub = threadIdx.x >> 3, part = threadIdx.x & 7; // row within the step, 8-key group
+    if (a.vec_ok && (tile + 1) * PF_KT <= a.n_kv) {
+        const int sub = lane >> 3, part = lane & 7; // row within the step, 8-key group
         for (int r = r0 + sub; r < r1; r += 8) {
-            const int4_t v = *(const int4_t *) (mp + (uint64_t) r * nbm1 + ((uint64_t) tile * PF_KT + part * 8) * 2);
+            const int4_t v = *(const int4_t *) (mp + (uint64_t) r * a.nbm1 + ((uint64_t) tile * PF_KT + part * 8) * 2);
             uint32_t byte = 0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -69,27 +91,27 @@ __global__ __launch_bounds__(64) void pf_mask_flags_kernel(const char * mask, ui
             }
             any_visible |= byte != 0;
             any_hidden  |= byte != 0xFFu;
-            bits[(((uint64_t) mb * n_q + r) * n_tiles + tile) * 8 + part] = (uint8_t) byte;
+            a.bits[(((uint64_t) mb * a.n_q + r) * a.n_tiles + tile) * 8 + part] = (uint8_t) byte;
         }
     } else {
-        const int key = tile * PF_KT + threadIdx.x;
+        const int key = tile * PF_KT + lane;
         for (int r = r0; r < r1; ++r) {
             bool vis = false;
-            if (key < n_kv) {
-                const uint16_t h = ((const uint16_t *) (mp + (uint64_t) r * nbm1))[key];
+            if (key < a.n_kv) {
+                const uint16_t h = ((const uint16_t *) (mp + (uint64_t) r * a.nbm1))[key];
                 vis = h != 0xFC00u;
                 any_nonzero |= vis && (h & 0x7FFFu) != 0;
             }
             any_visible |= vis;
             any_hidden  |= !vis;
             const uint64_t row_bits = __builtin_amdgcn_ballot_w64(vis);
-            if (threadIdx.x == 0) *(uint64_t *) (bits + (((uint64_t) mb * n_q + r) * n_tiles + tile) * 8) = row_bits;
+            if (lane == 0) *(uint64_t *) (a.bits + (((uint64_t) mb * a.n_q + r) * a.n_tiles + tile) * 8) = row_bits;
         }
     }
     const bool vis = __builtin_amdgcn_ballot_w64(any_visible) != 0;
     const bool nz  = __builtin_amdgcn_ballot_w64(any_nonzero) != 0;
     const bool hid = __builtin_amdgcn_ballot_w64(any_hidden) != 0;
-    if (threadIdx.x == 0) flags[((uint64_t) mb * n_rb + rb) * n_tiles + tile] = !vis ? 0 : (nz ? 2 : (hid ? 3 : 1));
+    if (lane == 0) a.flags[((uint64_t) mb * a.n_rb + rb) * a.n_tiles + tile] = !vis ? 0 : (nz ? 2 : (hid ? 3 : 1));
 }
 
 // ---- the tiled kernel ---------------------------------------------------------------------------------------------
@@ -143,14 +165,11 @@ __device__ __forceinline__ half8_t pf_tr8(const lds_char * p) {
 }
 
 // F32 K and V of one (batch entry, KV head) as f16 planes [key][64]: K rounded, V as high and low halves
-__global__ __launch_bounds__(256) void pf_convert_kernel(const char * k, const char * v, uint64_t nbk1, uint64_t nbk2, uint64_t nbk3,
-                                                         uint64_t nbv1, uint64_t nbv2, uint64_t nbv3, int n_kv, int Hkv,
-                                                         _Float16 * k16, _Float16 * vhi, _Float16 * vlo) {
-    const int unit = blockIdx.x * 256 + threadIdx.x; // 8 values each
-    const int key = unit >> 3, part = unit & 7, g = blockIdx.y, b = blockIdx.z;
-    if (key >= n_kv) return;
-    const float4_t * kp = (const float4_t *) (k + (uint64_t) key * nbk1 + (uint64_t) g * nbk2 + (uint64_t) b * nbk3) + 2 * part;
-    const float4_t * vp = (const float4_t *) (v + (uint64_t) key * nbv1 + (uint64_t) g * nbv2 + (uint64_t) b * nbv3) + 2 * part;
+__device__ __forceinline__ void pf_convert_unit(const pf_prep_args & a, int unit, int g, int b) { // 8 values each
+    const int key = unit >> 3, part = unit & 7;
+    if (key >= a.n_kv) return;
+    const float4_t * kp = (const float4_t *) (a.k + (uint64_t) key * a.nbk1 + (uint64_t) g * a.nbk2 + (uint64_t) b * a.nbk3) + 2 * part;
+    const float4_t * vp = (const float4_t *) (a.v + (uint64_t) key * a.nbv1 + (uint64_t) g * a.nbv2 + (uint64_t) b * a.nbv3) + 2 * part;
     const float4_t k0 = kp[0], k1 = kp[1], v0 = vp[0], v1 = vp[1];
     half8_t kh, vh, vl;
 #pragma unroll
@@ -160,10 +179,91 @@ __global__ __launch_bounds__(256) void pf_convert_kernel(const char * k, const c
         vl[i]     = (_Float16) (v0[i] - (float) vh[i]);
         vl[4 + i] = (_Float16) (v1[i] - (float) vh[4 + i]);
     }
-    const uint64_t o = (((uint64_t) b * Hkv + g) * n_kv + key) * 64 + 8 * part;
-    *(half8_t *) (k16 + o) = kh;
-    *(half8_t *) (vhi + o) = vh;
-    *(half8_t *) (vlo + o) = vl;
+    const uint64_t o = (((uint64_t) b * a.Hkv + g) * a.n_kv + key) * 64 + 8 * part;
+    *(half8_t *) (a.k16 + o) = kh;
+    *(half8_t *) (a.vhi + o) = vh;
+    *(half8_t *) (a.vlo + o) = vl;
+}
+
+// One cache write and its sum in the order of GGML_OP_SUM's kernels here (glue.hip).  Beyond 16 Ki units that is blocks of
+// 1024 threads: block b's thread t walks units 1024 b + t, + 128 * 1024, ..., a wave adds its lanes by butterfly, a block's 16
+// wave totals are added in order.  A work-group of 256 threads stands for one such block, each of its waves for four of the
+// block's: four units of a thread are requested together.
+template <bool VEC>
+__device__ __forceinline__ void pf_store_large(const kvs_side & s, uint32_t b, double * total, double * part) {
+    const uint32_t n = kvs_units(s, VEC);
+    double acc[4] = { 0.0, 0.0, 0.0, 0.0 };
+    for (uint32_t base = b * 1024 + threadIdx.x; base < n; base += PF_TOTALS * 1024) {
+        float v[4][VEC ? 4 : 1];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) if (base + 256 * p < n) kvs_fetch<VEC>(s, base + 256 * p, v[p]);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) if (base + 256 * p < n) kvs_apply<VEC>(s, base + 256 * p, true, v[p], acc[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const double t = vx_wave_sum(acc[p]);
+        if ((threadIdx.x & 63) == 0) part[4 * p + (threadIdx.x >> 6)] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < 16; ++w) t += part[w];
+        *total = t;
+    }
+}
+
+// One launch for what three did (the cache write, the mask's flags, the f16 images): each is a trip to memory and its
+// latency at a prompt's size.  Two sequences of 512 tokens: 4.8 + 4.1 + 3.9 us as launches of their own, and 4.5 for the
+// scalar that the attention now adds up itself; 24 layers 3067 -> 2876 us, 16 x 4096 tokens 86.5 -> 85.7 ms.
+__global__ __launch_bounds__(256) void pf_prep_kernel(const pf_prep_args a) {
+    __shared__ double part[16];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
+    int i = blockIdx.x;
+    if (i < a.n_store) {
+        if (a.store_large) {
+            const bool second = i >= a.n_tk; // (uniform)
+            const kvs_side & s = second ? a.vs : a.ks;
+            const uint32_t b = (uint32_t) (second ? i - a.n_tk : i);
+            double * total = a.totals + (second ? PF_TOTALS : 0) + b;
+            if (s.vec) pf_store_large<true>(s, b, total, part);
+            else       pf_store_large<false>(s, b, total, part);
+        } else { // 16 waves a side
+            const bool second = i >= 4;
+            const kvs_side & s = second ? a.vs : a.ks;
+            const uint32_t w = (uint32_t) (4 * (i & 3) + wave);
+            const double t = s.vec ? kvs_mid_wave<true>(s, w, (uint32_t) lane) : kvs_mid_wave<false>(s, w, (uint32_t) lane);
+            if (lane == 0) a.totals[(second ? PF_TOTALS : 0) + w] = t;
+        }
+        return;
+    }
+    i -= a.n_store;
+    if (i < a.n_mask) {
+        const int unit = 4 * i + wave;
+        if (unit < a.n_units) pf_mask_unit(a, unit, lane);
+        return;
+    }
+    i -= a.n_mask;
+    const int kb = i % a.key_blocks, bg = i / a.key_blocks;
+    pf_convert_unit(a, kb * 256 + (int) threadIdx.x, bg % a.Hkv, bg / a.Hkv);
+}
+
+// the ordering scalar of a large write's totals, for every work-group of the attention kernel to read
+__global__ __launch_bounds__(128) void pf_scalar_kernel(const double * totals, int n_tk, int n_tv, float scale, float bias, float * out) {
+    __shared__ double part[2][PF_TOTALS];
+    __shared__ double sum[2];
+    const int t = threadIdx.x;
+    part[0][t] = t < n_tk ? totals[t] : 0.0;
+    part[1][t] = t < n_tv ? totals[PF_TOTALS + t] : 0.0;
+    __syncthreads();
+    if ((t & 63) == 0) { // a wave a side
+        double s = 0.0;
+        const int n = t ? n_tv : n_tk;
+        for (int i = 0; i < n; ++i) s += part[t >> 6][i];
+        sum[t >> 6] = s;
+    }
+    __syncthreads();
+    if (t == 0) *out = kvs_scalar((float) sum[0], (float) sum[1], scale, bias);
 }
 
 // VLO: V comes with a low-half image (a.vl).  NCB: 32-column blocks per wave.
@@ -179,6 +279,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
     __shared__ uint16_t tile_list[PF_MAX_TILES];
     __shared__ uint8_t  tile_flag[PF_MAX_TILES];
     __shared__ int      n_active_s;
+    __shared__ float    y_s;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -246,6 +347,20 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             base += __builtin_popcountll(bal);
         }
         if (lane == 0) n_active_s = base;
+    } else if (wave == 1 && a.totals) { // the cache write's ordering scalar: k's totals in the low half of the wave, v's in the high
+        const int n = hl ? a.n_tv : a.n_tk;
+        double tot[PF_TOTALS_INLINE / 32];
+#pragma unroll
+        for (int u = 0; u < PF_TOTALS_INLINE / 32; ++u) tot[u] = 32 * u + cl < n ? a.totals[hl * PF_TOTALS + 32 * u + cl] : 0.0;
+        double t = 0.0;
+        const int nmax = max(a.n_tk, a.n_tv); // (zeros behind a side's own count change nothing: a sum from +0.0 is never -0.0)
+#pragma unroll
+        for (int u = 0; u < PF_TOTALS_INLINE / 32; ++u) {
+            if (32 * u >= nmax) break;
+            for (int i2 = 0; i2 < min(32, nmax - 32 * u); ++i2) t += __shfl(tot[u], (lane & 32) + i2, 64);
+        }
+        const float sum = (float) t, sv = __shfl(sum, 32, 64);
+        if (lane == 0) y_s = kvs_scalar(sum, sv, a.sync_scale, a.sync_bias);
     }
     __syncthreads();
     const int n_active = __builtin_amdgcn_readfirstlane(n_active_s);
@@ -603,6 +718,8 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
     int lane_e = threadIdx.x & 63; // (worked out again rather than kept alive through the walk)
     asm volatile("" : "+v"(lane_e));
     const int hl_e = lane_e >> 5, cl_e = lane_e & 31;
+    const bool  has_add = a.totals || a.add1;
+    const float addend = a.totals ? y_s : a.add1 ? *a.add1 : 0.0f;
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         const int  col = wave * (32 * NCB) + cb * 32 + cl_e;
@@ -627,8 +744,9 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
+#pragma clang fp contract(off) // (the normalised value is rounded before the addend joins it, as two nodes would)
                     float4_t r = float4_t{o[cb][dt][4 * q4], o[cb][dt][4 * q4 + 1], o[cb][dt][4 * q4 + 2], o[cb][dt][4 * q4 + 3]} * inv;
-                    if (a.add1) r += *a.add1;
+                    if (has_add) r += addend;
                     asm volatile("" : "+v"(r)); // the fp32 value the node holds, formed as such, then rounded
                     *(half4_t *) (tb + ((uint64_t) dt * a.tile_tt * 64 + 16 * q4) * 8) = half4_t{(_Float16) r[0], (_Float16) r[1], (_Float16) r[2], (_Float16) r[3]};
                 }
@@ -638,8 +756,9 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
+#pragma clang fp contract(off) // (the normalised value is rounded before the addend joins it, as two nodes would)
                     float4_t r = float4_t{o[cb][dt][4 * q4], o[cb][dt][4 * q4 + 1], o[cb][dt][4 * q4 + 2], o[cb][dt][4 * q4 + 3]} * inv;
-                    if (a.add1) r += *a.add1;
+                    if (has_add) r += addend;
                     *(float4_t *) (out + 32 * dt + 8 * q4 + 4 * hl_e) = r;
                 }
         }
@@ -673,6 +792,14 @@ bool vx_fattn_prefill_accepts(const vx_tensor * q, const vx_tensor * k, float lo
     // too few work-groups: the wave kernel spreads wider (one stream of 512 tokens, 32 blocks of 256 columns run as 64 of
     // 128: 19 us here against 28 us there; 256 tokens, 16 blocks: 15 us against 14 us)
     return (int64_t) n_rb * n_groups >= 32;
+}
+
+// whether a cache write's slot and a tensor share bytes (by their extents)
+static bool pf_overlaps(const kvs_side & s, const vx_tensor * t) {
+    uint64_t sb = s.dst_f16 ? 2 : 4, tb = vx_type_size(t->type);
+    for (int i = 0; i < 4; ++i) { sb += (uint64_t) (s.ned[i] - 1) * s.nbd[i]; tb += (uint64_t) (t->ne[i] - 1) * t->nb[i]; }
+    const char * t0 = (const char *) t->data;
+    return s.d < t0 + tb && t0 < s.d + sb;
 }
 
 vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
@@ -728,32 +855,68 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
         if (rc != VX_OK) return rc;
         ws = (char *) p;
     }
-    if (front) { // the caller's launches first: they own the front of the block, and leave the addend there
-        const vx_status rc = front->launch(ws, front->ctx, st);
-        if (rc != VX_OK) return rc;
-        a.add1 = (const float *) (ws + front->addend_at);
+    pf_prep_args p = {};
+    p.key_blocks = 1;
+    a.totals = nullptr; a.n_tk = a.n_tv = 0; a.sync_scale = a.sync_bias = 0.0f;
+    if (front) { // the cache write's totals and scalar lie at the front of the block
+        p.ks = *front->ks; p.vs = *front->vs;
+        if (front->base) *front->base = ws;
+        p.totals = (double *) ws;
+        p.store_large = front->store_large;
+        const int64_t uk = kvs_host_units(p.ks), uv = kvs_host_units(p.vs);
+        a.n_tk = p.store_large ? (int) std::min<int64_t>(PF_TOTALS, (uk + 1023) / 1024) : 16;
+        a.n_tv = p.store_large ? (int) std::min<int64_t>(PF_TOTALS, (uv + 1023) / 1024) : 16;
+        p.n_tk = a.n_tk;
+        p.n_store = p.store_large ? a.n_tk + a.n_tv : 8;
+        if (std::max(a.n_tk, a.n_tv) <= PF_TOTALS_INLINE) a.totals = p.totals;
+        else a.add1 = (const float *) (ws + VX_PF_SCALAR_AT);
+        a.sync_scale = front->scale; a.sync_bias = front->bias;
         if (front->tiles) {
             a.tile_out = (_Float16 *) (ws + front->tiles_at);
             a.tile_tt = front->tile_tt; a.tile_bs = front->tile_bs; a.tile_ts = front->tile_ts;
         }
         ws += front_bytes;
     }
+    int64_t blocks = p.n_store;
+    p.n_q = n_q; p.n_kv = n_kv; p.RB = RB; p.n_rb = n_rb; p.n_tiles = n_tiles;
     if (mask) {
-        vx_launch(pf_mask_flags_kernel, dim3((unsigned) n_tiles, (unsigned) n_rb, (unsigned) (a.nem2 * a.nem3)), dim3(64), 0, st,
-            a.mask, a.nbm1, a.nbm2, a.nbm3, a.nem2, n_q, n_kv, RB, n_rb, n_tiles,
-            (int) ((uintptr_t) a.mask % 16 == 0 && a.nbm1 % 16 == 0 && a.nbm2 % 16 == 0 && a.nbm3 % 16 == 0), (uint8_t *) ws + bits_bytes,
-            (uint8_t *) ws);
-        VX_LAUNCH_CHECK();
-        a.bits = (const uint8_t *) ws;
-        a.flags = (const uint8_t *) ws + bits_bytes;
+        p.mask = a.mask; p.nbm1 = a.nbm1; p.nbm2 = a.nbm2; p.nbm3 = a.nbm3; p.nem2 = a.nem2;
+        p.vec_ok = (uintptr_t) a.mask % 16 == 0 && a.nbm1 % 16 == 0 && a.nbm2 % 16 == 0 && a.nbm3 % 16 == 0;
+        p.bits = (uint8_t *) ws; p.flags = (uint8_t *) ws + bits_bytes;
+        const int64_t units = (int64_t) n_tiles * n_rb * a.nem2 * a.nem3;
+        if (units > 0x7ffffff0) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext: launch too large");
+        p.n_units = (int) units;
+        p.n_mask = (int) ((units + 3) / 4);
+        blocks += p.n_mask;
+        a.bits = p.bits;
+        a.flags = p.flags;
     }
     if (a.kv_f32) {
-        _Float16 * k16 = (_Float16 *) (ws + flag_bytes), * vhi = (_Float16 *) (ws + flag_bytes + plane), * vlo = (_Float16 *) (ws + flag_bytes + 2 * plane);
-        vx_launch(pf_convert_kernel, dim3((unsigned) ((n_kv * 8 + 255) / 256), (unsigned) Hkv, (unsigned) k->ne[3]), dim3(256), 0, st,
-            a.k, a.v, a.nbk1, a.nbk2, a.nbk3, a.nbv1, a.nbv2, a.nbv3, n_kv, Hkv, k16, vhi, vlo);
-        VX_LAUNCH_CHECK();
-        a.k = (const char *) k16; a.v = (const char *) vhi; a.vl = (const char *) vlo;
+        p.k16 = (_Float16 *) (ws + flag_bytes); p.vhi = (_Float16 *) (ws + flag_bytes + plane); p.vlo = (_Float16 *) (ws + flag_bytes + 2 * plane);
+        p.k = a.k; p.v = a.v;
+        p.nbk1 = a.nbk1; p.nbk2 = a.nbk2; p.nbk3 = a.nbk3; p.nbv1 = a.nbv1; p.nbv2 = a.nbv2; p.nbv3 = a.nbv3;
+        p.Hkv = Hkv; p.key_blocks = (n_kv * 8 + 255) / 256;
+        blocks += (int64_t) p.key_blocks * Hkv * k->ne[3];
+        a.k = (const char *) p.k16; a.v = (const char *) p.vhi; a.vl = (const char *) p.vlo;
         a.nbk1 = a.nbv1 = 128; a.nbk2 = a.nbv2 = (uint64_t) n_kv * 128; a.nbk3 = a.nbv3 = (uint64_t) Hkv * n_kv * 128;
+    }
+    if (blocks > 0x7fffffff) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext: launch too large");
+    if (p.n_store && (pf_overlaps(p.ks, k) || pf_overlaps(p.ks, v) || pf_overlaps(p.vs, k) || pf_overlaps(p.vs, v) ||
+                      (mask && (pf_overlaps(p.ks, mask) || pf_overlaps(p.vs, mask))))) { // (what the rest reads is being written: one after the other)
+        pf_prep_args first = p;
+        first.n_mask = 0;
+        vx_launch(pf_prep_kernel, dim3((unsigned) p.n_store), dim3(256), 0, st, first);
+        VX_LAUNCH_CHECK();
+        blocks -= p.n_store;
+        p.n_store = 0;
+    }
+    if (blocks) {
+        vx_launch(pf_prep_kernel, dim3((unsigned) blocks), dim3(256), 0, st, p);
+        VX_LAUNCH_CHECK();
+    }
+    if (front && !a.totals) {
+        vx_launch(pf_scalar_kernel, dim3(1), dim3(PF_TOTALS), 0, st, (const double *) p.totals, a.n_tk, a.n_tv, a.sync_scale, a.sync_bias, (float *) a.add1);
+        VX_LAUNCH_CHECK();
     }
     const dim3 grid((unsigned) (n_rb * n_groups)), block(64 * PF_WAVES);
     if (half_cols) {

@@ -1078,20 +1078,6 @@ __global__ __launch_bounds__(1024) void kv_store_large_kernel(const kvs_args a, 
 // but one work-group storing and adding 2 x 64 Ki values is 17 us.  Here every wave of that block is a work-group of its
 // own (16 per cache) and leaves its total where the kernel behind adds the block totals in order: the same additions in
 // the same order, the zeros of the 112 further slots change nothing.
-template <bool VEC>
-__device__ __forceinline__ double kvs_mid_wave(const kvs_side & s, uint32_t w, uint32_t lane) {
-    const uint32_t n = kvs_units(s, VEC);
-    double acc = 0.0;
-    if (n <= VX_SUM_ONE_WAVE_UNITS) { // (uniform) a sum of one wave's size: its order, by the first wave
-        if (w) return 0.0;
-        for (uint32_t e = lane; e < n; e += 64) kvs_unit<VEC>(s, e, true, acc);
-        return vx_wave_sum(acc);
-    }
-    if (w * 64 >= n) return 0.0;
-    for (uint32_t e = w * 64 + lane; e < n; e += 1024) kvs_unit<VEC>(s, e, true, acc);
-    return vx_wave_sum(acc);
-}
-
 template <bool VK, bool VV>
 __global__ __launch_bounds__(64) void kv_store_mid_kernel(const kvs_args a, double * partials) {
     const bool     second = blockIdx.x >= 16; // uniform
@@ -1117,12 +1103,6 @@ __device__ __forceinline__ float kvs_scalar_of_totals(const kvs_args & a, const 
     }
     __syncthreads();
     return y_s;
-}
-
-// the scalar alone, for a consumer that adds it itself (the prefill attention's epilogue)
-__global__ __launch_bounds__(256) void kv_sync_scalar_kernel(const kvs_args a, const double * partials, float * y_out) {
-    const float y = kvs_scalar_of_totals(a, partials);
-    if (threadIdx.x == 0) *y_out = y;
 }
 
 __global__ __launch_bounds__(256) void kv_sync_add1_kernel(const kvs_args a, const double * partials) {
@@ -1976,26 +1956,15 @@ extern "C" vx_status vx_kv_store_sync(const vx_tensor * k, const vx_tensor * k_s
     return VX_OK;
 }
 
-// The cache write and the ordering scalar of vx_kv_store_sync without its ADD1: the scalar goes to y_out for a kernel
-// launched behind this call on the same stream to add.  partials: 2 * SUM_BLOCKS doubles of device memory.
-bool vx_kv_store_scalar_ok(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot) {
+// Whether an attention launch may take the cache write along (vx_pf_front) and which form its sums have: one block's
+// or many blocks' (*large).
+bool vx_kv_store_scalar_ok(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot, bool * large) {
+    if (large) *large = false;
     // (a prompt's or a prefill's write: attention shapes with a smaller one do not reach the kernel that adds the scalar)
-    return k && k_slot && v && v_slot && (kvs_mid(k, k_slot, v, v_slot) || kvs_large(k, k_slot, v, v_slot));
+    if (!k || !k_slot || !v || !v_slot) return false;
+    if (kvs_mid(k, k_slot, v, v_slot)) return true;
+    if (!kvs_large(k, k_slot, v, v_slot)) return false;
+    if (large) *large = true;
+    return true;
 }
 
-vx_status vx_kv_store_scalar(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot,
-                             float scale, float bias, void * partials, float * y_out, hipStream_t st) {
-    if (!vx_kv_store_scalar_ok(k, k_slot, v, v_slot)) return vx_fail(VX_ERR_UNSUPPORTED, "kv_store_scalar: shapes vx_kv_store_sync does not take");
-    kvs_args a;
-    kvs_side_fill(a.k, k, k_slot);
-    kvs_side_fill(a.v, v, v_slot);
-    a.x = nullptr; a.d = nullptr;
-    for (int i = 0; i < 4; ++i) { a.ne[i] = 0; a.nbx[i] = 0; a.nbd[i] = 0; }
-    a.scale = scale; a.bias = bias;
-    a.dense4 = 0;
-    a.defer = nullptr;
-    kvs_launch_store(a, kvs_mid(k, k_slot, v, v_slot), (double *) partials, st);
-    vx_launch(kv_sync_scalar_kernel, dim3(1), dim3(256), 0, st, a, (const double *) partials, y_out);
-    VX_LAUNCH_CHECK();
-    return VX_OK;
-}

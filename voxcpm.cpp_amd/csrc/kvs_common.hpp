@@ -40,6 +40,8 @@ static inline void kvs_side_fill(kvs_side & o, const vx_tensor * src, const vx_t
     o.src_dense = vx_is_contiguous(src) && (uintptr_t) src->data % 16 == 0;
 }
 
+static inline int64_t kvs_host_units(const kvs_side & a) { return a.ned[0] / (a.vec ? 4 : 1) * a.ned[1] * a.ned[2] * a.ned[3]; }
+
 #ifdef __HIPCC__
 // Unit e of the slot (4 consecutive elements when VEC, else one): fetch from the source, optionally store,
 // add to acc in element order -- the inner step of GGML_OP_SUM's walk over the written slot.
@@ -121,6 +123,21 @@ __device__ __forceinline__ double kvs_wave_total(const kvs_side & a, int lane, b
     }
     if (w < 16) total += 0.0; // their zeros, added once (it only matters for the sign of a zero total)
     return total;
+}
+
+// Wave w of the 16 that one block's sum consists of, by a wave of its own: stores its units and returns its total.
+template <bool VEC>
+__device__ __forceinline__ double kvs_mid_wave(const kvs_side & s, uint32_t w, uint32_t lane) {
+    const uint32_t n = kvs_units(s, VEC);
+    double acc = 0.0;
+    if (n <= VX_SUM_ONE_WAVE_UNITS) { // (uniform) a sum of one wave's size: its order, by the first wave
+        if (w) return 0.0;
+        for (uint32_t e = lane; e < n; e += 64) kvs_unit<VEC>(s, e, true, acc);
+        return vx_wave_sum(acc);
+    }
+    if (w * 64 >= n) return 0.0;
+    for (uint32_t e = w * 64 + lane; e < n; e += 1024) kvs_unit<VEC>(s, e, true, acc);
+    return vx_wave_sum(acc);
 }
 
 // both cache writes of a step at once: the two sides' loads are in flight together

@@ -87,13 +87,17 @@ void   vx_derived_abandon(const vx_derived_key & key, hipStream_t stream); // a 
 // so that the first call of the entry point does no set-up work
 vx_status vx_fattn_static_setup(void);
 
-// Work that a caller of vx_fattn_prefill wants launched in front of the attention's own kernels, with a piece of the
-// call's workspace block to itself: `bytes` (a multiple of 256) at the front of the block, handed to `launch` once the
-// block is known; the float at `addend_at` bytes into it is then the attention's addend.
+// A cache write that vx_fattn_prefill takes along: slots stored and summed by work-groups of the launch that prepares the
+// attention's operands, the ordering scalar (scale * (sum k + sum v) + bias) added to the attention's result.  `bytes` (a
+// multiple of 256, at least VX_PF_FRONT) at the front of the call's workspace block are its own: totals, scalar, tiles.
+struct kvs_side;
+constexpr size_t VX_PF_FRONT = 4096, VX_PF_SCALAR_AT = 2048; // 2 x 128 totals, then the scalar
 struct vx_pf_front {
-    size_t bytes, addend_at;
-    vx_status (*launch)(void * front, void * ctx, hipStream_t stream);
-    void * ctx;
+    size_t bytes;
+    const kvs_side * ks, * vs;
+    bool   store_large; // vx_kv_store_scalar_ok's form of the sums
+    float  scale, bias;
+    void ** base;       // where to leave the block's address (or null)
     // optionally the result leaves as the pre-tiled product kernel's f16 activation tiles (k = head * 64 + d) at
     // tiles_at bytes into the front instead of being stored to dst: tile_tt 16-token tiles per k block; tile_bs tiles
     // per batch entry (0: the sequences are flattened into one token dimension, tile_ts tokens apart)
@@ -116,11 +120,8 @@ bool      vx_proj_tiles_ok(const vx_tensor * w, const vx_tensor * x, const vx_te
 vx_status vx_proj_tiles_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale,
                             int act_mode, const void * tiles, size_t ws_offset, hipStream_t stream);
 
-// vx_kv_store_sync's cache write and ordering scalar without the ADD1 (glue.hip): the scalar is left in *y_out
-// (device memory), partials are 2 KiB of device memory
-bool      vx_kv_store_scalar_ok(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot);
-vx_status vx_kv_store_scalar(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot,
-                             float scale, float bias, void * partials, float * y_out, hipStream_t stream);
+// whether vx_fattn_prefill may take this cache write along (glue.hip); *large: sums of many blocks
+bool vx_kv_store_scalar_ok(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot, bool * large = nullptr);
 
 // whether vx_fattn_prefill would take this shape (k describes all keys)
 bool vx_fattn_prefill_accepts(const vx_tensor * q, const vx_tensor * k, float logit_softcap);
