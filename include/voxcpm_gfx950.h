@@ -342,7 +342,9 @@ VX_API int vx_supports_flash_attn_ext_store(const vx_tensor * q, const vx_tensor
  * fp32 nor read back and laid out again.  attn describes that output as the projection reads it ([hidden, tokens] with
  * the sequences one after the other, or [hidden, tokens, batch]; dense, the attention result's own memory order): its
  * memory is NOT written -- for callers whose only reader of it is the projection.  Where vx_flash_attn_ext_store applies
- * and the projection alone would run on the pre-tiled kernel (Q8_0, VX_ACT_FLOAT) -- what the supports function reports;
+ * and the projection alone would run on the pre-tiled kernel (Q8_0, VX_ACT_FLOAT) -- and for prompts of 17 tokens up whose
+ * attention is one key range a wave (256 keys; the projection's activation pass then adds the ordering scalar) -- what the
+ * supports function reports;
  * other shapes run as the separate calls, through attn's memory.  dst and the cache contents equal the separate calls'. */
 VX_API vx_status vx_flash_attn_ext_store_proj(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
                                               const float * sinks, const vx_tensor * k_src, const vx_tensor * k_slot,

@@ -51,3 +51,38 @@ def test_attention_reads_the_written_slots(pkg, gpu):
                                       None), "over the slots")
     torch.cuda.synchronize()
     assert torch.equal(kc, kc2) and torch.equal(vc, vc2) and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,T", [(1, 17), (1, 32), (1, 33), (1, 45), (2, 64), (1, 129), (3, 100), (1, 203), (1, 256), (5, 203)])
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("poison", [False, True])
+def test_short_prompt_block(pkg, gpu, B, T, f16, poison):
+    """A prompt's attention, cache write, o projection and update as one call against the calls it stands for, bit for bit."""
+    import torch
+    from test_gpu_fused import q8_dev
+    say(f"short prompt's attention block as one call B={B} T={T} f16 cache={f16} poison={poison}")
+    L, d = pkg.lib(), pkg.desc
+    H, Hkv, D, hidden = 16, 2, 64, 1024
+    g = rng("prep-short", B, T)
+    q, k, v = (dev(g.standard_normal((B, T, h, D)).astype("float32")) for h in (H, Hkv, Hkv))
+    if poison:
+        v[B - 1, T // 2, 1, 3] = float("nan")
+    res = dev(g.standard_normal((B * T, hidden)).astype("float32"))
+    wd = pkg.desc_q8(w := q8_dev((0.05 * g.standard_normal((hidden, hidden))).astype("float32"))[0], hidden)
+    mask = torch.full((T, T), float("-inf"), dtype=torch.float16, device="cuda").triu(1).contiguous()
+    kc1, vc1, kc2, vc2 = (torch.zeros((B, Hkv, T + 3, D), dtype=torch.float16 if f16 else torch.float32, device="cuda") for _ in range(4))
+    slot = lambda c: c[:, :, 2:2 + T].transpose(1, 2)
+    qkv = [d(t.transpose(1, 2)) for t in (q, k, v)]
+    a, o1 = torch.empty((B, T, H, D), device="cuda"), torch.empty_like(res)
+    ok(pkg, L.vx_flash_attn_ext(*qkv, d(mask), None, d(a), 0.125, 0.0, 0.0, None), "flash_attn_ext")
+    ok(pkg, L.vx_kv_store_sync(d(k), d(slot(kc1)), d(v), d(slot(vc1)), d(a), d(a), 0.25, 0.5, None), "kv_store_sync")
+    ok(pkg, L.vx_mul_mat_scale_add(wd, d(a.view(B * T, hidden)), d(res), d(o1), 0.7, pkg.ACT_FLOAT, None), "mul_mat_scale_add")
+    b, o2 = torch.full((B * T, hidden), 7.0, device="cuda"), torch.full_like(res, 5.0)
+    tail = (d(k), d(slot(kc2)), d(v), d(slot(vc2)), d(b), wd, d(res), d(o2))
+    one = L.vx_supports_flash_attn_ext_store_proj(*qkv, d(mask), *tail, 0.0, pkg.ACT_FLOAT)
+    assert one == (B * T <= 1024)
+    ok(pkg, L.vx_flash_attn_ext_store_proj(*qkv, d(mask), None, *tail, 0.125, 0.0, 0.0, 0.25, 0.5, 0.7, pkg.ACT_FLOAT, None), "one call")
+    torch.cuda.synchronize()
+    assert torch.equal(kc1.view(torch.uint8), kc2.view(torch.uint8)) and torch.equal(vc1.view(torch.uint8), vc2.view(torch.uint8))
+    assert torch.equal(torch.isnan(o1), torch.isnan(o2)) and torch.equal(o1.nan_to_num(3.0), o2.nan_to_num(3.0))
+    assert bool(torch.isnan(o2).any()) == poison and (not one or bool((b == 7.0).all()))

@@ -57,6 +57,8 @@ struct fa_args {
     kvs_side kvs_k, kvs_v;
     float kvs_scale, kvs_bias;
     int has_kvs;
+    double * kvs_totals; // PRE: 16 wave totals a side, and the grid's slices in front that form them
+    int pre_slices;
     float * kvs_out; // the scalar, written by the first kernel's extra block and read by every merge block
     const char * k2; const char * v2;
     uint64_t nbk1b, nbk2b, nbk3b, nbv1b, nbv2b, nbv3b;
@@ -140,7 +142,11 @@ __device__ __forceinline__ void fa_finish(const fa_args & a, float4_t acc, float
 // left them): they are rounded to f16, to nearest even, while they are loaded -- exactly what a CPY node to an F16
 // tensor in front of a CONCAT would have stored.
 // HALF: the whole key range is at most 16 keys (chosen by the host: one range, one pair of tensors).
-template <int D, bool KV_F32, bool HAS_MASK, bool SOFTCAP, int TWO_SEG, bool HALF = false>
+// PRE: the cache write of the same attention block rides along (a prompt too short for the tiled kernel): 32 waves in front
+// store the slots and leave the totals of GGML_OP_SUM's 16 waves a side, which the o projection's activation pass adds up
+// and adds to this kernel's result.  The two launches it replaces (5.0 + 4.2 us of a 45-token prompt's layer of 55) were
+// one work-group's trip to memory and a pass over the result.
+template <int D, bool KV_F32, bool HAS_MASK, bool SOFTCAP, int TWO_SEG, bool HALF = false, bool PRE = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fattn_cols16_kernel(const fa_args a) {
     constexpr int NP  = D / 32;          // MFMAs along the head dimension
     constexpr int SEG = D / 4;           // elements of a row owned by lane-group j
@@ -149,6 +155,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fa
     const int lane = threadIdx.x;
     const int j = lane >> 4, c = lane & 15;
 
+    if constexpr (PRE) {
+        if ((int) blockIdx.z < a.pre_slices) {
+            const uint32_t i = blockIdx.z * gridDim.x + blockIdx.x, w = i & 15;
+            if (i >= 32) return;
+            double t; // (two branches: a reference to either argument would be a copy of one in scratch memory)
+            if (i >= 16) t = a.kvs_v.vec ? kvs_mid_wave<true>(a.kvs_v, w, (uint32_t) lane) : kvs_mid_wave<false>(a.kvs_v, w, (uint32_t) lane);
+            else         t = a.kvs_k.vec ? kvs_mid_wave<true>(a.kvs_k, w, (uint32_t) lane) : kvs_mid_wave<false>(a.kvs_k, w, (uint32_t) lane);
+            if (lane == 0) a.kvs_totals[(i >= 16 ? VX_KVS_V_AT : 0) + w] = t;
+            return;
+        }
+    }
     // With the cache write folded in, the grid has one more slice in front: its first wave forms the two sums and leaves
     // the scalar for the merge kernel, its other waves store the slots.  (One wave reads
     // the step's keys and values: when every merge block formed the sums itself, sixteen streams' 512 blocks asked the
@@ -176,7 +193,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fa
         }
     }
     // the grid is (column tile, key range, batch entry x KV head): dispatched in the same order as one flat index
-    const int ct = blockIdx.x, sp = blockIdx.y, bg = (int) blockIdx.z - ((TWO_SEG != 0 && a.has_kvs) ? 1 : 0);
+    const int ct = blockIdx.x, sp = blockIdx.y, bg = (int) blockIdx.z - (PRE ? a.pre_slices : (TWO_SEG != 0 && a.has_kvs) ? 1 : 0);
     const int b  = fa_div(bg, a.inv_hkv);
     const int g  = bg - b * a.Hkv;
     const int tile = bg * a.n_col_tiles + ct;
@@ -937,7 +954,14 @@ void launch_dec64(const fa_args & a, hipStream_t st) {
 
 template <int D, bool KV_F32>
 void launch_cols16(const fa_args & a, hipStream_t st) {
-    const dim3 grid((unsigned) a.n_col_tiles, (unsigned) a.n_splits, (unsigned) (a.ne3 * a.Hkv + (a.has_kvs ? 1 : 0))), block(64);
+    const dim3 grid((unsigned) a.n_col_tiles, (unsigned) a.n_splits, (unsigned) (a.ne3 * a.Hkv + (a.has_kvs ? 1 : 0) + a.pre_slices)), block(64);
+    if constexpr (D == 64) {
+        if (a.pre_slices) { // (one pair of tensors, one key range, no soft cap)
+            if (a.mask) vx_launch(fattn_cols16_kernel<D, KV_F32, true, false, 0, false, true>, grid, block, 0, st, a);
+            else        vx_launch(fattn_cols16_kernel<D, KV_F32, false, false, 0, false, true>, grid, block, 0, st, a);
+            return;
+        }
+    }
     if constexpr (D == 64 && !KV_F32) {
         if (a.k2 && a.seg2_f32) { // an F16 cache and the step's F32 keys
             if (a.softcap != 0.0f) vx_launch(fattn_cols16_kernel<D, false, true, true, 2>, grid, block, 0, st, a);
@@ -1006,7 +1030,7 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
                         const float * addend, const vx_tensor * dst, float scale, float max_bias, float logit_softcap,
                         hipStream_t st, const vx_tensor * ks_src = nullptr, const vx_tensor * ks_slot = nullptr,
                         const vx_tensor * vs_src = nullptr, const vx_tensor * vs_slot = nullptr, float kvs_scale = 0.0f,
-                        float kvs_bias = 0.0f, void * fixed_ws = nullptr, size_t fixed_ws_bytes = 0);
+                        float kvs_bias = 0.0f, void * fixed_ws = nullptr, size_t fixed_ws_bytes = 0, double * kvs_totals = nullptr);
 
 extern "C" vx_status vx_flash_attn_ext_add1(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v,
                                             const vx_tensor * mask, const float * sinks, const float * addend,
@@ -1192,11 +1216,39 @@ static bool pf_proj_geometry(const vx_tensor * q, const vx_tensor * attn, const 
     return (int64_t) B * T < ((int64_t) 1 << 31);
 }
 
+// A prompt too short for the tiled kernel, in one key range (up to 256 keys, or more sequences than leave a range to cut):
+// the general kernel with the cache write beside it, its result in fp32 in the workspace, the scalar added by the
+// projection's activation pass -- three launches instead of five: a 45-token prompt through 24 layers 1317 -> 1111 us, 203
+// tokens 1746 -> 1589.  (Decode-sized calls stay with the entry points of their
+// own; f16 keys without a mask beyond 64 are the streaming kernel's, whose arithmetic is another.)
+static bool short_store_proj_ok(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask, const vx_tensor * k_src,
+                                const vx_tensor * k_slot, const vx_tensor * v_src, const vx_tensor * v_slot, const vx_tensor * attn,
+                                const vx_tensor * w_o, const vx_tensor * residual, const vx_tensor * dst, float logit_softcap, int act_mode) {
+    const vx_tensor ad = pf_attn_shape(q, attn);
+    if (!vx_supports_flash_attn_ext(q, k, v, mask, &ad) || logit_softcap != 0.0f || q->ne[0] != 64 || q->ne[1] <= 16) return false;
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || (uintptr_t) attn->data % 16) return false;
+    if (vx_fattn_prefill_accepts(q, k, 0.0f) || (k->type == VX_TYPE_F16 && !mask)) return false;
+    int n_splits, chunk;
+    fa_split_plan(fa_tiles(q, k), (int) k->ne[1], &n_splits, &chunk);
+    if (n_splits != 1 || (q->ne[1] * (q->ne[2] / k->ne[2])) >= (1 << 22) || q->ne[3] * k->ne[2] > 65000) return false;
+    if (!kvs_side_ok(k_src, k_slot, (int64_t) 1 << 24) || !kvs_side_ok(v_src, v_slot, (int64_t) 1 << 24)) return false;
+    kvs_side sk, sv;
+    kvs_side_fill(sk, k_src, k_slot);
+    kvs_side_fill(sv, v_src, v_slot);
+    if (kvs_host_units(sk) > 16 * 1024 || kvs_host_units(sv) > 16 * 1024) return false; // (sums of one block each)
+    for (const vx_tensor * r : { q, k, v, mask }) // (what the attention reads while the slots are written)
+        if (r && (kvs_overlaps(sk, r) || kvs_overlaps(sv, r))) return false;
+    const int64_t hidden = q->ne[0] * q->ne[2], N = q->ne[1] * q->ne[3];
+    return attn->type == VX_TYPE_F32 && vx_is_contiguous(attn) && attn->ne[0] == hidden && attn->ne[1] == N && attn->ne[2] == 1 && attn->ne[3] == 1 &&
+           vx_proj_add_ok(w_o, attn, residual, dst, act_mode);
+}
+
 extern "C" int vx_supports_flash_attn_ext_store_proj(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
                                                      const vx_tensor * k_src, const vx_tensor * k_slot, const vx_tensor * v_src,
                                                      const vx_tensor * v_slot, const vx_tensor * attn, const vx_tensor * w_o,
                                                      const vx_tensor * residual, const vx_tensor * dst, float logit_softcap, int act_mode) {
     if (!attn || !q) return 0;
+    if (short_store_proj_ok(q, k, v, mask, k_src, k_slot, v_src, v_slot, attn, w_o, residual, dst, logit_softcap, act_mode)) return 1;
     const vx_tensor ad = pf_attn_shape(q, attn);
     if (!vx_supports_flash_attn_ext_store(q, k, v, mask, k_src, k_slot, v_src, v_slot, &ad, logit_softcap)) return 0;
     vx_pf_front front{};
@@ -1228,6 +1280,20 @@ extern "C" vx_status vx_flash_attn_ext_store_proj(const vx_tensor * q, const vx_
         const vx_status rc = vx_flash_attn_ext_store(q, k, v, mask, sinks, k_src, k_slot, v_src, v_slot, &ad, scale, max_bias, logit_softcap, sync_scale,
                                                      sync_bias, stream);
         return rc != VX_OK ? rc : vx_mul_mat_scale_add(w_o, attn, residual, dst, res_scale, act_mode, stream);
+    }
+    if (short_store_proj_ok(q, k, v, mask, k_src, k_slot, v_src, v_slot, attn, w_o, residual, dst, logit_softcap, act_mode)) {
+        vx_tensor out = *attn;
+        const size_t out_bytes = ((size_t) vx_nelements(attn) * 4 + 255) & ~(size_t) 255;
+        void * ws = nullptr; // one block for both phases, as below
+        vx_status rc = vx_workspace((hipStream_t) stream, PF_STORE_FRONT + out_bytes + vx_proj_add_bytes(w_o, attn), &ws);
+        if (rc != VX_OK) return rc;
+        out.data = (char *) ws + PF_STORE_FRONT;
+        const vx_tensor ao = pf_attn_shape(q, &out);
+        rc = fa_run(q, k, v, nullptr, nullptr, k, v, mask, sinks, nullptr, &ao, scale, max_bias, 0.0f, (hipStream_t) stream, k_src, k_slot, v_src, v_slot,
+                    sync_scale, sync_bias, nullptr, 0, (double *) ws);
+        if (rc != VX_OK) return rc;
+        return vx_proj_add_run(w_o, &out, residual, dst, res_scale, act_mode, (const double *) ws, sync_scale, sync_bias, PF_STORE_FRONT + out_bytes,
+                               (hipStream_t) stream);
     }
     pf_store_sides sides;
     vx_pf_front front{};
@@ -1305,10 +1371,11 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
                         const vx_tensor * kall, const vx_tensor * vall, const vx_tensor * mask, const float * sinks,
                         const float * addend, const vx_tensor * dst, float scale, float max_bias, float logit_softcap,
                         hipStream_t st, const vx_tensor * ks_src, const vx_tensor * ks_slot, const vx_tensor * vs_src,
-                        const vx_tensor * vs_slot, float kvs_scale, float kvs_bias, void * fixed_ws, size_t fixed_ws_bytes) {
+                        const vx_tensor * vs_slot, float kvs_scale, float kvs_bias, void * fixed_ws, size_t fixed_ws_bytes, double * kvs_totals) {
     (void) vall;
     fa_args a;
     a.has_kvs = 0; a.kvs_out = nullptr;
+    a.kvs_totals = nullptr; a.pre_slices = 0;
     a.k2 = k2 ? (const char *) k2->data : nullptr; a.v2 = v2 ? (const char *) v2->data : nullptr;
     a.nbk1b = k2 ? k2->nb[1] : 0; a.nbk2b = k2 ? k2->nb[2] : 0; a.nbk3b = k2 ? k2->nb[3] : 0;
     a.nbv1b = v2 ? v2->nb[1] : 0; a.nbv2b = v2 ? v2->nb[2] : 0; a.nbv3b = v2 ? v2->nb[3] : 0;
@@ -1343,7 +1410,13 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
     const int64_t tiles = (int64_t) a.ne3 * a.Hkv * a.n_col_tiles;
 
     fa_split_plan(tiles, a.n_kv, &a.n_splits, &a.chunk);
-    if (ks_src) {
+    if (kvs_totals) {
+        if (a.n_splits != 1 || q->ne[0] != 64 || k2 || logit_softcap != 0.0f) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext_store_proj: one key range");
+        kvs_side_fill(a.kvs_k, ks_src, ks_slot);
+        kvs_side_fill(a.kvs_v, vs_src, vs_slot);
+        a.kvs_totals = kvs_totals;
+        a.pre_slices = (32 + a.n_col_tiles - 1) / a.n_col_tiles;
+    } else if (ks_src) {
         if (a.n_splits == 1) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext_kv2_store: needs a key count that is split across waves");
         kvs_side_fill(a.kvs_k, ks_src, ks_slot);
         kvs_side_fill(a.kvs_v, vs_src, vs_slot);
@@ -1356,7 +1429,7 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
     const int D = (int) q->ne[0];
     const bool f32 = k->type == VX_TYPE_F32;
 
-    const bool dec = fa_dec64_takes(a, D, f32);
+    const bool dec = !kvs_totals && fa_dec64_takes(a, D, f32);
 
     if (a.n_splits > 1) {
         const size_t o_bytes  = (size_t) nblocks * 16 * D * sizeof(float);

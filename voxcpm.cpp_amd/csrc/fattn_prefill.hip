@@ -26,7 +26,7 @@ constexpr int PF_WAVES = 4;
 constexpr int PF_COLS  = 256; // columns per work-group
 constexpr int PF_KT    = 64;  // keys per tile
 constexpr int PF_MAX_TILES = 1024;
-constexpr int PF_TOTALS = 128;       // block totals of one sum of a cache write, at most
+constexpr int PF_TOTALS = VX_KVS_V_AT;       // block totals of one sum of a cache write, at most
 constexpr int PF_TOTALS_INLINE = 64; // up to here a wave of every attention work-group adds them (two sequences of 512 tokens: 32 a side; beside
                                      // the tile list that takes less than the 4.5 us of a launch for one number), beyond pf_scalar_kernel does
 
@@ -794,14 +794,6 @@ bool vx_fattn_prefill_accepts(const vx_tensor * q, const vx_tensor * k, float lo
     return (int64_t) n_rb * n_groups >= 32;
 }
 
-// whether a cache write's slot and a tensor share bytes (by their extents)
-static bool pf_overlaps(const kvs_side & s, const vx_tensor * t) {
-    uint64_t sb = s.dst_f16 ? 2 : 4, tb = vx_type_size(t->type);
-    for (int i = 0; i < 4; ++i) { sb += (uint64_t) (s.ned[i] - 1) * s.nbd[i]; tb += (uint64_t) (t->ne[i] - 1) * t->nb[i]; }
-    const char * t0 = (const char *) t->data;
-    return s.d < t0 + tb && t0 < s.d + sb;
-}
-
 vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
                            const float * sinks, const float * addend, const vx_tensor * dst, float scale, float max_bias,
                            float logit_softcap, hipStream_t st, const vx_pf_front * front) {
@@ -901,8 +893,8 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
         a.nbk1 = a.nbv1 = 128; a.nbk2 = a.nbv2 = (uint64_t) n_kv * 128; a.nbk3 = a.nbv3 = (uint64_t) Hkv * n_kv * 128;
     }
     if (blocks > 0x7fffffff) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext: launch too large");
-    if (p.n_store && (pf_overlaps(p.ks, k) || pf_overlaps(p.ks, v) || pf_overlaps(p.vs, k) || pf_overlaps(p.vs, v) ||
-                      (mask && (pf_overlaps(p.ks, mask) || pf_overlaps(p.vs, mask))))) { // (what the rest reads is being written: one after the other)
+    if (p.n_store && (kvs_overlaps(p.ks, k) || kvs_overlaps(p.ks, v) || kvs_overlaps(p.vs, k) || kvs_overlaps(p.vs, v) ||
+                      (mask && (kvs_overlaps(p.ks, mask) || kvs_overlaps(p.vs, mask))))) { // (what the rest reads is being written: one after the other)
         pf_prep_args first = p;
         first.n_mask = 0;
         vx_launch(pf_prep_kernel, dim3((unsigned) p.n_store), dim3(256), 0, st, first);

@@ -21,6 +21,7 @@
 // [16.6 + 4.4 for the K cut's second launch], gate/up pair 10.9 [20.7]; 45 tokens: 3.7 [5.8], 6.7 [9.9 + 6.0], 6.0 [7.3 +
 // 7.3 + 3.4]; 1024 tokens: 7.5 [10], 17.7 [26 + 5.5], 38 [46].
 #include "gemm_mid.hpp"
+#include "kvs_common.hpp"
 #include "mm_common.hpp"
 
 #include <cstdlib>
@@ -352,6 +353,8 @@ struct gm_acts {
     int           ne12, N, K, n_tt, n_kb, row_blocks;
     const float * norm_w;
     float         eps;
+    const double * totals;  // a cache write's wave totals: its scalar joins every value before the rounding
+    float         sync_scale, sync_bias;
     half8_t *     xt;
     // rotation angles of the launch behind (blocks from row_blocks on)
     const int32_t * pos; const float * ff;
@@ -408,10 +411,16 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
             put(lane + 64 * cc, h);
         }
     } else {
-        for (int iv0 = lane; iv0 < nvec; iv0 += 64 * 4) {
+        float y = 0.0f;
+        for (int iv0 = lane; iv0 < nvec; iv0 += 64 * 4) { // (nvec is a multiple of 64: whole waves)
             float4_t v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = ((const float4_t *) row)[min(iv0 + 64 * u, nvec - 1)];
+            if (a.totals) { // (uniform) the ADD1 node
+                if (iv0 == lane) y = kvs_scalar_of_16(a.totals, lane, a.sync_scale, a.sync_bias);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] += y;
+            }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 if (iv0 + 64 * u >= nvec) break;
@@ -530,6 +539,7 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
         p.N = a.N; p.K = (int) c.K; p.n_tt = a.n_tt; p.n_kb = a.n_kb;
         p.row_blocks = 4 * a.n_tt;
         p.norm_w = c.norm_w; p.eps = c.norm_eps;
+        p.totals = c.add_totals; p.sync_scale = c.add_scale; p.sync_bias = c.add_bias;
         p.xt = (half8_t *) base;
         int blocks = p.row_blocks;
         if (rotate) {

@@ -26,6 +26,8 @@ struct vx_gm_call {
     uint64_t      nb11, nb12, nb13;
     const float * norm_w;
     float         norm_eps;
+    const double * add_totals;    // a cache write's wave totals, whose ordering scalar is added to every activation (no norm), or null
+    float         add_scale, add_bias;
     const void *  tile_in;
     int           tile_tt;        // 16-token tiles per k block of tile_in / tile_out
     void *        tile_out;       // gate/up pair: results as the next product's f16 activation tiles instead of dst

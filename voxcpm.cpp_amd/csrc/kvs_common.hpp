@@ -42,6 +42,16 @@ static inline void kvs_side_fill(kvs_side & o, const vx_tensor * src, const vx_t
 
 static inline int64_t kvs_host_units(const kvs_side & a) { return a.ned[0] / (a.vec ? 4 : 1) * a.ned[1] * a.ned[2] * a.ned[3]; }
 
+// whether a cache write's slot and a tensor share bytes (by their extents)
+static inline bool kvs_overlaps(const kvs_side & s, const vx_tensor * t) {
+    uint64_t sb = s.dst_f16 ? 2 : 4, tb = vx_type_size(t->type);
+    for (int i = 0; i < 4; ++i) { sb += (uint64_t) (s.ned[i] - 1) * s.nbd[i]; tb += (uint64_t) (t->ne[i] - 1) * t->nb[i]; }
+    const char * t0 = (const char *) t->data;
+    return s.d < t0 + tb && t0 < s.d + sb;
+}
+
+constexpr int VX_KVS_V_AT = 128; // where the second side's totals lie in an array of both
+
 #ifdef __HIPCC__
 // Unit e of the slot (4 consecutive elements when VEC, else one): fetch from the source, optionally store,
 // add to acc in element order -- the inner step of GGML_OP_SUM's walk over the written slot.
@@ -125,19 +135,41 @@ __device__ __forceinline__ double kvs_wave_total(const kvs_side & a, int lane, b
     return total;
 }
 
+// the scalar the reference adds to the attention output: (sum(k_slot) + sum(v_slot)) * scale + bias
+__device__ __forceinline__ float kvs_scalar(float sk, float sv, float scale, float bias) {
+    const float t = sk + sv;                                       // the ADD node
+    return bias == 0.0f ? t * scale : fmaf(t, scale, bias);        // the SCALE node
+}
+
 // Wave w of the 16 that one block's sum consists of, by a wave of its own: stores its units and returns its total.
+// Eight of a lane's units are requested together (one trip instead of eight), then taken in order.
 template <bool VEC>
 __device__ __forceinline__ double kvs_mid_wave(const kvs_side & s, uint32_t w, uint32_t lane) {
     const uint32_t n = kvs_units(s, VEC);
+    const bool     one = n <= VX_SUM_ONE_WAVE_UNITS; // (uniform) a sum of one wave's size: its order, by the first wave
+    if (one ? w != 0 : w * 64 >= n) return 0.0;
+    const uint32_t step = one ? 64 : 1024;
+    constexpr int  UB = 8;
     double acc = 0.0;
-    if (n <= VX_SUM_ONE_WAVE_UNITS) { // (uniform) a sum of one wave's size: its order, by the first wave
-        if (w) return 0.0;
-        for (uint32_t e = lane; e < n; e += 64) kvs_unit<VEC>(s, e, true, acc);
-        return vx_wave_sum(acc);
+    for (uint32_t base = w * 64 + lane; base < n; base += step * UB) {
+        float v[UB][VEC ? 4 : 1];
+#pragma unroll
+        for (int i = 0; i < UB; ++i) if (base + step * i < n) kvs_fetch<VEC>(s, base + step * i, v[i]);
+#pragma unroll
+        for (int i = 0; i < UB; ++i) if (base + step * i < n) kvs_apply<VEC>(s, base + step * i, true, v[i], acc);
     }
-    if (w * 64 >= n) return 0.0;
-    for (uint32_t e = w * 64 + lane; e < n; e += 1024) kvs_unit<VEC>(s, e, true, acc);
     return vx_wave_sum(acc);
+}
+
+// The two sums of 16 wave totals a side (k's at 0, v's at VX_KVS_V_AT) as the ordering scalar, by every lane of a wave:
+// k's totals in its low half, v's in the high.
+__device__ __forceinline__ float kvs_scalar_of_16(const double * totals, int lane, float scale, float bias) {
+    const double tot = (lane & 31) < 16 ? totals[(lane >> 5) * VX_KVS_V_AT + (lane & 31)] : 0.0;
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t += __shfl(tot, (lane & 32) + i, 64);
+    const float sum = (float) t;
+    return kvs_scalar(__shfl(sum, 0, 64), __shfl(sum, 32, 64), scale, bias);
 }
 
 // both cache writes of a step at once: the two sides' loads are in flight together
@@ -190,9 +222,4 @@ __device__ __forceinline__ void kvs_wave_totals(const kvs_side & k, const kvs_si
     if (wv < 16) tv += 0.0;
 }
 
-// the scalar the reference adds to the attention output: (sum(k_slot) + sum(v_slot)) * scale + bias
-__device__ __forceinline__ float kvs_scalar(float sk, float sv, float scale, float bias) {
-    const float t = sk + sv;                                       // the ADD node
-    return bias == 0.0f ? t * scale : fmaf(t, scale, bias);        // the SCALE node
-}
 #endif

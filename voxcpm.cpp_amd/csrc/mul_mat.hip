@@ -3009,6 +3009,30 @@ bool vx_proj_tiles_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor 
     return true;
 }
 
+bool vx_proj_add_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, int act_mode) {
+    mm_args b;
+    bool mid = false;
+    return proj_tiles_fill(b, mid, w, x, residual, dst, 0.0f, act_mode) && mid;
+}
+
+size_t vx_proj_add_bytes(const vx_tensor * w, const vx_tensor * x) { return vx_gm_tile_bytes(w->ne[0], x->ne[1], 1); }
+
+vx_status vx_proj_add_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale, int act_mode,
+                          const double * totals, float sync_scale, float sync_bias, size_t ws_offset, hipStream_t st) {
+    mm_args b;
+    bool mid = false;
+    vx_gm_call c;
+    if (!proj_tiles_fill(b, mid, w, x, residual, dst, scale, act_mode) || !mid) return vx_fail(VX_ERR_UNSUPPORTED, "projection with a scalar: a shape outside the kernel");
+    if (!w->data || !residual->data || !dst->data || !x->data) return vx_fail(VX_ERR_INVALID, "projection with a scalar: null data");
+    b.ws_offset = ws_offset;
+    if (!mid_fill(c, b, 1, WT_Q8)) return vx_fail(VX_ERR_UNSUPPORTED, "projection with a scalar: a shape outside the kernel");
+    c.add_totals = totals; c.add_scale = sync_scale; c.add_bias = sync_bias;
+    const vx_status rc = vx_gm_run(c, st);
+    if (rc != VX_OK) return rc;
+    VX_LAUNCH_CHECK();
+    return VX_OK;
+}
+
 vx_status vx_proj_tiles_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale,
                             int act_mode, const void * tiles, size_t ws_offset, hipStream_t st) {
     mm_args b;

@@ -120,6 +120,14 @@ bool      vx_proj_tiles_ok(const vx_tensor * w, const vx_tensor * x, const vx_te
 vx_status vx_proj_tiles_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale,
                             int act_mode, const void * tiles, size_t ws_offset, hipStream_t stream);
 
+// vx_mul_mat_scale_add of a Q8_0 projection whose F32 activations x get the ordering scalar of a cache write (16 totals a
+// side, as kvs_scalar_of_16 takes them) added first.  _ok: gemm_mid.hip's kernel runs the product, whose activation pass adds it.
+// _bytes: what the run takes of the workspace behind the caller's ws_offset bytes.
+bool      vx_proj_add_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, int act_mode);
+size_t    vx_proj_add_bytes(const vx_tensor * w, const vx_tensor * x);
+vx_status vx_proj_add_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale, int act_mode,
+                          const double * totals, float sync_scale, float sync_bias, size_t ws_offset, hipStream_t stream);
+
 // whether vx_fattn_prefill may take this cache write along (glue.hip); *large: sums of many blocks
 bool vx_kv_store_scalar_ok(const vx_tensor * k, const vx_tensor * k_slot, const vx_tensor * v, const vx_tensor * v_slot, bool * large = nullptr);
 
