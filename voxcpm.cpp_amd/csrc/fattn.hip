@@ -57,9 +57,11 @@ struct fa_args {
     kvs_side kvs_k, kvs_v;
     float kvs_scale, kvs_bias;
     int has_kvs;
-    double * kvs_totals; // PRE: 16 wave totals a side, and the grid's slices in front that form them
-    int pre_slices;
-    float * kvs_out; // the scalar, written by the first kernel's extra block and read by every merge block
+    int pre_slices;      // PRE: the grid's slices in front that form the totals of the write's sums
+    union {
+        float *  kvs_out;    // the scalar, written by the first kernel's extra block and read by every merge block
+        double * kvs_totals; // PRE: 16 wave totals a side
+    };
     const char * k2; const char * v2;
     uint64_t nbk1b, nbk2b, nbk3b, nbv1b, nbv2b, nbv3b;
     int n_kv1;
@@ -1375,7 +1377,7 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
     (void) vall;
     fa_args a;
     a.has_kvs = 0; a.kvs_out = nullptr;
-    a.kvs_totals = nullptr; a.pre_slices = 0;
+    a.pre_slices = 0;
     a.k2 = k2 ? (const char *) k2->data : nullptr; a.v2 = v2 ? (const char *) v2->data : nullptr;
     a.nbk1b = k2 ? k2->nb[1] : 0; a.nbk2b = k2 ? k2->nb[2] : 0; a.nbk3b = k2 ? k2->nb[3] : 0;
     a.nbv1b = v2 ? v2->nb[1] : 0; a.nbv2b = v2 ? v2->nb[2] : 0; a.nbv3b = v2 ? v2->nb[3] : 0;

@@ -216,11 +216,14 @@ __device__ __forceinline__ void pf_store_large(const kvs_side & s, uint32_t b, d
 // One launch for what three did (the cache write, the mask's flags, the f16 images): each is a trip to memory and its
 // latency at a prompt's size.  Two sequences of 512 tokens: 4.8 + 4.1 + 3.9 us as launches of their own, and 4.5 for the
 // scalar that the attention now adds up itself; 24 layers 3067 -> 2876 us, 16 x 4096 tokens 86.5 -> 85.7 ms.
+// STORE is a parameter of its own because the write's four units in flight cost every wave of the launch 98 registers, half
+// the waves a SIMD can hold (a causal attention of 4096 tokens without a write 74.6 -> 71.9 us a call).
+template <bool STORE>
 __global__ __launch_bounds__(256) void pf_prep_kernel(const pf_prep_args a) {
     __shared__ double part[16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
     int i = blockIdx.x;
-    if (i < a.n_store) {
+    if (STORE && i < a.n_store) {
         if (a.store_large) {
             const bool second = i >= a.n_tk; // (uniform)
             const kvs_side & s = second ? a.vs : a.ks;
@@ -237,7 +240,7 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(const pf_prep_args a) {
         }
         return;
     }
-    i -= a.n_store;
+    if constexpr (STORE) i -= a.n_store;
     if (i < a.n_mask) {
         const int unit = 4 * i + wave;
         if (unit < a.n_units) pf_mask_unit(a, unit, lane);
@@ -897,13 +900,14 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
                       (mask && (kvs_overlaps(p.ks, mask) || kvs_overlaps(p.vs, mask))))) { // (what the rest reads is being written: one after the other)
         pf_prep_args first = p;
         first.n_mask = 0;
-        vx_launch(pf_prep_kernel, dim3((unsigned) p.n_store), dim3(256), 0, st, first);
+        vx_launch(pf_prep_kernel<true>, dim3((unsigned) p.n_store), dim3(256), 0, st, first);
         VX_LAUNCH_CHECK();
         blocks -= p.n_store;
         p.n_store = 0;
     }
     if (blocks) {
-        vx_launch(pf_prep_kernel, dim3((unsigned) blocks), dim3(256), 0, st, p);
+        if (p.n_store) vx_launch(pf_prep_kernel<true>, dim3((unsigned) blocks), dim3(256), 0, st, p);
+        else           vx_launch(pf_prep_kernel<false>, dim3((unsigned) blocks), dim3(256), 0, st, p);
         VX_LAUNCH_CHECK();
     }
     if (front && !a.totals) {
