@@ -408,7 +408,7 @@ VX_API vx_status vx_norm_mul_mat_swiglu(const vx_tensor * x, const vx_tensor * n
 VX_API int vx_supports_norm_mul_mat_swiglu(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate,
                                            const vx_tensor * up, const vx_tensor * dst);
 /* the same call at prompt and prefill sizes (vx_supports_mul_mat_swiglu_tiled's shapes where the activations are laid out in
- * tiles beforehand: up to 1024 tokens, and on the pre-tiled Q8_0 kernel beyond): the norm and its weight are applied by the pass that lays the activations out in tiles, x is read once and the
+ * tiles beforehand: up to 3072 tokens (F16 weights 1152), and on the pre-tiled Q8_0 kernel beyond): the norm and its weight are applied by the pass that lays the activations out in tiles, x is read once and the
  * normalised tensor is never stored.  Same bits as RMS_NORM, MUL, then vx_mul_mat_swiglu. */
 VX_API int vx_supports_norm_mul_mat_swiglu_tiled(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate,
                                                  const vx_tensor * up, const vx_tensor * dst, int act_mode);

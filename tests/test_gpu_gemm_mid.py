@@ -1,4 +1,4 @@
-"""GPU: the product kernel for 17 to 1024 tokens (csrc/gemm_mid.hip) at the edges of its tiles -- ragged token and row tiles,
+"""GPU: the product kernel for 17 to 3072 tokens (F16 weights: 1152) (csrc/gemm_mid.hip) at the edges of its tiles -- ragged token and row tiles,
 the shortest and longest K it takes, a batch, both weight types -- and the groups built on it against their separate calls."""
 import numpy as np
 import pytest
@@ -16,7 +16,8 @@ def dequant(q, K):
 
 
 @pytest.mark.parametrize("M,K,N,nb", [(16, 1024, 17, 1), (1000, 1024, 33, 1), (128, 768, 64, 2), (1024, 1024, 203, 1), (40, 2304, 31, 3),
-                                      (1024, 4096, 129, 1), (520, 4096, 17, 1), (4096, 1024, 65, 1), (1024, 1024, 1024, 1), (72, 16384, 100, 1)])
+                                      (1024, 4096, 129, 1), (520, 4096, 17, 1), (4096, 1024, 65, 1), (1024, 1024, 1024, 1), (72, 16384, 100, 1),
+                                      (136, 1024, 1152, 1), (136, 1024, 1153, 1), (72, 4096, 1536, 2), (136, 1024, 3073, 1)])
 @pytest.mark.parametrize("wtype", ["q8", "f16"])
 def test_products(pkg, gpu, monkeypatch, M, K, N, nb, wtype):
     import torch
@@ -99,3 +100,8 @@ def test_groups_equal_their_separate_calls(pkg, gpu, T, B, wtype):
     ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, wg, wu, wd, d(x), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp_tiled")
     torch.cuda.synchronize()
     assert same_bits(o1, o2)
+
+
+@pytest.mark.parametrize("T,B,wtype", [(1500, 2, "q8"), (3072, 1, "q8"), (1152, 1, "f16")])
+def test_groups_at_the_last_token_counts(pkg, gpu, T, B, wtype):
+    test_groups_equal_their_separate_calls(pkg, gpu, T, B, wtype)

@@ -1,4 +1,4 @@
-// gemm_mid.hip -- MUL_MAT for some tens to a thousand tokens (a prompt, concurrent LocDiT requests): Q8_0 / F16 weights.
+// gemm_mid.hip -- MUL_MAT for some tens to a few thousand tokens (a prompt, concurrent LocDiT requests): Q8_0 / F16 weights.
 //
 // What bounds these products is neither the matrix cores nor HBM (a 203-token layer is 6 GFLOP and 16 MB of weights) but
 // what each of the chip's 256 compute units has to bring in and issue for its small tile, and the time until its first
@@ -486,10 +486,12 @@ bool gm_go(int tile, int epi, const gm_args & a, int gx, int gy, int nbatch, hip
 bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch) {
     const char * e = getenv("VX_GEMM_MID"); // 0: the kernels of mul_mat.hip for these shapes (read on every call: a test compares the two)
     if (e && atoi(e) == 0) return false;
-    (void) wtype;
     // (VX_GEMM_Q8T, when it is set, decides between the two prefill kernels for every product of 1024 tokens or more)
     if (N >= 1024 && getenv("VX_GEMM_Q8T")) return false;
-    if (N <= 16 || N * nbatch > 1024 || nbatch > 65535) return false;
+    // Up to where this kernel's 64 x 128 tiles, beat the LDS-tiled and pre-tiled
+    // kernels' 128 x 128.  Q8_0, 24 layers of one prompt: 1200 tokens 6270 -> 3818 us, 2048 6834 -> 5205, 2600 8990 -> 7156, but
+    // 4000 9639 -> 10114; F16, 56 products: 1100 tokens 1343 -> 1260 us, 1537 1417 -> 1463.
+    if (N <= 16 || N * nbatch > (wtype == VX_GM_Q8 ? 3072 : 1152) || nbatch > 65535) return false;
     // K of whole 256s (the stages).  Up to 16 tokens are the streaming kernel's; what it takes beyond them with K of 513 to
     // 1024 it sums in this kernel's order, and with K above 2048 it takes nothing beyond them: elsewhere a call that one of
     // the two had to decline (alignment, VX_ACT_Q8's groups) would differ from its neighbours in the last bit.

@@ -1,4 +1,4 @@
-// gemm_mid.hpp -- the product kernel for some tens to a thousand tokens (gemm_mid.hip), as mul_mat.hip calls it.
+// gemm_mid.hpp -- the product kernel for some tens to a few thousand tokens (gemm_mid.hip), as mul_mat.hip calls it.
 #pragma once
 #include "vx_common.hpp"
 #include "rope_common.hpp"
