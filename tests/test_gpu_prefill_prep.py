@@ -86,3 +86,32 @@ def test_short_prompt_block(pkg, gpu, B, T, f16, poison):
     assert torch.equal(kc1.view(torch.uint8), kc2.view(torch.uint8)) and torch.equal(vc1.view(torch.uint8), vc2.view(torch.uint8))
     assert torch.equal(torch.isnan(o1), torch.isnan(o2)) and torch.equal(o1.nan_to_num(3.0), o2.nan_to_num(3.0))
     assert bool(torch.isnan(o2).any()) == poison and (not one or bool((b == 7.0).all()))
+
+
+@pytest.mark.parametrize("B,T,H,M", [(2, 1536, 64, 8192), (2, 600, 16, 1024), (3, 517, 16, 1000)])
+@pytest.mark.parametrize("batched", [True, False])
+def test_prefill_block_by_sequence(pkg, gpu, B, T, H, M, batched):
+    """Attention, cache write, o projection and update as one call, the attention's result a batch of sequences or flattened: the bits
+    of the three calls either way, whichever product kernel a single call of that shape runs on."""
+    import torch
+    from test_gpu_fused import q8_dev
+    say(f"prefill attention block as one call B={B} T={T} heads={H} rows={M} batched={batched}")
+    L, d = pkg.lib(), pkg.desc
+    Hkv, D, hidden = H // 8, 64, H * 64
+    g = rng("prep-batch", B, T, H)
+    q, k, v = (dev(g.standard_normal((B, T, h, D)).astype("float32")) for h in (H, Hkv, Hkv))
+    shape = (B, 1, T, hidden) if batched else (B * T, hidden)
+    res = dev(g.standard_normal((B, 1, T, M) if batched else (B * T, M)).astype("float32"))
+    wd = pkg.desc_q8(w := q8_dev((0.05 * g.standard_normal((M, hidden))).astype("float32"))[0], hidden)
+    kc1, vc1, kc2, vc2 = (torch.zeros((B, Hkv, T, D), device="cuda") for _ in range(4))
+    slot = lambda c: c.transpose(1, 2)
+    qkv = [d(t.transpose(1, 2)) for t in (q, k, v)]
+    a, o1, b, o2 = torch.empty(shape, device="cuda"), torch.empty_like(res), torch.empty(shape, device="cuda"), torch.full_like(res, 5.0)
+    ok(pkg, L.vx_flash_attn_ext(*qkv, None, None, d(a.view(B, T, H, D)), 0.125, 0.0, 0.0, None), "flash_attn_ext")
+    ok(pkg, L.vx_kv_store_sync(d(k), d(slot(kc1)), d(v), d(slot(vc1)), d(a.view(B, T, H, D)), d(a.view(B, T, H, D)), 0.25, 0.5, None), "kv_store_sync")
+    ok(pkg, L.vx_mul_mat_scale_add(wd, d(a), d(res), d(o1), 0.7, pkg.ACT_FLOAT, None), "mul_mat_scale_add")
+    tail = (d(k), d(slot(kc2)), d(v), d(slot(vc2)), d(b), wd, d(res), d(o2))
+    assert L.vx_supports_flash_attn_ext_store_proj(*qkv, None, *tail, 0.0, pkg.ACT_FLOAT) == 1
+    ok(pkg, L.vx_flash_attn_ext_store_proj(*qkv, None, None, *tail, 0.125, 0.0, 0.0, 0.25, 0.5, 0.7, pkg.ACT_FLOAT, None), "one call")
+    torch.cuda.synchronize()
+    assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2) and torch.equal(o1, o2)

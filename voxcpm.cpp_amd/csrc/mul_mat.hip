@@ -2954,8 +2954,8 @@ extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w,
 }
 
 // A projection with its residual update whose activations a kernel in front of it (the prefill attention's epilogue) has
-// left as this kernel's f16 tiles: vx_mul_mat_scale_add without its activation pass.  Taken where the separate call runs
-// on the pre-tiled kernel, so the bits are the same.
+// left as the product kernel's f16 tiles: vx_mul_mat_scale_add without its activation pass.  Taken where the separate call
+// runs on gemm_mid.hip's kernel (mid) or on the pre-tiled one, on the same of the two, so the bits are the same.
 static bool proj_tiles_fill(mm_args & b, bool & mid, const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale, int act_mode) {
     if (!w || !x || !residual || !dst || act_mode != VX_ACT_FLOAT || gemm_lds_mode() == 0) return false;
     if (w->type != VX_TYPE_Q8_0 || w->ne[2] != 1 || w->ne[3] != 1 || x->type != VX_TYPE_F32 || !vx_is_contiguous(x)) return false;
@@ -2975,9 +2975,9 @@ static bool proj_tiles_fill(mm_args & b, bool & mid, const vx_tensor * w, const 
     b.w_aligned = ((uintptr_t) w->data % 4 == 0) && w->nb[1] % 4 == 0;
     b.x_aligned = ((uintptr_t) x->data % 16 == 0) && x->nb[1] % 16 == 0 && x->nb[2] % 16 == 0 && x->nb[3] % 16 == 0;
     const int64_t nbatch = x->ne[2] * x->ne[3];
-    {   // gemm_mid.hip's kernel, as the separate call would run it (sequences flattened into one token dimension, as the graphs have them)
+    {   // gemm_mid.hip's kernel, wherever the separate call would run on it (sequences flattened into one token dimension or a batch)
         vx_gm_call c;
-        mid = b.x_aligned && nbatch == 1 && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 && mid_fill(c, b, (int) nbatch, WT_Q8);
+        mid = b.x_aligned && nbatch <= 65535 && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 && mid_fill(c, b, (int) nbatch, WT_Q8);
         if (mid) return true;
     }
     // (what launch_gemm_lds asks for before it hands a product to the pre-tiled kernel)
