@@ -105,3 +105,39 @@ def test_groups_equal_their_separate_calls(pkg, gpu, T, B, wtype):
 @pytest.mark.parametrize("T,B,wtype", [(1500, 2, "q8"), (3072, 1, "q8"), (1152, 1, "f16")])
 def test_groups_at_the_last_token_counts(pkg, gpu, T, B, wtype):
     test_groups_equal_their_separate_calls(pkg, gpu, T, B, wtype)
+
+
+@pytest.mark.parametrize("N", [45, 100, 300, 1024])
+def test_kernel_switches_mean_what_they_say(pkg, gpu, monkeypatch, N):
+    """The switches that name another kernel, at shapes of this one: VX_GEMM_LDS=2 rounds q * d once to f16 on the tiled kernels, 0 is the
+    register-operand kernels, VX_GEMM_Q8T chooses between the prefill kernels; a switch set to its default changes nothing."""
+    import torch
+    say(f"kernel switches at N={N}")
+    L, d = pkg.lib(), pkg.desc
+    K, M = 4096, 1024
+    g = rng("mid-switches", N)
+    w = (0.05 * g.standard_normal((M, K))).astype(np.float32)
+    wd = pkg.desc_q8(wq := q8_dev(w)[0], K)
+    x = dev(g.standard_normal((N, K)).astype(np.float32))
+
+    def product(**env):
+        for name in ("VX_GEMM_MID", "VX_GEMM_LDS", "VX_GEMM_Q8T"):
+            monkeypatch.delenv(name, raising=False)
+        for name, value in env.items():
+            monkeypatch.setenv(name, value)
+        out = torch.empty((N, M), dtype=torch.float32, device="cuda")
+        ok(pkg, L.vx_mul_mat(wd, d(x), d(out), pkg.ACT_FLOAT, None), "mul_mat")
+        torch.cuda.synchronize()
+        return out
+
+    plain = product()
+    for name, value in (("VX_GEMM_MID", "1"), ("VX_GEMM_LDS", "1"), ("VX_GEMM_Q8T", "1")):
+        assert same_bits(plain, product(**{name: value})), (name, value)
+    for value in ("0", "2"):
+        assert same_bits(product(VX_GEMM_LDS=value), product(VX_GEMM_LDS=value, VX_GEMM_MID="0")), value
+        if N >= 1024:
+            assert same_bits(product(VX_GEMM_Q8T=value), product(VX_GEMM_Q8T=value, VX_GEMM_MID="0")), value
+    # the folded scale is another rounding of every weight: about 2^-12 of the result away, the sums' order some 2^-22
+    x16, w64 = x.half().double(), torch.from_numpy(dequant(wq.cpu().numpy(), K)).cuda()
+    away = lambda t: float((t.double() - x16 @ w64.T).norm() / (x16 @ w64.T).norm())
+    assert away(plain) < 1e-6 and away(product(VX_GEMM_LDS="2")) > 2e-5

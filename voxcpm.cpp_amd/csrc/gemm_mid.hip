@@ -484,10 +484,11 @@ bool gm_go(int tile, int epi, const gm_args & a, int gx, int gy, int nbatch, hip
 } // namespace
 
 bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch) {
-    const char * e = getenv("VX_GEMM_MID"); // 0: the kernels of mul_mat.hip for these shapes (read on every call: a test compares the two)
-    if (e && atoi(e) == 0) return false;
-    // (VX_GEMM_Q8T, when it is set, decides between the two prefill kernels for every product of 1024 tokens or more)
-    if (N >= 1024 && getenv("VX_GEMM_Q8T")) return false;
+    // Switches, read on every call.  VX_GEMM_MID=0: the kernels of mul_mat.hip for these shapes.  VX_GEMM_LDS other than 1 and, from
+    // 1024 tokens on, VX_GEMM_Q8T other than 1 ask for one of those kernels by name (another rounding of the weights, the older
+    // kernels, one prefill kernel or the other): then it is that kernel that runs.
+    auto is = [](const char * name, int by_default) { const char * e = getenv(name); return e ? atoi(e) : by_default; };
+    if (is("VX_GEMM_MID", 1) == 0 || is("VX_GEMM_LDS", 1) != 1 || (N >= 1024 && is("VX_GEMM_Q8T", 1) != 1)) return false;
     // Up to where this kernel's 64 x 128 tiles, beat the LDS-tiled and pre-tiled
     // kernels' 128 x 128.  Q8_0, 24 layers of one prompt: 1200 tokens 6270 -> 3818 us, 2048 6834 -> 5205, 2600 8990 -> 7156, but
     // 4000 9639 -> 10114; F16, 56 products: 1100 tokens 1343 -> 1260 us, 1537 1417 -> 1463.
