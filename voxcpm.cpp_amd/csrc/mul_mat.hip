@@ -2657,7 +2657,7 @@ extern "C" int vx_supports_mul_mat_swiglu_tiled(const vx_tensor * gate, const vx
     if (up->type != gate->type) return 0;
     for (int i = 0; i < 4; ++i) if (up->ne[i] != gate->ne[i] || up->nb[i] != gate->nb[i]) return 0;
     if (mid_split(gate, up, src1)) return 0;
-    if (src1->ne[1] <= 64 && !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0])) return act_mode == VX_ACT_FLOAT && swiglu_mid_ok(gate, up, src1, nullptr, dst);
+    if (src1->ne[1] <= 64 && !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]) && act_mode == VX_ACT_FLOAT && swiglu_mid_ok(gate, up, src1, nullptr, dst)) return 1;
     // (neither the pair nor one product on its own may be a shape of the streaming kernel: it sums the K blocks in another order)
     return !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]) && !gemv_shape_ok(src1->ne[1], gate->ne[1], gate->ne[0]) &&
            gemm_lds_swiglu_ok(gate, up, src1, dst, act_mode);
@@ -2740,7 +2740,7 @@ static vx_status swiglu_run(const vx_tensor * gate, const vx_tensor * up, const 
     const bool tiled = norm_w ? norm_swiglu_tiled_ok(src1, norm_w, gate, up, dst, act_mode) : vx_supports_mul_mat_swiglu_tiled(gate, up, src1, dst, act_mode) != 0;
     if (!tiled && !vx_supports_mul_mat_swiglu(gate, up, src1, dst))
         return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat_swiglu: two Q8_0/F16 matrices of one layout, a token count the streaming kernel takes "
-                       "(or, with f16 activations, 64 tokens or more for the tiled kernel: vx_supports_mul_mat_swiglu_tiled)");
+                       "(or, with f16 activations, one that a tiled kernel takes: vx_supports_mul_mat_swiglu_tiled)");
     if ((uintptr_t) src1->data % 4 || (uintptr_t) dst->data % 4 || (gate->type == VX_TYPE_F16 && (((uintptr_t) gate->data | (uintptr_t) up->data) % 2)))
         return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat_swiglu: misaligned tensor data");
     mm_args a = {};
