@@ -313,17 +313,16 @@ def test_supports_truth_table_node_groups(pkg):
     assert lib.vx_supports_kv_store_sync(k_src, slot, None, slot, attn, attn) == 0
 
 
-@pytest.mark.parametrize("K,at_63", [(1024, 1), (4096, 1), (128, 0), (1536, 0)])
+@pytest.mark.parametrize("K,at_63", [(1024, 1), (768, 1), (128, 0), (1536, 0)])
 def test_gate_up_pair_around_64_tokens(pkg, monkeypatch, K, at_63):
-    """The pair on the tiled kernels: from 64 tokens on wherever the LDS-tiled kernel walks its K whole (at K = 4096 these tiles have it
-    cut), below that only where gemm_mid.hip's kernel takes it."""
+    """The pair on the tiled kernels: from 64 tokens on at any K of whole 128s that is not cut, below that only where gemm_mid.hip's
+    kernel takes it."""
     tiled = pkg.lib().vx_supports_mul_mat_swiglu_tiled
     w = q8(pkg, [K, 8192, 1, 1])
     ask = lambda n: tiled(w, w, f32(pkg, [K, n, 1, 1]), f32(pkg, [8192, n, 1, 1]), pkg.ACT_FLOAT)
     assert [ask(n) for n in (63, 64, 65)] == [at_63, 1, 1]
     monkeypatch.setenv("VX_GEMM_MID", "0")
-    whole = int(K < 2048)
-    assert [ask(n) for n in (63, 64, 65)] == [0, whole, whole]
+    assert [ask(n) for n in (63, 64, 65)] == [0, 1, 1]
 
 
 def test_ops_validate_before_touching_the_device(pkg):

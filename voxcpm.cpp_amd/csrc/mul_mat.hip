@@ -2975,10 +2975,12 @@ static bool proj_tiles_fill(mm_args & b, bool & mid, const vx_tensor * w, const 
     b.w_aligned = ((uintptr_t) w->data % 4 == 0) && w->nb[1] % 4 == 0;
     b.x_aligned = ((uintptr_t) x->data % 16 == 0) && x->nb[1] % 16 == 0 && x->nb[2] % 16 == 0 && x->nb[3] % 16 == 0;
     const int64_t nbatch = x->ne[2] * x->ne[3];
-    {   // gemm_mid.hip's kernel, wherever the separate call would run on it (sequences flattened into one token dimension or a batch)
+    {   // gemm_mid.hip's kernel, wherever the separate call would run on it: sequences flattened into one token dimension, as the graphs
+        // have them; a batch of sequences runs as the separate calls there
         vx_gm_call c;
-        mid = b.x_aligned && nbatch <= 65535 && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 && mid_fill(c, b, (int) nbatch, WT_Q8);
-        if (mid) return true;
+        const bool alone = nbatch <= 65535 && mid_fill(c, b, (int) nbatch, WT_Q8);
+        mid = alone && nbatch == 1 && b.x_aligned && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0;
+        if (alone) return mid;
     }
     // (what launch_gemm_lds asks for before it hands a product to the pre-tiled kernel)
     if ((uint64_t) b.M * b.nb01 >= (1ull << 32) || (uint64_t) 256 * b.nb11 + 256 >= (1ull << 32) || (uint64_t) 256 * b.nb1 + 1024 >= (1ull << 32) ||
