@@ -450,6 +450,19 @@ def test_row_rotations_reproduce_the_xor_butterfly():
             assert len(set(a.tolist())) == 1   # every lane holds the same total
 
 
+def test_direct_lds_loads_set_m0_themselves():
+    """A direct load into LDS goes where M0 points, and the compiler writes M0 as it likes between two asm statements: every
+    statement with such a load sets it first."""
+    import glob, os, re
+    seen = 0
+    for f in glob.glob(os.path.join(os.path.dirname(__file__), "..", "voxcpm.cpp_amd", "csrc", "*.hip")):
+        for text in re.findall(r"asm volatile\((.*?)\);", open(f).read(), re.S):
+            if "load_lds" in text:
+                seen += 1
+                assert 0 <= text.find("s_mov_b32 m0") < text.find("load_lds"), (f, text)
+    assert seen >= 5
+
+
 def test_hot_kernels_do_not_spill():
     """The build keeps every kernel's resource remarks beside its object file.  The kernels on the timed paths must not
     use scratch memory: a few spilled registers cost the 128 x 128 GEMM tile a quarter of its speed once, and no parity

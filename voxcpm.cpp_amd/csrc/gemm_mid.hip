@@ -46,6 +46,20 @@ struct gm_args {
 
 enum { GM_PLAIN = 0, GM_SWIGLU = 1, GM_SEGS = 2 };
 
+// N consecutive 1 KB tiles from global memory (uniform base + lane offset) into LDS at lds + 16 lane: one statement, since the
+// compiler may write M0 between two
+template <int N> __device__ __forceinline__ void gm_dma_tiles(uint32_t off, const char * base, uint32_t lds) {
+    static_assert(N == 1 || N == 2 || N == 4, "instances of gm_kernel");
+    if constexpr (N == 1)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+    else if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(off), "s"(base), "s"(lds)
+                     : "memory");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %0, %1 offset:2048\n\tglobal_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(off), "s"(base), "s"(lds) : "memory");
+}
+
 template <int N> __device__ __forceinline__ void gm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
 
 template <int WT, int MT, int NT, int RW, int KG, int CH, int S>
@@ -142,12 +156,8 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
                 for (int kb = 0; kb < 4 * CH; ++kb) { // NT consecutive tiles of a k block (past the last token tile: the next block's, dropped at the store)
                     const char * p = xsrc + (int64_t) (st * 4 * CH + kb) * a.n_tt * 1024;
 #pragma unroll
-                    for (int t0 = 0; t0 < NT; t0 += 4) {
-                        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(loff), "s"(p + t0 * 1024), "s"(base + (uint32_t) (kb * NT + t0) * 1024) : "memory");
-                        if (t0 + 1 < NT) asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(loff), "s"(p + t0 * 1024) : "memory");
-                        if (t0 + 2 < NT) asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(loff), "s"(p + t0 * 1024) : "memory");
-                        if (t0 + 3 < NT) asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(loff), "s"(p + t0 * 1024) : "memory");
-                    }
+                    for (int t0 = 0; t0 < NT; t0 += 4)
+                        gm_dma_tiles<(NT < 4 ? NT : 4)>(loff, p + t0 * 1024, base + (uint32_t) (kb * NT + t0) * 1024);
                 }
             };
             constexpr int L = sh::XINST;
