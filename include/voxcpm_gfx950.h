@@ -73,11 +73,13 @@ VX_API vx_status    vx_memset(void * dst, int value, size_t bytes, vx_stream str
 VX_API vx_status    vx_stream_create(vx_stream * stream);
 VX_API vx_status    vx_stream_destroy(vx_stream stream);
 VX_API vx_status    vx_stream_synchronize(vx_stream stream);
-/* The per-stream workspace (split-KV partials, split-K partials, block sums, mask classification).  It grows on
+/* The per-stream workspace (split-KV partials, split-K partials, block sums, mask classification, activation tiles and what
+ * one call hands from launch to launch).  It grows on
  * demand; a block that was handed out keeps its address and stays allocated until vx_stream_destroy, also after a
  * larger block has replaced it, so launches already queued and HIP graphs already captured from the stream stay
  * valid.  A call that would have to grow the workspace while the stream is being captured returns
- * VX_ERR_UNSUPPORTED: reserve the largest size first.  No counterpart in the reference (ggml-cpu takes its scratch
+ * VX_ERR_UNSUPPORTED: reserve the largest size first.  (Products of 17 to 3072 tokens and the calls built on them -- the kernel
+ * of gemm_mid.hip -- allocate beside the capture instead: a graph that begins with one needs no reservation.)  No counterpart in the reference (ggml-cpu takes its scratch
  * from the compute plan's work buffer, ggml/src/ggml-cpu/ggml-cpu.c:2700-2935). */
 VX_API vx_status    vx_workspace_reserve(vx_stream stream, size_t bytes);
 /* current block, its size and the number of superseded blocks still held for this stream (any out pointer may be NULL) */

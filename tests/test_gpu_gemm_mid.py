@@ -1,5 +1,7 @@
 """GPU: the product kernel for 17 to 3072 tokens (F16 weights: 1152) (csrc/gemm_mid.hip) at the edges of its tiles -- ragged token and row tiles,
 the shortest and longest K it takes, a batch, both weight types -- and the groups built on it against their separate calls."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -141,3 +143,43 @@ def test_kernel_switches_mean_what_they_say(pkg, gpu, monkeypatch, N):
     x16, w64 = x.half().double(), torch.from_numpy(dequant(wq.cpu().numpy(), K)).cuda()
     away = lambda t: float((t.double() - x16 @ w64.T).norm() / (x16 @ w64.T).norm())
     assert away(plain) < 1e-6 and away(product(VX_GEMM_LDS="2")) > 2e-5
+
+
+@pytest.mark.parametrize("K,M,N,wtype", [(1024, 1024, 45, "q8"), (1024, 1024, 1100, "q8"), (1024, 4096, 1100, "f16")])
+def test_first_call_of_a_stream_under_capture(pkg, gpu, K, M, N, wtype):
+    """Products whose other kernels use no scratch memory: a graph may begin with one on a stream that never ran anything, and so may
+    the gate/up pair.  Replayed with direct calls of another size (the workspace grows) between the replays."""
+    import torch
+    say(f"capture without a reservation K={K} M={M} N={N} weights={wtype}")
+    L, d = pkg.lib(), pkg.desc
+    g = rng("mid-capture", K, M, N)
+    keep = []
+
+    def weight():
+        w = (0.05 * g.standard_normal((M, K))).astype(np.float32)
+        keep.append(q8_dev(w)[0] if wtype == "q8" else dev(w.astype(np.float16)))
+        return pkg.desc_q8(keep[-1], K) if wtype == "q8" else d(keep[-1])
+
+    w, up = weight(), weight()
+    x, big = (dev(g.standard_normal((n, K)).astype(np.float32)) for n in (N, 1152))
+    want, want2, out, out2, other = (torch.zeros(n, M, device="cuda") for n in (N, N, N, N, 1152))
+    ok(pkg, L.vx_mul_mat(w, d(x), d(want), pkg.ACT_FLOAT, None), "direct")
+    ok(pkg, L.vx_mul_mat_swiglu(w, up, d(x), d(want2), pkg.ACT_FLOAT, None), "direct pair")
+    torch.cuda.synchronize()
+    s = C.c_void_p()        # (a stream of its own: torch's come from a pool and may have a workspace already)
+    ok(pkg, L.vx_stream_create(C.byref(s)), "stream")
+    ok(pkg, L.vx_graph_begin(s), "begin")
+    rc = L.vx_mul_mat(w, d(x), d(out), pkg.ACT_FLOAT, s), L.vx_mul_mat_swiglu(w, up, d(x), d(out2), pkg.ACT_FLOAT, s)
+    graph = C.c_void_p()
+    ok(pkg, L.vx_graph_end(s, C.byref(graph)), "end")
+    assert rc == (0, 0) and graph.value
+    for _ in range(3):
+        out.zero_(), out2.zero_()
+        torch.cuda.synchronize()
+        ok(pkg, L.vx_graph_launch(graph, s), "replay")
+        ok(pkg, L.vx_stream_synchronize(s), "sync")
+        assert same_bits(out, want) and same_bits(out2, want2)
+        ok(pkg, L.vx_mul_mat(w, d(big), d(other), pkg.ACT_FLOAT, s), "direct call between")
+        ok(pkg, L.vx_stream_synchronize(s), "sync")
+    ok(pkg, L.vx_graph_destroy(graph), "graph")
+    ok(pkg, L.vx_stream_destroy(s), "stream")

@@ -1287,7 +1287,7 @@ extern "C" vx_status vx_flash_attn_ext_store_proj(const vx_tensor * q, const vx_
         vx_tensor out = *attn;
         const size_t out_bytes = ((size_t) vx_nelements(attn) * 4 + 255) & ~(size_t) 255;
         void * ws = nullptr; // one block for both phases, as below
-        vx_status rc = vx_workspace((hipStream_t) stream, PF_STORE_FRONT + out_bytes + vx_proj_add_bytes(w_o, attn), &ws);
+        vx_status rc = vx_workspace((hipStream_t) stream, PF_STORE_FRONT + out_bytes + vx_proj_add_bytes(w_o, attn), &ws, true);
         if (rc != VX_OK) return rc;
         out.data = (char *) ws + PF_STORE_FRONT;
         const vx_tensor ao = pf_attn_shape(q, &out);

@@ -541,7 +541,7 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
     const size_t xt_bytes = c.tile_in ? 0 : vx_gm_tile_bytes(c.K, c.N, nbatch), tab_bytes = rotate ? (size_t) c.N * 32 * sizeof(float2) : 0;
     void * ws = nullptr;
     if (xt_bytes + tab_bytes) {
-        const vx_status rc = vx_workspace(st, c.ws_offset + xt_bytes + tab_bytes, &ws);
+        const vx_status rc = vx_workspace(st, c.ws_offset + xt_bytes + tab_bytes, &ws, true);
         if (rc != VX_OK) return rc;
     }
     char * base = (char *) ws + c.ws_offset;

@@ -2932,7 +2932,7 @@ extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w,
     void * ws = nullptr;
     (void) take_ws_status();
     if (mid) { // one request for all the group needs: its pieces lie in one block, also when it grows
-        const vx_status rc = vx_workspace(st, tiles + vx_gm_tile_bytes(a.K, a.N, nbatch), &ws);
+        const vx_status rc = vx_workspace(st, tiles + vx_gm_tile_bytes(a.K, a.N, nbatch), &ws, true);
         if (rc != VX_OK) return rc;
         const int wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
         a.ws_offset = tiles; a.tile_out = ws; a.tile_tt = tile_tt;

@@ -64,8 +64,9 @@ inline void vx_launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_by
 
 // per-stream scratch memory, grown on demand.  A block stays allocated at its address until the stream is
 // destroyed, also after a larger one has replaced it (ws_policy.hpp), so launches already queued and graphs
-// already captured keep valid arguments; growth during a stream capture is refused.
-vx_status vx_workspace(hipStream_t stream, size_t bytes, void ** ptr);
+// already captured keep valid arguments; growth during a stream capture is refused, except where a call says in_capture:
+// the products of gemm_mid.hip, whose shapes ran on kernels without scratch memory before that one took them over.
+vx_status vx_workspace(hipStream_t stream, size_t bytes, void ** ptr, bool in_capture = false);
 
 // Copies derived from pinned weights (vx_weights_pin), kept from call to call.  vx_derived_get returns the copy for `key`
 // (the calling stream is made to wait for the kernel that filled it, if that ran on another stream), or a new block of

@@ -227,21 +227,27 @@ vx_status vx_fail(vx_status st, const char * fmt, ...) {
     return st;
 }
 
-vx_status vx_workspace(hipStream_t stream, size_t bytes, void ** ptr) {
+vx_status vx_workspace(hipStream_t stream, size_t bytes, void ** ptr, bool in_capture) {
     int dev = 0;
     VX_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     vx_ws_state & ws = g_ws[ws_key(dev, stream)];
-    bool capturing = false;
+    bool captured = false;
     if (bytes > ws.cur.bytes) { // only a growing request needs to know
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &cs) != hipSuccess) (void) hipGetLastError();
-        capturing = cs != hipStreamCaptureStatusNone;
+        captured = cs != hipStreamCaptureStatusNone;
     }
     hipError_t err = hipSuccess;
-    const vx_ws_result r = vx_ws_request(ws, bytes, capturing, [&](size_t want) -> void * {
+    const vx_ws_result r = vx_ws_request(ws, bytes, captured && !in_capture, [&](size_t want) -> void * {
         void * p = nullptr;
-        err      = hipMalloc(&p, want);
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed; // (this thread's own allocation, no part of any capture)
+        if (captured) err = hipThreadExchangeStreamCaptureMode(&mode);
+        if (err == hipSuccess) {
+            err = hipMalloc(&p, want);
+            if (captured) (void) hipThreadExchangeStreamCaptureMode(&mode);
+        }
+        if (err != hipSuccess) (void) hipGetLastError();
         return err == hipSuccess ? p : nullptr;
     }, ptr);
     if (r == VX_WS_CAPTURING)

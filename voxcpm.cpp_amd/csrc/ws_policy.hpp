@@ -7,7 +7,8 @@
 // allocates a new block and retires the old one; retired blocks are released when the stream is destroyed.
 // Each growth at least doubles the block, so all retired blocks together are smaller than the live one.
 // Growth while the stream is being captured is refused (an allocation must not be recorded into a graph):
-// reserve the largest size before capturing.
+// reserve the largest size before capturing.  A caller that allocates beside the capture (hipMalloc with the thread's capture
+// mode relaxed, which records nothing) asks with capturing = false.
 #pragma once
 
 #include <cstddef>
