@@ -444,19 +444,22 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
 }
 
 // ---- tile choice -----------------------------------------------------------------------------------------------------
-// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages); what a work-group costs, measured: microseconds
-// per 128 of K and fixed, and how many of them a compute unit holds
+// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages); what a work-group costs, measured with Q8_0 weights:
+// microseconds per 128 of K and fixed
 #define GM_TILES(X) \
-    X(0, 1, 1, 1, 2, 3, 0.127f, 0.95f, 4) \
-    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f, 2) \
-    X(2, 2, 2, 1, 2, 3, 0.190f, 1.40f, 2) \
-    X(3, 2, 4, 1, 1, 3, 0.276f, 1.30f, 2) \
-    X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f, 2) \
-    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f, 1)
+    X(0, 1, 1, 1, 2, 3, 0.127f, 0.95f) \
+    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f) \
+    X(2, 2, 2, 1, 2, 3, 0.190f, 1.40f) \
+    X(3, 2, 4, 1, 1, 3, 0.276f, 1.30f) \
+    X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
+    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f)
 constexpr int GM_N_TILES = 6;
-struct gm_tile { int rows, toks, mt; float per_step, fixed; int per_cu; };
+// lone: a compute unit's LDS holds one work-group (F16 rows are twice the bytes: more of the tiles)
+struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2]; };
 const gm_tile gm_tiles[GM_N_TILES] = {
-#define X(I, MT, NT, RW, CH, S, A_, B_, OCC) { 16 * MT * RW, 16 * NT, MT, A_, B_, OCC },
+#define X(I, MT, NT, RW, CH, S, A_, B_)                                                          \
+    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, 4, CH, S>::LDS > 160 * 1024, \
+                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, 4, CH, S>::LDS > 160 * 1024 } },
     GM_TILES(X)
 #undef X
 };
@@ -477,7 +480,7 @@ bool gm_launch(const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
 template <int WT>
 bool gm_go(int tile, int epi, const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
     switch (tile) {
-#define X(I, MT, NT, RW, CH, S, A_, B_, OCC)                                                                              \
+#define X(I, MT, NT, RW, CH, S, A_, B_)                                                                                   \
         case I:                                                                                                         \
             if (epi == GM_PLAIN) return gm_launch<WT, MT, NT, RW, CH, S, GM_PLAIN>(a, gx, gy, nbatch, st);              \
             if constexpr (MT % 2 == 0) {                                                                                \
@@ -578,7 +581,7 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
         const float one = g.fixed + g.per_step * (float) (c.K / 128);
         // (work-groups that share a compute unit share its vector units: the fixed part of one hides behind the other's products)
         const float per_cu = (float) ((wgs + 255) / 256);
-        const float us = per_cu <= 1.0f ? one : g.per_cu == 1 ? per_cu * one : one + (per_cu - 1.0f) * (g.per_step * (float) (c.K / 128) + 0.3f * g.fixed);
+        const float us = per_cu <= 1.0f ? one : g.lone[c.wtype] ? per_cu * one : one + (per_cu - 1.0f) * (g.per_step * (float) (c.K / 128) + 0.3f * g.fixed);
         if (best < 0 || us < best_us) { best = t; best_us = us; }
     }
     const gm_tile & g = gm_tiles[best];
