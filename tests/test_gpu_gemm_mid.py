@@ -183,3 +183,36 @@ def test_first_call_of_a_stream_under_capture(pkg, gpu, K, M, N, wtype):
         ok(pkg, L.vx_stream_synchronize(s), "sync")
     ok(pkg, L.vx_graph_destroy(graph), "graph")
     ok(pkg, L.vx_stream_destroy(s), "stream")
+
+
+@pytest.mark.parametrize("M,last,wtype", [(1024, 192, "q8"), (4096, 48, "q8"), (1024, 64, "f16"), (128, 1024, "f16")])
+def test_small_products_keep_the_streaming_kernel(pkg, gpu, monkeypatch, M, last, wtype):
+    """Where both kernels give the same bits the streaming one runs up to `last` tokens: it needs no scratch memory, so a stream that
+    never ran anything else still has none.  The two sides of the line against the streaming kernel alone."""
+    import torch
+    say(f"streaming kernel up to {last} tokens x {M} rows, weights={wtype}")
+    L, d = pkg.lib(), pkg.desc
+    K = 1024
+    g = rng("mid-small", M, last)
+    w = (0.05 * g.standard_normal((M, K))).astype(np.float32)
+    wg = q8_dev(w)[0] if wtype == "q8" else dev(w.astype(np.float16))
+    wd = pkg.desc_q8(wg, K) if wtype == "q8" else d(wg)
+    for N in (17, last, last + 1):
+        x, res = dev(g.standard_normal((N, K)).astype(np.float32)), dev(g.standard_normal((N, M)).astype(np.float32))
+        out, upd, old, old_upd = (torch.empty(N, M, device="cuda") for _ in range(4))
+        torch.cuda.synchronize()
+        s, ptr, size = C.c_void_p(), C.c_void_p(), C.c_size_t()
+        ok(pkg, L.vx_stream_create(C.byref(s)), "stream")
+        ok(pkg, L.vx_mul_mat(wd, d(x), d(out), pkg.ACT_FLOAT, s), "mul_mat")
+        ok(pkg, L.vx_mul_mat_scale_add(wd, d(x), d(res), d(upd), 0.7, pkg.ACT_FLOAT, s), "mul_mat_scale_add")
+        ok(pkg, L.vx_stream_synchronize(s), "sync")
+        ok(pkg, L.vx_workspace_info(s, C.byref(ptr), C.byref(size), None), "info")
+        assert (size.value == 0) == (N <= last), (N, size.value)
+        ok(pkg, L.vx_stream_destroy(s), "stream")
+        with monkeypatch.context() as m:
+            m.setenv("VX_GEMM_MID", "0")
+            if M * N <= 256 * 1024 or (M <= 1024 and N <= 448):     # (what the streaming kernel takes at all)
+                ok(pkg, L.vx_mul_mat(wd, d(x), d(old), pkg.ACT_FLOAT, None), "streaming")
+                ok(pkg, L.vx_mul_mat_scale_add(wd, d(x), d(res), d(old_upd), 0.7, pkg.ACT_FLOAT, None), "streaming")
+                torch.cuda.synchronize()
+                assert same_bits(out, old) and same_bits(upd, old_upd), N

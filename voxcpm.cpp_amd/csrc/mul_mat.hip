@@ -2524,10 +2524,32 @@ bool launch_mid(const mm_args & a, int nbatch, int wt, hipStream_t st) {
     return true;
 }
 
+// Products (and k + v, q + k + v without a norm) that both this file's streaming kernel and gemm_mid.hip's take, with the same
+// bits: the streaming kernel needs no activation pass in front and wins while tokens x rows is small.  K = 1024, graphs of a
+// dozen products, streaming / the other, microseconds: Q8_0 1024 rows x 45 tokens 4.7 / 6.0, x 160 6.3 / 7.6, x 203 8.6 / 7.8;
+// 128 x 448 4.6 / 6.9; 4096 x 45 6.3 / 7.9, x 64 9.3 / 7.8; k + v and a rotation x 512 0.96 of the other's time, x 800 1.43.
+// F16 1024 x 64 5.8 / 6.4, x 80 6.8 / 6.7; 128 x 1000 7.5 / 8.8, x 1152 10.5 / 9.3.  With a norm the activation pass pays at
+// every count (it is formed once instead of by every work-group), and so it does for a gate/up pair.
+bool stream_first(const mm_args & a, int nbatch, int wt) {
+    if (a.w2 || a.norm_w || a.tile_in || a.N <= 16 || a.K > 1024) return false;
+    const int64_t work = a.M * a.N * nbatch;
+    if (wt == WT_Q8) return work * a.K <= 192 * 1024 * 1024;
+    int64_t rows = a.nseg > 0 ? 0 : a.M;
+    for (int i = 0; i < a.nseg; ++i) rows = rows > a.seg[i].M ? rows : a.seg[i].M;
+    return work <= (rows <= 128 ? 128 : 64) * 1024;
+}
+
+// whichever of the two takes the call (the streaming kernel needs every matrix to be its shape)
+template <int WT, bool ACT_Q8>
+bool launch_stream_or_mid(const mm_args & a, int nbatch, hipStream_t st) {
+    if constexpr (ACT_Q8) return launch_gemv<WT, true>(a, nbatch, st);
+    else if (stream_first(a, nbatch, WT)) return launch_gemv<WT, false>(a, nbatch, st) || launch_mid(a, nbatch, WT, st);
+    else return launch_mid(a, nbatch, WT, st) || launch_gemv<WT, false>(a, nbatch, st);
+}
+
 template <int WT, bool ACT_Q8>
 void launch(const mm_args & a, int nbatch, hipStream_t st) {
-    if constexpr (WT != WT_F32 && !ACT_Q8) { if (launch_mid(a, nbatch, WT, st)) return; }
-    if constexpr (WT != WT_F32) { if (launch_gemv<WT, ACT_Q8>(a, nbatch, st)) return; }
+    if constexpr (WT != WT_F32) { if (launch_stream_or_mid<WT, ACT_Q8>(a, nbatch, st)) return; }
     if constexpr (WT != WT_F32 && !ACT_Q8) { if (launch_gemm_lds<WT>(a, nbatch, st) || ws_failed()) return; }
     if constexpr (WT != WT_F32) { if (launch_gemm128<WT, ACT_Q8>(a, nbatch, st)) return; }
     if (a.N <= 16) {
@@ -2811,13 +2833,9 @@ extern "C" vx_status vx_mul_mat_scale_add(const vx_tensor * src0, const vx_tenso
     hipStream_t st = (hipStream_t) stream;
     bool ok = false;
     (void) take_ws_status();
-    if (src0->type == VX_TYPE_F16 || act_mode == VX_ACT_FLOAT) {
-        ok = launch_mid(a, nbatch, src0->type == VX_TYPE_F16 ? WT_F16 : WT_Q8, st);
-        if (ws_failed()) return take_ws_status();
-    }
-    if (ok) {}
-    else if (src0->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
-    else                                 ok = launch_gemv<WT_F16, false>(a, nbatch, st);
+    if (src0->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_stream_or_mid<WT_Q8, true>(a, nbatch, st) : launch_stream_or_mid<WT_Q8, false>(a, nbatch, st);
+    else                            ok = launch_stream_or_mid<WT_F16, false>(a, nbatch, st);
+    if (ws_failed()) return take_ws_status();
     if (!ok) { // not the streaming kernel's shape: the tiled kernels with K cut (see vx_supports_mul_mat_scale_add)
         if (src0->type == VX_TYPE_Q8_0) {
             if (act_mode == VX_ACT_Q8) ok = launch_mm_cut<WT_Q8, true>(a, nbatch, st);
@@ -3253,9 +3271,8 @@ extern "C" vx_status vx_kv_proj_rope(const vx_tensor * wk, const vx_tensor * wv,
     hipStream_t st = (hipStream_t) stream;
     bool ok;
     (void) take_ws_status();
-    if ((act_mode == VX_ACT_FLOAT || wk->type == VX_TYPE_F16) && launch_mid(a, nbatch, wk->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16, st)) ok = true;
-    else if (wk->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
-    else                          ok = launch_gemv<WT_F16, false>(a, nbatch, st);
+    if (wk->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_stream_or_mid<WT_Q8, true>(a, nbatch, st) : launch_stream_or_mid<WT_Q8, false>(a, nbatch, st);
+    else                          ok = launch_stream_or_mid<WT_F16, false>(a, nbatch, st);
     if (ws_failed()) return take_ws_status();
     if (!ok) return vx_fail(VX_ERR_UNSUPPORTED, "kv_proj_rope: shape outside the streaming kernel");
     VX_LAUNCH_CHECK();
@@ -3371,9 +3388,8 @@ static vx_status qkv_run(const vx_tensor * norm_w, float eps, const vx_tensor * 
     hipStream_t st = (hipStream_t) stream;
     bool ok;
     (void) take_ws_status();
-    if ((act_mode == VX_ACT_FLOAT || wq->type == VX_TYPE_F16) && launch_mid(a, nbatch, wq->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16, st)) ok = true;
-    else if (wq->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_gemv<WT_Q8, true>(a, nbatch, st) : launch_gemv<WT_Q8, false>(a, nbatch, st);
-    else                          ok = launch_gemv<WT_F16, false>(a, nbatch, st);
+    if (wq->type == VX_TYPE_Q8_0) ok = act_mode == VX_ACT_Q8 ? launch_stream_or_mid<WT_Q8, true>(a, nbatch, st) : launch_stream_or_mid<WT_Q8, false>(a, nbatch, st);
+    else                          ok = launch_stream_or_mid<WT_F16, false>(a, nbatch, st);
     if (ws_failed()) return take_ws_status();
     if (!ok) return vx_fail(VX_ERR_UNSUPPORTED, "qkv_proj_rope: shape outside the streaming kernel");
     VX_LAUNCH_CHECK();
