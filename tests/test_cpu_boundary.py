@@ -237,6 +237,8 @@ def test_supports_truth_table_node_groups(pkg):
     assert order(K, 2, 1024) == order(K, 16, 4096) == 8 and order(K, 17, 4096) == 4 and order(K, 112, 1024) == 4 and order(K, 14, 1024) == 16
     assert order(4096, 2, 1024) == order(4096, 112, 1024) == 16
     assert order(K, 0, 1024) == 0 and order(33, 2, 1024) == 0
+    assert order(K, 300, 8192) == order(K, 300, 4096) and order(K, 2048, 4096) == order(K, 2048, 1024)
+    assert order(K, 2048, 8192) != order(K, 2048, 4096) and order(4096, 600, 128) != order(4096, 600, 1024)   # rows that gemm_mid.hip leaves
     # gate / up / SwiGLU: both matrices count as rows
     wg = q8(pkg, [K, 4096, 1, 1])
     ffn = lambda n: f32(pkg, [4096, n, 1, 1])

@@ -216,3 +216,36 @@ def test_small_products_keep_the_streaming_kernel(pkg, gpu, monkeypatch, M, last
                 ok(pkg, L.vx_mul_mat_scale_add(wd, d(x), d(res), d(old_upd), 0.7, pkg.ACT_FLOAT, None), "streaming")
                 torch.cuda.synchronize()
                 assert same_bits(out, old) and same_bits(upd, old_upd), N
+
+
+@pytest.mark.parametrize("K,M,N,wtype", [(1024, 8192, 2048, "q8"), (1024, 16384, 400, "q8"), (4096, 11264, 1024, "q8"), (4096, 128, 600, "q8"),
+                                         (8192, 200, 45, "q8"), (1024, 50000, 97, "q8"), (1024, 8200, 500, "f16")])
+def test_rows_that_other_kernels_serve(pkg, gpu, monkeypatch, K, M, N, wtype):
+    """Wide matrices at many tokens and few rows with a long K: the kernels behind VX_GEMM_MID=0, alone and (where it is one call) as a pair."""
+    import torch
+    say(f"rows outside the mid-size kernel K={K} M={M} N={N} weights={wtype}")
+    L, d = pkg.lib(), pkg.desc
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+
+    def weight():
+        if wtype == "f16":
+            w = (0.05 * torch.randn(M, K, generator=gen, device="cuda")).half()
+            return w, d(w)
+        w = torch.randint(0, 256, (M, K // 32, 34), generator=gen, device="cuda", dtype=torch.uint8)
+        w[:, :, :2] = torch.tensor([0, 0x10], dtype=torch.uint8, device="cuda")     # scales of 2^-11
+        w = w.view(M, -1)
+        return w, pkg.desc_q8(w, K)
+
+    (w, wd), (u, ud) = weight(), weight()
+    x = torch.randn(N, K, generator=gen, device="cuda")
+    outs = []
+    for mid in (None, "0"):
+        if mid:
+            monkeypatch.setenv("VX_GEMM_MID", mid)
+        out, pair = torch.full((N, M), 5.0, device="cuda"), torch.full((N, M), 5.0, device="cuda")
+        ok(pkg, L.vx_mul_mat(wd, d(x), d(out), pkg.ACT_FLOAT, None), "mul_mat")
+        if L.vx_supports_mul_mat_swiglu_tiled(wd, ud, d(x), d(pair), pkg.ACT_FLOAT):
+            ok(pkg, L.vx_mul_mat_swiglu(wd, ud, d(x), d(pair), pkg.ACT_FLOAT, None), "pair")
+        torch.cuda.synchronize()
+        outs.append((out, pair))
+    assert same_bits(outs[0][0], outs[1][0]) and same_bits(outs[0][1], outs[1][1])

@@ -496,26 +496,43 @@ bool gm_go(int tile, int epi, const gm_args & a, int gx, int gy, int nbatch, hip
 
 } // namespace
 
-bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch) {
+// Rows of a matrix that the kernels of mul_mat.hip serve better (`tokens` of the whole call; a gate/up pair goes by one matrix's rows).
+// Measured with graphs of several weights and, for the pre-tiled kernel, pinned ones; these / here, microseconds:
+//   * over 6144 rows and from 1024 tokens on, where the pre-tiled kernel fills the chip with the pair's 256 x 128 tiles: K 4096, pairs of
+//     11264 rows x 1024 tokens 215 / 294, 14336 x 2048 499 / 739; 16384 rows x 2048 299 / 421 (8192 x 1024: 121 / 108);
+//   * over 6144 rows with K up to 1024, where the 128 x 128 tiles of the LDS-tiled kernel fill it: Q8_0 16384 rows x 300 tokens 32 / 30,
+//     x 512 37 / 43; F16 16384 x 200 23.7 / 25.0, x 448 32 / 44, 8192 x 200 17.6 / 14.9, x 337 17.5 / 20.8, x 800 31 / 40;
+//   * a vocabulary's 73448 rows: K 1024 x 64 tokens 1.4 of the time here, x 100 0.96, x 512 0.84, K 4096 x 100 1.3, x 300 0.93;
+//   * few rows and a long K, which those kernels cut across work-groups: K 4096, 128 rows x 300 tokens 1.33, x 512 0.91, x 2048 0.77;
+//     K 8192, 128 rows x 45 0.97, x 512 0.74.
+static bool gm_rows_ok(int wtype, int64_t K, int64_t tokens, int64_t M) {
+    if (M <= 256 && (K >= 8192 || (K >= 4096 && tokens >= 512))) return false;
+    if (M <= 6144) return true;
+    if (M > 49152 && tokens > 96) return false;
+    const int64_t tiles = (M + 255) / 256 * ((tokens + 127) / 128);
+    if (wtype == VX_GM_Q8 && tokens >= 1024 && tiles >= 320 && tiles * K >= 512 * 1024) return false;
+    return K > 1024 || M * tokens <= (wtype == VX_GM_Q8 ? 5120 : 2560) * 1024;
+}
+
+bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M) {
     // Switches, read on every call.  VX_GEMM_MID=0: the kernels of mul_mat.hip for these shapes.  VX_GEMM_LDS other than 1 and, from
     // 1024 tokens on, VX_GEMM_Q8T other than 1 ask for one of those kernels by name (another rounding of the weights, the older
     // kernels, one prefill kernel or the other): then it is that kernel that runs.
     auto is = [](const char * name, int by_default) { const char * e = getenv(name); return e ? atoi(e) : by_default; };
     if (is("VX_GEMM_MID", 1) == 0 || is("VX_GEMM_LDS", 1) != 1 || (N >= 1024 && is("VX_GEMM_Q8T", 1) != 1)) return false;
-    // Up to where this kernel's 64 x 128 tiles, beat the LDS-tiled and pre-tiled
-    // kernels' 128 x 128.  Q8_0, 24 layers of one prompt: 1200 tokens 6270 -> 3818 us, 2048 6834 -> 5205, 2600 8990 -> 7156, but
+    // Up to where this kernel's 64 x 128 tiles beat the LDS-tiled and pre-tiled kernels' larger ones in a layer of 1024 / 4096 rows.  Q8_0, 24 layers of one prompt: 1200 tokens 6270 -> 3818 us, 2048 6834 -> 5205, 2600 8990 -> 7156, but
     // 4000 9639 -> 10114; F16, 56 products: 1100 tokens 1343 -> 1260 us, 1537 1417 -> 1463.
     if (N <= 16 || N * nbatch > (wtype == VX_GM_Q8 ? 3072 : 1152) || nbatch > 65535) return false;
     // K of whole 256s (the stages).  Up to 16 tokens are the streaming kernel's; what it takes beyond them with K of 513 to
     // 1024 it sums in this kernel's order, and with K above 2048 it takes nothing beyond them: elsewhere a call that one of
     // the two had to decline (alignment, VX_ACT_Q8's groups) would differ from its neighbours in the last bit.
-    return K % 256 == 0 && ((K > 512 && K <= 1024) || (K > 2048 && K <= 16384));
+    return K % 256 == 0 && ((K > 512 && K <= 1024) || (K > 2048 && K <= 16384)) && gm_rows_ok(wtype, K, N * nbatch, M);
 }
 
 bool vx_gm_takes(const vx_gm_call & c) {
-    if (!vx_gm_region(c.wtype, c.K, c.N, (int64_t) c.ne12 * c.ne13)) return false;
     auto al16 = [](const void * p, uint64_t s) { return (uintptr_t) p % 16 == 0 && s % 16 == 0; };
     for (int i = 0; i < c.nmat; ++i) {
+        if (!vx_gm_region(c.wtype, c.K, c.N, (int64_t) c.ne12 * c.ne13, c.mat[i].M)) return false;
         if (!al16(c.mat[i].w, c.mat[i].nb01) || c.mat[i].M < 1) return false;
         if (c.nmat > 1 && c.mat[i].M % 64) return false;
     }

@@ -41,9 +41,10 @@ struct vx_gm_call {
     size_t        ws_offset;      // bytes at the start of the stream's workspace that the caller keeps
 };
 
-// The region of K and token counts this kernel serves for a weight type.  It does not depend on the number of rows, so that
-// a product and every group it is part of are formed by the same kernel, in the same order of every sum.
-bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch);
+// Whether this kernel serves a product of M rows, K columns and N * nbatch tokens.  The rows of one matrix decide, for a gate/up pair
+// as for gate or up alone, and a group of several matrices needs the answer for each: a product and every group it is part of
+// are formed by the same kernel, in the same order of every sum.
+bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M);
 // region, and operands on the boundaries its loads need (dst only needs 4-byte aligned values)
 bool vx_gm_takes(const vx_gm_call & c);
 size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch); // f16 activation tiles of a product

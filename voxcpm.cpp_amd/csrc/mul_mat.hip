@@ -2635,7 +2635,7 @@ extern "C" vx_status vx_mul_mat(const vx_tensor * src0, const vx_tensor * src1, 
 // gemm_mid.hip's kernel serves gate and up alone as well as the pair, but each only on 16-byte boundaries: a pair of which one
 // matrix is on such a boundary and the other is not would be summed in another order than the two products by themselves.
 static bool mid_split(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1) {
-    return vx_gm_region(gate->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, gate->ne[0], src1->ne[1], src1->ne[2] * src1->ne[3]) &&
+    return vx_gm_region(gate->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, gate->ne[0], src1->ne[1], src1->ne[2] * src1->ne[3], gate->ne[1]) &&
            ((uintptr_t) gate->data % 16 == 0) != ((uintptr_t) up->data % 16 == 0);
 }
 
@@ -3120,7 +3120,11 @@ extern "C" int vx_supports_qkv_proj_rope(const vx_tensor * wq, const vx_tensor *
 // qkv_proj / gate_up_proj) compares the two before promising identical bits.
 extern "C" int vx_mul_mat_sum_order(int64_t K, int64_t tokens, int64_t M) {
     if (K < 32 || K % 32 || tokens < 1 || M < 1) return 0;
-    return gemv_waves_for(K, tokens, M);
+    // (shapes of gemm_mid.hip's kernel but for their rows, with either weight type: another kernel's order)
+    int by_rows = 0;
+    for (int wt : { VX_GM_Q8, VX_GM_F16 })
+        if (vx_gm_region(wt, K, tokens, 1, 1024) && !vx_gm_region(wt, K, tokens, 1, M)) by_rows |= 64 << wt;
+    return gemv_waves_for(K, tokens, M) + by_rows;
 }
 
 static vx_status qkv_run(const vx_tensor * norm_w, float eps, const vx_tensor * wq, const vx_tensor * wk, const vx_tensor * wv,
@@ -3152,7 +3156,10 @@ static bool qkv_tiled_fill(mm_args & a, bool & mid, const vx_tensor * norm_w, fl
     a.w_aligned = 1;
     a.nseg = 3;
     const int nbatch = (int) x->ne[3];
-    const bool mid_ok = vx_gm_region(wq->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, a.K, a.N, nbatch);
+    int in_mid = 0; // matrices of gemm_mid.hip's kernel: all three, or none
+    for (const vx_tensor * w : ws) in_mid += vx_gm_region(wq->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, a.K, a.N, nbatch, w->ne[1]);
+    if (in_mid != 0 && in_mid != 3) return false;
+    const bool mid_ok = in_mid == 3;
     for (int i = 0; i < 3; ++i) {
         const vx_tensor * w = ws[i];
         if ((wq->type != VX_TYPE_Q8_0 && wq->type != VX_TYPE_F16) || w->type != wq->type || w->ne[0] != wq->ne[0] || w->ne[2] != 1 || w->ne[3] != 1 || !vx_positive(w) ||
