@@ -249,3 +249,30 @@ def test_rows_that_other_kernels_serve(pkg, gpu, monkeypatch, K, M, N, wtype):
         torch.cuda.synchronize()
         outs.append((out, pair))
     assert same_bits(outs[0][0], outs[1][0]) and same_bits(outs[0][1], outs[1][1])
+
+
+# (rows wide enough for the pre-tiled kernel on the side that is not the mid-size kernel's: K 512, an ffn width off the 256s)
+@pytest.mark.parametrize("K,F,M,N", [(1024, 5504, 5504, 3072), (512, 11008, 5632, 3000), (1024, 5632, 5504, 3072)])
+def test_mlp_with_one_product_on_each_kernel(pkg, gpu, K, F, M, N):
+    """norm + gate/up + SwiGLU + down + update as one call where the two products by themselves run on different kernels."""
+    import torch
+    say(f"mlp K={K} ffn={F} rows={M} tokens={N}")
+    L, d = pkg.lib(), pkg.desc
+    gen = torch.Generator(device="cuda").manual_seed(F + N)
+
+    def weight(m, k):
+        w = torch.randint(0, 256, (m, k // 32, 34), generator=gen, device="cuda", dtype=torch.uint8)
+        w[:, :, :2] = torch.tensor([0, 0x0c], dtype=torch.uint8, device="cuda")     # scales of 2^-12
+        return w.view(m, -1)
+
+    wg, wu, wd = weight(F, K), weight(F, K), weight(M, F)
+    gd, ud, dd = pkg.desc_q8(wg, K), pkg.desc_q8(wu, K), pkg.desc_q8(wd, F)
+    x, nw = torch.randn(N, K, generator=gen, device="cuda"), 1 + 0.1 * torch.randn(K, generator=gen, device="cuda")
+    res = torch.randn(N, M, generator=gen, device="cuda")
+    act, o1, o2 = torch.empty(N, F, device="cuda"), torch.empty(N, M, device="cuda"), torch.full((N, M), 5.0, device="cuda")
+    ok(pkg, L.vx_norm_mul_mat_swiglu(d(x), d(nw), 1e-5, gd, ud, d(act), pkg.ACT_FLOAT, None), "pair")
+    ok(pkg, L.vx_mul_mat_scale_add(dd, d(act), d(res), d(o1), 0.3, pkg.ACT_FLOAT, None), "down")
+    assert L.vx_supports_mlp_tiled(d(x), d(nw), gd, ud, dd, d(res), d(o2), pkg.ACT_FLOAT) == 1
+    ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, gd, ud, dd, d(res), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp")
+    torch.cuda.synchronize()
+    assert same_bits(o1, o2)

@@ -2875,11 +2875,12 @@ extern "C" vx_status vx_mul_mat_scale_add(const vx_tensor * src0, const vx_tenso
 }
 
 // mlp_forward and the residual update behind it at prefill sizes (src/minicpm.cpp:718-747, 775-786): RMS_NORM, MUL, gate, up,
-// SwiGLU, down, SCALE, ADD.  Three launches on the pre-tiled kernel: the activation pass with the norm, the gate/up pair
+// SwiGLU, down, SCALE, ADD.  Three launches on gemm_mid.hip's kernel, the pre-tiled one or one product each: the activation pass with the norm, the gate/up pair
 // whose epilogue writes silu(g) * u as f16 tiles, and the down projection that takes those tiles as they are, with the
 // update in its epilogue.  The intermediate [tokens x ffn] tensor is neither stored in fp32 nor read back and re-laid-out
 // (at 65536 tokens x 4096: a gigabyte each way).  Every value is rounded where the separate calls round it: same bits.
-static bool mlp_fill(mm_args & a, mm_args & b, bool & mid, const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
+struct mlp_route { bool a_mid, b_mid; }; // which of the two products is gemm_mid.hip's kernel's, as it would be in a call of its own
+static bool mlp_fill(mm_args & a, mm_args & b, mlp_route & r, const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
                      const vx_tensor * down, const vx_tensor * residual, float scale, const vx_tensor * dst, int act_mode) {
     if (!x || !norm_w || !gate || !up || !down || !residual || !dst) return false;
     if (down->type != gate->type || (down->type != VX_TYPE_Q8_0 && down->type != VX_TYPE_F16) || down->ne[2] != 1 || down->ne[3] != 1 || gate->ne[2] != 1 || gate->ne[3] != 1) return false;
@@ -2910,63 +2911,54 @@ static bool mlp_fill(mm_args & a, mm_args & b, bool & mid, const vx_tensor * x, 
     b.w_aligned = ((uintptr_t) down->data % 4 == 0) && down->nb[1] % 4 == 0;
     b.x_aligned = 1;
     const int nbatch = (int) (x->ne[2] * x->ne[3]);
-    {   // both products on gemm_mid.hip's kernel, as the separate calls would run them
-        const int wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
-        vx_gm_call c;
-        mm_args d = b;
-        d.tile_in = x->data; // (taken over as tiles: the activations' own alignment does not matter)
-        mid = (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 && mid_fill(c, a, nbatch, wt) && mid_fill(c, d, nbatch, wt);
-        if (mid) return true;
-        if (wt != WT_Q8) return false;
-    }
-    // both products on the pre-tiled kernel, as the separate calls would run them
-    return gemm_lds_mode() != 0 && b.w_aligned && (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0 &&
-           gemm_q8t_takes(a, nbatch, true) && gemm_q8t_takes(b, nbatch, false) && (uint64_t) 256 * b.rnb1 + 1024 < (1ull << 32);
+    const int wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
+    const bool stores = (uintptr_t) dst->data % 4 == 0 && (uintptr_t) residual->data % 4 == 0;
+    vx_gm_call c;
+    mm_args d = b;
+    d.tile_in = x->data; // (taken over as tiles: the activations' own alignment does not matter)
+    r.a_mid = mid_fill(c, a, nbatch, wt);
+    r.b_mid = mid_fill(c, d, nbatch, wt);
+    if (r.a_mid && r.b_mid) return stores;
+    // (what the pre-tiled kernel would not take of one product alone is nothing for this call)
+    return wt == WT_Q8 && stores && gemm_lds_mode() != 0 && b.w_aligned && gemm_q8t_takes(a, nbatch, true) && gemm_q8t_takes(b, nbatch, false) &&
+           (uint64_t) 256 * b.rnb1 + 1024 < (1ull << 32);
 }
 
 extern "C" int vx_supports_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, const vx_tensor * gate, const vx_tensor * up, const vx_tensor * down,
                                      const vx_tensor * residual, const vx_tensor * dst, int act_mode) {
     mm_args a = {}, b = {};
-    bool mid = false;
-    return mlp_fill(a, b, mid, x, norm_w, 0.0f, gate, up, down, residual, 0.0f, dst, act_mode);
+    mlp_route r;
+    return mlp_fill(a, b, r, x, norm_w, 0.0f, gate, up, down, residual, 0.0f, dst, act_mode);
 }
 
 extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
                                   const vx_tensor * down, const vx_tensor * residual, float scale, const vx_tensor * dst, int act_mode, vx_stream stream) {
     mm_args a = {}, b = {};
-    bool mid = false;
-    if (!mlp_fill(a, b, mid, x, norm_w, eps, gate, up, down, residual, scale, dst, act_mode))
+    mlp_route r;
+    if (!mlp_fill(a, b, r, x, norm_w, eps, gate, up, down, residual, scale, dst, act_mode))
         return vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the shapes of vx_supports_norm_mul_mat_swiglu_tiled, a Q8_0 down projection that the pre-tiled kernel takes, "
                        "an F32 residual of dst's shape");
     if (!x->data || !norm_w->data || !gate->data || !up->data || !down->data || !residual->data || !dst->data) return vx_fail(VX_ERR_INVALID, "mlp_tiled: null data");
     if (!(eps >= 0.0f)) return vx_fail(VX_ERR_INVALID, "mlp_tiled: eps must be >= 0");
     const int nbatch = (int) (x->ne[2] * x->ne[3]);
     hipStream_t st = (hipStream_t) stream;
-    // the tiles between the two products: whole 128-token tiles of the pair (it writes every token of its tiles), at the front of
-    // the workspace; both products put what they need behind them (a block that a later, larger request replaces stays valid)
-    // (gemm_mid.hip's kernel: the tiles of the tokens that exist)
+    // the tiles between the two products at the front of the workspace, all they need behind them (a block that a later, larger
+    // request replaces stays valid): whole 128-token tiles where the pre-tiled kernel writes or reads them, else those of the
+    // tokens that exist
+    const bool   mid = r.a_mid && r.b_mid;
+    const int    wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
     const int    tile_tt = mid ? (int) ((a.N + 15) / 16) : (int) ((a.N + QT_TOKS - 1) / QT_TOKS) * (QT_TOKS / 16);
     const size_t tiles   = ((mid ? vx_gm_tile_bytes(a.M, a.N, nbatch) : (size_t) nbatch * (size_t) (a.M / 32) * (size_t) tile_tt * 1024) + 255) & ~(size_t) 255;
     void * ws = nullptr;
     (void) take_ws_status();
-    if (mid) { // one request for all the group needs: its pieces lie in one block, also when it grows
-        const vx_status rc = vx_workspace(st, tiles + vx_gm_tile_bytes(a.K, a.N, nbatch), &ws, true);
-        if (rc != VX_OK) return rc;
-        const int wt = gate->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16;
-        a.ws_offset = tiles; a.tile_out = ws; a.tile_tt = tile_tt;
-        b.tile_in = ws; b.tile_tt = tile_tt;
-        if (!launch_mid(a, nbatch, wt, st) || ws_failed()) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the gate/up product could not be launched");
-        if (!launch_mid(b, nbatch, wt, st) || ws_failed()) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the down projection could not be launched");
-        VX_LAUNCH_CHECK();
-        return VX_OK;
-    }
-    const vx_status rc = vx_workspace(st, tiles, &ws);
+    const vx_status rc = vx_workspace(st, tiles + (r.a_mid ? vx_gm_tile_bytes(a.K, a.N, nbatch) : 0), &ws, mid);
     if (rc != VX_OK) return rc;
     a.ws_offset = tiles; a.tile_out = ws; a.tile_tt = tile_tt;
     b.ws_offset = tiles; b.tile_in = ws;  b.tile_tt = tile_tt;
     const bool fold = gemm_lds_mode() == 2;
-    if (!launch_gemm_q8t<true>(a, nbatch, st, fold)) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the gate/up product could not be launched");
-    if (!launch_gemm_q8t<false>(b, nbatch, st, fold)) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the down projection could not be launched");
+    const bool ok = (r.a_mid ? launch_mid(a, nbatch, wt, st) : launch_gemm_q8t<true>(a, nbatch, st, fold)) && !ws_failed() &&
+                    (r.b_mid ? launch_mid(b, nbatch, wt, st) : launch_gemm_q8t<false>(b, nbatch, st, fold));
+    if (!ok || ws_failed()) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: a product could not be launched");
     VX_LAUNCH_CHECK();
     return VX_OK;
 }
