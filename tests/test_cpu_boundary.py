@@ -327,6 +327,22 @@ def test_gate_up_pair_around_64_tokens(pkg, monkeypatch, K, at_63):
     assert [ask(n) for n in (63, 64, 65)] == [0, 1, 1]
 
 
+def test_pairs_off_the_16_bytes_are_taken(pkg):
+    """gate and up on different boundaries: refused by nothing that took them when both lie on the same one."""
+    lib = pkg.lib()
+
+    def at(off):
+        w = q8(pkg, [1024, 4096, 1, 1])
+        w.data = 0x10000 + off      # (looked at, not read)
+        return w
+
+    for n, off, stream, tiled in ((20, 2, 1, 0), (20, 4, 1, 0), (100, 2, 0, 0), (100, 4, 0, 1), (2000, 8, 0, 1)):
+        x, dst = f32(pkg, [1024, n, 1, 1]), f32(pkg, [4096, n, 1, 1])
+        for g, u in ((at(0), at(off)), (at(off), at(0))):
+            assert lib.vx_supports_mul_mat_swiglu(g, u, x, dst) == stream, (n, off)
+            assert lib.vx_supports_mul_mat_swiglu_tiled(g, u, x, dst, pkg.ACT_FLOAT) == tiled, (n, off)
+
+
 def test_ops_validate_before_touching_the_device(pkg):
     """Contract violations are reported by status + message; nothing is launched."""
     lib = pkg.lib()

@@ -276,3 +276,52 @@ def test_mlp_with_one_product_on_each_kernel(pkg, gpu, K, F, M, N):
     ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, gd, ud, dd, d(res), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp")
     torch.cuda.synchronize()
     assert same_bits(o1, o2)
+
+
+@pytest.mark.parametrize("F,N,shift", [(4096, 20, 4), (4096, 24, 2), (4096, 100, 4), (4096, 1500, 8), (5504, 3072, 4)])
+@pytest.mark.parametrize("which", ["gate", "up"])
+def test_pair_with_one_matrix_off_the_16_bytes(pkg, gpu, F, N, shift, which):
+    """Taken as before and with the bits of gate and up by themselves, of which one runs on another kernel then; with the norm in front and
+    with the down projection behind where those are one call."""
+    import torch
+    say(f"split pair ffn={F} tokens={N} shift={shift} {which}")
+    L, d = pkg.lib(), pkg.desc
+    K, M = 1024, 5504
+    gen = torch.Generator(device="cuda").manual_seed(F + N)
+
+    def weight(m, k, at=0):
+        w = torch.randint(0, 256, (m, k // 32, 34), generator=gen, device="cuda", dtype=torch.uint8)
+        w[:, :, :2] = torch.tensor([0, 0x0c], dtype=torch.uint8, device="cuda")
+        flat = torch.zeros(w.numel() + 16, dtype=torch.uint8, device="cuda")
+        flat[at:at + w.numel()] = w.view(-1)
+        return flat[at:at + w.numel()].view(m, -1)
+
+    wg, wu, wd = weight(F, K, shift if which == "gate" else 0), weight(F, K, shift if which == "up" else 0), weight(M, F)
+    gd, ud, dd = pkg.desc_q8(wg, K), pkg.desc_q8(wu, K), pkg.desc_q8(wd, F)
+    x, nw = torch.randn(N, K, generator=gen, device="cuda"), 1 + 0.1 * torch.randn(K, generator=gen, device="cuda")
+    res = torch.randn(N, M, generator=gen, device="cuda")
+    new = lambda m: torch.full((N, m), 5.0, device="cuda")
+    n, want, got, got_n, o1, o2 = new(K), new(F), new(F), new(F), new(M), new(M)
+    ok(pkg, L.vx_rms_norm_mul(d(x), d(nw), d(n), 1e-5, None), "norm")
+
+    def apart(src):
+        g, u, out = new(F), new(F), new(F)
+        ok(pkg, L.vx_mul_mat(gd, d(src), d(g), pkg.ACT_FLOAT, None), "gate")
+        ok(pkg, L.vx_mul_mat(ud, d(src), d(u), pkg.ACT_FLOAT, None), "up")
+        ok(pkg, L.vx_glu(pkg.GLU_SWIGLU, d(g), d(u), d(out), 0, None), "glu")
+        return out
+
+    want = apart(x)
+    ok(pkg, L.vx_mul_mat_swiglu(gd, ud, d(x), d(got), pkg.ACT_FLOAT, None), "pair")
+    torch.cuda.synchronize()
+    assert same_bits(got, want)
+    if N in (20, 24, 3072):
+        want = apart(n)
+        ok(pkg, L.vx_norm_mul_mat_swiglu(d(x), d(nw), 1e-5, gd, ud, d(got_n), pkg.ACT_FLOAT, None), "norm + pair")
+        torch.cuda.synchronize()
+        assert same_bits(got_n, want)
+    if N == 3072:
+        ok(pkg, L.vx_mul_mat_scale_add(dd, d(want), d(res), d(o1), 0.3, pkg.ACT_FLOAT, None), "down")
+        ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, gd, ud, dd, d(res), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp")
+        torch.cuda.synchronize()
+        assert same_bits(o1, o2)

@@ -2632,19 +2632,11 @@ extern "C" vx_status vx_mul_mat(const vx_tensor * src0, const vx_tensor * src1, 
 // MUL_MAT(gate) , MUL_MAT(up) , GLU(SWIGLU split) as one launch for decode-sized token counts
 // (MiniCPMModel::mlp_forward, src/minicpm.cpp:718-747).  Both products are formed exactly as vx_mul_mat
 // forms them (same block order, same reduction order), so the result equals the three separate nodes'.
-// gemm_mid.hip's kernel serves gate and up alone as well as the pair, but each only on 16-byte boundaries: a pair of which one
-// matrix is on such a boundary and the other is not would be summed in another order than the two products by themselves.
-static bool mid_split(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1) {
-    return vx_gm_region(gate->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, gate->ne[0], src1->ne[1], src1->ne[2] * src1->ne[3], gate->ne[1]) &&
-           ((uintptr_t) gate->data % 16 == 0) != ((uintptr_t) up->data % 16 == 0);
-}
-
 extern "C" int vx_supports_mul_mat_swiglu(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * dst) {
     if (!vx_supports_mul_mat(gate, src1, dst) || !up) return 0;
     if (gate->type != VX_TYPE_Q8_0 && gate->type != VX_TYPE_F16) return 0;
     if (up->type != gate->type) return 0;
     for (int i = 0; i < 4; ++i) if (up->ne[i] != gate->ne[i] || up->nb[i] != gate->nb[i]) return 0;
-    if (mid_split(gate, up, src1)) return 0;
     return gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]);
 }
 
@@ -2678,7 +2670,6 @@ extern "C" int vx_supports_mul_mat_swiglu_tiled(const vx_tensor * gate, const vx
     if (gate->type != VX_TYPE_Q8_0 && gate->type != VX_TYPE_F16) return 0;
     if (up->type != gate->type) return 0;
     for (int i = 0; i < 4; ++i) if (up->ne[i] != gate->ne[i] || up->nb[i] != gate->nb[i]) return 0;
-    if (mid_split(gate, up, src1)) return 0;
     if (src1->ne[1] <= 64 && !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]) && act_mode == VX_ACT_FLOAT && swiglu_mid_ok(gate, up, src1, nullptr, dst)) return 1;
     // (neither the pair nor one product on its own may be a shape of the streaming kernel: it sums the K blocks in another order)
     return !gemv_shape_ok(src1->ne[1], 2 * gate->ne[1], gate->ne[0]) && !gemv_shape_ok(src1->ne[1], gate->ne[1], gate->ne[0]) &&
@@ -2754,6 +2745,44 @@ extern "C" vx_status vx_norm_mul_mat_swiglu(const vx_tensor * x, const vx_tensor
     return swiglu_run(gate, up, x, norm_w, eps, dst, act_mode, stream);
 }
 
+// gemm_mid.hip's kernel wants its matrices on 16-byte boundaries: a pair of which only one matrix lies on one would be summed in
+// another order than gate and up by themselves.  (The streaming kernel, which takes such a pair at its own shapes, sums as that one.)
+static bool mid_split(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1) {
+    return vx_gm_region(gate->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, gate->ne[0], src1->ne[1], src1->ne[2] * src1->ne[3], gate->ne[1]) &&
+           ((uintptr_t) gate->data % 16 == 0) != ((uintptr_t) up->data % 16 == 0);
+}
+// Such a pair at the tiled kernels' shapes (Q8_0, where 4-byte boundaries do): the norm, the two products and the GLU as launches of
+// their own, `at` bytes into the workspace.
+static vx_status swiglu_apart(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * dst,
+                              size_t at, hipStream_t st) {
+    auto dense = [](vx_tensor t) {
+        for (int i = 1; i < 4; ++i) t.nb[i] = (i == 1 ? 4 : t.nb[i - 1]) * (uint64_t) t.ne[i - 1];
+        return t;
+    };
+    auto bytes = [](const vx_tensor & t) { return ((size_t) vx_nelements(&t) * 4 + 255) & ~(size_t) 255; };
+    vx_tensor xn = norm_w ? dense(*x) : *x, g = dense(*dst);
+    const size_t front = at + (norm_w ? bytes(xn) : 0) + bytes(g);
+    void * ws = nullptr;
+    vx_status rc = vx_workspace(st, front, &ws, true);
+    if (rc != VX_OK) return rc;
+    g.data = (char *) ws + front - bytes(g);
+    if (norm_w) {
+        xn.data = (char *) ws + at;
+        rc = vx_rms_norm_mul(x, norm_w, &xn, eps, (vx_stream) st);
+        if (rc != VX_OK) return rc;
+    }
+    for (int i = 0; i < 2; ++i) {
+        const vx_tensor * w = i ? up : gate;
+        mm_args a = {};
+        swiglu_fill(a, w, w, &xn, nullptr, 0.0f, i ? dst : &g);
+        a.w2 = nullptr;
+        a.ws_offset = front; // (a larger block that it asks for leaves this one's contents where they are)
+        launch<WT_Q8, false>(a, (int) (x->ne[2] * x->ne[3]), st);
+        if (ws_failed()) return take_ws_status();
+    }
+    return vx_glu(VX_GLU_SWIGLU, &g, dst, dst, 0, (vx_stream) st);
+}
+
 static vx_status swiglu_run(const vx_tensor * gate, const vx_tensor * up, const vx_tensor * src1, const vx_tensor * norm_w, float eps,
                             const vx_tensor * dst, int act_mode, vx_stream stream) {
     if (!gate || !up || !src1 || !dst || !gate->data || !up->data || !src1->data || !dst->data)
@@ -2765,6 +2794,10 @@ static vx_status swiglu_run(const vx_tensor * gate, const vx_tensor * up, const 
                        "(or, with f16 activations, one that a tiled kernel takes: vx_supports_mul_mat_swiglu_tiled)");
     if ((uintptr_t) src1->data % 4 || (uintptr_t) dst->data % 4 || (gate->type == VX_TYPE_F16 && (((uintptr_t) gate->data | (uintptr_t) up->data) % 2)))
         return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat_swiglu: misaligned tensor data");
+    if (tiled && mid_split(gate, up, src1)) {
+        (void) take_ws_status();
+        return swiglu_apart(gate, up, src1, norm_w, eps, dst, 0, (hipStream_t) stream);
+    }
     mm_args a = {};
     swiglu_fill(a, gate, up, src1, norm_w, eps, dst);
     const int nbatch = (int) (src1->ne[2] * src1->ne[3]);
@@ -2879,7 +2912,7 @@ extern "C" vx_status vx_mul_mat_scale_add(const vx_tensor * src0, const vx_tenso
 // whose epilogue writes silu(g) * u as f16 tiles, and the down projection that takes those tiles as they are, with the
 // update in its epilogue.  The intermediate [tokens x ffn] tensor is neither stored in fp32 nor read back and re-laid-out
 // (at 65536 tokens x 4096: a gigabyte each way).  Every value is rounded where the separate calls round it: same bits.
-struct mlp_route { bool a_mid, b_mid; }; // which of the two products is gemm_mid.hip's kernel's, as it would be in a call of its own
+struct mlp_route { bool a_mid, b_mid, apart; }; // which of the two products is gemm_mid.hip's kernel's, as it would be in a call of its own; a split pair
 static bool mlp_fill(mm_args & a, mm_args & b, mlp_route & r, const vx_tensor * x, const vx_tensor * norm_w, float eps, const vx_tensor * gate, const vx_tensor * up,
                      const vx_tensor * down, const vx_tensor * residual, float scale, const vx_tensor * dst, int act_mode) {
     if (!x || !norm_w || !gate || !up || !down || !residual || !dst) return false;
@@ -2916,6 +2949,7 @@ static bool mlp_fill(mm_args & a, mm_args & b, mlp_route & r, const vx_tensor * 
     vx_gm_call c;
     mm_args d = b;
     d.tile_in = x->data; // (taken over as tiles: the activations' own alignment does not matter)
+    r.apart = mid_split(gate, up, x);
     r.a_mid = mid_fill(c, a, nbatch, wt);
     r.b_mid = mid_fill(c, d, nbatch, wt);
     if (r.a_mid && r.b_mid) return stores;
@@ -2951,6 +2985,23 @@ extern "C" vx_status vx_mlp_tiled(const vx_tensor * x, const vx_tensor * norm_w,
     const size_t tiles   = ((mid ? vx_gm_tile_bytes(a.M, a.N, nbatch) : (size_t) nbatch * (size_t) (a.M / 32) * (size_t) tile_tt * 1024) + 255) & ~(size_t) 255;
     void * ws = nullptr;
     (void) take_ws_status();
+    if (r.apart) { // the pair's result in F32, for the down projection's own activation pass
+        vx_tensor act = *dst;
+        act.ne[0] = gate->ne[1];
+        act.nb[1] = b.nb11; act.nb[2] = b.nb12; act.nb[3] = b.nb13;
+        const size_t act_bytes = ((size_t) vx_nelements(&act) * 4 + 255) & ~(size_t) 255;
+        vx_status rc = vx_workspace(st, act_bytes, &ws);
+        if (rc != VX_OK) return rc;
+        act.data = ws;
+        rc = swiglu_apart(gate, up, x, norm_w, eps, &act, act_bytes, st);
+        if (rc != VX_OK) return rc;
+        b.x = (const char *) ws;
+        b.ws_offset = act_bytes;
+        const bool ok = r.b_mid ? launch_mid(b, nbatch, wt, st) : launch_gemm_lds<WT_Q8>(b, nbatch, st);
+        if (!ok || ws_failed()) return ws_failed() ? take_ws_status() : vx_fail(VX_ERR_UNSUPPORTED, "mlp_tiled: the down projection could not be launched");
+        VX_LAUNCH_CHECK();
+        return VX_OK;
+    }
     const vx_status rc = vx_workspace(st, tiles + (r.a_mid ? vx_gm_tile_bytes(a.K, a.N, nbatch) : 0), &ws, mid);
     if (rc != VX_OK) return rc;
     a.ws_offset = tiles; a.tile_out = ws; a.tile_tt = tile_tt;
