@@ -34,9 +34,6 @@ struct pf_args {
     const char * q; const char * k; const char * v; const char * vl; const char * mask;
     const float * sinks;
     const float * add1; // optional scalar added to every output element (a fused GGML_OP_ADD1)
-    const double * totals; // or the block totals of a cache write's two sums (n_tk of k at 0, n_tv of v at PF_TOTALS), which give that scalar
-    int n_tk, n_tv;
-    float sync_scale, sync_bias;
     _Float16 * tile_out; // optional: the result as f16 activation tiles of the product that follows, instead of dst
     uint32_t tile_tt, tile_bs, tile_ts;
     float * dst;
@@ -49,18 +46,25 @@ struct pf_args {
     float scale2, max_bias, m0, m1; // scale2 = scale * log2(e)
     uint32_t n_head_log2;
     int kv_f32;
+    const double * totals; // instead of add1 the block totals of a cache write's two sums (n_tk of k at 0, n_tv of v at PF_TOTALS), which give that scalar
+    int n_tk, n_tv;
+    float sync_scale, sync_bias;
 };
 
 // What the launch in front of the attention kernel prepares, each by work-groups of its own: the cache write of the same
 // attention block (n_store work-groups), the mask's tile flags (n_mask), the f16 images of F32 K / V (the rest).
+struct pf_mask_args {
+    const char * mask;
+    uint64_t nbm1, nbm2, nbm3;
+    int nem2, n_q, n_kv, RB, n_rb, n_tiles, vec_ok, n_units;
+    uint8_t * flags; uint8_t * bits;
+};
 struct pf_prep_args {
     kvs_side ks, vs;
     double * totals;
     int store_large, n_tk, n_store; // the SUMs' form (below); work-groups (large) or totals of the k side; work-groups of both
-    const char * mask;
-    uint64_t nbm1, nbm2, nbm3;
-    int nem2, n_q, n_kv, RB, n_rb, n_tiles, vec_ok, n_units, n_mask;
-    uint8_t * flags; uint8_t * bits;
+    pf_mask_args m;
+    int n_mask, n_kv;
     const char * k; const char * v;
     uint64_t nbk1, nbk2, nbk3, nbv1, nbv2, nbv3;
     int Hkv, key_blocks;
@@ -72,8 +76,7 @@ struct pf_prep_args {
 // any row of the block; 1 every entry is zero; 2 some entry is a finite non-zero value; 3 zeros and -inf only.  For the
 // last kind the rows' visibility is also left as one bit per key (bits[mask batch][row][tile], keys past n_kv cleared),
 // so that the attention kernel applies such a tile -- a causal mask's diagonal -- from 8 bytes per row.
-__device__ __forceinline__ void pf_mask_unit(const pf_prep_args & a, int unit, int lane) {
-    const int tile = unit % a.n_tiles, rb = (unit / a.n_tiles) % a.n_rb, mb = unit / a.n_tiles / a.n_rb;
+__device__ __forceinline__ void pf_mask_unit(const pf_mask_args & a, int tile, int rb, int mb, int lane) {
     const char * mp = a.mask + (uint64_t) (mb % a.nem2) * a.nbm2 + (uint64_t) (mb / a.nem2) * a.nbm3;
     const int r0 = rb * a.RB, r1 = min(a.n_q, (rb + 1) * a.RB);
     bool any_visible = false, any_nonzero = false, any_hidden = false;
@@ -215,9 +218,9 @@ __device__ __forceinline__ void pf_store_large(const kvs_side & s, uint32_t b, d
 
 // One launch for what three did (the cache write, the mask's flags, the f16 images): each is a trip to memory and its
 // latency at a prompt's size.  Two sequences of 512 tokens: 4.8 + 4.1 + 3.9 us as launches of their own, and 4.5 for the
-// scalar that the attention now adds up itself; 24 layers 3067 -> 2876 us, 16 x 4096 tokens 86.5 -> 85.7 ms.
+// scalar that the attention now adds up itself; 24 layers 3067 -> 2876 us (16 x 4096 tokens: no difference beyond noise).
 // STORE is a parameter of its own because the write's four units in flight cost every wave of the launch 98 registers, half
-// the waves a SIMD can hold (a causal attention of 4096 tokens without a write 74.6 -> 71.9 us a call).
+// the waves a SIMD can hold (F32 keys and values without a write are left for the other instance).
 template <bool STORE>
 __global__ __launch_bounds__(256) void pf_prep_kernel(const pf_prep_args a) {
     __shared__ double part[16];
@@ -243,12 +246,22 @@ __global__ __launch_bounds__(256) void pf_prep_kernel(const pf_prep_args a) {
     if constexpr (STORE) i -= a.n_store;
     if (i < a.n_mask) {
         const int unit = 4 * i + wave;
-        if (unit < a.n_units) pf_mask_unit(a, unit, lane);
+        if (unit < a.m.n_units) pf_mask_unit(a.m, unit % a.m.n_tiles, (unit / a.m.n_tiles) % a.m.n_rb, unit / a.m.n_tiles / a.m.n_rb, lane);
         return;
     }
     i -= a.n_mask;
     const int kb = i % a.key_blocks, bg = i / a.key_blocks;
     pf_convert_unit(a, kb * 256 + (int) threadIdx.x, bg % a.Hkv, bg / a.Hkv);
+}
+
+// The mask's units alone (f16 keys and values, no cache write): the grid is (W key tiles, row block, mask batch), a wave a tile.
+// (Arguments one by one: the first of them come in registers, where a struct's fields are a trip to memory, 0.2 of 3 us.)
+template <int W>
+__global__ __launch_bounds__(64 * W) void pf_mask_kernel(const char * mask, uint64_t nbm1, uint64_t nbm2, uint64_t nbm3, int nem2, int n_q, int n_kv, int RB,
+                                                         int n_rb, int n_tiles, int vec_ok, uint8_t * flags, uint8_t * bits) {
+    const pf_mask_args a = { mask, nbm1, nbm2, nbm3, nem2, n_q, n_kv, RB, n_rb, n_tiles, vec_ok, 0, flags, bits };
+    const int tile = W * (int) blockIdx.x + __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
+    if (tile < n_tiles) pf_mask_unit(a, tile, blockIdx.y, blockIdx.z, threadIdx.x & 63);
 }
 
 // the ordering scalar of a large write's totals, for every work-group of the attention kernel to read
@@ -269,8 +282,9 @@ __global__ __launch_bounds__(128) void pf_scalar_kernel(const double * totals, i
     if (t == 0) *out = kvs_scalar((float) sum[0], (float) sum[1], scale, bias);
 }
 
-// VLO: V comes with a low-half image (a.vl).  NCB: 32-column blocks per wave.
-template <bool VLO, int NCB>
+// VLO: V comes with a low-half image (a.vl).  NCB: 32-column blocks per wave.  SUMS: the addend is the ordering scalar of a.totals
+// (an instance of its own: as a test in every instance it cost the calls without a cache write 1 %, 2048 causal tokens 38.7 -> 39.1 us).
+template <bool VLO, int NCB, bool SUMS = false>
 __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_kernel(const pf_args a) {
     constexpr int D = 64;
     constexpr int PF_STAGES = VLO ? 3 : PF_STAGES_MAX; // (three stages of K, V and V low leave room for two work-groups on a compute unit)
@@ -282,7 +296,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
     __shared__ uint16_t tile_list[PF_MAX_TILES];
     __shared__ uint8_t  tile_flag[PF_MAX_TILES];
     __shared__ int      n_active_s;
-    __shared__ float    y_s;
+    __shared__ float    y_s; // SUMS
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -350,7 +364,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             base += __builtin_popcountll(bal);
         }
         if (lane == 0) n_active_s = base;
-    } else if (wave == 1 && a.totals) { // the cache write's ordering scalar: k's totals in the low half of the wave, v's in the high
+    } else if (SUMS && wave == 1) { // the cache write's ordering scalar: k's totals in the low half of the wave, v's in the high
         const int n = hl ? a.n_tv : a.n_tk;
         double tot[PF_TOTALS_INLINE / 32];
 #pragma unroll
@@ -721,8 +735,8 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
     int lane_e = threadIdx.x & 63; // (worked out again rather than kept alive through the walk)
     asm volatile("" : "+v"(lane_e));
     const int hl_e = lane_e >> 5, cl_e = lane_e & 31;
-    const bool  has_add = a.totals || a.add1;
-    const float addend = a.totals ? y_s : a.add1 ? *a.add1 : 0.0f;
+    const bool  has_add = SUMS || a.add1;
+    const float addend = SUMS ? y_s : a.add1 ? *a.add1 : 0.0f;
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         const int  col = wave * (32 * NCB) + cb * 32 + cl_e;
@@ -873,18 +887,19 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
         ws += front_bytes;
     }
     int64_t blocks = p.n_store;
-    p.n_q = n_q; p.n_kv = n_kv; p.RB = RB; p.n_rb = n_rb; p.n_tiles = n_tiles;
+    p.n_kv = n_kv;
+    p.m.n_q = n_q; p.m.n_kv = n_kv; p.m.RB = RB; p.m.n_rb = n_rb; p.m.n_tiles = n_tiles;
     if (mask) {
-        p.mask = a.mask; p.nbm1 = a.nbm1; p.nbm2 = a.nbm2; p.nbm3 = a.nbm3; p.nem2 = a.nem2;
-        p.vec_ok = (uintptr_t) a.mask % 16 == 0 && a.nbm1 % 16 == 0 && a.nbm2 % 16 == 0 && a.nbm3 % 16 == 0;
-        p.bits = (uint8_t *) ws; p.flags = (uint8_t *) ws + bits_bytes;
+        p.m.mask = a.mask; p.m.nbm1 = a.nbm1; p.m.nbm2 = a.nbm2; p.m.nbm3 = a.nbm3; p.m.nem2 = a.nem2;
+        p.m.vec_ok = (uintptr_t) a.mask % 16 == 0 && a.nbm1 % 16 == 0 && a.nbm2 % 16 == 0 && a.nbm3 % 16 == 0;
+        p.m.bits = (uint8_t *) ws; p.m.flags = (uint8_t *) ws + bits_bytes;
         const int64_t units = (int64_t) n_tiles * n_rb * a.nem2 * a.nem3;
         if (units > 0x7ffffff0) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext: launch too large");
-        p.n_units = (int) units;
+        p.m.n_units = (int) units;
         p.n_mask = (int) ((units + 3) / 4);
         blocks += p.n_mask;
-        a.bits = p.bits;
-        a.flags = p.flags;
+        a.bits = p.m.bits;
+        a.flags = p.m.flags;
     }
     if (a.kv_f32) {
         p.k16 = (_Float16 *) (ws + flag_bytes); p.vhi = (_Float16 *) (ws + flag_bytes + plane); p.vlo = (_Float16 *) (ws + flag_bytes + 2 * plane);
@@ -905,7 +920,15 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
         blocks -= p.n_store;
         p.n_store = 0;
     }
-    if (blocks) {
+    if (blocks && blocks == p.n_mask && n_rb <= 65535 && a.nem2 * a.nem3 <= 65535) {
+        // Up to four units a compute unit go out one by one (a causal call of 512 tokens 16.2 us against 16.3 with four to a work-group,
+        // 16 x 256 18.5 / 18.9), more of them by fours (2048: 38.4 us against 39.1, 4096: 72.1 / 73.8).
+        const dim3 grid((unsigned) n_tiles, (unsigned) n_rb, (unsigned) (a.nem2 * a.nem3));
+        const pf_mask_args & m = p.m;
+        if (m.n_units <= 1024) vx_launch(pf_mask_kernel<1>, grid, dim3(64), 0, st, m.mask, m.nbm1, m.nbm2, m.nbm3, m.nem2, m.n_q, m.n_kv, m.RB, m.n_rb, m.n_tiles, m.vec_ok, m.flags, m.bits);
+        else vx_launch(pf_mask_kernel<4>, dim3((grid.x + 3) / 4, grid.y, grid.z), dim3(256), 0, st, m.mask, m.nbm1, m.nbm2, m.nbm3, m.nem2, m.n_q, m.n_kv, m.RB, m.n_rb, m.n_tiles, m.vec_ok, m.flags, m.bits);
+        VX_LAUNCH_CHECK();
+    } else if (blocks) {
         if (p.n_store) vx_launch(pf_prep_kernel<true>, dim3((unsigned) blocks), dim3(256), 0, st, p);
         else           vx_launch(pf_prep_kernel<false>, dim3((unsigned) blocks), dim3(256), 0, st, p);
         VX_LAUNCH_CHECK();
@@ -915,7 +938,11 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
         VX_LAUNCH_CHECK();
     }
     const dim3 grid((unsigned) (n_rb * n_groups)), block(64 * PF_WAVES);
-    if (half_cols) {
+    if (a.totals) {
+        if (!half_cols)    vx_launch(pf_kernel<false, 2, true>, grid, block, 0, st, a);
+        else if (a.kv_f32) vx_launch(pf_kernel<true, 1, true>, grid, block, 0, st, a);
+        else               vx_launch(pf_kernel<false, 1, true>, grid, block, 0, st, a);
+    } else if (half_cols) {
         if (a.kv_f32) vx_launch(pf_kernel<true, 1>, grid, block, 0, st, a);
         else          vx_launch(pf_kernel<false, 1>, grid, block, 0, st, a);
     } else {
