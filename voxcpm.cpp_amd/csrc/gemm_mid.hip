@@ -514,14 +514,10 @@ static bool gm_rows_ok(int wtype, int64_t K, int64_t tokens, int64_t M) {
     return K > 1024 || M * tokens <= (wtype == VX_GM_Q8 ? 5120 : 2560) * 1024;
 }
 
-bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M) {
-    // Switches, read on every call.  VX_GEMM_MID=0: the kernels of mul_mat.hip for these shapes.  VX_GEMM_LDS other than 1 and, from
-    // 1024 tokens on, VX_GEMM_Q8T other than 1 ask for one of those kernels by name (another rounding of the weights, the older
-    // kernels, one prefill kernel or the other): then it is that kernel that runs.
-    auto is = [](const char * name, int by_default) { const char * e = getenv(name); return e ? atoi(e) : by_default; };
-    if (is("VX_GEMM_MID", 1) == 0 || is("VX_GEMM_LDS", 1) != 1 || (N >= 1024 && is("VX_GEMM_Q8T", 1) != 1)) return false;
-    // Up to where this kernel's 64 x 128 tiles beat the LDS-tiled and pre-tiled kernels' larger ones in a layer of 1024 / 4096 rows.  Q8_0, 24 layers of one prompt: 1200 tokens 6270 -> 3818 us, 2048 6834 -> 5205, 2600 8990 -> 7156, but
-    // 4000 9639 -> 10114; F16, 56 products: 1100 tokens 1343 -> 1260 us, 1537 1417 -> 1463.
+bool vx_gm_shape(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M) {
+    // Up to where this kernel's 64 x 128 tiles beat the LDS-tiled and pre-tiled kernels' larger ones in a layer of 1024 / 4096 rows.
+    // Q8_0, 24 layers of one prompt: 1200 tokens 6270 -> 3818 us, 2048 6834 -> 5205, 2600 8990 -> 7156, but 4000 9639 -> 10114;
+    // F16, 56 products: 1100 tokens 1343 -> 1260 us, 1537 1417 -> 1463.
     if (N <= 16 || N * nbatch > (wtype == VX_GM_Q8 ? 3072 : 1152) || nbatch > 65535) return false;
     // K of whole 256s (the stages).  Up to 16 tokens are the streaming kernel's; what it takes beyond them with K of 513 to
     // 1024 it sums in this kernel's order, and with K above 2048 it takes nothing beyond them: elsewhere a call that one of
@@ -529,17 +525,25 @@ bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M) {
     return K % 256 == 0 && ((K > 512 && K <= 1024) || (K > 2048 && K <= 16384)) && gm_rows_ok(wtype, K, N * nbatch, M);
 }
 
+bool vx_gm_on(int64_t N) {
+    // Switches, read on every call.  VX_GEMM_MID=0: the kernels of mul_mat.hip for these shapes.  VX_GEMM_LDS other than 1 and, from
+    // 1024 tokens on, VX_GEMM_Q8T other than 1 ask for one of those kernels by name (another rounding of the weights, the older
+    // kernels, one prefill kernel or the other): then it is that kernel that runs.
+    auto is = [](const char * name, int by_default) { const char * e = getenv(name); return e ? atoi(e) : by_default; };
+    return is("VX_GEMM_MID", 1) != 0 && is("VX_GEMM_LDS", 1) == 1 && (N < 1024 || is("VX_GEMM_Q8T", 1) == 1);
+}
+
 bool vx_gm_takes(const vx_gm_call & c) {
     auto al16 = [](const void * p, uint64_t s) { return (uintptr_t) p % 16 == 0 && s % 16 == 0; };
     for (int i = 0; i < c.nmat; ++i) {
-        if (!vx_gm_region(c.wtype, c.K, c.N, (int64_t) c.ne12 * c.ne13, c.mat[i].M)) return false;
+        if (!vx_gm_shape(c.wtype, c.K, c.N, (int64_t) c.ne12 * c.ne13, c.mat[i].M)) return false;
         if (!al16(c.mat[i].w, c.mat[i].nb01) || c.mat[i].M < 1) return false;
         if (c.nmat > 1 && c.mat[i].M % 64) return false;
     }
     if (c.w2 && !al16(c.w2, 0)) return false;
     if (!c.tile_in && !(al16(c.x, c.nb11) && c.nb12 % 16 == 0 && c.nb13 % 16 == 0)) return false;
     if (c.norm_w && (c.K > 1024 || (uintptr_t) c.norm_w % 16)) return false;
-    return true;
+    return vx_gm_on(c.N);
 }
 
 size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch) {

@@ -44,7 +44,9 @@ struct vx_gm_call {
 // Whether this kernel serves a product of M rows, K columns and N * nbatch tokens.  The rows of one matrix decide, for a gate/up pair
 // as for gate or up alone, and a group of several matrices needs the answer for each: a product and every group it is part of
 // are formed by the same kernel, in the same order of every sum.
-bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M);
+bool vx_gm_shape(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M);
+bool vx_gm_on(int64_t N); // and whether the environment leaves it in place
+static inline bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M) { return vx_gm_shape(wtype, K, N, nbatch, M) && vx_gm_on(N); }
 // region, and operands on the boundaries its loads need (dst only needs 4-byte aligned values)
 bool vx_gm_takes(const vx_gm_call & c);
 size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch); // f16 activation tiles of a product

@@ -3166,8 +3166,8 @@ extern "C" int vx_mul_mat_sum_order(int64_t K, int64_t tokens, int64_t M) {
     // (shapes of gemm_mid.hip's kernel but for their rows, with either weight type: another kernel's order)
     int by_rows = 0;
     for (int wt : { VX_GM_Q8, VX_GM_F16 })
-        if (vx_gm_region(wt, K, tokens, 1, 1024) && !vx_gm_region(wt, K, tokens, 1, M)) by_rows |= 64 << wt;
-    return gemv_waves_for(K, tokens, M) + by_rows;
+        if (vx_gm_shape(wt, K, tokens, 1, 1024) && !vx_gm_shape(wt, K, tokens, 1, M)) by_rows |= 64 << wt;
+    return gemv_waves_for(K, tokens, M) + (by_rows && vx_gm_on(tokens) ? by_rows : 0);
 }
 
 static vx_status qkv_run(const vx_tensor * norm_w, float eps, const vx_tensor * wq, const vx_tensor * wk, const vx_tensor * wv,
@@ -3200,7 +3200,8 @@ static bool qkv_tiled_fill(mm_args & a, bool & mid, const vx_tensor * norm_w, fl
     a.nseg = 3;
     const int nbatch = (int) x->ne[3];
     int in_mid = 0; // matrices of gemm_mid.hip's kernel: all three, or none
-    for (const vx_tensor * w : ws) in_mid += vx_gm_region(wq->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, a.K, a.N, nbatch, w->ne[1]);
+    for (const vx_tensor * w : ws) in_mid += vx_gm_shape(wq->type == VX_TYPE_Q8_0 ? VX_GM_Q8 : VX_GM_F16, a.K, a.N, nbatch, w->ne[1]);
+    if (in_mid && !vx_gm_on(a.N)) in_mid = 0;
     if (in_mid != 0 && in_mid != 3) return false;
     const bool mid_ok = in_mid == 3;
     for (int i = 0; i < 3; ++i) {
