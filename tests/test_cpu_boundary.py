@@ -343,6 +343,15 @@ def test_pairs_off_the_16_bytes_are_taken(pkg):
             assert lib.vx_supports_mul_mat_swiglu_tiled(g, u, x, dst, pkg.ACT_FLOAT) == tiled, (n, off)
 
 
+@pytest.mark.parametrize("heads,tokens,want", [(16, 65536, 1), (28, 65536, 1), (29, 65536, 0), (64, 8192, 0), (64, 2048, 1)])
+def test_norm_qkv_announces_what_it_can_launch(pkg, heads, tokens, want):
+    """norm + q/k/v + rotation beyond gemm_mid.hip's tokens: the pre-tiled kernel's form of several matrices holds 2048 rows."""
+    K, D, Hkv = 1024, 64, 2
+    wq, wk, nw, x = q8(pkg, [K, heads * D, 1, 1]), q8(pkg, [K, Hkv * D, 1, 1]), f32(pkg, [K, 1, 1, 1]), f32(pkg, [K, tokens, 1, 1])
+    q, k, v = f32(pkg, [D, heads, tokens, 1]), f32(pkg, [D, Hkv, tokens, 1]), f32(pkg, [Hkv * D, tokens, 1, 1])
+    assert pkg.lib().vx_supports_norm_qkv_proj_rope_tiled(x, nw, wq, wk, wk, q, k, v, D, 2, pkg.ACT_FLOAT) == want
+
+
 def test_ops_validate_before_touching_the_device(pkg):
     """Contract violations are reported by status + message; nothing is launched."""
     lib = pkg.lib()

@@ -1846,6 +1846,7 @@ vx_status take_ws_status() { const vx_status rc = t_ws_status; t_ws_status = VX_
 // bring 50 KB in from L2: no single unit bounds it; what is left is the waves of a work-group meeting at a barrier every
 // block and the issue of the direct loads (a fifth of the time when they are taken out).
 constexpr int QT_ROWS = 256, QT_TOKS = 128, QT_STAGES = 2;
+constexpr int QT_SEG_ROWS = 8 * QT_ROWS; // rows of all matrices of a launch over several: a group of 32 work-groups holds all the row tiles
 constexpr int QT_STAGE_BYTES = (QT_ROWS + QT_TOKS) / 16 * 1024 + QT_ROWS * 4;
 constexpr size_t QT_LDS = (size_t) QT_STAGES * QT_STAGE_BYTES;
 
@@ -2359,7 +2360,7 @@ bool launch_gemm_q8t(const mm_args & a, int nbatch, hipStream_t st, bool fold) {
     const int64_t wunits = (int64_t) q.n_kb * q.n_rt * 64, xunits = (int64_t) ((q.n_kb + QT_ACT_UNROLL - 1) / QT_ACT_UNROLL) * q.n_tt * 64;
     if ((wunits + 255) / 256 > 0x7fffffff || (xunits + 255) / 256 > 0x7fffffff) return false;
     const int gx = (q.n_rt + 15) / 16, gy = (q.n_tt + 7) / 8, Gx = (gx + 3) / 4, Gy = (gy + 7) / 8;
-    if (segs && gx > 8) return false; // (the segment form's groups hold all the row tiles)
+    if (segs && a.M > QT_SEG_ROWS) return false;
     // groups of 32 work-groups, dealt to the XCDs in turn: 4 row tiles x 8 token tiles, or (segments) all gx row tiles x 32 / gx token tiles
     const int64_t groups = segs ? ((int64_t) gy + 32 / gx - 1) / (32 / gx) : (int64_t) Gx * Gy;
     const int64_t blocks = (groups + 7) / 8 * 8 * 32;
@@ -3232,7 +3233,7 @@ static bool qkv_tiled_fill(mm_args & a, bool & mid, const vx_tensor * norm_w, fl
         mid = norm_w->data && n_dims == 64 && q_dst->ne[0] == 64 && k_dst->ne[0] == 64 && q_dst->ne[2] == k_dst->ne[2] && mid_fill(c, a, nbatch, wq->type == VX_TYPE_Q8_0 ? WT_Q8 : WT_F16);
         return mid;
     }
-    if (wq->type != VX_TYPE_Q8_0) return false;
+    if (wq->type != VX_TYPE_Q8_0 || a.M > QT_SEG_ROWS) return false;
     return a.w_aligned && a.x_aligned && norm_w->data && (uintptr_t) norm_w->data % 16 == 0 && gemm_q8t_takes(a, nbatch, false);
 }
 
