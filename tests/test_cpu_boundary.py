@@ -507,7 +507,7 @@ def test_hot_kernels_do_not_spill():
         assert len(names) == len(sizes), f
         scratch.update({n: int(s) for n, s in zip(names, sizes)})
     assert len(scratch) > 250
-    hot = [r"gemm_q8t_kernel", r"qt_weights_kernel", r"qt_acts_kernel", r"qt_acts_norm_kernel", r"qt_rope_table_kernel", r"rope_heads_kernel", r"kv_sync_add1_kernel", r"kv_sync_scalar_kernel", r"kv_store_mid_kernel", "kv_sync_scalar_kernel", r"fattn_dec64_kernel", r"gemm_lds_kernel", r"gemv_dma_kernel", r"gemv_kernel", r"mm_kernel", r"mm_splitk_reduce_kernel", r"fattn_merge_kernel",
+    hot = [r"gemm_q8t_kernel", r"qt_weights_kernel", r"qt_acts_kernel", r"qt_acts_norm_kernel", r"qt_rope_table_kernel", r"rope_heads_kernel", r"kv_sync_add1_kernel", r"kv_store_mid_kernel", r"gm_kernel", r"gm_acts_kernel", r"pf_prep_kernel", r"pf_mask_kernel", r"pf_scalar_kernel", r"fattn_dec64_kernel", r"gemm_lds_kernel", r"gemv_dma_kernel", r"gemv_kernel", r"mm_kernel", r"mm_splitk_reduce_kernel", r"fattn_merge_kernel",
            r"fattn_cols16_kernelILi64ELb0", r"pf_kernel", r"small_graph_dense_kernel", r"small_graph_kernel", r"rms_norm_kernel",
            r"rope_kernel", r"concat_many_kernel"]
     known = [r"fattn_cols16_kernelILi(64|128)ELb1", r"fattn_cols16_kernelILi128ELb0ELb1ELb[01]ELi1", r"kv_store_sync_kernel",

@@ -325,3 +325,56 @@ def test_pair_with_one_matrix_off_the_16_bytes(pkg, gpu, F, N, shift, which):
         ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, gd, ud, dd, d(res), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp")
         torch.cuda.synchronize()
         assert same_bits(o1, o2)
+
+
+@pytest.mark.parametrize("T,B", [(17, 3), (45, 2), (203, 2), (517, 2)])
+@pytest.mark.parametrize("wtype", ["q8", "f16"])
+@pytest.mark.parametrize("poison", [False, True])
+def test_groups_by_sequence(pkg, gpu, T, B, wtype, poison):
+    """norm + q/k/v + rope, k + v + rope and the MLP with the sequences in a dimension of their own and strided rows, against separate calls;
+    a NaN and an infinity stay in their tokens."""
+    import torch
+    say(f"layer groups by sequence T={T} B={B} weights={wtype} poison={poison}")
+    L, d = pkg.lib(), pkg.desc
+    K, H, Hkv, F = 1024, 16, 2, 2304
+    gen = torch.Generator(device="cuda").manual_seed(T * B)
+    keep = []
+
+    def weight(m, k):
+        w = 0.05 * torch.randn(m, k, generator=gen, device="cuda")
+        keep.append(q8_dev(w.cpu().numpy())[0] if wtype == "q8" else w.half())
+        return pkg.desc_q8(keep[-1], k) if wtype == "q8" else d(keep[-1])
+
+    wq, wk, wv, wg, wu, wd = weight(K, K), weight(128, K), weight(128, K), weight(F, K), weight(F, K), weight(K, F)
+    wide = torch.randn(B, T + 2, K + 32, generator=gen, device="cuda")
+    if poison:
+        wide[0, T // 2, 5], wide[B - 1, T - 1, 7] = float("nan"), float("inf")
+    x, nw = wide[:, :T, :K], 1 + 0.1 * torch.randn(K, generator=gen, device="cuda")
+    x4 = x.unsqueeze(1)                                             # [K, T, 1, B]
+    pos, ff = torch.arange(5, 5 + T, dtype=torch.int32, device="cuda"), 1 + torch.rand(32, generator=gen, device="cuda")
+    rope = (64, 2, 32768, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+    new = lambda *s: torch.full(s, 9.0, device="cuda")
+    n, q1, k1, v1, q2, k2, v2, k3, v3 = (new(B, 1, T, K), new(B, T, H, 64), new(B, T, Hkv, 64), new(B, 1, T, 128), new(B, T, H, 64), new(B, T, Hkv, 64),
+                                         new(B, 1, T, 128), new(B, T, Hkv, 64), new(B, 1, T, 128))
+    ok(pkg, L.vx_rms_norm_mul(d(x4), d(nw), d(n), 1e-5, None), "norm")
+    for w, t in ((wq, q1), (wk, k1), (wv, v1)):
+        ok(pkg, L.vx_mul_mat(w, d(n), d(t.view(B, 1, T, -1)), pkg.ACT_FLOAT, None), "mul_mat")
+        if t is not v1:
+            ok(pkg, L.vx_rope(d(t), pos.data_ptr(), ff.data_ptr(), d(t), *rope, None), "rope")
+    ok(pkg, L.vx_norm_qkv_proj_rope(d(x4), d(nw), 1e-5, wq, wk, wv, pos.data_ptr(), ff.data_ptr(), d(q2), d(k2), d(v2), *rope, pkg.ACT_FLOAT, None), "qkv")
+    ok(pkg, L.vx_kv_proj_rope(wk, wv, d(n), pos.data_ptr(), ff.data_ptr(), d(k3), d(v3), *rope, pkg.ACT_FLOAT, None), "kv")
+    gate, up, act, o1, o2 = new(B, T, F), new(B, T, F), new(B, T, F), new(B, T, K), new(B, T, K)
+    n3 = n[:, 0]
+    ok(pkg, L.vx_mul_mat(wg, d(n3), d(gate), pkg.ACT_FLOAT, None), "gate")
+    ok(pkg, L.vx_mul_mat(wu, d(n3), d(up), pkg.ACT_FLOAT, None), "up")
+    ok(pkg, L.vx_glu(pkg.GLU_SWIGLU, d(gate), d(up), d(act), 0, None), "glu")
+    ok(pkg, L.vx_mul_mat_scale_add(wd, d(act), d(x), d(o1), 0.3, pkg.ACT_FLOAT, None), "down")
+    assert L.vx_supports_mlp_tiled(d(x), d(nw), wg, wu, wd, d(x), d(o2), pkg.ACT_FLOAT) == (B * T <= (3072 if wtype == "q8" else 1152))
+    if B * T <= 1152 or wtype == "q8":
+        ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, wg, wu, wd, d(x), 0.3, d(o2), pkg.ACT_FLOAT, None), "mlp")
+    torch.cuda.synchronize()
+    for a, b in ((q1, q2), (k1, k2), (v1, v2), (k1, k3), (v1, v3), (o1, o2)):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a.nan_to_num(3.0, 4.0, 5.0), b.nan_to_num(3.0, 4.0, 5.0))
+    bad = {(0, T // 2), (B - 1, T - 1)} if poison else set()
+    assert {tuple(i) for i in torch.nonzero(~torch.isfinite(o2).all(2)).tolist()} == bad
+    assert {tuple(i) for i in torch.nonzero(~torch.isfinite(v2[:, 0]).all(2)).tolist()} == bad
