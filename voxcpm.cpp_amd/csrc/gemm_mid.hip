@@ -62,7 +62,9 @@ template <int N> __device__ __forceinline__ void gm_dma_tiles(uint32_t off, cons
 
 template <int N> __device__ __forceinline__ void gm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
 
-template <int WT, int MT, int NT, int RW, int KG, int CH, int S>
+constexpr int KG = 4; // waves of a row group, over the k blocks: the streaming kernel's four waves
+
+template <int WT, int MT, int NT, int RW, int CH, int S>
 struct gm_shape {
     static constexpr int NC = KG * RW, NWAVES = NC + 2;       // compute waves; one wave brings the weights, one the activations
     static constexpr int ROWS = 16 * MT * RW, TOKS = 16 * NT;
@@ -76,11 +78,12 @@ struct gm_shape {
     static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
 };
 
-template <int WT, int MT, int NT, int RW, int KG, int CH, int S, int EPI>
+template <int WT, int MT, int NT, int RW, int CH, int S, int EPI>
 __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a) {
-    using sh = gm_shape<WT, MT, NT, RW, KG, CH, S>;
+    using sh = gm_shape<WT, MT, NT, RW, CH, S>;
     static_assert((CH == 1 || CH == 2) && 4 * CH % KG == 0, "stages of 128 or 256 k, whole steps");
-    static_assert(EPI == GM_PLAIN || MT % 2 == 0, "pairs of row tiles inside a wave");
+    static_assert(EPI == GM_PLAIN || MT == 2, "pairs of row tiles inside a wave");
+    static_assert(S == 3, "what the waits below count");
     extern __shared__ __align__(1024) char gm_smem[];
     typedef __attribute__((address_space(3))) char lds_char;
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
     // first row of local row tile lt (wave row rw holds lt = rw * MT + m)
     auto row_of = [&](int lt) {
         if constexpr (EPI == GM_SWIGLU) return tx * (sh::ROWS / 2) + 16 * (lt >> 1);      // even tiles W, odd tiles the same rows of W2
-        if constexpr (EPI == GM_SEGS && MT == 2) { // 32 rows a wave: (d .. d + 15, d + 32 .. d + 47) of one head
+        if constexpr (EPI == GM_SEGS) { // 32 rows a wave: (d .. d + 15, d + 32 .. d + 47) of one head
             const int q = tx * RW + lt / MT;
             return (q >> 1) * 64 + 16 * (q & 1) + 32 * (lt % MT);
         }
@@ -141,7 +144,6 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
             for (int st = 0; st < nst; ++st) {
                 const int younger = min(st == 0 ? S - 1 : S - 2, nst - 1 - st);
                 if (younger >= S - 2) gm_wait<L * (S - 2)>();
-                else if (S > 3 && younger == 1) gm_wait<L>();
                 else gm_wait<0>();
                 __builtin_amdgcn_s_barrier();
                 if (st > 0 && st - 1 + S < nst) issue(st - 1 + S, buf);
@@ -168,7 +170,6 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
             for (int st = 0; st < nst; ++st) {
                 const int younger = min(st == 0 ? S - 1 : S - 2, nst - 1 - st);
                 if (younger >= S - 2) gm_wait<L * (S - 2)>();
-                else if (S > 3 && younger == 1) gm_wait<L>();
                 else gm_wait<0>();
                 __builtin_amdgcn_s_barrier();
                 if (st > 0 && st - 1 + S < nst) issue(st - 1 + S, buf);
@@ -458,16 +459,16 @@ constexpr int GM_N_TILES = 6;
 struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2]; };
 const gm_tile gm_tiles[GM_N_TILES] = {
 #define X(I, MT, NT, RW, CH, S, A_, B_)                                                          \
-    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, 4, CH, S>::LDS > 160 * 1024, \
-                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, 4, CH, S>::LDS > 160 * 1024 } },
+    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, CH, S>::LDS > 160 * 1024, \
+                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, CH, S>::LDS > 160 * 1024 } },
     GM_TILES(X)
 #undef X
 };
 
 template <int WT, int MT, int NT, int RW, int CH, int S, int EPI>
 bool gm_launch(const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
-    using sh = gm_shape<WT, MT, NT, RW, 4, CH, S>;
-    auto kern = gm_kernel<WT, MT, NT, RW, 4, CH, S, EPI>;
+    using sh = gm_shape<WT, MT, NT, RW, CH, S>;
+    auto kern = gm_kernel<WT, MT, NT, RW, CH, S, EPI>;
     static bool raised = false;
     if (!raised && sh::LDS > 64 * 1024) {
         if (hipFuncSetAttribute((const void *) kern, hipFuncAttributeMaxDynamicSharedMemorySize, sh::LDS) != hipSuccess) { (void) hipGetLastError(); return false; }
