@@ -16,10 +16,11 @@
 //     vector instruction every four cycles, so an exactly scaled 16 x 16 x 32 product costs its own slot and four
 //     additions, 20 cycles against the matrix core's 16, plus the conversions -- 7 slots in all at two row tiles x eight
 //     token tiles a wave.
-// Measured on cold weights (microseconds a launch, without the 3 us of the activation pass, which the norm's launch was
-// before; in brackets the streaming / LDS-tiled kernels of mul_mat.hip): 203 tokens: 1024 x 1024 4.7 [10.7], 1024 x 4096 8.8
-// [16.6 + 4.4 for the K cut's second launch], gate/up pair 10.9 [20.7]; 45 tokens: 3.7 [5.8], 6.7 [9.9 + 6.0], 6.0 [7.3 +
-// 7.3 + 3.4]; 1024 tokens: 7.5 [10], 17.7 [26 + 5.5], 38 [46].
+// Under the tracer, microseconds a launch in a stack of 24 layers (the activation pass, which the norm's launch was before, is
+// 3.4 to 4.8 of its own): 45 tokens: norm + q / k / v + rope 6.6, gate/up pair 7.6, o and down 7.5 on average; 1024 tokens: 12, 39, o
+// 10, down 23.  Whole prompts against the streaming / LDS-tiled kernels of mul_mat.hip and the launches around them: 45 tokens
+// 1729 -> 1108 us, 203 2329 -> 1579, 2 x 512 4408 -> 2850.  Counters of the pair at 1024 tokens: 10.4 vector instructions a matrix
+// instruction, epilogue and GLU included; they issue in half of the SIMDs' cycles and the matrix cores are busy in a fifth.
 #include "gemm_mid.hpp"
 #include "kvs_common.hpp"
 #include "mm_common.hpp"
