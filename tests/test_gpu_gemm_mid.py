@@ -183,6 +183,20 @@ def test_first_call_of_a_stream_under_capture(pkg, gpu, K, M, N, wtype):
         ok(pkg, L.vx_stream_synchronize(s), "sync")
     ok(pkg, L.vx_graph_destroy(graph), "graph")
     ok(pkg, L.vx_stream_destroy(s), "stream")
+    # the same under a capture that forbids other threads' unsafe calls as well (torch's)
+    ok(pkg, L.vx_stream_create(C.byref(s)), "stream")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.ExternalStream(s.value)):
+        rc = L.vx_mul_mat(w, d(x), d(out), pkg.ACT_FLOAT, s)
+    assert rc == 0
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert same_bits(out, want)
+    del g
+    ok(pkg, L.vx_stream_destroy(s), "stream")
 
 
 @pytest.mark.parametrize("M,last,wtype", [(1024, 192, "q8"), (4096, 48, "q8"), (1024, 64, "f16"), (128, 1024, "f16")])
