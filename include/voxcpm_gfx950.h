@@ -514,6 +514,34 @@ VX_API int vx_supports_get_rows(const vx_tensor * table, const vx_tensor * rows,
 VX_API int vx_supports_concat(const vx_tensor * src0, const vx_tensor * src1, const vx_tensor * dst, int dim);
 VX_API int vx_supports_sum(const vx_tensor * src, const vx_tensor * dst);
 
+/* ---- a decoder stack over a few token rows as one call ------------------------------------------------
+ * MiniCPMModel::forward_step / forward (src/minicpm.cpp:572-846) for at most 16 token rows: n_layer layers of rms_norm, q / k / v
+ * with their rotations, attention, o projection and residual update, rms_norm, SwiGLU MLP and residual update, then the final
+ * rms_norm; Q8_0 weights, activations in float (VX_ACT_FLOAT).  Either a decode step -- one token of each of `batch` sequences,
+ * n_past cached keys, the step's keys and values written to the caches (write_kv; the ordering scalar of the graph's cache write,
+ * (sum k + sum v) * sync_scale + sync_bias, is added to the attention's result) -- or whole sequences of n_tokens that attend to
+ * themselves and leave no cache (n_past 0; mask: F16 [n_tokens][n_tokens] or NULL).  The results are the bits of the separate calls.
+ * x and out: dense F32 [batch][n_tokens][hidden].  Weight rows are dense Q8_0 blocks, norms dense F32.  cache_nb1 / nb2 / nb3: byte
+ * strides of a cache's rows, heads and sequences, the same for K and V of every layer.  positions: n_tokens int32 on the device.
+ * No counterpart in ggml-cpu, which runs the nodes one by one. */
+#define VX_STACK_MAX_LAYERS 32
+typedef struct vx_stack_layer {
+    const void * q_proj, * k_proj, * v_proj, * o_proj, * gate_proj, * up_proj, * down_proj;
+    const void * input_norm, * post_norm;
+    void * k_cache, * v_cache;
+} vx_stack_layer;
+typedef struct vx_stack {
+    const vx_stack_layer * layers;
+    const void * x; void * out; const void * norm;
+    const int32_t * positions; const float * rope_factors; const void * mask;
+    uint64_t mask_nb1, cache_nb1, cache_nb2, cache_nb3;
+    int32_t n_layer, batch, n_tokens, n_past, hidden, ffn, n_heads, n_kv_heads, head_dim, kv_type, write_kv, rope_n_ctx_orig;
+    float   eps, residual_scale, attn_scale, sync_scale, sync_bias;
+    float   rope_base, rope_freq_scale, rope_ext_factor, rope_attn_factor, rope_beta_fast, rope_beta_slow;
+} vx_stack;
+VX_API int vx_supports_stack(const vx_stack * stack);
+VX_API vx_status vx_stack_run(const vx_stack * stack, vx_stream stream);
+
 #ifdef __cplusplus
 }
 #endif

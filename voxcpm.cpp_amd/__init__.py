@@ -46,6 +46,23 @@ class VxSmallNode(C.Structure):
     ]
 
 
+class VxStackLayer(C.Structure):
+    _fields_ = [(n, C.c_void_p) for n in ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj",
+                                          "input_norm", "post_norm", "k_cache", "v_cache")]
+
+
+class VxStack(C.Structure):
+    _fields_ = ([("layers", C.POINTER(VxStackLayer))] +
+                [(n, C.c_void_p) for n in ("x", "out", "norm", "positions", "rope_factors", "mask")] +
+                [(n, C.c_uint64) for n in ("mask_nb1", "cache_nb1", "cache_nb2", "cache_nb3")] +
+                [(n, C.c_int32) for n in ("n_layer", "batch", "n_tokens", "n_past", "hidden", "ffn", "n_heads", "n_kv_heads", "head_dim",
+                                          "kv_type", "write_kv", "rope_n_ctx_orig")] +
+                [(n, C.c_float) for n in ("eps", "residual_scale", "attn_scale", "sync_scale", "sync_bias", "rope_base", "rope_freq_scale",
+                                          "rope_ext_factor", "rope_attn_factor", "rope_beta_fast", "rope_beta_slow")])
+
+
+ERR_UNSUPPORTED = 2
+STACK_MAX_LAYERS = 32
 SMALL_DST_PRIVATE = 1
 
 EXPORTS = [
@@ -63,7 +80,7 @@ EXPORTS = [
     "vx_supports_cpy", "vx_supports_concat", "vx_supports_sum",
     "vx_arange", "vx_repeat", "vx_get_rows", "vx_supports_arange", "vx_supports_repeat", "vx_supports_get_rows",
     "vx_small_graph", "vx_supports_small_node", "vx_mul_mat_sum_order",
-    "vx_rms_norm_mul", "vx_scale_add", "vx_add_scale", "vx_flash_attn_ext_add1", "vx_mul_mat_swiglu", "vx_supports_mul_mat_swiglu", "vx_supports_mul_mat_swiglu_tiled", "vx_mul_mat_scale_add", "vx_supports_mul_mat_scale_add", "vx_kv_store_sync", "vx_supports_kv_store_sync", "vx_flash_attn_ext_kv2", "vx_supports_flash_attn_ext_kv2", "vx_flash_attn_ext_kv2_store", "vx_supports_flash_attn_ext_kv2_store", "vx_flash_attn_ext_store", "vx_supports_flash_attn_ext_store", "vx_flash_attn_ext_store_proj", "vx_supports_flash_attn_ext_store_proj", "vx_qkv_proj_rope", "vx_supports_qkv_proj_rope", "vx_kv_proj_rope", "vx_supports_kv_proj_rope", "vx_norm_qkv_proj_rope", "vx_supports_norm_qkv_proj_rope", "vx_norm_mul_mat_swiglu", "vx_supports_norm_qkv_proj_rope_tiled", "vx_supports_mlp_tiled", "vx_mlp_tiled", "vx_supports_norm_mul_mat_swiglu_tiled", "vx_supports_norm_mul_mat_swiglu", "vx_supports_rms_norm_mul", "vx_supports_fused_pair",
+    "vx_rms_norm_mul", "vx_scale_add", "vx_add_scale", "vx_flash_attn_ext_add1", "vx_mul_mat_swiglu", "vx_supports_mul_mat_swiglu", "vx_supports_mul_mat_swiglu_tiled", "vx_mul_mat_scale_add", "vx_supports_mul_mat_scale_add", "vx_kv_store_sync", "vx_supports_kv_store_sync", "vx_flash_attn_ext_kv2", "vx_supports_flash_attn_ext_kv2", "vx_flash_attn_ext_kv2_store", "vx_supports_flash_attn_ext_kv2_store", "vx_flash_attn_ext_store", "vx_supports_flash_attn_ext_store", "vx_flash_attn_ext_store_proj", "vx_supports_flash_attn_ext_store_proj", "vx_qkv_proj_rope", "vx_supports_qkv_proj_rope", "vx_kv_proj_rope", "vx_supports_kv_proj_rope", "vx_norm_qkv_proj_rope", "vx_supports_norm_qkv_proj_rope", "vx_norm_mul_mat_swiglu", "vx_supports_norm_qkv_proj_rope_tiled", "vx_supports_mlp_tiled", "vx_mlp_tiled", "vx_supports_norm_mul_mat_swiglu_tiled", "vx_supports_norm_mul_mat_swiglu", "vx_supports_rms_norm_mul", "vx_supports_fused_pair", "vx_supports_stack", "vx_stack_run",
 ]
 
 BIN_ADD, BIN_SUB, BIN_MUL, BIN_DIV = 0, 1, 2, 3
@@ -170,6 +187,8 @@ def lib():
     l.vx_supports_kv_store_sync.argtypes = [TP, TP, TP, TP, TP, TP]
     l.vx_flash_attn_ext_kv2.argtypes = [TP, TP, TP, TP, TP, TP, f32p, TP, C.c_float, C.c_float, C.c_float, vp]
     l.vx_supports_flash_attn_ext_kv2.argtypes = [TP, TP, TP, TP, TP, TP, TP]
+    l.vx_supports_stack.argtypes = [C.POINTER(VxStack)]
+    l.vx_stack_run.argtypes = [C.POINTER(VxStack), vp]
     l.vx_flash_attn_ext_kv2_store.argtypes = [TP, TP, TP, TP, TP, TP, f32p, TP, TP, TP, TP, TP] + [C.c_float] * 5 + [vp]
     l.vx_supports_flash_attn_ext_kv2_store.argtypes = [TP] * 11
     l.vx_flash_attn_ext_store.argtypes = [TP, TP, TP, TP, f32p, TP, TP, TP, TP, TP] + [C.c_float] * 5 + [vp]

@@ -25,7 +25,8 @@ import math
 
 import numpy as np
 
-from . import (ACT_FLOAT, BIN_ADD, BIN_MUL, F16, F32, GLU_SWIGLU, _p, _stream, check, desc, desc_q8, lib)
+from . import (ACT_FLOAT, BIN_ADD, BIN_MUL, ERR_UNSUPPORTED, F16, F32, GLU_SWIGLU, STACK_MAX_LAYERS, VxStack, VxStackLayer, _p, _stream, check,
+               desc, desc_q8, lib)
 
 WEIGHT_NAMES = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
 
@@ -326,8 +327,15 @@ class MiniCPMBackbone:
         o2 = out.view(N, self.hidden)
         norm(cur_x, self.final_norm, o2)
 
+        stack = self._stack(x, out, pos, T, n_past, mask, write_kv, attn_factor) if fuse else None
+
         def run():
             st = _stream()
+            if stack is not None:   # all of it as one resident launch, the same bits
+                rc = L.vx_stack_run(stack, st)
+                if rc != ERR_UNSUPPORTED:
+                    check(rc, "vx_stack_run")
+                    return
             for fn, args in calls:
                 rc = fn(*args, st)
                 if rc:
@@ -337,6 +345,41 @@ class MiniCPMBackbone:
         run.calls = calls           # (function, arguments) in launch order, for tools that time parts of a step
         run.n_calls = len(calls)
         return run, out
+
+    def _stack(self, x, out, pos, T, n_past, mask, write_kv, attn_factor):
+        """The whole plan as vx_stack_run's argument where that takes it (a decode step, or one pass without a cache, of at
+        most 16 token rows), else None."""
+        torch = self.torch
+        if self.act_mode != ACT_FLOAT or self.n_layer > STACK_MAX_LAYERS or (mask is not None and (mask.dim() != 2 or mask.stride(1) != 1)):
+            return None
+        if mask is not None and (mask.dtype != torch.float16 or mask.shape[0] < T or mask.shape[1] != T):
+            return None
+        layers = (VxStackLayer * self.n_layer)()
+        kc = self.k_cache[0]
+        es = kc.element_size()
+        for li, s in enumerate(layers):
+            w, nrm = self.weights[li], self.norms[li]
+            for name in WEIGHT_NAMES:
+                rows, k = w[name]
+                want = {"o_proj": (self.hidden, self.n_heads * self.D), "gate_proj": (self.ffn, self.hidden), "up_proj": (self.ffn, self.hidden),
+                        "down_proj": (self.hidden, self.ffn), "q_proj": (self.n_heads * self.D, self.hidden)}.get(name, (self.n_kv * self.D, self.hidden))
+                if not rows.is_contiguous() or (rows.shape[0], k) != want:
+                    return None
+                setattr(s, name, rows.data_ptr())
+            s.input_norm, s.post_norm = _p(nrm["input_layernorm"]), _p(nrm["post_layernorm"])
+            for t in (self.k_cache[li], self.v_cache[li]):
+                if t.stride() != kc.stride() or t.stride(3) != 1:
+                    return None
+            s.k_cache, s.v_cache = self.k_cache[li].data_ptr(), self.v_cache[li].data_ptr()
+        st = VxStack(layers=layers, x=x.data_ptr(), out=out.data_ptr(), norm=_p(self.final_norm), positions=_p(pos), rope_factors=_p(self.rope_factors),
+                     mask=_p(mask), mask_nb1=0 if mask is None else 2 * mask.stride(0), cache_nb1=es * kc.stride(2), cache_nb2=es * kc.stride(1),
+                     cache_nb3=es * kc.stride(0), n_layer=self.n_layer, batch=self.batch, n_tokens=T, n_past=n_past, hidden=self.hidden, ffn=self.ffn,
+                     n_heads=self.n_heads, n_kv_heads=self.n_kv, head_dim=self.D, kv_type=F16 if self.kv_dtype == torch.float16 else F32,
+                     write_kv=int(bool(write_kv)), rope_n_ctx_orig=self.rope_original_max, eps=self.eps,
+                     residual_scale=self.residual_scale if self.use_mup else 1.0, attn_scale=1.0 / math.sqrt(self.D), sync_scale=0.0, sync_bias=0.0,
+                     rope_base=self.rope_base, rope_freq_scale=1.0, rope_ext_factor=0.0, rope_attn_factor=attn_factor, rope_beta_fast=32.0,
+                     rope_beta_slow=1.0)
+        return st if lib().vx_supports_stack(st) else None
 
     def forward(self, x, n_past=0, mask=None, write_kv=True):
         """MiniCPMModel::forward / forward_step: x (batch, n_tokens, hidden) -> same shape."""

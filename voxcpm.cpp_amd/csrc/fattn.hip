@@ -35,6 +35,7 @@
 #include <type_traits>
 #include "vx_common.hpp"
 #include "kvs_common.hpp"
+#include "stack.hpp"
 
 #include <cmath>
 #include <cstdlib>
@@ -994,6 +995,17 @@ void launch_cols16_pre(const fa_args & a, hipStream_t st) {
 }
 
 } // namespace
+
+bool vx_fattn_stack_plan(int64_t tiles, int n_kv, bool f16, int * n_splits, int * chunk) {
+    fa_args a{};
+    a.n_kv = n_kv;
+    if (f16 && n_kv > 64 && !fa_dec64_takes(a, 64, false)) return false;
+    fa_split_plan(tiles, n_kv, n_splits, chunk);
+    return true;
+}
+bool vx_fattn_stack_self(int64_t tokens, int64_t gqa) {
+    return tokens <= 16 && tokens * gqa < 256; // (from 256 columns on the LDS-tiled kernel may take it)
+}
 
 extern "C" int vx_supports_flash_attn_ext(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v,
                                           const vx_tensor * mask, const vx_tensor * dst) {

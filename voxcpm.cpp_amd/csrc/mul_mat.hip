@@ -27,6 +27,7 @@
 #include "mm_common.hpp"
 #include "gemm_mid.hpp"
 #include "rope_common.hpp"
+#include "stack.hpp"
 
 #include <cstdlib>
 #include <type_traits>
@@ -3162,6 +3163,9 @@ extern "C" int vx_supports_qkv_proj_rope(const vx_tensor * wq, const vx_tensor *
 // products with equal K, token count of the call and number are summed identically.  It depends on the row count, so a backend
 // that runs a product over a row range of a matrix in place of the product over the whole matrix (the reference's row-fused
 // qkv_proj / gate_up_proj) compares the two before promising identical bits.
+int vx_gemv_waves(int64_t K, int64_t tokens, int64_t M) { return gemv_waves_for(K, tokens, M); }
+int vx_gemv_dma_slot(int64_t K) { return gemv_dma_slot(K); }
+
 extern "C" int vx_mul_mat_sum_order(int64_t K, int64_t tokens, int64_t M) {
     if (K < 32 || K % 32 || tokens < 1 || M < 1) return 0;
     // (shapes of gemm_mid.hip's kernel but for their rows, with either weight type: another kernel's order)
