@@ -908,7 +908,7 @@ __global__ __launch_bounds__(64) void fattn_dec64_kernel(const fa_args a) {
             const bool  vis   = cm != -INFINITY;
             const float delta = !vis ? 0.0f : (seen ? fmaxf(cm, 0.0f) : cm);
             seen = seen || vis;
-            const float f = __builtin_amdgcn_exp2f(-delta);
+            const float f = __builtin_amdgcn_exp2f(-fmaxf(delta, 0.0f)); // (a first reference below zero scales sums of zero: by 1, not by what may be inf)
             s[0] -= delta;
             s[1] -= delta;
             negm -= delta;

@@ -586,7 +586,9 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             const float delta = !vis ? 0.0f : (seen[cb] ? fmaxf(cm, 0.0f) : cm);
             seen[cb] = seen[cb] || vis;
             if (__builtin_amdgcn_ballot_w64(delta != 0.0f) == 0) return; // nothing moves (wave-uniform)
-            const float f = __builtin_amdgcn_exp2f(-delta);
+            // (a column's first reference may lie anywhere below zero -- scores of -200, a mask of the lowest finite value -- and what it
+            // would scale is zero: by 1, not by an exponential that overflows, 0 * inf)
+            const float f = __builtin_amdgcn_exp2f(-fmaxf(delta, 0.0f));
             s -= delta;
             if (same_cb_inflight) s_inflight -= delta; // scores already formed against the old reference
             negm[cb] -= delta;
