@@ -1,4 +1,5 @@
-"""GPU: prefill attention (csrc/fattn_prefill.hip, pf_kernel) against the same attention in float64; scores far below zero there and
+"""GPU: prefill attention (csrc/fattn_prefill.hip, pf_kernel) against the same attention in float64: two teams of waves with one tile
+or none for the second, an odd last tile, columns that one team or nobody sees, both sides of the rule's line; scores far below zero there and
 in the decode kernel (csrc/fattn.hip, fattn_dec64_kernel)."""
 import pytest
 
@@ -54,3 +55,33 @@ def test_first_scores_far_below_zero(pkg, gpu, B, n_q, n, case, f16):
     if f16:
         k, v = k.half(), v.half()
     check(q, k, v, mask, 0.125, None, gpu.flash_attn_ext(q, k, v, mask, 0.125))
+
+
+def masks(kind, n_q, n_kv, g):
+    import torch
+    i, j = torch.arange(n_q)[:, None] + (n_kv - n_q), torch.arange(n_kv)[None]
+    vis = {"causal": j <= i, "one tile": (j // 64 == min(3, (n_kv - 1) // 64)) & (i >= 0), "second team only": (j // 64 == 1) & (i % 3 > 0),
+           "either team": (j // 64) % 2 == (i // 5) % 2, "hidden rows": (j <= i) & (i % 7 > 0), "all hidden": (j < 0) & (i >= 0), "values": j <= i + 100}[kind]
+    m = torch.where(vis, torch.from_numpy(g.standard_normal((n_q, n_kv)).astype("float32")) if kind == "values" else torch.tensor(0.0), torch.tensor(float("-inf")))
+    if kind == "either team":
+        m[3::11] = -65504.0     # the lowest finite value is a value, not a hidden key
+    return m.half().view(1, 1, n_q, n_kv).contiguous().cuda()
+
+
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("B,n_q,n_kv,kind,sinks", [
+    (1, 512, 512, "causal", False), (1, 257, 64, "one tile", False), (1, 300, 333, "one tile", True), (1, 260, 100, "second team only", True),
+    (2, 270, 460, "either team", False), (1, 523, 523, "hidden rows", True), (1, 256, 300, "all hidden", False), (1, 400, 777, "values", False),
+    (1, 513, 1025, None, True), (1, 2048, 2048, "causal", False), (1, 2049, 2049, "causal", False), (2, 1170, 1170, "causal", False),
+    (2, 1500, 1500, "causal", False), (2, 1700, 1700, "causal", False), (4, 520, 520, "causal", False), (1, 2049, 2049, None, False)])
+def test_prefill_attention_by_two_teams(pkg, gpu, B, n_q, n_kv, kind, sinks, f16):
+    import torch
+    say(f"prefill attention, two teams: {B} x {n_q}/{n_kv} {kind} sinks={sinks} f16={f16}")
+    H, Hkv, D, scale = 16, 2, 64, 0.125
+    g = rng("teams", B, n_q, n_kv)
+    q, k, v = (dev(g.standard_normal((B, h, n, D)).astype("float32")) for h, n in ((H, n_q), (Hkv, n_kv), (Hkv, n_kv)))
+    if f16:
+        k, v = k.half(), v.half()
+    mask = masks(kind, n_q, n_kv, g) if kind else None
+    sk = dev(g.standard_normal(H).astype("float32")) if sinks else None
+    check(q, k, v, mask, scale, sk, gpu.flash_attn_ext(q, k, v, mask, scale, sinks=sk))

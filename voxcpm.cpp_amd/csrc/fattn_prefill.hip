@@ -159,6 +159,13 @@ __device__ __forceinline__ void pf_dma4(const char * base, uint32_t off, uint32_
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
 }
 
+// Two probabilities to f16, to nearest (v_cvt_pk_f16_f32).  Rounded toward zero, a column's reference key alone would keep its value,
+// 1, while all others lose half a unit on average: with two references a column (two teams) that was 0.8 % of the whole error.
+__device__ __forceinline__ half2_t pf_cvt2(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    return __builtin_convertvector(f2{a, b}, half2_t);
+}
+
 __device__ __forceinline__ half8_t pf_tr8(const lds_char * p) {
     typedef short short4_t __attribute__((ext_vector_type(4)));
     typedef short short8_t __attribute__((ext_vector_type(8)));
@@ -284,22 +291,27 @@ __global__ __launch_bounds__(128) void pf_scalar_kernel(const double * totals, i
 
 // VLO: V comes with a low-half image (a.vl).  NCB: 32-column blocks per wave.  SUMS: the addend is the ordering scalar of a.totals
 // (an instance of its own: as a test in every instance it cost the calls without a cache write 1 %, 2048 causal tokens 38.7 -> 39.1 us).
-template <bool VLO, int NCB, bool SUMS = false>
-__global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_kernel(const pf_args a) {
+// TEAMS: sets of PF_WAVES waves over the same columns, each with every TEAMS-th active tile and stages of its own, their (O, sum,
+// reference) joined through LDS at the end.  A wave alone on its SIMD leaves half of the issue slots empty (0.92 us a tile; two that
+// share the SIMD take 0.62 us each), so a row block walks 64 tiles in about 45 us where one team takes 62; against a cut of the
+// key range into work-groups of their own nothing goes through memory and no launch follows.  One sequence of 4096 tokens 72 -> 64 us.
+template <bool VLO, int NCB, bool SUMS = false, int TEAMS = 1>
+__global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_kernel(const pf_args a) {
     constexpr int D = 64;
     constexpr int PF_STAGES = VLO ? 3 : PF_STAGES_MAX; // (three stages of K, V and V low leave room for two work-groups on a compute unit)
     constexpr int NL = VLO ? 6 : 4; // direct loads per wave and tile (a tile that needs its visibility bits has one more)
-    __shared__ __attribute__((aligned(1024))) char k_lds[PF_STAGES][PF_KSTAGE];
-    __shared__ __attribute__((aligned(1024))) char v_lds[PF_STAGES][PF_VSTAGE];
-    __shared__ __attribute__((aligned(1024))) char vl_lds[VLO ? PF_STAGES : 1][VLO ? PF_VSTAGE : 16];
-    __shared__ __attribute__((aligned(256))) uint32_t bits_lds[PF_STAGES][64]; // visibility bits of the block's rows: 8 bytes per row
+    __shared__ __attribute__((aligned(1024))) char k_lds[TEAMS][PF_STAGES][PF_KSTAGE];
+    __shared__ __attribute__((aligned(1024))) char v_lds[TEAMS][PF_STAGES][PF_VSTAGE];
+    __shared__ __attribute__((aligned(1024))) char vl_lds[VLO ? TEAMS : 1][VLO ? PF_STAGES : 1][VLO ? PF_VSTAGE : 16];
+    __shared__ __attribute__((aligned(256))) uint32_t bits_lds[TEAMS][PF_STAGES][64]; // visibility bits of the block's rows: 8 bytes per row
     __shared__ uint16_t tile_list[PF_MAX_TILES];
     __shared__ uint8_t  tile_flag[PF_MAX_TILES];
     __shared__ int      n_active_s;
     __shared__ float    y_s; // SUMS
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wid  = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = TEAMS == 1 ? wid : wid % PF_WAVES, team = TEAMS == 1 ? 0 : wid / PF_WAVES;
     const int hl = lane >> 5, cl = lane & 31;
 
     // ---- which (batch, kv head, row block): heavy (late) row blocks first; blocks of one
@@ -338,7 +350,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
     }
 
     // ---- active key tiles of this row block
-    if (wave == 0) {
+    if (wid == 0) {
         int base = 0;
         for (int t0 = 0; t0 < a.n_tiles; t0 += 64) {
             const int t = t0 + lane;
@@ -364,7 +376,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             base += __builtin_popcountll(bal);
         }
         if (lane == 0) n_active_s = base;
-    } else if (SUMS && wave == 1) { // the cache write's ordering scalar: k's totals in the low half of the wave, v's in the high
+    } else if (SUMS && wid == 1) { // the cache write's ordering scalar: k's totals in the low half of the wave, v's in the high
         const int n = hl ? a.n_tv : a.n_tk;
         double tot[PF_TOTALS_INLINE / 32];
 #pragma unroll
@@ -380,7 +392,8 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
         if (lane == 0) y_s = kvs_scalar(sum, sv, a.sync_scale, a.sync_bias);
     }
     __syncthreads();
-    const int n_active = __builtin_amdgcn_readfirstlane(n_active_s);
+    const int n_all = __builtin_amdgcn_readfirstlane(n_active_s);
+    const int n_active = TEAMS == 1 ? n_all : (n_all - team + TEAMS - 1) / TEAMS; // this team's: tiles team, team + TEAMS, ... of the list
 
     // Softmax bookkeeping.  Probabilities are taken relative to a per-column *reference* that trails the running maximum:
     // the S^T accumulator starts at -reference (the same value in a lane's 16 registers: a lane holds one column).  The
@@ -406,10 +419,10 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const char * kg = a.k + (uint64_t) g * a.nbk2 + (uint64_t) (b / a.rk3) * a.nbk3;
         const char * vg = a.v + (uint64_t) g * a.nbv2 + (uint64_t) (b / a.rk3) * a.nbv3;
         const char * vlg = VLO ? a.vl + (uint64_t) g * a.nbv2 + (uint64_t) (b / a.rk3) * a.nbv3 : nullptr;
-        const uint32_t k_base = (uint32_t) (uintptr_t) (lds_char *) &k_lds[0][0];
-        const uint32_t v_base = (uint32_t) (uintptr_t) (lds_char *) &v_lds[0][0];
-        const uint32_t vl_base = (uint32_t) (uintptr_t) (lds_char *) &vl_lds[0][0];
-        const uint32_t bits_base = (uint32_t) (uintptr_t) (lds_char *) &bits_lds[0][0];
+        const uint32_t k_base = (uint32_t) (uintptr_t) (lds_char *) &k_lds[team][0][0];
+        const uint32_t v_base = (uint32_t) (uintptr_t) (lds_char *) &v_lds[team][0][0];
+        const uint32_t vl_base = (uint32_t) (uintptr_t) (lds_char *) &vl_lds[VLO ? team : 0][0][0];
+        const uint32_t bits_base = (uint32_t) (uintptr_t) (lds_char *) &bits_lds[team][0][0];
         // the rows' visibility bits of a tile (used when the tile's flag is 3): lane = (row lane / 2, dword lane % 2); every
         // wave fetches the block's 256 bytes (the same bytes to the same place), only for tiles that need them
         const char * bits_src = a.bits ? (const char *) a.bits + ((uint64_t) (b % a.nem3) * a.nem2 * a.n_q) * a.n_tiles * 8 : a.q;
@@ -440,7 +453,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
         int dma_last = 0, dma_stage = 0, dma_tile = 0;
         bool dma_bits = false;
         auto issue_setup = [&](int idx, int stage) {
-            const int at = min(idx, n_active - 1);
+            const int at = TEAMS * min(idx, n_active - 1) + team;
             const int tile = __builtin_amdgcn_readfirstlane(tile_list[at]);
             dma_kt = kg + (uint64_t) tile * PF_KT * a.nbk1;
             dma_vt = vg + (uint64_t) tile * PF_KT * a.nbv1;
@@ -497,15 +510,15 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
         {
             const int r8 = cl & 7;
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) kad[kk] = (uint32_t) ((cl >> 3) * PF_KBLK + r8 * 128 + (((2 * kk + hl) ^ r8) << 4));
+            for (int kk = 0; kk < 4; ++kk) kad[kk] = (uint32_t) (team * PF_STAGES * PF_KSTAGE + (cl >> 3) * PF_KBLK + r8 * 128 + (((2 * kk + hl) ^ r8) << 4));
             const int i = lane & 15, gg = (lane >> 4) & 1;
 #pragma unroll
             for (int dt = 0; dt < 2; ++dt)
-                vad[dt] = (uint32_t) ((4 * hl + (i >> 2)) * 128 + (((4 * dt + 2 * gg + ((i & 3) >> 1)) ^ (2 * (i >> 2))) << 4) + 8 * (i & 1));
+                vad[dt] = (uint32_t) (team * PF_STAGES * PF_VSTAGE + (4 * hl + (i >> 2)) * 128 + (((4 * dt + 2 * gg + ((i & 3) >> 1)) ^ (2 * (i >> 2))) << 4) + 8 * (i & 1));
         }
-        const lds_char * const k_lds0 = (const lds_char *) &k_lds[0][0];
-        const lds_char * const v_lds0 = (const lds_char *) &v_lds[0][0];
-        const lds_char * const vl_lds0 = (const lds_char *) &vl_lds[0][0];
+        const lds_char * const k_lds0 = (const lds_char *) &k_lds[0][0][0]; // (a team's own lie in the lane's offset)
+        const lds_char * const v_lds0 = (const lds_char *) &v_lds[0][0][0];
+        const lds_char * const vl_lds0 = (const lds_char *) &vl_lds[0][0][0];
 
         // The walk is a software pipeline over *units* (a 32-key block x one of the wave's 32-column blocks; 2 NCB per tile,
         // column blocks alternating).  A step handles unit u as 8 groups of { one matrix instruction; exp2, exp2, convert,
@@ -551,7 +564,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
                 const int rl  = col < ncols_blk ? (col >> a.gqa_sh) : 0;
                 uint32_t w;
                 if (a.bits) {
-                    w = bits_lds[stage][2 * rl + kb];
+                    w = bits_lds[team][stage][2 * rl + kb];
                 } else { // no mask: the bounds
                     const int left = a.n_kv - tile * PF_KT - 32 * kb;
                     w = left >= 32 ? 0xFFFFFFFFu : (left <= 0 ? 0u : (1u << left) - 1u);
@@ -597,13 +610,12 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
             l[cb] *= f;
         };
         auto probs = [&](const float16_t & s, int4_t (&pb)[2], float & lt) {
-            typedef __fp16 fp16x2 __attribute__((ext_vector_type(2)));
             half2_t acc = half2_t{(_Float16) 0.0f, (_Float16) 0.0f};
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const fp16x2 pr = __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_exp2f(s[2 * i]), __builtin_amdgcn_exp2f(s[2 * i + 1]));
+                const half2_t pr = pf_cvt2(__builtin_amdgcn_exp2f(s[2 * i]), __builtin_amdgcn_exp2f(s[2 * i + 1]));
                 pb[i >> 2][i & 3] = __builtin_bit_cast(int, pr);
-                acc += __builtin_bit_cast(half2_t, pr);
+                acc += pr;
             }
             lt = (float) acc[0] + (float) acc[1];
         };
@@ -629,8 +641,8 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
 
         for (int it = 0; it < n_active; ++it) {
             const int  stage  = it % PF_STAGES, stage1 = (it + 1) % PF_STAGES;
-            const int  tile   = __builtin_amdgcn_readfirstlane(tile_list[it]);
-            const int  flag   = __builtin_amdgcn_readfirstlane(tile_flag[it]); // 1 plain, 2 mask values, 3 visibility bits
+            const int  tile   = __builtin_amdgcn_readfirstlane(tile_list[TEAMS * it + team]);
+            const int  flag   = __builtin_amdgcn_readfirstlane(tile_flag[TEAMS * it + team]); // 1 plain, 2 mask values, 3 visibility bits
 
 #pragma unroll
             for (int k = 0; k < NU; ++k) {
@@ -658,7 +670,6 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
                 }
                 float lt = 0.0f;
                 half2_t acc2 = half2_t{(_Float16) 0.0f, (_Float16) 0.0f};
-                typedef __fp16 fp16x2 __attribute__((ext_vector_type(2)));
                 // matrix instruction i of the step, and the operand reads that follow it
                 auto mat = [&](int i) {
                     if (i < 4) {
@@ -692,18 +703,18 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
                     mat(i);
                     const float na = __builtin_amdgcn_exp2f(sbuf[cur][2 * i]), nb = __builtin_amdgcn_exp2f(sbuf[cur][2 * i + 1]);
                     if (i > 0) {
-                        const fp16x2 pr = __builtin_amdgcn_cvt_pkrtz(ea, eb);
+                        const half2_t pr = pf_cvt2(ea, eb);
                         pbuf[cur][(i - 1) >> 2][(i - 1) & 3] = __builtin_bit_cast(int, pr);
-                        acc2 += __builtin_bit_cast(half2_t, pr);
+                        acc2 += pr;
                     }
                     ea = na;
                     eb = nb;
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 {
-                    const fp16x2 pr = __builtin_amdgcn_cvt_pkrtz(ea, eb);
+                    const half2_t pr = pf_cvt2(ea, eb);
                     pbuf[cur][1][3] = __builtin_bit_cast(int, pr);
-                    acc2 += __builtin_bit_cast(half2_t, pr);
+                    acc2 += pr;
                 }
                 lt = (float) acc2[0] + (float) acc2[1];
                 asm volatile("" : "+v"(lt));
@@ -732,6 +743,37 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
         pv_all(NCB - 1, pbuf[(NU - 1) & 1]); // the last unit's
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the loads issued past the last tile
     }
+    if constexpr (TEAMS == 2) {
+        static_assert(NCB == 1, "the hand-over below is one column block's");
+        // The walk's barriers are the work-group's: one in front, one a tile.  The second team makes up for the tile it has
+        // not, or for a walk it has not at all.  (A loop of its own: a wave's count is uniform.)
+        const int mine = n_active > 0 ? n_active + 1 : 0, most = n_all > 0 ? (n_all + 1) / 2 + 1 : 0;
+        for (int i = mine; i < most; ++i) asm volatile("s_barrier" ::: "memory");
+        __syncthreads(); // nobody reads a stage any more, and every direct load has landed
+        // the second team's sums through its own stages: o by register and lane, then the column's L and reference
+        float * const po = (float *) &k_lds[1][0][0] + wave * (16 + 2) * 64, * const po1 = (float *) &v_lds[1][0][0] + wave * 16 * 64;
+        static_assert(PF_WAVES * 18 * 64 * 4 <= PF_STAGES * PF_KSTAGE && PF_WAVES * 16 * 64 * 4 <= PF_STAGES * PF_VSTAGE, "room for a team's sums");
+        l[0] += __shfl_xor(l[0], 32, 64); // (the two lanes of a column hold disjoint keys)
+        if (team == 1) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) { po[r * 64 + lane] = o[0][0][r]; po1[r * 64 + lane] = o[0][1][r]; }
+            po[16 * 64 + lane] = l[0];
+            po[17 * 64 + lane] = -negm[0][0];
+        }
+        __syncthreads();
+        if (team == 1) return;
+        const float L1 = po[16 * 64 + lane], M1 = po[17 * 64 + lane], M0 = -negm[0][0];
+        // (a column that saw no key has the sum 0 and no reference; one that did has at least its largest score's 1)
+        const float m  = l[0] == 0.0f ? M1 : L1 == 0.0f ? M0 : fmaxf(M0, M1);
+        const float f0 = l[0] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(M0 - m), f1 = L1 == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(M1 - m);
+        l[0] = l[0] * f0 + L1 * f1;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            o[0][0][r] = o[0][0][r] * f0 + po[r * 64 + lane] * f1;
+            o[0][1][r] = o[0][1][r] * f0 + po1[r * 64 + lane] * f1;
+            negm[0][r] = -m;
+        }
+    }
 
     // ---- finish: lane (hl, cl), d block dt, register r holds d = 32 dt + 8 (r / 4) + 4 hl + r % 4 of column cl
     int lane_e = threadIdx.x & 63; // (worked out again rather than kept alive through the walk)
@@ -745,7 +787,7 @@ __global__ __launch_bounds__(64 * PF_WAVES) __attribute__((amdgpu_waves_per_eu(2
         const bool ok  = col < ncols_blk;
         const int  row = row0 + (ok ? (col >> a.gqa_sh) : 0);
         const int  hd  = g * a.gqa + (ok ? (col & (a.gqa - 1)) : 0);
-        float L = l[cb] + __shfl_xor(l[cb], 32, 64); // the two lanes of a column hold disjoint keys
+        float L = TEAMS == 2 ? l[cb] : l[cb] + __shfl_xor(l[cb], 32, 64); // the two lanes of a column hold disjoint keys
         float M = -negm[cb][0]; // the reference the sums are relative to
         float ms = 1.0f;
         if (a.sinks) { // ggml/src/ggml-cpu/ops.cpp:8598-8615, in the log2 domain
@@ -811,6 +853,20 @@ bool vx_fattn_prefill_accepts(const vx_tensor * q, const vx_tensor * k, float lo
     // too few work-groups: the wave kernel spreads wider (one stream of 512 tokens, 32 blocks of 256 columns run as 64 of
     // 128: 19 us here against 28 us there; 256 tokens, 16 blocks: 15 us against 14 us)
     return (int64_t) n_rb * n_groups >= 32;
+}
+
+// Whether a grid of 128-column work-groups runs as two teams of waves over the same columns (pf_kernel's TEAMS) instead of one.
+// Up to a work-group for each of 256 compute units the second team runs on what would be idle issue slots; it costs nothing where the
+// walk is a few tiles.  Beyond, the work-groups come one after another where two of one team would share a compute unit, which
+// repays itself only where a long walk ends the call: with a mask (most of a causal mask's work-groups are short; without one all
+// are alike) and tiles enough for the number of work-groups.  Us a call, one team / two, f16 keys and values, causal:
+//   256 work-groups: 2048 tokens 38.2 / 31.1, 2 x 1024 24.3 / 21.5, 4 x 512 17.7 / 17.7; 512 new of 4096 keys (64) 62.7 / 45.5
+//   beyond: 2300 tokens (288 work-groups) 47.8 / 39.2, 4096 (512) 73.9 / 66.4, 2 x 1200 (300) 29.7 / 27.9;
+//   the line: 2 x 1500 (376) 36.6 / 35.9, 2 x 1700 (428) 39.6 / 39.9, 2 x 2048 (512) 41.1 / 41.5; 4 x 700 (352) 23.4 / 26.8.
+//   No mask: 2048 tokens (256) 32.8 / 27.9, 2300 (288) 47.6 / 54.3, 4096 (512) 91.3 / 93.2.  F32 keys and values alike.
+static bool pf_two_teams(int64_t n_wg, int n_tiles, bool masked) {
+    if (n_wg <= 256) return true;
+    return masked && n_wg <= 512 && n_tiles * (700 - n_wg) >= 7500;
 }
 
 vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
@@ -939,13 +995,18 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
         vx_launch(pf_scalar_kernel, dim3(1), dim3(PF_TOTALS), 0, st, (const double *) p.totals, a.n_tk, a.n_tv, a.sync_scale, a.sync_bias, (float *) a.add1);
         VX_LAUNCH_CHECK();
     }
-    const dim3 grid((unsigned) (n_rb * n_groups)), block(64 * PF_WAVES);
+    const dim3 grid((unsigned) (n_rb * n_groups)), block(64 * PF_WAVES), block2(2 * 64 * PF_WAVES);
+    const bool two = half_cols && pf_two_teams((int64_t) n_rb * n_groups, n_tiles, mask != nullptr);
     if (a.totals) {
         if (!half_cols)    vx_launch(pf_kernel<false, 2, true>, grid, block, 0, st, a);
+        else if (a.kv_f32 && two) vx_launch(pf_kernel<true, 1, true, 2>, grid, block2, 0, st, a);
+        else if (two)      vx_launch(pf_kernel<false, 1, true, 2>, grid, block2, 0, st, a);
         else if (a.kv_f32) vx_launch(pf_kernel<true, 1, true>, grid, block, 0, st, a);
         else               vx_launch(pf_kernel<false, 1, true>, grid, block, 0, st, a);
     } else if (half_cols) {
-        if (a.kv_f32) vx_launch(pf_kernel<true, 1>, grid, block, 0, st, a);
+        if (a.kv_f32 && two) vx_launch(pf_kernel<true, 1, false, 2>, grid, block2, 0, st, a);
+        else if (two)      vx_launch(pf_kernel<false, 1, false, 2>, grid, block2, 0, st, a);
+        else if (a.kv_f32) vx_launch(pf_kernel<true, 1>, grid, block, 0, st, a);
         else          vx_launch(pf_kernel<false, 1>, grid, block, 0, st, a);
     } else {
         vx_launch(pf_kernel<false, 2>, grid, block, 0, st, a);
