@@ -149,18 +149,22 @@ __device__ __forceinline__ void fa_finish(const fa_args & a, float4_t acc, float
 // store the slots and leave the totals of GGML_OP_SUM's 16 waves a side, which the o projection's activation pass adds up
 // and adds to this kernel's result.  The two launches it replaces (5.0 + 4.2 us of a 45-token prompt's layer of 55) were
 // one work-group's trip to memory and a pass over the result.
-template <int D, bool KV_F32, bool HAS_MASK, bool SOFTCAP, int TWO_SEG, bool HALF = false, bool PRE = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fattn_cols16_kernel(const fa_args a) {
+// NW: waves that share a column tile's one key range, each with every NW-th tile of 32 keys; their (O, max, sum) meet in LDS
+// (fa_shared_takes below has the figures; the F32 form gets the registers of a wave alone on its SIMD, with 256 it spills).
+template <int D, bool KV_F32, bool HAS_MASK, bool SOFTCAP, int TWO_SEG, bool HALF = false, bool PRE = false, int NW = 1>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 && KV_F32 ? 1 : 2))) void fattn_cols16_kernel(const fa_args a) {
     constexpr int NP  = D / 32;          // MFMAs along the head dimension
     constexpr int SEG = D / 4;           // elements of a row owned by lane-group j
     constexpr int ES  = KV_F32 ? 4 : 2;  // bytes per K/V element
 
-    const int lane = threadIdx.x;
+    static_assert(NW == 1 || (TWO_SEG == 0 && !HALF), "waves share a range of one pair of tensors");
+    const int lane = NW == 1 ? threadIdx.x : threadIdx.x & 63;
+    const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
     const int j = lane >> 4, c = lane & 15;
 
     if constexpr (PRE) {
         if ((int) blockIdx.z < a.pre_slices) {
-            const uint32_t i = blockIdx.z * gridDim.x + blockIdx.x, w = i & 15;
+            const uint32_t i = (blockIdx.z * gridDim.x + blockIdx.x) * NW + (uint32_t) wave, w = i & 15;
             if (i >= 32) return;
             double t; // (two branches: a reference to either argument would be a copy of one in scratch memory)
             if (i >= 16) t = a.kvs_v.vec ? kvs_mid_wave<true>(a.kvs_v, w, (uint32_t) lane) : kvs_mid_wave<false>(a.kvs_v, w, (uint32_t) lane);
@@ -340,7 +344,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fa
     } else if constexpr (HALF) {
         load_half0(kv0, t0);
     } else {
-        load_tile(kv0, t0);
+        load_tile(NW == 1 ? kv0 : min(kv0 + 32 * wave, kv0 + ((kv1 - kv0 - 1) / 32) * 32), t0);
     }
 
     // ---- Q^T operand: column c, elements d = SEG*j + 8p + i, split into hi + lo
@@ -486,12 +490,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fa
     if constexpr (HALF) {
         consume(t0, kv0, std::true_type{});
     } else {
-        for (int kb = kv0; kb < kv1p; kb += 64) {
-            load_tile(min(kb + 32, klast), t1);
+        for (int kb = kv0 + 32 * wave; kb < kv1p; kb += 64 * NW) {
+            load_tile(min(kb + 32 * NW, klast), t1);
             consume(t0, kb, std::false_type{});
-            if (kb + 32 >= kv1p) break;
-            load_tile(min(kb + 64, klast), t0);
-            consume(t1, kb + 32, std::false_type{});
+            if (kb + 32 * NW >= kv1p) break;
+            load_tile(min(kb + 64 * NW, klast), t0);
+            consume(t1, kb + 32 * NW, std::false_type{});
         }
     }
     if constexpr (TWO_SEG == 2) {
@@ -503,6 +507,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void fa
 
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if constexpr (NW > 1) { // each wave ends with a share of the (p, u) tiles, added in the waves' order
+        __shared__ float4_t o_s[NW][NP * 2][64];
+        __shared__ float2   ml_s[NW][16];
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) o_s[wave][2 * p + u][lane] = o[p][u];
+        if (j == 0) ml_s[wave][c] = make_float2(m, l);
+        __syncthreads();
+        if (!col_ok) return;
+        float M = -INFINITY, L = 0.0f, f[NW];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) { f[w] = ml_s[w][c].x; M = fmaxf(M, f[w]); }
+        const float shift = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) { f[w] = __builtin_amdgcn_exp2f(f[w] - shift); L += ml_s[w][c].y * f[w]; }
+        const bool  has_sink = a.sinks != nullptr, has_addend = a.add1 != nullptr;
+        const float sink = has_sink ? a.sinks[head] : 0.0f, addend = has_addend ? *a.add1 : 0.0f;
+        for (int pu = wave; pu < NP * 2; pu += NW) {
+            float4_t acc = float4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int w = 0; w < NW; ++w) acc += o_s[w][pu][lane] * f[w];
+            fa_finish(a, acc, M, L, b, iq1, head, D, SEG * (2 * (pu & 1) + (j >> 1)) + 8 * (pu >> 1) + 4 * (j & 1), has_sink, sink, has_addend, addend);
+        }
+        return;
+    }
     if (!col_ok) return;
 
     // lane (j,c), tile (p,u), register r holds d = SEG*(2u + j/2) + 8p + 4*(j%2) + r of column c
@@ -635,7 +665,7 @@ void fa_split_plan(int64_t tiles, int n_kv, int * n_splits, int * chunk_out) {
     static const int min_chunk = [] { const char * e = getenv("VX_FA_MIN_CHUNK"); const int v = e ? atoi(e) : 0; return v >= 32 ? v / 32 * 32 : 32; }();
     *n_splits  = 1;
     *chunk_out = (n_kv + 31) / 32 * 32;
-    // Up to 256 keys one wave finishes (0.5 us per 32-key step) before a split plus the merge
+    // Up to 256 keys one wave (or four that share the range, fa_shared_takes) finishes (0.5 us per 32-key step) before a split plus the merge
     // launch would.
     static const int waves_per_cu = [] { const char * e = getenv("VX_FA_WAVES_PER_CU"); const int v = e ? atoi(e) : 0; return v >= 1 && v <= 32 ? v : 4; }();
     if (tiles < (int64_t) waves_per_cu * num_cus() && n_kv > 256) {
@@ -992,6 +1022,29 @@ void launch_cols16_pre(const fa_args & a, hipStream_t st) {
     const dim3 grid((unsigned) a.n_col_tiles, 1, (unsigned) (a.ne3 * a.Hkv + a.pre_slices)), block(64);
     if (a.mask) vx_launch(fattn_cols16_kernel<64, KV_F32, true, false, 0, false, true>, grid, block, 0, st, a);
     else        vx_launch(fattn_cols16_kernel<64, KV_F32, false, false, 0, false, true>, grid, block, 0, st, a);
+}
+constexpr int FA_SHARED_WAVES = 4;
+template <bool KV_F32>
+void launch_cols16_shared(const fa_args & a, hipStream_t st) {
+    constexpr int W = FA_SHARED_WAVES;
+    const dim3 grid((unsigned) a.n_col_tiles, 1, (unsigned) (a.ne3 * a.Hkv + a.pre_slices)), block(64 * W);
+    if (a.pre_slices) {
+        if (a.mask) vx_launch(fattn_cols16_kernel<64, KV_F32, true, false, 0, false, true, W>, grid, block, 0, st, a);
+        else        vx_launch(fattn_cols16_kernel<64, KV_F32, false, false, 0, false, true, W>, grid, block, 0, st, a);
+    } else {
+        if (a.mask) vx_launch(fattn_cols16_kernel<64, KV_F32, true, false, 0, false, false, W>, grid, block, 0, st, a);
+        else        vx_launch(fattn_cols16_kernel<64, KV_F32, false, false, 0, false, false, W>, grid, block, 0, st, a);
+    }
+}
+// Whether four waves share a column tile's keys: a short prompt leaves compute units with one wave each, which then walks all keys
+// alone (0.7 us per 32 of them with F32 keys and values, 0.45 with f16).  Up to a work-group per compute unit the four run at once;
+// beyond, the F32 form's registers (one wave a SIMD) let no second work-group in and the call takes longer.  Us a call, causal, one
+// wave / four: F32 33 tokens 5.84 / 4.79, 45 5.87 / 4.90, 128 8.54 / 6.75, 203 12.2 / 8.60, 250 13.9 / 9.32, 2 x 127 (256 tiles) 8.73
+// / 6.83, 16 x 40 (640) 7.47 / 12.0; f16 64 4.04 / 4.14, 70 4.63 / 4.24, 203 7.15 / 5.38, 16 x 60 (960) 5.75 / 9.23 (two waves' worth
+// of keys gain nothing there: more than 64).  The error against float64 is up to a fifth lower: shorter chains.  (From seventeen query
+// rows on: a decode step's sums have an order of their own, which the resident stack repeats.)
+bool fa_shared_takes(const fa_args & a, int D, bool kv_f32, int64_t tiles) {
+    return a.n_splits == 1 && D == 64 && !a.k2 && a.softcap == 0.0f && a.n_q > 16 && a.n_kv > (kv_f32 ? 32 : 64) && tiles <= num_cus();
 }
 
 } // namespace
@@ -1432,7 +1485,7 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
         kvs_side_fill(a.kvs_k, ks_src, ks_slot);
         kvs_side_fill(a.kvs_v, vs_src, vs_slot);
         a.kvs_totals = kvs_totals;
-        a.pre_slices = (32 + a.n_col_tiles - 1) / a.n_col_tiles;
+        a.pre_slices = 1;
     } else if (ks_src) {
         if (a.n_splits == 1) return vx_fail(VX_ERR_UNSUPPORTED, "flash_attn_ext_kv2_store: needs a key count that is split across waves");
         kvs_side_fill(a.kvs_k, ks_src, ks_slot);
@@ -1447,6 +1500,11 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
     const bool f32 = k->type == VX_TYPE_F32;
 
     const bool dec = !kvs_totals && fa_dec64_takes(a, D, f32);
+    const bool shared = !dec && fa_shared_takes(a, D, f32, tiles);
+    if (a.pre_slices) { // 32 waves' work-groups in front
+        const int in_front = shared ? 32 / FA_SHARED_WAVES : 32;
+        a.pre_slices = (in_front + a.n_col_tiles - 1) / a.n_col_tiles;
+    }
 
     if (a.n_splits > 1) {
         const size_t o_bytes  = (size_t) nblocks * 16 * D * sizeof(float);
@@ -1466,7 +1524,7 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
     }
 
     if (dec) launch_dec64(a, st);
-    else if (a.pre_slices) {} // (below)
+    else if (a.pre_slices || shared) {} // (below)
     else if (D == 64) { if (f32) launch_cols16<64, true>(a, st); else launch_cols16<64, false>(a, st); }
     else         { if (f32) launch_cols16<128, true>(a, st); else launch_cols16<128, false>(a, st); }
     VX_LAUNCH_CHECK();
@@ -1477,7 +1535,10 @@ static vx_status fa_run(const vx_tensor * q, const vx_tensor * k, const vx_tenso
         else         vx_launch(fattn_merge_kernel<128>, grid, mblock, 0, st, a);
         VX_LAUNCH_CHECK();
     }
-    if (a.pre_slices) {
+    if (shared) {
+        if (f32) launch_cols16_shared<true>(a, st); else launch_cols16_shared<false>(a, st);
+        VX_LAUNCH_CHECK();
+    } else if (a.pre_slices) {
         if (f32) launch_cols16_pre<true>(a, st); else launch_cols16_pre<false>(a, st);
         VX_LAUNCH_CHECK();
     }
