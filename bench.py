@@ -336,7 +336,7 @@ def backbone_bench(pkg, timer, side, threads, with_cpu, layers=LAYERS, batch=2, 
     torch.cuda.synchronize()
     t_step = (time.perf_counter() - t0) / (per * 4)
     kvb = layers * 2 * batch * HKV * (prefill + steps // 2) * D * es
-    res = {"decode_steps_per_s": 1.0 / t_step, "ms_per_step": t_step * 1e3, "launches_per_step": n_calls,
+    res = {"decode_steps_per_s": 1.0 / t_step, "ms_per_step": t_step * 1e3, "separate_calls_per_step": n_calls,
            "weight_GB/s": weight_bytes / t_step / 1e9, "hbm_frac_weights_plus_kv": (weight_bytes + kvb) / t_step / 1e9 / HBM_PEAK_GBS,
            "prefill_ms": t_prefill * 1e3, "prefill_tokens_per_s": batch * prefill / t_prefill,
            "prefill_ms_weights_not_pinned": t_prefill_unpinned * 1e3,
