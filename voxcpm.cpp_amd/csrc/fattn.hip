@@ -1041,8 +1041,9 @@ void launch_cols16_shared(const fa_args & a, hipStream_t st) {
 // beyond, the F32 form's registers (one wave a SIMD) let no second work-group in and the call takes longer.  Us a call, causal, one
 // wave / four: F32 33 tokens 5.84 / 4.79, 45 5.87 / 4.90, 128 8.54 / 6.75, 203 12.2 / 8.60, 250 13.9 / 9.32, 2 x 127 (256 tiles) 8.73
 // / 6.83, 16 x 40 (640) 7.47 / 12.0; f16 64 4.04 / 4.14, 70 4.63 / 4.24, 203 7.15 / 5.38, 16 x 60 (960) 5.75 / 9.23 (two waves' worth
-// of keys gain nothing there: more than 64).  The error against float64 is up to a fifth lower: shorter chains.  (From seventeen query
-// rows on: a decode step's sums have an order of their own, which the resident stack repeats.)
+// of keys gain nothing there: more than 64).  Eight waves instead of four: F32 130 tokens 7.59, but 203 9.40 and 250 11.4.  The error
+// against float64 is up to a fifth lower: shorter chains.  (From seventeen query rows on: a decode step's sums have an order of their
+// own, which the resident stack repeats.)
 bool fa_shared_takes(const fa_args & a, int D, bool kv_f32, int64_t tiles) {
     return a.n_splits == 1 && D == 64 && !a.k2 && a.softcap == 0.0f && a.n_q > 16 && a.n_kv > (kv_f32 ? 32 : 64) && tiles <= num_cus();
 }
