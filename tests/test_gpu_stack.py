@@ -189,3 +189,35 @@ def test_two_streams_at_once(gpu, env):
     torch.cuda.synchronize()
     for _, _, out, want, _ in jobs:
         assert torch.equal(out, want)
+
+
+# A process of its own each, since the library reads the switch once.
+MANY_TOKENS = """
+import os, sys
+sys.path[:0] = [{root!r}, {tests!r}]
+import torch, __graft_entry__, test_gpu_stack as t
+gpu = __graft_entry__.load_package()
+gpu.check(gpu.lib().vx_init(0), "vx_init")
+def taken(batch, T, past):
+    m = t.build(gpu, 1, batch, past + T, True)
+    x = torch.zeros((batch, T, 1024), device="cuda")
+    pos = torch.arange(past, past + T, dtype=torch.int32, device="cuda")
+    return m._stack(x, torch.empty_like(x), pos, T, past, None, past > 0, 1.0) is not None
+print([taken(*s) for s in ((1, 1, 40), (4, 1, 40), (8, 1, 40), (9, 1, 40), (16, 1, 700), (1, 8, 0), (1, 9, 0), (2, 7, 0))])
+"""
+
+
+def test_slots_that_no_instance_has_are_refused(gpu):
+    """VX_GEMV_MANY_TOKENS above the row count gives products of 9 to 16 rows eight slots; the launch for more than eight rows has sixteen."""
+    import subprocess
+    import sys
+    say("stack: VX_GEMV_MANY_TOKENS")
+    tests = os.path.dirname(os.path.abspath(__file__))
+    code = MANY_TOKENS.format(root=os.path.dirname(tests), tests=tests)
+    for many, want in ((None, [True] * 8), ("100", [True, True, True, False, False, True, False, False])):
+        env = {k: v for k, v in os.environ.items() if k not in ("VX_GEMV_MANY_TOKENS", "VX_STACK")}
+        if many:
+            env["VX_GEMV_MANY_TOKENS"] = many
+        got = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+        assert got.returncode == 0, got.stderr[-2000:]
+        assert got.stdout.strip().splitlines()[-1] == str(want), (many, got.stdout)

@@ -1286,6 +1286,7 @@ bool vs_fill(const vx_stack * s, vs_args & a, vs_plan & p) {
     p.nwa = vx_gemv_waves(a.hidden, N, a.hidden);
     if ((p.nwa != 8 && p.nwa != 16) || vx_gemv_waves(a.hidden, N, a.hkv * 64) != p.nwa) return false;
     if (vx_gemv_waves(a.hidden, N, a.ffn) != 8 || vx_gemv_waves(a.ffn, N, a.hidden) != 16) return false;
+    if (N > 8 && p.nwa != 16) return false; // (the instances for more than eight rows have sixteen; VX_GEMV_MANY_TOKENS may ask for eight)
     p.tpw = N > 8 ? 2 : 1;
     p.halves = p.tpw;
     for (int l = 0; l < s->n_layer; ++l) {
