@@ -49,3 +49,31 @@ def test_waves_share_a_range(pkg, gpu, B, H, Hkv, n_q, n_kv, kind, sinks, f16):
             bound = (2.0 ** -10 * (2 + size) if streamed else 2.0 ** -20 * (2 * size + 1)) * vv.abs().max()
             err = (got[b, :, h] - want).abs().max()
             assert float(err) <= float(bound), (b, h, float(err), float(bound))
+
+
+@pytest.mark.parametrize("kinds", ["f32", "f16", "f16 cache, f32 step"])
+@pytest.mark.parametrize("B,H,Hkv,T,n_past,masked", [
+    (1, 16, 2, 40, 100, True), (2, 16, 2, 17, 17, True), (1, 16, 2, 33, 160, False), (1, 16, 2, 64, 31, True), (1, 16, 2, 20, 128, True),
+    (1, 16, 2, 100, 5, True), (1, 6, 2, 45, 66, False), (1, 16, 2, 128, 128, True), (2, 16, 2, 127, 129, True), (3, 16, 2, 86, 50, True),
+    (1, 16, 2, 17, 47, True), (1, 16, 2, 17, 48, True), (1, 16, 2, 16, 100, True)])
+def test_two_segments_are_shared_as_one(pkg, gpu, B, H, Hkv, T, n_past, masked, kinds):
+    """Cached keys and the step's own as two pairs of tensors against the two joined: the same bits, on both sides of the rule (17 rows,
+    33 / 65 keys, 256 tiles), with the boundary on a multiple of 32, beside it, in the first tile and in each wave's tiles."""
+    import torch
+    say(f"attention over two segments, waves share a range: {B} x {T}/{n_past}+{T} heads {H}/{Hkv} mask={masked} {kinds}")
+    L, d, n_kv = pkg.lib(), pkg.desc, n_past + T
+    g = rng("shared2", B, T, n_past)
+    first = torch.float32 if kinds == "f32" else torch.float16
+    second = torch.float16 if kinds == "f16" else torch.float32
+    q = dev(g.standard_normal((B, H, T, 64)).astype("float32"))
+    kp, vp = (dev(g.standard_normal((B, Hkv, n_past + 7, 64)).astype("float32")).to(first)[:, :, :n_past] for _ in range(2))
+    kc, vc = (dev(g.standard_normal((B, T, Hkv, 64)).astype("float32")).to(second).transpose(1, 2) for _ in range(2))
+    i, j = torch.arange(T)[:, None] + n_past, torch.arange(n_kv)[None]
+    mask = torch.where((j <= i) & (i % 7 > 0), 0.0, float("-inf")).half().view(1, 1, T, n_kv).contiguous().cuda() if masked else None
+    kall, vall = (torch.cat([p, c.to(first)], 2).contiguous() for p, c in ((kp, kc), (vp, vc)))
+    want = gpu.flash_attn_ext(q, kall, vall, mask, 0.125)
+    got = torch.full_like(want, 3.0)
+    assert L.vx_supports_flash_attn_ext_kv2(d(q), d(kp), d(kc), d(vp), d(vc), d(mask), d(got)) == 1
+    pkg.check(L.vx_flash_attn_ext_kv2(d(q), d(kp), d(kc), d(vp), d(vc), d(mask), None, d(got), 0.125, 0.0, 0.0, None), "kv2")
+    torch.cuda.synchronize()
+    assert torch.equal(want, got)

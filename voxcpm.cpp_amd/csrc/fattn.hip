@@ -149,7 +149,8 @@ __device__ __forceinline__ void fa_finish(const fa_args & a, float4_t acc, float
 // store the slots and leave the totals of GGML_OP_SUM's 16 waves a side, which the o projection's activation pass adds up
 // and adds to this kernel's result.  The two launches it replaces (5.0 + 4.2 us of a 45-token prompt's layer of 55) were
 // one work-group's trip to memory and a pass over the result.
-// NW: waves that share a column tile's one key range, each with every NW-th tile of 32 keys; their (O, max, sum) meet in LDS
+// NW: waves that share a column tile's one key range, each with every NW-th tile of 32 keys, wherever its rows lie; their (O, max, sum)
+// meet in LDS
 // (fa_shared_takes below has the figures; the F32 form gets the registers of a wave alone on its SIMD, with 256 it spills).
 template <int D, bool KV_F32, bool HAS_MASK, bool SOFTCAP, int TWO_SEG, bool HALF = false, bool PRE = false, int NW = 1>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 && KV_F32 ? 1 : 2))) void fattn_cols16_kernel(const fa_args a) {
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
     constexpr int SEG = D / 4;           // elements of a row owned by lane-group j
     constexpr int ES  = KV_F32 ? 4 : 2;  // bytes per K/V element
 
-    static_assert(NW == 1 || (TWO_SEG == 0 && !HALF), "waves share a range of one pair of tensors");
+    static_assert(NW == 1 || !HALF, "waves share a range of more than one tile");
     const int lane = NW == 1 ? threadIdx.x : threadIdx.x & 63;
     const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
     const int j = lane >> 4, c = lane & 15;
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
     // the scalar for the merge kernel, its other waves store the slots.  (One wave reads
     // the step's keys and values: when every merge block formed the sums itself, sixteen streams' 512 blocks asked the
     // same few cache lines at once and the merge took 9 us instead of 4.)
-    if constexpr (TWO_SEG != 0) {
+    if constexpr (TWO_SEG != 0 && NW == 1) { // (waves that share a range have no merge kernel to leave it for)
         if (a.has_kvs && blockIdx.z == 0) {
             if (blockIdx.x != 0) return;
             if (blockIdx.y == 0) { // the sums, in GGML_OP_SUM's order, by one wave (no stores: their index arithmetic is the others' work)
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
         }
     }
     // the grid is (column tile, key range, batch entry x KV head): dispatched in the same order as one flat index
-    const int ct = blockIdx.x, sp = blockIdx.y, bg = (int) blockIdx.z - (PRE ? a.pre_slices : (TWO_SEG != 0 && a.has_kvs) ? 1 : 0);
+    const int ct = blockIdx.x, sp = blockIdx.y, bg = (int) blockIdx.z - (PRE ? a.pre_slices : (TWO_SEG != 0 && NW == 1 && a.has_kvs) ? 1 : 0);
     const int b  = fa_div(bg, a.inv_hkv);
     const int g  = bg - b * a.Hkv;
     const int tile = bg * a.n_col_tiles + ct;
@@ -333,14 +334,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
 
     // two tiles alternate in registers: while one is consumed the other is in flight
     kv_tile<NP, KV_F32> t0, t1, t2;
-    const int kmix = max(kv0, pure); // first tile of the lane-by-lane part (TWO_SEG == 2)
+    // first tile of the lane-by-lane part (TWO_SEG == 2): this wave's first that lies at or behind the boundary (kv0 is 0 where waves share)
+    const int kmix = max(kv0, pure) + (NW == 1 ? 0 : 32 * ((wave - pure / 32) & (NW - 1)));
     // A range of at most 16 keys (LocDiT's 14-token sequence) is half a tile: the second half's loads, conversions and
     // products would all be of keys that are switched off.  (A kernel of its own, not a branch: tile loads in a branch
     // would hold back every request behind it until their conversions have their data.)
     static_assert(!HALF || TWO_SEG == 0, "the half-tile kernel reads one pair of tensors");
     if constexpr (TWO_SEG == 2) {
         if (kmix < kv1) load_mixed(kmix, t2);  // requested first, consumed last
-        if (kv0 < kv1p) load_tile(kv0, t0);
+        if (kv0 + 32 * wave < kv1p) load_tile(kv0 + 32 * wave, t0);
     } else if constexpr (HALF) {
         load_half0(kv0, t0);
     } else {
@@ -499,7 +501,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW > 1 
         }
     }
     if constexpr (TWO_SEG == 2) {
-        for (int kb = kmix; kb < kv1; kb += 32) {
+        for (int kb = kmix; kb < kv1; kb += 32 * NW) {
             if (kb != kmix) load_mixed(kb, t2);
             consume(t2, kb, std::false_type{});
         }
@@ -1028,7 +1030,17 @@ template <bool KV_F32>
 void launch_cols16_shared(const fa_args & a, hipStream_t st) {
     constexpr int W = FA_SHARED_WAVES;
     const dim3 grid((unsigned) a.n_col_tiles, 1, (unsigned) (a.ne3 * a.Hkv + a.pre_slices)), block(64 * W);
-    if (a.pre_slices) {
+    if (a.k2) { // the same tiles to the same waves as for the two pairs joined: the same bits
+        if constexpr (!KV_F32) {
+            if (a.seg2_f32) {
+                if (a.mask) vx_launch(fattn_cols16_kernel<64, false, true, false, 2, false, false, W>, grid, block, 0, st, a);
+                else        vx_launch(fattn_cols16_kernel<64, false, false, false, 2, false, false, W>, grid, block, 0, st, a);
+                return;
+            }
+        }
+        if (a.mask) vx_launch(fattn_cols16_kernel<64, KV_F32, true, false, 1, false, false, W>, grid, block, 0, st, a);
+        else        vx_launch(fattn_cols16_kernel<64, KV_F32, false, false, 1, false, false, W>, grid, block, 0, st, a);
+    } else if (a.pre_slices) {
         if (a.mask) vx_launch(fattn_cols16_kernel<64, KV_F32, true, false, 0, false, true, W>, grid, block, 0, st, a);
         else        vx_launch(fattn_cols16_kernel<64, KV_F32, false, false, 0, false, true, W>, grid, block, 0, st, a);
     } else {
@@ -1043,9 +1055,11 @@ void launch_cols16_shared(const fa_args & a, hipStream_t st) {
 // / 6.83, 16 x 40 (640) 7.47 / 12.0; f16 64 4.04 / 4.14, 70 4.63 / 4.24, 203 7.15 / 5.38, 16 x 60 (960) 5.75 / 9.23 (two waves' worth
 // of keys gain nothing there: more than 64).  Eight waves instead of four: F32 130 tokens 7.59, but 203 9.40 and 250 11.4.  The error
 // against float64 is up to a fifth lower: shorter chains.  (From seventeen query rows on: a decode step's sums have an order of their
-// own, which the resident stack repeats.)
+// own, which the resident stack repeats.)  Keys in two pairs of tensors go by the same rule: vx_flash_attn_ext_kv2 promises the bits of
+// the joined call.  Its call, one wave / four: F32 40 rows behind 100 keys 10.7 / 8.5, 120 behind 130 15.5 / 9.7; an f16 cache and
+// F32 rows 7.8 / 6.7 and 11.3 / 7.5.
 bool fa_shared_takes(const fa_args & a, int D, bool kv_f32, int64_t tiles) {
-    return a.n_splits == 1 && D == 64 && !a.k2 && a.softcap == 0.0f && a.n_q > 16 && a.n_kv > (kv_f32 ? 32 : 64) && tiles <= num_cus();
+    return a.n_splits == 1 && D == 64 && a.softcap == 0.0f && a.n_q > 16 && a.n_kv > (kv_f32 ? 32 : 64) && tiles <= num_cus();
 }
 
 } // namespace
