@@ -1085,7 +1085,7 @@ __device__ __forceinline__ void vs_product(vs_const_args * ap, vs_ctx & k, int p
             }
         }
         float res[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (wid == end && (p == VS_O || p == VS_D)) { // the residual values of this work-group's rows: lane (j, c) has tokens 4 j .. 4 j + 3 of column c
+        if (wid == end && (p == VS_O || p == VS_D)) { // the residual values of this work-group's rows, its own stores: lane (j, c) has tokens 4 j .. 4 j + 3 of column c
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t e = (uint32_t) ((4 * j + r) * a.hidden + u * a.ro + c);
@@ -1130,6 +1130,10 @@ __device__ __forceinline__ void vs_product(vs_const_args * ap, vs_ctx & k, int p
         if (k.full && wid == W - 4 + p && l + 1 < a.n_layer) vs_fetch(vs_fresh(ap), k, p, l + 1, u, vs_fresh(lane0));
         if (wid != end) continue;
         vs_finish_product<NWA>(vs_fresh(ap), k, p, l, u, vs_fresh(lane0), res);
+        // The o projection of the next layer reads these values back as its residual, by another wave and without a look: they are in memory
+        // before this wave passes a barrier.  (Everybody else waits for the same trip: 550 -> 551.5 us a step of two rows, where looking for
+        // the empty slot's pattern at the o projection's end took 567.  What down reads back has been seen by this work-group's gate / up rows.)
+        if (p == VS_D) vs_wait_vm0();
     }
 }
 
