@@ -523,6 +523,9 @@ VX_API int vx_supports_sum(const vx_tensor * src, const vx_tensor * dst);
  * themselves and leave no cache (n_past 0; mask: F16 [n_tokens][n_tokens] or NULL).  The results are the bits of the separate calls.
  * x and out: dense F32 [batch][n_tokens][hidden].  Weight rows are dense Q8_0 blocks, norms dense F32.  cache_nb1 / nb2 / nb3: byte
  * strides of a cache's rows, heads and sequences, the same for K and V of every layer.  positions: n_tokens int32 on the device.
+ * The launch's work-groups wait for each other's values.  Only those that run take part, so every wait ends; each is bounded all the
+ * same (about 0.2 s), and should one run out, the token rows that miss a value are NaN in out and in their cache slots, whatever the
+ * call returned.
  * No counterpart in ggml-cpu, which runs the nodes one by one. */
 #define VX_STACK_MAX_LAYERS 32
 typedef struct vx_stack_layer {

@@ -111,7 +111,10 @@ __device__ __forceinline__ void vs_dma16_nt(const char * base, uint32_t off, uin
 // ---- the exchange
 struct vs_xch {
     __amdgpu_buffer_rsrc_t r;
-    int dead; // a wait was given up (uniform per wave): nothing waits any more, so that the grid drains
+    // a wait was given up (uniform per wave): nothing waits any more, so that the grid drains.  What is missing stays the pattern, a NaN in
+    // F32 and in f16, and every use of it -- norm, product, softmax weight, sum, residual -- gives NaN: the token rows that depend on it end
+    // as NaN in all their columns (the next norm's sum is NaN), the others are right.
+    int dead;
     __device__ __forceinline__ int4_t ld(uint32_t off) const { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, VS_DEV); }
     __device__ __forceinline__ void st(uint32_t off, float v) const {
         const int b = __builtin_bit_cast(int, v);
@@ -1221,7 +1224,6 @@ __global__ __launch_bounds__(64 * W) void stack_kernel(const vs_args) {
     }
     // ---- the final norm: a row each for the first work-groups
     const vs_args & a = vs_fresh(ap);
-    if (k.x.dead && lane == 0) __hip_atomic_store(a.ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (k.wid == 0) {
         const int nv = a.hidden >> 8;
         const uint32_t x_at = (uint32_t) (n_layer - 1) * a.layer_bytes + a.o_x;
@@ -1231,8 +1233,7 @@ __global__ __launch_bounds__(64 * W) void stack_kernel(const vs_args) {
             vx_rms_row r;
 #pragma unroll
             for (int cc = 0; cc < 8; ++cc) r.v[cc] = __builtin_bit_cast(float4, v[cc]);
-            float sc = vx_rms_row_scale(r, a.hidden, lane, a.eps);
-            if (k.x.dead || __hip_atomic_load(a.ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) sc = __builtin_nanf("");
+            const float sc = vx_rms_row_scale(r, a.hidden, lane, a.eps);
 #pragma unroll
             for (int cc = 0; cc < 8; ++cc)
                 if (cc < nv) ((float4_t *) (a.out + (size_t) t * a.hidden))[lane + 64 * cc] = vs_f4(v[cc]) * sc * ((const float4_t *) a.norm)[lane + 64 * cc];
