@@ -79,8 +79,10 @@ VX_API vx_status    vx_stream_synchronize(vx_stream stream);
  * larger block has replaced it, so launches already queued and HIP graphs already captured from the stream stay
  * valid.  A call that would have to grow the workspace while the stream is being captured returns
  * VX_ERR_UNSUPPORTED: reserve the largest size first.  (Products of 17 to 3072 tokens and the calls built on them -- the kernel
- * of gemm_mid.hip -- allocate beside the capture instead: a graph that begins with one needs no reservation.)  No counterpart in the reference (ggml-cpu takes its scratch
- * from the compute plan's work buffer, ggml/src/ggml-cpu/ggml-cpu.c:2700-2935). */
+ * of gemm_mid.hip -- and vx_stack_run allocate beside the capture instead: a graph that begins with one needs no reservation.)
+ * Calls that use it and overlap in time need a stream each: graphs captured on one stream replay one after the other.  No
+ * counterpart in the reference (ggml-cpu takes its scratch from the compute plan's work buffer,
+ * ggml/src/ggml-cpu/ggml-cpu.c:2700-2935). */
 VX_API vx_status    vx_workspace_reserve(vx_stream stream, size_t bytes);
 /* current block, its size and the number of superseded blocks still held for this stream (any out pointer may be NULL) */
 VX_API vx_status    vx_workspace_info(vx_stream stream, void ** ptr, size_t * bytes, int * retired_blocks);
@@ -543,7 +545,13 @@ typedef struct vx_stack {
     float   rope_base, rope_freq_scale, rope_ext_factor, rope_attn_factor, rope_beta_fast, rope_beta_slow;
 } vx_stack;
 VX_API int vx_supports_stack(const vx_stack * stack);
+/* The values pass through an area of memory that belongs to one run at a time: two runs that share it must not overlap in time.
+ * vx_stack_run takes it from the stream's workspace (allocated beside a capture where it has to grow), so graphs captured on one stream
+ * share it and replay one after the other.  vx_stack_run_in is given the area (16-byte boundary, vx_stack_area_bytes of it; 0: a
+ * stack that is refused), on whichever stream: a plan that keeps an area of its own runs and replays beside any other. */
 VX_API vx_status vx_stack_run(const vx_stack * stack, vx_stream stream);
+VX_API size_t    vx_stack_area_bytes(const vx_stack * stack);
+VX_API vx_status vx_stack_run_in(const vx_stack * stack, void * area, size_t area_bytes, vx_stream stream);
 
 #ifdef __cplusplus
 }

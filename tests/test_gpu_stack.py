@@ -221,3 +221,54 @@ def test_slots_that_no_instance_has_are_refused(gpu):
         got = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
         assert got.returncode == 0, got.stderr[-2000:]
         assert got.stdout.strip().splitlines()[-1] == str(want), (many, got.stdout)
+
+
+def test_graphs_of_one_stream_replay_side_by_side(gpu, env):
+    """Two plans recorded on the same stream and replayed on two others at once: a plan's exchange area is its own."""
+    import torch
+    say("stack: two graphs of one capture stream on two streams")
+    env.pop("VX_STACK", None)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    side, jobs = torch.cuda.Stream(), []
+    for i in range(2):
+        m = build(gpu, 4, 2, 41, False)     # (one key range: nothing of the separate calls' lies in the workspace either)
+        for c in m.k_cache + m.v_cache:
+            c[:, :, :40] = torch.randn((2, 2, 40, 64), generator=gen, device="cuda")
+        run, out = m.plan(torch.randn((2, 1, 1024), generator=gen, device="cuda"), 1, 40)
+        run()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            run()
+        jobs.append((torch.cuda.Stream(), g, out, out.clone(), m, run))
+    for _ in range(5):
+        for _, _, out, _, _, _ in jobs:
+            out.zero_()
+        torch.cuda.synchronize()
+        for _ in range(8):
+            for s, g, _, _, _, _ in jobs:
+                with torch.cuda.stream(s):
+                    g.replay()
+        torch.cuda.synchronize()
+        for _, _, out, want, _, _ in jobs:
+            assert torch.equal(out, want)
+
+
+def test_areas_that_do_not_fit_are_refused(gpu, env):
+    import torch
+    from voxcpm_cpp_amd import lib
+    say("stack: the caller's area")
+    env.pop("VX_STACK", None)
+    m = build(gpu, 1, 2, 41, False)
+    x = torch.zeros((2, 1, 1024), device="cuda")
+    run, out = m.plan(x, 1, 40)
+    st = m._stack(x, out, run._keep[0], 1, 40, None, True, 1.0)
+    n = lib().vx_stack_area_bytes(st)
+    area = torch.empty(n + 16, dtype=torch.uint8, device="cuda")
+    assert n > 256
+    for at, size in ((0, n), (area.data_ptr(), n - 1), (area.data_ptr() + 8, n)):
+        assert lib().vx_stack_run_in(st, at, size, None) == 3   # VX_ERR_INVALID
+    assert lib().vx_stack_run_in(st, area.data_ptr() + 16, n, None) == 0
+    torch.cuda.synchronize()
+    st.n_tokens = 17
+    assert lib().vx_stack_area_bytes(st) == 0 and lib().vx_stack_run_in(st, area.data_ptr(), n, None) == 2

@@ -328,13 +328,16 @@ class MiniCPMBackbone:
         norm(cur_x, self.final_norm, o2)
 
         stack = self._stack(x, out, pos, T, n_past, mask, write_kv, attn_factor) if fuse else None
+        if stack is not None:   # (the plan's own exchange area: a graph of it replays beside graphs of other plans)
+            area = new(L.vx_stack_area_bytes(stack), dtype=torch.uint8)
+            keep.append(area)
 
         def run():
             st = _stream()
             if stack is not None:   # all of it as one resident launch, the same bits
-                rc = L.vx_stack_run(stack, st)
+                rc = L.vx_stack_run_in(stack, area.data_ptr(), area.numel(), st)
                 if rc != ERR_UNSUPPORTED:
-                    check(rc, "vx_stack_run")
+                    check(rc, "vx_stack_run_in")
                     return
             for fn, args in calls:
                 rc = fn(*args, st)
@@ -347,7 +350,7 @@ class MiniCPMBackbone:
         return run, out
 
     def _stack(self, x, out, pos, T, n_past, mask, write_kv, attn_factor):
-        """The whole plan as vx_stack_run's argument where that takes it (a decode step, or one pass without a cache, of at
+        """The whole plan as vx_stack_run_in's argument where that takes it (a decode step, or one pass without a cache, of at
         most 16 token rows), else None."""
         torch = self.torch
         if self.act_mode != ACT_FLOAT or self.n_layer > STACK_MAX_LAYERS or (mask is not None and (mask.dim() != 2 or mask.stride(1) != 1)):

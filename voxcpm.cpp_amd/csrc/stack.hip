@@ -1415,20 +1415,21 @@ extern "C" int vx_supports_stack(const vx_stack * s) {
     return vs_fill(s, a, p) ? 1 : 0;
 }
 
-extern "C" vx_status vx_stack_run(const vx_stack * s, vx_stream stream) {
+extern "C" size_t vx_stack_area_bytes(const vx_stack * s) {
     vs_args a;
     vs_plan p;
-    if (!vs_fill(s, a, p))
-        return vx_fail(VX_ERR_UNSUPPORTED, "stack: at most 16 token rows; a decode step of one token a sequence, or sequences without a cache; Q8_0 weights on 16-byte boundaries");
-    hipStream_t st = (hipStream_t) stream;
-    void * ws = nullptr;
-    const vx_status rc = vx_workspace(st, p.ws_bytes, &ws, true);
-    if (rc != VX_OK) return rc;
-    a.ctl = (uint32_t *) ws;
-    a.xch = (char *) ws + 256;
+    return vs_fill(s, a, p) ? p.ws_bytes : 0;
+}
+
+static vx_status vs_refused() {
+    return vx_fail(VX_ERR_UNSUPPORTED, "stack: at most 16 token rows; a decode step of one token a sequence, or sequences without a cache; Q8_0 weights on 16-byte boundaries");
+}
+static vx_status vs_run(vs_args & a, vs_plan & p, void * area, hipStream_t st) {
+    a.ctl = (uint32_t *) area;
+    a.xch = (char *) area + 256;
     const uint32_t n16 = (uint32_t) (p.ws_bytes / 16);
     const unsigned blocks = (n16 + 255) / 256 < 2048 ? (n16 + 255) / 256 : 2048;
-    vx_launch(stack_clear_kernel, dim3(blocks), dim3(256), 0, st, (int4_t *) ws, n16);
+    vx_launch(stack_clear_kernel, dim3(blocks), dim3(256), 0, st, (int4_t *) area, n16);
     VX_LAUNCH_CHECK();
     // fewer work-groups than compute units leave the others to other streams (read on every call; any number gives the same bits)
     if (const char * e = getenv("VX_STACK_GROUPS")) { const int n = atoi(e); if (n >= 1 && n < p.grid) p.grid = n; }
@@ -1438,4 +1439,22 @@ extern "C" vx_status vx_stack_run(const vx_stack * s, vx_stream stream) {
         case VS_F16_SHORT: return vs_launch<VS_F16_SHORT>(a, p, st);
         default:           return vs_launch<VS_SELF>(a, p, st);
     }
+}
+
+extern "C" vx_status vx_stack_run(const vx_stack * s, vx_stream stream) {
+    vs_args a;
+    vs_plan p;
+    if (!vs_fill(s, a, p)) return vs_refused();
+    void * ws = nullptr;
+    const vx_status rc = vx_workspace((hipStream_t) stream, p.ws_bytes, &ws, true);
+    return rc != VX_OK ? rc : vs_run(a, p, ws, (hipStream_t) stream);
+}
+
+extern "C" vx_status vx_stack_run_in(const vx_stack * s, void * area, size_t bytes, vx_stream stream) {
+    vs_args a;
+    vs_plan p;
+    if (!vs_fill(s, a, p)) return vs_refused();
+    if (!area || !al16(area) || bytes < p.ws_bytes)
+        return vx_fail(VX_ERR_INVALID, "stack: the area must be %zu bytes on a 16-byte boundary", p.ws_bytes);
+    return vs_run(a, p, area, (hipStream_t) stream);
 }
