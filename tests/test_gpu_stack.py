@@ -272,3 +272,18 @@ def test_areas_that_do_not_fit_are_refused(gpu, env):
     torch.cuda.synchronize()
     st.n_tokens = 17
     assert lib().vx_stack_area_bytes(st) == 0 and lib().vx_stack_run_in(st, area.data_ptr(), n, None) == 2
+
+
+def test_ordering_scalar_is_the_graphs(gpu, env):
+    """The sums over k and v are formed in another order than the separate calls': right where the scale is zero, refused elsewhere."""
+    import torch
+    from voxcpm_cpp_amd import lib
+    say("stack: the ordering scalar's scale")
+    env.pop("VX_STACK", None)
+    m = build(gpu, 1, 2, 41, False)
+    x = torch.zeros((2, 1, 1024), device="cuda")
+    run, out = m.plan(x, 1, 40)
+    st = m._stack(x, out, run._keep[0], 1, 40, None, True, 1.0)
+    for scale, bias, want in ((0.0, 0.0, 1), (0.0, 0.5, 1), (0.125, 0.0, 0), (0.125, 0.5, 0), (float("nan"), 0.0, 0)):
+        st.sync_scale, st.sync_bias = scale, bias
+        assert lib().vx_supports_stack(st) == want, (scale, bias)

@@ -1274,6 +1274,7 @@ bool vs_fill(const vx_stack * s, vs_args & a, vs_plan & p) {
     if (s->hidden != s->n_heads * 64 || s->hidden % 1024 || s->hidden > 2048 || s->ffn % 2048 || s->ffn < 2048 || s->ffn > 4096) return false;
     if (N * s->n_kv_heads > 32) return false;
     const bool decode = s->write_kv != 0;
+    if (decode && s->sync_scale != 0.0f) return false; // (vs_addend's order of sums shows in any but a product with zero)
     if (decode ? (s->n_tokens != 1 || s->n_past < 1 || s->mask != nullptr) : s->n_past != 0) return false;
     if (s->kv_type != VX_TYPE_F32 && s->kv_type != VX_TYPE_F16) return false;
     if (!al16(s->x) || !al16(s->out) || !al16(s->norm) || (s->mask && ((uintptr_t) s->mask % 2 || s->mask_nb1 % 2))) return false;
