@@ -287,3 +287,22 @@ def test_ordering_scalar_is_the_graphs(gpu, env):
     for scale, bias, want in ((0.0, 0.0, 1), (0.0, 0.5, 1), (0.125, 0.0, 0), (0.125, 0.5, 0), (float("nan"), 0.0, 0)):
         st.sync_scale, st.sync_bias = scale, bias
         assert lib().vx_supports_stack(st) == want, (scale, bias)
+
+
+def test_norm_weights_of_another_layout_stay_with_the_separate_calls(gpu, env):
+    """The launch reads dense F32 norm weights; what the separate calls refuse or read otherwise is not its own."""
+    import torch
+    say("stack: norm weights")
+    env.pop("VX_STACK", None)
+    m = build(gpu, 2, 2, 41, False)
+    x = torch.zeros((2, 1, 1024), device="cuda")
+    pos = torch.full((1,), 40, dtype=torch.int32, device="cuda")
+    taken = lambda: m._stack(x, torch.empty_like(x), pos, 1, 40, None, True, 1.0) is not None
+    assert taken()
+    for li, name in ((-1, "norm"), (1, "input_layernorm"), (0, "post_layernorm")):
+        good = m.final_norm if li < 0 else m.norms[li][name]
+        for bad in (good[:8].contiguous(), good.half(), torch.stack([good, good], 1)[:, 0]):
+            m.set_norm(li, name, bad)
+            assert not taken(), (name, bad.dtype, bad.shape, bad.stride())
+        m.set_norm(li, name, good)
+    assert taken()

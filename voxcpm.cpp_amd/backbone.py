@@ -357,6 +357,9 @@ class MiniCPMBackbone:
             return None
         if mask is not None and (mask.dtype != torch.float16 or mask.shape[0] < T or mask.shape[1] != T):
             return None
+        for nw in [self.final_norm] + [n[k] for n in self.norms for k in ("input_layernorm", "post_layernorm")]:
+            if nw is None or nw.dtype != torch.float32 or nw.numel() != self.hidden or nw.shape[-1] != self.hidden or not nw.is_contiguous():
+                return None     # (the launch reads `hidden` dense values; the separate calls look at the descriptor)
         layers = (VxStackLayer * self.n_layer)()
         kc = self.k_cache[0]
         es = kc.element_size()
