@@ -1318,10 +1318,15 @@ bool vs_fill(const vx_stack * s, vs_args & a, vs_plan & p) {
         p.mode = f32 ? VS_F32 : a.n_past + 1 > 64 ? VS_F16 : VS_F16_SHORT;
         // Where the separate calls are the faster ones (us a step of 24 layers, separate / here): with more than eight rows what every
         // work-group stages outweighs the launches -- 16 rows over 6144 keys of an f16 cache 1070 / 1131, over 700 keys 953 / 912, over 40
-        // keys 1260 / 890; 9 rows of an F32 cache over 300 keys 853 / 862, 16 over 200 keys 1436 / 1100; 8 rows of an F32 cache over
-        // 300 keys 831 / 736, over 2000 keys 934 / 949.  Up to seven rows it is the faster one everywhere (one row 767 / 524 over 37 keys,
-        // 729 / 534 over 8000; six rows over 8000 keys 904 / 825).
-        const int most = N > 8 ? (f32 ? 256 : 1024) : N == 8 && f32 ? 1024 : 1 << 30;
+        // keys 1260 / 890; 9 rows of an F32 cache over 300 keys 853 / 862, 16 over 200 keys 1436 / 1100.  Up to eight rows, an F32 cache
+        // (the attention's tiles in registers are seven waves' work here and a whole grid's there) over 300, 2000, 4000 and 8000 keys:
+        //   rows 1  675 / 538   712 / 552   763 / 598   826 / 647      5  789 / 688   858 / 832   918 / 879  1032 / 963
+        //        2  703 / 583   754 / 641   794 / 683   867 / 741      6  802 / 695   878 / 869   940 / 910  1080 / 1022
+        //        4  777 / 621   829 / 718   880 / 768   970 / 840      7  822 / 739   911 / 963   980 / 1023 1157 / 1164
+        // seven rows over 1000 keys 849 / 822, over 1400 878 / 873, over 1535 879 / 885; eight over 400 831 / 756, over 1023 874 / 843, over 2000 934 / 949.
+        // An f16 cache over 300, 2000 and 8000 keys: one row 717 / 499, 716 / 519, 706 / 549; five 794 / 602, 786 / 723, 847 / 823; eight
+        // 800 / 666, 841 / 808, 979 / 936.
+        const int most = N > 8 ? (f32 ? 256 : 1024) : !f32 || N < 7 ? 1 << 30 : N == 7 ? 1408 : 1024;
         if (a.n_past + 1 > most || (N > 8 && a.n_splits > 32)) return false;
     } else {
         // (14 rows, a ten-step solve: 1352 / 1280 us; one pass of 16 rows 130 / 133)
