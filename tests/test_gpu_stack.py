@@ -306,3 +306,24 @@ def test_norm_weights_of_another_layout_stay_with_the_separate_calls(gpu, env):
             assert not taken(), (name, bad.dtype, bad.shape, bad.stride())
         m.set_norm(li, name, good)
     assert taken()
+
+
+def test_a_plan_can_keep_the_separate_calls(gpu, env):
+    import torch
+    say("stack: resident = False")
+    env.pop("VX_STACK", None)
+    m = build(gpu, 2, 2, 41, False)
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    for c in m.k_cache + m.v_cache:
+        c[:, :, :40] = torch.randn((2, 2, 40, 64), generator=gen, device="cuda")
+    x = torch.randn((2, 1, 1024), generator=gen, device="cuda")
+    outs = []
+    for resident in (True, False):
+        m.resident = resident
+        run, out = m.plan(x, 1, 40)
+        areas = [t for t in run._keep if isinstance(t, torch.Tensor) and t.dtype == torch.uint8]
+        assert len(areas) == int(resident)
+        run()
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.equal(*outs)

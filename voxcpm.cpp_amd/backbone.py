@@ -45,6 +45,11 @@ class MiniCPMBackbone:
         self.residual_scale = float(np.float32(scale_depth) / np.sqrt(np.float32(max(1, n_layer)))) if use_mup else 1.0
         self.act_mode = act_mode
         self.fuse_pairs = fuse_pairs
+        # Whether plans of a few token rows run as one resident launch where that takes them.  It holds every compute unit for the whole
+        # step: alone, or beside kernels of other kinds, the step is up to half as fast again, but steps on streams of their own come one
+        # after another where the separate calls' kernels interleave (us for one step on each stream, one row: two streams 895 separate,
+        # 1019 resident; three 968, 1700).  A program that steps several plans at once sets it to False before it makes them.
+        self.resident = True
         self.rope_base, self.rope_original_max = rope_base, rope_original_max
         self.kv_dtype = torch.float16 if kv_f16 else torch.float32
         dev = "cuda"
@@ -327,7 +332,7 @@ class MiniCPMBackbone:
         o2 = out.view(N, self.hidden)
         norm(cur_x, self.final_norm, o2)
 
-        stack = self._stack(x, out, pos, T, n_past, mask, write_kv, attn_factor) if fuse else None
+        stack = self._stack(x, out, pos, T, n_past, mask, write_kv, attn_factor) if fuse and self.resident else None
         if stack is not None:   # (the plan's own exchange area: a graph of it replays beside graphs of other plans)
             area = new(L.vx_stack_area_bytes(stack), dtype=torch.uint8)
             keep.append(area)
