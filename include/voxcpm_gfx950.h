@@ -523,6 +523,8 @@ VX_API int vx_supports_sum(const vx_tensor * src, const vx_tensor * dst);
  * n_past cached keys, the step's keys and values written to the caches (write_kv; the ordering scalar of the graph's cache write,
  * (sum k + sum v) * sync_scale + sync_bias, is added to the attention's result) -- or whole sequences of n_tokens that attend to
  * themselves and leave no cache (n_past 0; mask: F16 [n_tokens][n_tokens] or NULL).  The results are the bits of the separate calls.
+ * Taken: hidden 1024 in 16 heads of 64, ffn 4096 (2048: up to four rows), at most VX_STACK_MAX_LAYERS layers, 32 (row, KV head) pairs
+ * and a number of cached keys up to which it is faster than the separate calls; whole sequences: 14 rows in all.
  * (A step with a sync_scale other than zero, the graph's, is refused.)
  * x and out: dense F32 [batch][n_tokens][hidden].  Weight rows are dense Q8_0 blocks, norms dense F32.  cache_nb1 / nb2 / nb3: byte
  * strides of a cache's rows, heads and sequences, the same for K and V of every layer.  positions: n_tokens int32 on the device.

@@ -1274,8 +1274,9 @@ bool vs_fill(const vx_stack * s, vs_args & a, vs_plan & p) {
     if (!s || !s->layers || !s->x || !s->out || !s->norm || !s->positions) return false;
     if (s->n_layer < 1 || s->n_layer > VX_STACK_MAX_LAYERS || s->batch < 1 || s->n_tokens < 1 || s->n_past < 0) return false;
     const int64_t N = (int64_t) s->batch * s->n_tokens;
-    if (N > 16 || s->head_dim != 64 || s->n_heads < 1 || s->n_kv_heads < 1 || s->n_heads % s->n_kv_heads || s->n_heads / s->n_kv_heads > 16) return false;
-    if (s->hidden != s->n_heads * 64 || s->hidden % 1024 || s->hidden > 2048 || s->ffn % 2048 || s->ffn < 2048 || s->ffn > 4096) return false;
+    if (N > 16 || s->head_dim != 64 || s->n_kv_heads < 1 || s->n_heads % s->n_kv_heads || s->n_heads / s->n_kv_heads > 16) return false;
+    // (the slots below are those of sums over 1024 values)
+    if (s->hidden != 1024 || s->n_heads != 16 || (s->ffn != 2048 && s->ffn != 4096)) return false;
     if (N * s->n_kv_heads > 32) return false;
     const bool decode = s->write_kv != 0;
     if (decode && s->sync_scale != 0.0f) return false; // (vs_addend's order of sums shows in any but a product with zero)
