@@ -85,3 +85,54 @@ def test_prefill_attention_by_two_teams(pkg, gpu, B, n_q, n_kv, kind, sinks, f16
     mask = masks(kind, n_q, n_kv, g) if kind else None
     sk = dev(g.standard_normal(H).astype("float32")) if sinks else None
     check(q, k, v, mask, scale, sk, gpu.flash_attn_ext(q, k, v, mask, scale, sinks=sk))
+
+
+def wide_mask(kind, n):
+    import torch
+    i, j = torch.arange(n, device="cuda")[:, None], torch.arange(n, device="cuda")[None]
+    vis = {"causal": j <= i, "all": j < n + 0 * i, "late hidden": (j <= i + n) & (i < n - n // 10), "early hidden": (j >= 0) & (i >= n // 5), "nothing": (j < 0) & (i >= 0),
+           "window": (j <= i) & (j > i - 300), "prefix": (j <= i) | (j < n // 2), "values": j <= i + n}[kind]
+    m = torch.where(vis, torch.randn((n, n), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda") if kind == "values" else torch.tensor(0.0, device="cuda"),
+                    torch.tensor(float("-inf"), device="cuda"))
+    return m.half().view(1, 1, n, n).contiguous()
+
+
+# more row blocks than compute units: 258 (a second team with a block in two work-groups), 288, 465 (the rule's last at 32 tiles is 465), 512
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("B,H,Hkv,n,kind,sinks", [
+    (1, 16, 2, 2064, "all", False), (1, 16, 2, 2065, "window", True), (1, 16, 2, 2300, "late hidden", False), (1, 16, 2, 2300, "early hidden", True),
+    (1, 16, 2, 2300, "nothing", True), (1, 16, 2, 2300, "causal", False), (1, 16, 2, 2290, "prefix", False), (1, 16, 2, 3001, "values", False),
+    (1, 16, 2, 4096, "all", False), (1, 16, 2, 4095, "window", False), (1, 8, 8, 4096, "all", False), (1, 32, 4, 2113, "late hidden", False)])
+def test_teams_with_a_row_block_each(pkg, gpu, B, H, Hkv, n, kind, sinks, f16):
+    import torch
+    say(f"prefill attention, a row block a team: {B} x {n} heads {H}/{Hkv} {kind} sinks={sinks} f16={f16}")
+    g = rng("parted", B, n, H)
+    q, k, v = (dev(g.standard_normal((B, h, n, 64)).astype("float32")) for h in (H, Hkv, Hkv))
+    if f16:
+        k, v = k.half(), v.half()
+    mask = wide_mask(kind, n)
+    sk = dev(g.standard_normal(H).astype("float32")) if sinks else None
+    out = torch.full((B, n, H, 64), 7.0, device="cuda")
+    check(q, k, v, mask, 0.125, sk, gpu.flash_attn_ext(q, k, v, mask, 0.125, sinks=sk, out=out))
+
+
+@pytest.mark.parametrize("kind", ["all", "causal", "late hidden"])
+def test_cache_write_with_a_row_block_a_team(pkg, gpu, kind):
+    """The cache write's scalar joins both teams' rows: the bits of the call without a write (the scale is zero)."""
+    import torch
+    n, H, Hkv = 2300, 16, 2
+    say(f"prefill attention with a cache write, a row block a team: {kind}")
+    L, d = pkg.lib(), pkg.desc
+    g = rng("parted store", n)
+    q = dev(g.standard_normal((1, H, n, 64)).astype("float32"))
+    k, v = (dev(g.standard_normal((1, n, Hkv, 64)).astype("float32")) for _ in range(2))
+    mask = wide_mask(kind, n)
+    kt, vt = k.transpose(1, 2), v.transpose(1, 2)
+    want = gpu.flash_attn_ext(q, kt, vt, mask, 0.125)
+    kc, vc = (torch.zeros((1, Hkv, n + 3, 64), device="cuda") for _ in range(2))
+    kw, vw = kc[:, :, :n].transpose(1, 2), vc[:, :, :n].transpose(1, 2)
+    got = torch.full_like(want, 7.0)
+    assert L.vx_supports_flash_attn_ext_store(d(q), d(kt), d(vt), d(mask), d(k), d(kw), d(v), d(vw), d(got), 0.0) == 1
+    pkg.check(L.vx_flash_attn_ext_store(d(q), d(kt), d(vt), d(mask), None, d(k), d(kw), d(v), d(vw), d(got), 0.125, 0.0, 0.0, 0.0, 0.0, None), "store")
+    torch.cuda.synchronize()
+    assert torch.equal(want, got) and torch.equal(kc[:, :, :n], kt) and torch.equal(vc[:, :, :n], vt)

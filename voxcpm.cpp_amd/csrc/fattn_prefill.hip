@@ -26,6 +26,7 @@ constexpr int PF_WAVES = 4;
 constexpr int PF_COLS  = 256; // columns per work-group
 constexpr int PF_KT    = 64;  // keys per tile
 constexpr int PF_MAX_TILES = 1024;
+constexpr int PF_PART = 256; // compute units: work-groups that stay where two teams walk a row block each
 constexpr int PF_TOTALS = VX_KVS_V_AT;       // block totals of one sum of a cache write, at most
 constexpr int PF_TOTALS_INLINE = 64; // up to here a wave of every attention work-group adds them (two sequences of 512 tokens: 32 a side; beside
                                      // the tile list that takes less than the 4.5 us of a launch for one number), beyond pf_scalar_kernel does
@@ -160,7 +161,9 @@ __device__ __forceinline__ void pf_dma4(const char * base, uint32_t off, uint32_
 }
 
 // Two probabilities to f16, to nearest (v_cvt_pk_f16_f32).  Rounded toward zero, a column's reference key alone would keep its value,
-// 1, while all others lose half a unit on average: with two references a column (two teams) that was 0.8 % of the whole error.
+// 1, while all others lose half a unit on average: with two references a column (two teams) that was 0.8 % of the whole error, and to
+// nearest the error is 10 % below either.  It costs 0.2 to 0.6 % (causal, toward zero / to nearest: 1 x 1024 20.9 / 21.0 us, 1 x 4096
+// 65.1 / 65.5, 16 x 1024 68.5 / 68.9, 16 x 2048 197.0 / 198.2).
 __device__ __forceinline__ half2_t pf_cvt2(float a, float b) {
     typedef float f2 __attribute__((ext_vector_type(2)));
     return __builtin_convertvector(f2{a, b}, half2_t);
@@ -292,10 +295,12 @@ __global__ __launch_bounds__(128) void pf_scalar_kernel(const double * totals, i
 // VLO: V comes with a low-half image (a.vl).  NCB: 32-column blocks per wave.  SUMS: the addend is the ordering scalar of a.totals
 // (an instance of its own: as a test in every instance it cost the calls without a cache write 1 %, 2048 causal tokens 38.7 -> 39.1 us).
 // TEAMS: sets of PF_WAVES waves over the same columns, each with every TEAMS-th active tile and stages of its own, their (O, sum,
-// reference) joined through LDS at the end.  A wave alone on its SIMD leaves half of the issue slots empty (0.92 us a tile; two that
+// reference) joined through LDS at the end -- or, in a grid of more work-groups than compute units whose walks are alike (pf_two_teams),
+// over a row block each.  A wave alone on its SIMD leaves half of the issue slots empty (0.92 us a tile; two that
 // share the SIMD take 0.62 us each), so a row block walks 64 tiles in about 45 us where one team takes 62; against a cut of the
 // key range into work-groups of their own nothing goes through memory and no launch follows.  One sequence of 4096 tokens 72 -> 64 us.
-template <bool VLO, int NCB, bool SUMS = false, int TEAMS = 1>
+// PART: whether a team may have a row block of its own (an instance of its own: in the others' code the choice cost 0.6 us of a call).
+template <bool VLO, int NCB, bool SUMS = false, int TEAMS = 1, bool PART = false>
 __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_kernel(const pf_args a) {
     constexpr int D = 64;
     constexpr int PF_STAGES = VLO ? 3 : PF_STAGES_MAX; // (three stages of K, V and V low leave room for two work-groups on a compute unit)
@@ -304,9 +309,9 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
     __shared__ __attribute__((aligned(1024))) char v_lds[TEAMS][PF_STAGES][PF_VSTAGE];
     __shared__ __attribute__((aligned(1024))) char vl_lds[VLO ? TEAMS : 1][VLO ? PF_STAGES : 1][VLO ? PF_VSTAGE : 16];
     __shared__ __attribute__((aligned(256))) uint32_t bits_lds[TEAMS][PF_STAGES][64]; // visibility bits of the block's rows: 8 bytes per row
-    __shared__ uint16_t tile_list[PF_MAX_TILES];
-    __shared__ uint8_t  tile_flag[PF_MAX_TILES];
-    __shared__ int      n_active_s;
+    __shared__ uint16_t tile_list[PART ? 2 * PF_MAX_TILES : PF_MAX_TILES];
+    __shared__ uint8_t  tile_flag[PART ? 2 * PF_MAX_TILES : PF_MAX_TILES];
+    __shared__ int      n_active_s[2];
     __shared__ float    y_s; // SUMS
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -316,9 +321,9 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
 
     // ---- which (batch, kv head, row block): heavy (late) row blocks first; blocks of one
     //      (batch, kv head) stay on one XCD (work-groups are dealt round-robin to 8 XCDs)
-    int grp, rb;
-    {
-        const int i = blockIdx.x;
+    int rb, g, b, row0, ncols_blk; // (ncols_blk: valid columns of the block)
+    auto block = [&](int i) {
+        int grp;
         if (a.xcd_map) {
             const int xcd = i & 7, slot = i >> 3;
             grp = (slot / a.n_rb) * 8 + xcd;
@@ -327,30 +332,49 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
             grp = i % a.n_groups;
             rb  = a.n_rb - 1 - i / a.n_groups;
         }
-    }
-    const int g = grp % a.Hkv, b = grp / a.Hkv;
-    const int row0 = rb * a.RB;
+        g = grp % a.Hkv;
+        b = grp / a.Hkv;
+        row0 = rb * a.RB;
+        ncols_blk = min(a.n_q - row0, a.RB) * a.gqa;
+    };
+    block(blockIdx.x);
+
+    // whether the teams walk a row block each: 64 of the mask's flags (4 row blocks x 16 tiles) say, see pf_two_teams
+    uint8_t sample = 0;
+    auto alike = [&]() {
+        const uint64_t bal = __builtin_amdgcn_ballot_w64(sample != 0);
+        int most = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) most = max(most, __builtin_popcountll((bal >> (16 * q)) & 0xFFFF));
+        return 3 * most <= __builtin_popcountll(bal);
+    };
+    if constexpr (PART) sample = a.flags[(((2 * (lane >> 4) + 1) * a.n_rb) >> 3) * a.n_tiles + (((2 * (lane & 15) + 1) * a.n_tiles) >> 5)];
 
     // ---- this wave's columns: lane (hl, cl) holds column cl of each block as the B operand's d = 16 kk + 8 hl .. + 7.
     //      The loads are issued before anything else (the tile list and the first tiles' copies are built while they fly).
-    const int ncols_blk = min(a.n_q - row0, a.RB) * a.gqa; // valid columns of the block
     float4_t qraw[NCB][4][2];
+    auto load_q = [&]() {
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-        const int  col = wave * (32 * NCB) + cb * 32 + cl;
-        const bool ok  = col < ncols_blk;
-        const int  row = row0 + (ok ? (col >> a.gqa_sh) : 0);
-        const int  hd  = g * a.gqa + (ok ? (col & (a.gqa - 1)) : 0);
-        const float * qp = (const float *) (a.q + (uint64_t) row * a.nbq1 + (uint64_t) hd * a.nbq2 + (uint64_t) b * a.nbq3) + 8 * hl;
+        for (int cb = 0; cb < NCB; ++cb) {
+            const int  col = wave * (32 * NCB) + cb * 32 + cl;
+            const bool ok  = col < ncols_blk;
+            const int  row = row0 + (ok ? (col >> a.gqa_sh) : 0);
+            const int  hd  = g * a.gqa + (ok ? (col & (a.gqa - 1)) : 0);
+            const float * qp = (const float *) (a.q + (uint64_t) row * a.nbq1 + (uint64_t) hd * a.nbq2 + (uint64_t) b * a.nbq3) + 8 * hl;
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            qraw[cb][kk][0] = ((const float4_t *) (qp + 16 * kk))[0];
-            qraw[cb][kk][1] = ((const float4_t *) (qp + 16 * kk))[1];
+            for (int kk = 0; kk < 4; ++kk) {
+                qraw[cb][kk][0] = ((const float4_t *) (qp + 16 * kk))[0];
+                qraw[cb][kk][1] = ((const float4_t *) (qp + 16 * kk))[1];
+            }
         }
+    };
+    load_q();
+    if constexpr (PART) {
+        if (blockIdx.x >= PF_PART && alike()) return; // (the second team of an earlier work-group has its block)
     }
 
-    // ---- active key tiles of this row block
-    if (wid == 0) {
+    // ---- active key tiles of this row block, by one wave: list and flags from `at` on, their number
+    auto list_tiles = [&](int at) {
         int base = 0;
         for (int t0 = 0; t0 < a.n_tiles; t0 += 64) {
             const int t = t0 + lane;
@@ -372,10 +396,14 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
             }
             const uint64_t bal = __builtin_amdgcn_ballot_w64(f != 0);
             const int pos = base + __builtin_popcountll(bal & ((1ull << lane) - 1));
-            if (f) { tile_list[pos] = (uint16_t) t; tile_flag[pos] = f; }
+            if (f) { tile_list[at + pos] = (uint16_t) t; tile_flag[at + pos] = f; }
             base += __builtin_popcountll(bal);
         }
-        if (lane == 0) n_active_s = base;
+        return base;
+    };
+    if (wid == 0) {
+        const int n = list_tiles(0);
+        if (lane == 0) n_active_s[0] = n;
     } else if (SUMS && wid == 1) { // the cache write's ordering scalar: k's totals in the low half of the wave, v's in the high
         const int n = hl ? a.n_tv : a.n_tk;
         double tot[PF_TOTALS_INLINE / 32];
@@ -391,9 +419,28 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
         const float sum = (float) t, sv = __shfl(sum, 32, 64);
         if (lane == 0) y_s = kvs_scalar(sum, sv, a.sync_scale, a.sync_bias);
     }
+    bool apart = false, idle = false; // (idle: a second team without a row block)
+    if constexpr (PART) {
+        static_assert(TEAMS == 2, "teams");
+        apart = alike();
+        if (apart && team == 1) {
+            idle = (int) blockIdx.x + PF_PART >= a.n_rb * a.n_groups;
+            if (!idle) {
+                block((int) blockIdx.x + PF_PART);
+                load_q();
+            }
+            if (wave == 0) {
+                const int n = idle ? 0 : list_tiles(PF_MAX_TILES);
+                if (lane == 0) n_active_s[1] = n;
+            }
+        }
+    }
     __syncthreads();
-    const int n_all = __builtin_amdgcn_readfirstlane(n_active_s);
-    const int n_active = TEAMS == 1 ? n_all : (n_all - team + TEAMS - 1) / TEAMS; // this team's: tiles team, team + TEAMS, ... of the list
+    const int n_first = __builtin_amdgcn_readfirstlane(n_active_s[0]);
+    const int n_all = apart ? max(n_first, __builtin_amdgcn_readfirstlane(n_active_s[1])) : n_first;
+    // this team's tiles: team, team + TEAMS, ... of the list, or the whole of its own
+    const int n_active = TEAMS == 1 ? n_all : apart ? __builtin_amdgcn_readfirstlane(n_active_s[team]) : (n_all - team + TEAMS - 1) / TEAMS;
+    const int list_step = apart ? 1 : TEAMS, list_at = apart ? team * PF_MAX_TILES : team;
 
     // Softmax bookkeeping.  Probabilities are taken relative to a per-column *reference* that trails the running maximum:
     // the S^T accumulator starts at -reference (the same value in a lane's 16 registers: a lane holds one column).  The
@@ -453,7 +500,7 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
         int dma_last = 0, dma_stage = 0, dma_tile = 0;
         bool dma_bits = false;
         auto issue_setup = [&](int idx, int stage) {
-            const int at = TEAMS * min(idx, n_active - 1) + team;
+            const int at = list_step * min(idx, n_active - 1) + list_at;
             const int tile = __builtin_amdgcn_readfirstlane(tile_list[at]);
             dma_kt = kg + (uint64_t) tile * PF_KT * a.nbk1;
             dma_vt = vg + (uint64_t) tile * PF_KT * a.nbv1;
@@ -641,8 +688,8 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
 
         for (int it = 0; it < n_active; ++it) {
             const int  stage  = it % PF_STAGES, stage1 = (it + 1) % PF_STAGES;
-            const int  tile   = __builtin_amdgcn_readfirstlane(tile_list[TEAMS * it + team]);
-            const int  flag   = __builtin_amdgcn_readfirstlane(tile_flag[TEAMS * it + team]); // 1 plain, 2 mask values, 3 visibility bits
+            const int  tile   = __builtin_amdgcn_readfirstlane(tile_list[list_step * it + list_at]);
+            const int  flag   = __builtin_amdgcn_readfirstlane(tile_flag[list_step * it + list_at]); // 1 plain, 2 mask values, 3 visibility bits
 
 #pragma unroll
             for (int k = 0; k < NU; ++k) {
@@ -744,16 +791,19 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the loads issued past the last tile
     }
     if constexpr (TEAMS == 2) {
-        static_assert(NCB == 1, "the hand-over below is one column block's");
-        // The walk's barriers are the work-group's: one in front, one a tile.  The second team makes up for the tile it has
+        // The walk's barriers are the work-group's: one in front, one a tile.  A team makes up for the tiles it has
         // not, or for a walk it has not at all.  (A loop of its own: a wave's count is uniform.)
-        const int mine = n_active > 0 ? n_active + 1 : 0, most = n_all > 0 ? (n_all + 1) / 2 + 1 : 0;
+        const int mine = n_active > 0 ? n_active + 1 : 0, most = n_all > 0 ? (apart ? n_all : (n_all + 1) / 2) + 1 : 0;
         for (int i = mine; i < most; ++i) asm volatile("s_barrier" ::: "memory");
+        if (idle) return;
+        l[0] += __shfl_xor(l[0], 32, 64); // (the two lanes of a column hold disjoint keys)
+    }
+    if (TEAMS == 2 && !apart) {
+        static_assert(TEAMS == 1 || NCB == 1, "the hand-over below is one column block's");
         __syncthreads(); // nobody reads a stage any more, and every direct load has landed
         // the second team's sums through its own stages: o by register and lane, then the column's L and reference
-        float * const po = (float *) &k_lds[1][0][0] + wave * (16 + 2) * 64, * const po1 = (float *) &v_lds[1][0][0] + wave * 16 * 64;
+        float * const po = (float *) &k_lds[TEAMS - 1][0][0] + wave * (16 + 2) * 64, * const po1 = (float *) &v_lds[TEAMS - 1][0][0] + wave * 16 * 64;
         static_assert(PF_WAVES * 18 * 64 * 4 <= PF_STAGES * PF_KSTAGE && PF_WAVES * 16 * 64 * 4 <= PF_STAGES * PF_VSTAGE, "room for a team's sums");
-        l[0] += __shfl_xor(l[0], 32, 64); // (the two lanes of a column hold disjoint keys)
         if (team == 1) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) { po[r * 64 + lane] = o[0][0][r]; po1[r * 64 + lane] = o[0][1][r]; }
@@ -855,18 +905,30 @@ bool vx_fattn_prefill_accepts(const vx_tensor * q, const vx_tensor * k, float lo
     return (int64_t) n_rb * n_groups >= 32;
 }
 
-// Whether a grid of 128-column work-groups runs as two teams of waves over the same columns (pf_kernel's TEAMS) instead of one.
-// Up to a work-group for each of 256 compute units the second team runs on what would be idle issue slots; it costs nothing where the
-// walk is a few tiles.  Beyond, the work-groups come one after another where two of one team would share a compute unit, which
-// repays itself only where a long walk ends the call: with a mask (most of a causal mask's work-groups are short; without one all
-// are alike) and tiles enough for the number of work-groups.  Us a call, one team / two, f16 keys and values, causal:
-//   256 work-groups: 2048 tokens 38.2 / 31.1, 2 x 1024 24.3 / 21.5, 4 x 512 17.7 / 17.7; 512 new of 4096 keys (64) 62.7 / 45.5
-//   beyond: 2300 tokens (288 work-groups) 47.8 / 39.2, 4096 (512) 73.9 / 66.4, 2 x 1200 (300) 29.7 / 27.9;
-//   the line: 2 x 1500 (376) 36.6 / 35.9, 2 x 1700 (428) 39.6 / 39.9, 2 x 2048 (512) 41.1 / 41.5; 4 x 700 (352) 23.4 / 26.8.
-//   No mask: 2048 tokens (256) 32.8 / 27.9, 2300 (288) 47.6 / 54.3, 4096 (512) 91.3 / 93.2.  F32 keys and values alike.
+// Whether a grid of 128-column work-groups runs with two teams of waves (pf_kernel's TEAMS) instead of one.
+// Up to a work-group for each of 256 compute units the second team runs on what would be idle issue slots, over the same columns; it
+// costs nothing where the walk is a few tiles.  Beyond, such work-groups come one after another where two of one team would share a
+// compute unit.  That repays itself where a few long walks end the call, as under a causal mask, and costs a prologue where all
+// walks are alike; which it is stands in the mask's flags, so the kernel decides: 64 of them, spread over rows and keys, and where
+// the longest of the four sampled walks is not a third longer than their mean, a work-group's teams take a row block each, placed as one
+// team's work-groups would be.  Us a call, f16 keys and values, one team / two over the same columns:
+//   256 work-groups: 2048 causal tokens 38.2 / 31.1, no mask 32.8 / 27.9, 2 x 1024 24.3 / 21.5, 4 x 512 17.7 / 17.7; 512 new of 4096 keys
+//   (64) 62.7 / 45.5.  No mask, beyond: 2300 tokens (288) 47.6 / 54.3, 4096 (512) 91.3 / 93.2.
+// One team / two over the same columns / by the flags:
+//   tokens (work-groups)   2064 (258)           2300 (288)           2700 (338)           3300 (414)           4096 (512)
+//   causal                 42.3  35.2  34.4     48.1  40.2  39.3     57.6  48.5  48.1     68.0  59.8  59.0     72.3  65.8  65.3
+//   all visible            52.6  61.4  52.8     60.1  68.7  60.1     73.0  81.3  73.4     87.5  93.7  84.8     99.9  103.6 98.8
+//   a third hidden behind  40.7  48.4  41.3     46.9  54.5  47.1     56.9  65.1  58.4     67.6  74.3  66.6     74.1  79.0  74.3
+//   half, then causal      41.4  43.4  42.2     47.4  47.9  46.6     57.0  57.5  57.3     68.8  71.1  70.6     76.6  80.0  79.5
+//   4 causal sequences     28.9  27.4  29.3     35.2  32.0  35.7     43.4  40.0  44.6     51.1  53.4  52.8     37.6  41.8  38.3
+//   window of 512          23.4  27.5  25.7     26.9  34.7  30.3     35.7  43.1  38.1     38.6  46.0  39.8     31.1  38.7  34.7
+// (the short walks lose what the second team's list and rows cost behind the decision).  F32 keys and values alike: causal 2300 59.9 / 49.8 /
+// 49.1, all visible 76.4 / 87.6 / 77.7.  With fewer tiles the causal call gains little and the others lose more: 2 x 1200 (300) causal
+// 29.7 / 28.4 / 29.0, half then causal 29.5 / 34.0; and towards 512 work-groups the causal walks are no longer few: 2 x 1700 (428) 39.2 /
+// 40.3, 2 x 2048 (512) 40.1 / 41.3.
 static bool pf_two_teams(int64_t n_wg, int n_tiles, bool masked) {
-    if (n_wg <= 256) return true;
-    return masked && n_wg <= 512 && n_tiles * (700 - n_wg) >= 7500;
+    if (n_wg <= PF_PART) return true;
+    return masked && n_wg <= 2 * PF_PART && n_tiles >= 32 && n_tiles * (700 - n_wg) >= 7500;
 }
 
 vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v, const vx_tensor * mask,
@@ -997,17 +1059,22 @@ vx_status vx_fattn_prefill(const vx_tensor * q, const vx_tensor * k, const vx_te
     }
     const dim3 grid((unsigned) (n_rb * n_groups)), block(64 * PF_WAVES), block2(2 * 64 * PF_WAVES);
     const bool two = half_cols && pf_two_teams((int64_t) n_rb * n_groups, n_tiles, mask != nullptr);
+    const bool part = two && n_rb * n_groups > PF_PART; // (with a mask only)
     if (a.totals) {
-        if (!half_cols)    vx_launch(pf_kernel<false, 2, true>, grid, block, 0, st, a);
-        else if (a.kv_f32 && two) vx_launch(pf_kernel<true, 1, true, 2>, grid, block2, 0, st, a);
-        else if (two)      vx_launch(pf_kernel<false, 1, true, 2>, grid, block2, 0, st, a);
-        else if (a.kv_f32) vx_launch(pf_kernel<true, 1, true>, grid, block, 0, st, a);
-        else               vx_launch(pf_kernel<false, 1, true>, grid, block, 0, st, a);
+        if (!half_cols)            vx_launch(pf_kernel<false, 2, true>, grid, block, 0, st, a);
+        else if (a.kv_f32 && part) vx_launch(pf_kernel<true, 1, true, 2, true>, grid, block2, 0, st, a);
+        else if (part)             vx_launch(pf_kernel<false, 1, true, 2, true>, grid, block2, 0, st, a);
+        else if (a.kv_f32 && two)  vx_launch(pf_kernel<true, 1, true, 2>, grid, block2, 0, st, a);
+        else if (two)              vx_launch(pf_kernel<false, 1, true, 2>, grid, block2, 0, st, a);
+        else if (a.kv_f32)         vx_launch(pf_kernel<true, 1, true>, grid, block, 0, st, a);
+        else                       vx_launch(pf_kernel<false, 1, true>, grid, block, 0, st, a);
     } else if (half_cols) {
-        if (a.kv_f32 && two) vx_launch(pf_kernel<true, 1, false, 2>, grid, block2, 0, st, a);
-        else if (two)      vx_launch(pf_kernel<false, 1, false, 2>, grid, block2, 0, st, a);
-        else if (a.kv_f32) vx_launch(pf_kernel<true, 1>, grid, block, 0, st, a);
-        else          vx_launch(pf_kernel<false, 1>, grid, block, 0, st, a);
+        if (a.kv_f32 && part)      vx_launch(pf_kernel<true, 1, false, 2, true>, grid, block2, 0, st, a);
+        else if (part)             vx_launch(pf_kernel<false, 1, false, 2, true>, grid, block2, 0, st, a);
+        else if (a.kv_f32 && two)  vx_launch(pf_kernel<true, 1, false, 2>, grid, block2, 0, st, a);
+        else if (two)              vx_launch(pf_kernel<false, 1, false, 2>, grid, block2, 0, st, a);
+        else if (a.kv_f32)         vx_launch(pf_kernel<true, 1>, grid, block, 0, st, a);
+        else                       vx_launch(pf_kernel<false, 1>, grid, block, 0, st, a);
     } else {
         vx_launch(pf_kernel<false, 2>, grid, block, 0, st, a);
     }
