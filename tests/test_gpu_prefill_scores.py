@@ -97,12 +97,12 @@ def wide_mask(kind, n):
     return m.half().view(1, 1, n, n).contiguous()
 
 
-# more row blocks than compute units: 258 (a second team with a block in two work-groups), 288, 465 (the rule's last at 32 tiles is 465), 512
+# more row blocks than compute units: 258 (two second teams with a block), 288, 376, 512, 264 dealt by XCD (8 KV heads); 532: one team
 @pytest.mark.parametrize("f16", [True, False])
 @pytest.mark.parametrize("B,H,Hkv,n,kind,sinks", [
     (1, 16, 2, 2064, "all", False), (1, 16, 2, 2065, "window", True), (1, 16, 2, 2300, "late hidden", False), (1, 16, 2, 2300, "early hidden", True),
     (1, 16, 2, 2300, "nothing", True), (1, 16, 2, 2300, "causal", False), (1, 16, 2, 2290, "prefix", False), (1, 16, 2, 3001, "values", False),
-    (1, 16, 2, 4096, "all", False), (1, 16, 2, 4095, "window", False), (1, 8, 8, 4096, "all", False), (1, 32, 4, 2113, "late hidden", False)])
+    (1, 16, 2, 4096, "all", False), (1, 16, 2, 4095, "window", False), (1, 8, 8, 4200, "all", False), (1, 8, 8, 4200, "early hidden", True), (1, 32, 4, 2113, "late hidden", False)])
 def test_teams_with_a_row_block_each(pkg, gpu, B, H, Hkv, n, kind, sinks, f16):
     import torch
     say(f"prefill attention, a row block a team: {B} x {n} heads {H}/{Hkv} {kind} sinks={sinks} f16={f16}")
@@ -136,3 +136,19 @@ def test_cache_write_with_a_row_block_a_team(pkg, gpu, kind):
     pkg.check(L.vx_flash_attn_ext_store(d(q), d(kt), d(vt), d(mask), None, d(k), d(kw), d(v), d(vw), d(got), 0.125, 0.0, 0.0, 0.0, 0.0, None), "store")
     torch.cuda.synchronize()
     assert torch.equal(want, got) and torch.equal(kc[:, :, :n], kt) and torch.equal(vc[:, :, :n], vt)
+
+
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("B,H,Hkv,n_q,n_kv,kind", [
+    (1, 8, 8, 512, 512, "causal"), (2, 8, 4, 400, 431, "causal"), (1, 16, 16, 300, 333, "hidden rows"), (1, 8, 8, 513, 513, "either team"), (1, 8, 4, 1025, 1025, None),
+    (8, 16, 4, 1024, 1024, "causal"), (8, 16, 4, 1000, 1030, "hidden rows"), (4, 8, 8, 2048, 2048, "causal"), (2, 12, 3, 512, 512, "causal")])
+def test_blocks_of_many_rows(pkg, gpu, B, H, Hkv, n_q, n_kv, kind, f16):
+    """Few heads to a KV head: more rows in a block than there are visibility bits in LDS (32), in blocks of 128 columns and of 256."""
+    import torch
+    say(f"prefill attention, blocks of many rows: {B} x {n_q}/{n_kv} heads {H}/{Hkv} {kind} f16={f16}")
+    g = rng("many rows", B, n_q, n_kv, H, Hkv)
+    q, k, v = (dev(g.standard_normal((B, h, n, 64)).astype("float32")) for h, n in ((H, n_q), (Hkv, n_kv), (Hkv, n_kv)))
+    if f16:
+        k, v = k.half(), v.half()
+    mask = masks(kind, n_q, n_kv, g) if kind else None
+    check(q, k, v, mask, 0.125, None, gpu.flash_attn_ext(q, k, v, mask, 0.125))

@@ -26,6 +26,7 @@ constexpr int PF_WAVES = 4;
 constexpr int PF_COLS  = 256; // columns per work-group
 constexpr int PF_KT    = 64;  // keys per tile
 constexpr int PF_MAX_TILES = 1024;
+constexpr int PF_BIT_ROWS = 32; // rows whose visibility bits of a tile fit the block's LDS: blocks of more rows (few heads to a KV head) take the mask's values
 constexpr int PF_PART = 256; // compute units: work-groups that stay where two teams walk a row block each
 constexpr int PF_TOTALS = VX_KVS_V_AT;       // block totals of one sum of a cache write, at most
 constexpr int PF_TOTALS_INLINE = 64; // up to here a wave of every attention work-group adds them (two sequences of 512 tokens: 32 a side; beside
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
     __shared__ __attribute__((aligned(1024))) char k_lds[TEAMS][PF_STAGES][PF_KSTAGE];
     __shared__ __attribute__((aligned(1024))) char v_lds[TEAMS][PF_STAGES][PF_VSTAGE];
     __shared__ __attribute__((aligned(1024))) char vl_lds[VLO ? TEAMS : 1][VLO ? PF_STAGES : 1][VLO ? PF_VSTAGE : 16];
-    __shared__ __attribute__((aligned(256))) uint32_t bits_lds[TEAMS][PF_STAGES][64]; // visibility bits of the block's rows: 8 bytes per row
+    __shared__ __attribute__((aligned(256))) uint32_t bits_lds[TEAMS][PF_STAGES][2 * PF_BIT_ROWS]; // visibility bits of the block's rows: 8 bytes per row
     __shared__ uint16_t tile_list[PART ? 2 * PF_MAX_TILES : PF_MAX_TILES];
     __shared__ uint8_t  tile_flag[PART ? 2 * PF_MAX_TILES : PF_MAX_TILES];
     __shared__ int      n_active_s[2];
@@ -393,6 +394,7 @@ __global__ __launch_bounds__(64 * PF_WAVES * TEAMS) __attribute__((amdgpu_waves_
                     f = 1;
                 }
                 if (f == 1 && (t + 1) * PF_KT > a.n_kv) f = 3; // partial tile: the bounds are visibility bits
+                if (f == 3 && a.flags && a.RB > PF_BIT_ROWS) f = 2; // (the values themselves say the same)
             }
             const uint64_t bal = __builtin_amdgcn_ballot_w64(f != 0);
             const int pos = base + __builtin_popcountll(bal & ((1ull << lane) - 1));
