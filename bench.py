@@ -672,6 +672,8 @@ PROFILE_RUNS = [
      [("sq1", SQ_SET_1), ("sq2", SQ_SET_2), ("fetch", "FETCH_SIZE"), ("write", "WRITE_SIZE")], "gemm|mm_|qt_"),
     ("backbone_decode_cfg4", "backbone", "Backbone decode step, 24 layers, batch 2, Q8_0 weights, f16 KV cache at ~520 keys (BASELINE config 4)", [], ""),
     ("backbone_decode_cfg5", "backbone16", "Backbone stack at BASELINE config 5 (batch 16, f16 KV 4096 -> 8192, prefill 16 x 4096)", [], ""),
+    ("step_1_kv37", "step_b1_kv37_f32", "A decode step of one sequence behind 37 keys through 24 layers (resident stack), Q8_0 weights, F32 KV cache, replayed from a HIP graph",
+     [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "stack"),
     ("prompt_1x45", "prompt_1x45_f32", "A prompt of 45 tokens through 24 layers, Q8_0 weights, F32 KV cache", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "gm_|fattn"),
     ("prompt_2x512", "prompt_2x512_f16", "Two prompts of 512 tokens through 24 layers, Q8_0 weights, f16 KV cache", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "gm_|pf_"),
     ("locdit_8_requests", "locdit_r8_l7", "One LocDiT estimator pass of eight concurrent requests, 4 layers, replayed from a HIP graph", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)],
@@ -793,7 +795,7 @@ def main():
     ap.add_argument("--profile-commands", metavar="RAW", default=None, help="print the rocprofv3 runs behind profiles/ (name, tab, command), outputs under RAW")
     ap.add_argument("--summarize", nargs=3, metavar=("RAW", "OUT", "COMMIT"), default=None, help="write profiles/*.txt from the raw output of those runs")
     ap.add_argument("--profile", choices=["decode5", "decode2", "prefill", "prefill1", "backbone", "backbone16", "cfm", "cfm8", "gemm", "peaks", "prompt_1x45_f32", "prompt_2x512_f16",
-                                              "locdit_r8_l7"], default=None,
+                                              "locdit_r8_l7", "step_b1_kv37_f32"], default=None,
                     help="run only this workload a few times (for rocprofv3) and print its figures")
     args = ap.parse_args()
     if args.profile_commands:
@@ -832,7 +834,7 @@ def main():
     if args.profile == "peaks":
         print(json.dumps({"profile": "peaks", **peaks_bench(timer)}))
         return
-    if args.profile in ("prompt_1x45_f32", "prompt_2x512_f16", "locdit_r8_l7"):   # passes of perf/cases.py's workload of that name
+    if args.profile in ("prompt_1x45_f32", "prompt_2x512_f16", "locdit_r8_l7", "step_b1_kv37_f32"):   # passes of perf/cases.py's workload of that name
         from perf import cases
         state = cases.prepare(next(c for c in cases.listed() if c["name"] == args.profile), 1)
         s = timer.run(lambda: cases.run(state), iters=20, warmup=3)
