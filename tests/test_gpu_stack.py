@@ -327,3 +327,16 @@ def test_a_plan_can_keep_the_separate_calls(gpu, env):
         outs.append(out)
     torch.cuda.synchronize()
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("n_kv,batch,past,f16", [(1, 4, 70, True), (1, 5, 40, False), (8, 4, 300, False), (8, 3, 33, True), (16, 1, 40, True), (16, 1, 20, False)])
+def test_numbers_of_kv_heads(gpu, env, n_kv, batch, past, f16):
+    """One to sixteen query heads to a KV head: other pairs a work-group, other columns of an attention unit."""
+    import torch
+    say(f"stack: 16 / {n_kv} heads, {batch} sequences behind {past} keys, f16 cache {f16}")
+    m = build(gpu, 2, batch, past + 1, f16, n_kv_heads=n_kv)
+    gen = torch.Generator(device="cuda").manual_seed(past)
+    for c in m.k_cache + m.v_cache:
+        c[:, :, :past] = torch.randn((batch, n_kv, past, 64), generator=gen, device="cuda")
+    x = torch.randn((batch, 1, 1024), generator=gen, device="cuda")
+    both(env, m, x, 1, past, groups=(None, 77))
