@@ -155,7 +155,10 @@ VX_API vx_status vx_soft_max(const vx_tensor * src, const vx_tensor * mask, cons
  * q [D, n_q, Hq, ne3] F32; k [D, n_kv, Hkv, ne3'] F16|F32; v like k; mask [n_kv, >=n_q,
  * ne32, ne33] F16 or NULL; sinks device float[Hq] or NULL; dst [D, Hq, n_q, ne3] F32
  * contiguous.  D (= DK = DV) in {64, 128}.  Row strides are free (permuted views and
- * KV-cache views are fine); the innermost dimension must be dense. */
+ * KV-cache views are fine); the innermost dimension must be dense.
+ * The order of a row's sums (and so its last bits) goes by the whole call -- query rows, keys, heads, sequences, from 2049 rows on a
+ * mask's shape too -- since these set how its keys are dealt: a sequence alone and the same sequence in a batch agree to rounding, not to the
+ * bit. */
 VX_API vx_status vx_flash_attn_ext(const vx_tensor * q, const vx_tensor * k, const vx_tensor * v,
                                    const vx_tensor * mask, const float * sinks, const vx_tensor * dst,
                                    float scale, float max_bias, float logit_softcap,

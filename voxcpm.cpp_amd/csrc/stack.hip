@@ -13,7 +13,8 @@
 //     units (16 KB; 2.5 for 64), against 4.6 to 6.2 us for data behind flags and 10.6 us for a release / acquire barrier.
 // Steps of 24 layers (us, separate calls / here): one sequence over 37 keys 767 / 524, over 8000 keys 729 / 534; two over 700 keys 718 /
 // 528; four 791 / 559; eight 846 / 693.  A layer of the one-token step is 20 us now: 6 of the attention, and for each product 1.4 of the
-// exchange, the sums' ends and the next activations' norm (1.0) and 0.5 to 1.4 of the products, whose LDS reads bound them.
+// exchange, the sums' ends and the next activations' norm (1.0) and 0.5 to 1.4 of the products.  Waves wait for 78 % of their cycles; a
+// SIMD issues vector work for 16 % of the time and matrix work for 2 %, LDS bank conflicts take 1 to 4 %: trips bound it.
 // Beside other work (one row, separate / here): next to a stream of large products 3358 / 663 us, of 203-token prompts 919 / 537, of
 // elementwise passes over 1 GiB 2635 / 1142 -- the launch keeps its compute units once it has them.  Next to others of its kind: one
 // step on each of two streams 895 / 1019, three 968 / 1700 (two that wait for the chip get half of it each, and without a whole
