@@ -136,7 +136,7 @@ def test_values_that_are_no_numbers_arrive(gpu, env, value):
 
 
 def test_first_call_under_a_capture_and_replays(gpu, env):
-    """A stream whose first call is recorded: the exchange area is allocated beside the capture, and every replay clears it."""
+    """A stream whose first call is recorded: every replay clears the plan's exchange area."""
     import torch
     say("stack: captured and replayed")
     m = build(gpu, 2, 2, 301, True)
@@ -340,3 +340,30 @@ def test_numbers_of_kv_heads(gpu, env, n_kv, batch, past, f16):
         c[:, :, :past] = torch.randn((batch, n_kv, past, 64), generator=gen, device="cuda")
     x = torch.randn((batch, 1, 1024), generator=gen, device="cuda")
     both(env, m, x, 1, past, groups=(None, 77))
+
+
+def test_the_streams_workspace_as_area_grows_beside_a_capture(gpu, env):
+    """vx_stack_run, whose area lies in the stream's workspace: recorded as the stream's first call, then replayed."""
+    import torch
+    from voxcpm_cpp_amd import lib
+    say("stack: vx_stack_run captured on a fresh stream")
+    env.pop("VX_STACK", None)
+    m = build(gpu, 2, 3, 301, True)
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    for c in m.k_cache + m.v_cache:
+        c[:, :, :300] = torch.randn((3, 2, 300, 64), generator=gen, device="cuda")
+    x = torch.randn((3, 1, 1024), generator=gen, device="cuda")
+    run, out = m.plan(x, 1, 300)
+    run()
+    torch.cuda.synchronize()
+    want = out.clone()
+    st = m._stack(x, out, run._keep[0], 1, 300, None, True, 1.0)
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        assert lib().vx_stack_run(st, torch.cuda.current_stream().cuda_stream) == 0
+    for _ in range(4):
+        out.zero_()
+        (torch.randn(1 << 20, device="cuda") * 2).sum().item()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
