@@ -37,6 +37,7 @@ struct gm_args {
     const half8_t * xt;            // [batch][k block][n_tt][64] operand tiles
     int           n_tt, n_kb;
     int           N, ne12;
+    int           xr;              // log2 of the XCDs that share out the row tiles (the others share out the token tiles)
     const char *  res;
     uint64_t      rnb1, rnb2, rnb3;
     float         res_scale;
@@ -91,7 +92,10 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
     const int j = lane >> 4, c = lane & 15;
     const int g = wid % KG, rw = wid / KG; // k group (block kb belongs to group kb mod KG), row group
 
-    int mi = 0, tx = blockIdx.x;
+    // (work-groups are dealt to the eight XCDs in turn, the grid's width is a multiple of 8)
+    const int xcd = blockIdx.x & 7;
+    int mi = 0, tx = (((int) blockIdx.x >> 3) << a.xr) + (xcd & ((1 << a.xr) - 1));
+    const int ty = ((int) blockIdx.y << (3 - a.xr)) + (xcd >> a.xr);
     if constexpr (EPI == GM_SEGS) {
         if (a.nmat > 1 && tx >= a.mat[1].wg0) mi = 1;
         if (a.nmat > 2 && tx >= a.mat[2].wg0) mi = 2;
@@ -99,8 +103,8 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
     }
     const vx_gm_mat & mt = a.mat[mi];
     const int M = mt.M;
-    if (tx * sh::ROWS >= (EPI == GM_SWIGLU ? 2 * M : M)) return; // padding of the grid
-    const int tt0 = blockIdx.y * NT;
+    if (tx * sh::ROWS >= (EPI == GM_SWIGLU ? 2 * M : M) || ty * sh::TOKS >= a.N) return; // padding of the grid
+    const int tt0 = ty * NT;
     const int batch = blockIdx.z;
     const int nst = a.n_kb / (4 * CH);
 
@@ -612,10 +616,19 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
     if (epi == GM_SWIGLU) gx = (2 * (int64_t) c.mat[0].M + g.rows - 1) / g.rows;
     else for (int i = 0; i < c.nmat; ++i) { a.mat[i].wg0 = (int) gx; gx += (c.mat[i].M + g.rows - 1) / g.rows; }
     const int64_t gy = (c.N + g.toks - 1) / g.toks;
-    // Row tile x of every token tile goes to XCD x mod 8 (work-groups are dealt round-robin, the grid's width a multiple of
-    // 8): its weights come into one L2.
-    if (gx > 8 && epi != GM_SEGS) gx = (gx + 7) / 8 * 8;
-    if (gx > 0x7fffffff || gy > 65535) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
-    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) gx, (int) gy, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) gx, (int) gy, nbatch, st);
+    // Which tiles an XCD takes: 1, 2, 4 or all 8 of them share out the row tiles, the rest the token tiles.  What the eight L2s
+    // bring in is every weight once per group of token tiles and every activation once per group of row tiles.
+    const double wbytes = (double) gx * g.rows * (c.K / 32) * (c.wtype == VX_GM_Q8 ? 34 : 64), xbytes = (double) c.N * c.K * 2;
+    double least = 0.0;
+    int64_t lx = 0, ly = 0, fill = 0;
+    for (int r = 3; r >= 0; --r) {
+        const int64_t nx = (gx + (1 << r) - 1) >> r, ny = (gy + (8 >> r) - 1) / (8 >> r), rounds = (nx * ny * nbatch + 31) / 32;
+        const double bytes = wbytes * (8 >> r) + xbytes * (1 << r);
+        if (lx && (rounds > fill || (rounds == fill && bytes >= least))) continue;
+        a.xr = r; least = bytes; lx = nx; ly = ny; fill = rounds;
+    }
+    gx = 8 * lx;
+    if (gx > 0x7fffffff || ly > 65535) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
+    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) gx, (int) ly, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) gx, (int) ly, nbatch, st);
     return ok ? VX_OK : vx_fail(VX_ERR_HIP, "mul_mat: the kernel could not be given its LDS");
 }
