@@ -37,6 +37,9 @@ struct gm_args {
     const half8_t * xt;            // [batch][k block][n_tt][64] operand tiles
     int           n_tt, n_kb;
     int           N, ne12;
+    const half8_t * wt;            // gd_kernel: the weights as operand tiles [k block][n_rt][64] ...
+    const float * wdt;             // ... and their scales, per 64 rows [16][4]
+    int           n_rt;            // 16-row tiles (of a pair's alternating ones)
     int           xr;              // log2 of the XCDs that share out the row tiles (the others share out the token tiles)
     const char *  res;
     uint64_t      rnb1, rnb2, rnb3;
@@ -362,6 +365,229 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
     }
 }
 
+// ---- the same product from weights that are laid out already ----------------------------------------------------------
+// Pinned Q8_0 weights may be at hand as f16 operand tiles (vx_qt_kept_tiles).  Then a compute wave has nothing to convert, which
+// is two of gm_kernel's seven vector slots a product, and owns 64 rows by itself: it fetches their tiles from memory straight into
+// the operand registers, four k blocks ahead, so that only the activations (which its three neighbours need as well) and the scales
+// pass through LDS, in stages of two k blocks with one barrier a stage.  What bounds it is the matrix core and the four scaled
+// additions of every product, which a SIMD overlaps only in part (25 cycles measured for the five, 16.5 and 9 for the two sides alone);
+// two work-groups a compute unit.  In a layer of 1024 tokens the pair of 4096 rows takes 28 us, 42.5 on gm_kernel; 24 layers 2769 -> 2481.
+// The k blocks are walked group by group (0, 4, 8 ..., then 1, 5, ...) and a group's sum is added to the total before the next
+// begins: gm_kernel's order of every sum, so which of the two runs does not show in the result.
+constexpr int GD_CT = 4, GD_ST = 3, GD_ROWS = 256, GD_TOKS = 16 * GD_CT;
+constexpr int GD_BLOCK = GD_CT * 1024, GD_STAGE = 2 * GD_BLOCK + 4 * 1024; // two blocks of token tiles, 1 KB of scales per wave (512 bytes of it read)
+constexpr int GD_LDS = GD_ST * GD_STAGE;
+
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gd_kernel(const gm_args a) {
+    extern __shared__ __align__(1024) char gm_smem[];
+    typedef __attribute__((address_space(3))) char lds_char;
+    typedef const __attribute__((address_space(3))) half8_t  lds_half8;
+    typedef const __attribute__((address_space(3))) float4_t lds_float4;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
+    const int j = lane >> 4, c = lane & 15;
+    const int xcd = blockIdx.x & 7;
+    const int tx = (((int) blockIdx.x >> 3) << a.xr) + (xcd & ((1 << a.xr) - 1)), ty = ((int) blockIdx.y << (3 - a.xr)) + (xcd >> a.xr);
+    if (tx * (GD_ROWS / 16) >= a.n_rt || ty * GD_TOKS >= a.N) return; // padding of the grid
+    const int batch = blockIdx.z, nkb = a.n_kb;
+    const int rtw = tx * (GD_ROWS / 16) + 4 * wid, tt0 = ty * GD_CT; // the wave's first row tile, the work-group's first token tile
+    const int n_rt4 = (a.n_rt + 3) & ~3;
+    const uint32_t smem0 = (uint32_t) (uintptr_t) (lds_char *) gm_smem, loff = (uint32_t) lane * 16;
+
+    // The k blocks in the order of the sums: in steps of four, from a group's last block to the next group's first (behind the last
+    // group blocks 4, 8 ... again: fetched for nothing).
+    const int n4 = nkb / 4;
+    // ---- a stage: wave w brings token tiles 2 (w mod 2), + 1 of block w / 2, and its own rows' scales of both blocks
+    // (past the last token tile: that one again, dropped at the store)
+    const int64_t xstr = (int64_t) a.n_tt * 1024;
+    const char * xsrc = (const char *) a.xt + ((int64_t) batch * nkb + (wid < 2 ? 0 : 4)) * xstr;
+    const uint32_t xo0 = (uint32_t) min(tt0 + 2 * (wid & 1), a.n_tt - 1) * 1024 + loff, xo1 = (uint32_t) min(tt0 + 2 * (wid & 1) + 1, a.n_tt - 1) * 1024 + loff;
+    const char * dsrc = (const char *) (a.wdt + min(rtw, n_rt4 - 4) * 16);
+    const int64_t dstr = (int64_t) n_rt4 * 64;
+    const uint32_t doff = (uint32_t) (lane & 16 ? 4 * dstr : 0) + (uint32_t) c * 16; // (lanes 32 on: the same again)
+    const uint32_t sdst = smem0 + (uint32_t) ((wid >> 1) * GD_BLOCK + 2 * (wid & 1) * 1024);
+    int sleft = n4 / 2; // stages of the group that are still to be requested
+    uint32_t ibuf = 0;
+    auto request = [&](int i) {
+        if (i < 2) {
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(i ? xo1 : xo0), "s"(xsrc), "s"(sdst + ibuf + i * 1024) : "memory");
+        } else {
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(doff), "s"(dsrc), "s"(smem0 + ibuf + 2 * GD_BLOCK + wid * 1024) : "memory");
+            const int64_t step = --sleft ? 8 : 9 - nkb;
+            sleft = sleft ? sleft : n4 / 2;
+            xsrc += step * xstr;
+            dsrc += step * dstr;
+            ibuf = ibuf + GD_STAGE == GD_ST * GD_STAGE ? 0 : ibuf + GD_STAGE;
+        }
+    };
+    // ---- the wave's weights: four row tiles a block
+    // (buffer loads: a base that stays, one 32-bit offset a lane and row tile, one scalar that walks the blocks; gd_takes keeps the
+    // matrix below 4 GiB)
+    const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *) a.wt, (short) 0, (int) ((uint32_t) nkb * (uint32_t) a.n_rt * 1024u), 0x00027000);
+    const uint32_t wstr = (uint32_t) a.n_rt * 1024u, wstep = 4 * wstr, wback = (uint32_t) (5 - nkb) * wstr;
+    uint32_t wsoff = 0;
+    int wleft = n4;
+    uint32_t woff[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) woff[rt] = (uint32_t) min(rtw + rt, a.n_rt - 1) * 1024 + loff;
+    half8_t b[4][4], x[GD_CT];
+    float4_t d[2];
+    auto fetch = [&](int set, int rt) {
+        b[set][rt] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, (int) woff[rt], (int) wsoff, 0));
+        if (rt == 3) {
+            wsoff += --wleft ? wstep : wback;
+            wleft = wleft ? wleft : n4;
+        }
+    };
+    float4_t acc[4][GD_CT], tot[4][GD_CT];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int tt = 0; tt < GD_CT; ++tt) { acc[rt][tt] = float4_t{0, 0, 0, 0}; tot[rt][tt] = float4_t{-0.0f, -0.0f, -0.0f, -0.0f}; } // (-0 + s is s)
+    auto stage_wait = [&](auto NC) { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(decltype(NC)::value) : "memory"); };
+    auto barrier = [&]() { __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fetch(0, i);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) request(i % 3);
+#pragma unroll
+    for (int i = 4; i < 16; ++i) fetch(i >> 2, i & 3);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) request(i);
+    stage_wait(std::integral_constant<int, 18>{}); // younger than stage 0: stages 1 and 2, the weight tiles of three blocks
+    barrier();
+    uint32_t rbuf = 0;
+#pragma unroll
+    for (int n = 0; n < GD_CT; ++n) x[n] = *(lds_half8 *) ((const lds_char *) gm_smem + n * 1024 + loff);
+    const uint32_t dof = 2 * GD_BLOCK + wid * 1024 + c * 16;
+    d[0] = *(lds_float4 *) ((const lds_char *) gm_smem + dof);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // A block: its operands (set P of the weights and scales, the tokens) are in registers; row by row its products are issued, their
+    // scaled additions two products behind, and what the row leaves free takes the next blocks' bytes.
+    auto block = [&](auto SET, auto LAST) {
+        constexpr int Q = decltype(SET)::value, P = Q & 1, T = 4 * GD_CT, LAG = 2;
+        constexpr bool more = !decltype(LAST)::value;
+        const uint32_t nbuf = rbuf + GD_STAGE == GD_ST * GD_STAGE ? 0 : rbuf + GD_STAGE;
+        const lds_char * nx = (const lds_char *) gm_smem + (P ? nbuf : rbuf + GD_BLOCK) + loff;
+        const lds_char * nd = (const lds_char *) gm_smem + (P ? nbuf : rbuf + 256) + dof;
+        float4_t blk[LAG + 1];
+#pragma unroll
+        for (int i = 0; i < T + LAG; ++i) {
+            const int rt = i / GD_CT, n = i % GD_CT;
+            if (i < T) {
+                blk[i % (LAG + 1)] = mfma16(x[n], b[Q][rt], float4_t{0, 0, 0, 0});
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (more) {
+                    if (P == 1 && i == GD_CT - 1) {
+                        // The next stage has landed once at most these are outstanding: younger than stage 1 are 19 loads, than stage 2 the
+                        // 15 of blocks 0 to 2, later 16.  Behind the barrier every wave has this stage's operands in registers: its
+                        // buffer takes the stage after next.
+                        stage_wait(std::integral_constant<int, 15>{});
+                        barrier();
+                    }
+                    if (P == 1 && i > GD_CT && i % GD_CT == 1) request(rt - 1);
+                    if (rt == 3) x[n] = *(lds_half8 *) (nx + n * 1024);
+                    if (rt == 2 && n == GD_CT - 1) d[1 - P] = *(lds_float4 *) nd;
+                    if (n == GD_CT - 1) fetch(Q, rt);
+                }
+            }
+            if (i >= LAG) {
+                const int p = i - LAG;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[p / GD_CT][p % GD_CT][r] = __builtin_fmaf(blk[p % (LAG + 1)][r], d[P][p / GD_CT], acc[p / GD_CT][p % GD_CT][r]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (P) rbuf = nbuf;
+    };
+    auto add_group = [&]() {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+            for (int n = 0; n < GD_CT; ++n) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) { tot[rt][n][r] += acc[rt][n][r]; acc[rt][n][r] = 0.0f; }
+                asm volatile("" : "+v"(tot[rt][n]), "+v"(acc[rt][n]));
+            }
+    };
+    using set0 = std::integral_constant<int, 0>;
+    using set1 = std::integral_constant<int, 1>;
+    using set2 = std::integral_constant<int, 2>;
+    using set3 = std::integral_constant<int, 3>;
+    auto four = [&](auto LAST) { block(set0{}, std::false_type{}); block(set1{}, std::false_type{}); block(set2{}, std::false_type{}); block(set3{}, LAST); };
+    const int turns = nkb / 16; // of a group
+    for (int g = 0; g < 3; ++g) {
+        for (int s = 0; s < turns; ++s) four(std::false_type{});
+        add_group();
+    }
+    for (int s = 0; s < turns - 1; ++s) four(std::false_type{});
+    four(std::true_type{});
+    add_group();
+    stage_wait(std::integral_constant<int, 0>{}); // (stages requested past the end have landed before the work-group's LDS is given back or used again)
+
+    // lane (j, c), tile (rt, n), register r: token 16 (tt0 + n) + 4 j + r, virtual row 16 (rtw + rt) + c
+    const int i12 = batch % a.ne12, i13 = batch / a.ne12;
+    const vx_gm_mat & mt = a.mat[0];
+    const int M = mt.M;
+    char * db = mt.dst + (uint64_t) i12 * mt.nb2 + (uint64_t) i13 * mt.nb3;
+    if constexpr (EPI == GM_SWIGLU) {
+        const int row0 = 8 * rtw; // the wave's 32 rows
+        if (a.tile_out) { // (uniform) rounded to f16 as the next product's activation pass would round it; whole tiles are written
+            __syncthreads(); // (the stages are read out: 4 KB of them for each wave's four tiles)
+            lds_char * mine = (lds_char *) gm_smem + wid * GD_CT * 1024;
+            if (row0 >= M) return;
+#pragma unroll
+            for (int n = 0; n < GD_CT; ++n)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float gt = tot[2 * p][n][r], u = tot[2 * p + 1][n][r];
+                        float h = (gt / (1.0f + expf(-gt))) * u;
+                        asm volatile("" : "+v"(h)); // the fp32 value the GLU node holds, formed as such
+                        *(__attribute__((address_space(3))) _Float16 *) (mine + n * 1024 + ((2 * p + (c >> 3)) * 16 + 4 * j + r) * 16 + (c & 7) * 2) = (_Float16) h;
+                    }
+            char * out = (char *) a.tile_out + (((uint64_t) batch * (uint32_t) (M >> 5) + (uint32_t) (row0 >> 5)) * (uint32_t) a.out_tt + (uint32_t) tt0) * 1024 + loff;
+#pragma unroll
+            for (int n = 0; n < GD_CT; ++n)
+                if (16 * (tt0 + n) < a.N) *(half8_t *) (out + n * 1024) = *(lds_half8 *) (mine + n * 1024 + loff);
+            return;
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int row = row0 + 16 * p + c;
+            if (row >= M) continue;
+#pragma unroll
+            for (int n = 0; n < GD_CT; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int   tok = 16 * (tt0 + n) + 4 * j + r;
+                    const float gt = tot[2 * p][n][r], u = tot[2 * p + 1][n][r];
+                    if (tok < a.N) *(float *) (db + (uint64_t) tok * mt.nb1 + (uint64_t) row * 4) = (gt / (1.0f + expf(-gt))) * u;
+                }
+        }
+    } else {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) {
+            const int row = 16 * (rtw + rt) + c;
+            if (row >= M) continue;
+#pragma unroll
+            for (int n = 0; n < GD_CT; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int tok = 16 * (tt0 + n) + 4 * j + r;
+                    if (tok >= a.N) continue;
+                    float val = tot[rt][n][r];
+                    if (a.res)
+                        val = scaled_residual(val, a.res_scale, *(const float *) (a.res + (uint64_t) i12 * a.rnb2 + (uint64_t) i13 * a.rnb3 + (uint64_t) tok * a.rnb1 + (uint64_t) row * 4));
+                    *(float *) (db + (uint64_t) tok * mt.nb1 + (uint64_t) row * 4) = val;
+                }
+        }
+    }
+}
+
 // ---- activations -> operand tiles ------------------------------------------------------------------------------------
 struct gm_acts {
     const char *  x;
@@ -557,6 +783,17 @@ size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch) {
     return (size_t) nbatch * (size_t) (K / 32) * (size_t) ((N + 15) / 16) * 1024 + 8192;
 }
 
+// Single products and pairs that gd_kernel takes where the weights' tiles are kept: from the number of its 256 x 64 tiles on at which
+// it beats gm_kernel's smaller ones.  gm_kernel / here, microseconds, activation pass included: 4096 x 1024 x 768 tokens (192 tiles)
+// 21.9 / 21.2, x 512 (128) 15.0 / 19.6, x 2048 42 / 32; 1024 x 4096 x 3000 (188) 64.9 / 58.8, x 2048 (128) 41 / 54.  A pair of 4096 rows
+// with its down projection behind it, by the token count: 256 (128 tiles) 27.2 / 31.0, 300 (160) 36.5 / 32.4, 512 38.7 / 34.7, 1024 62.8 / 49.5.
+static bool gd_takes(const vx_gm_call & c, int epi, int nbatch) {
+    if (c.wtype != VX_GM_Q8 || epi == GM_SEGS || c.K % 512) return false; // (a group's k blocks in whole fours)
+    const int64_t MV = c.w2 ? 2 * (int64_t) c.mat[0].M : c.mat[0].M;
+    if ((c.w2 && c.mat[0].M % 32) || (MV + 15) / 16 * (c.K / 32) >= (1 << 22)) return false;
+    return (MV + GD_ROWS - 1) / GD_ROWS * ((c.N + GD_TOKS - 1) / GD_TOKS) * nbatch >= (c.w2 ? 160 : 192);
+}
+
 vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
     const int nbatch = c.ne12 * c.ne13;
     gm_args a = {};
@@ -594,8 +831,38 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
         if (c.norm_w) vx_launch(gm_acts_kernel<true>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p);
         else          vx_launch(gm_acts_kernel<false>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p);
     }
-    // the tile whose work-groups finish first by the measured costs
     const int epi = c.w2 ? GM_SWIGLU : c.nmat > 1 ? GM_SEGS : GM_PLAIN;
+    // Which tiles an XCD takes: 1, 2, 4 or all 8 of them share out the row tiles, the rest the token tiles.  What the eight L2s
+    // bring in is every weight once per group of token tiles and every activation once per group of row tiles.
+    auto share = [&](int64_t gx, int64_t gy, double wbytes, int per_cu, int64_t & lx, int64_t & ly) {
+        const double xbytes = (double) c.N * c.K * 2;
+        double least = 0.0;
+        int64_t fill = 0;
+        lx = ly = 0;
+        for (int r = 3; r >= 0; --r) {
+            const int64_t nx = (gx + (1 << r) - 1) >> r, ny = (gy + (8 >> r) - 1) / (8 >> r), rounds = (nx * ny * nbatch + 32 * per_cu - 1) / (32 * per_cu);
+            const double bytes = wbytes * (8 >> r) + xbytes * (1 << r);
+            if (lx && (rounds > fill || (rounds == fill && bytes >= least))) continue;
+            a.xr = r; least = bytes; lx = nx; ly = ny; fill = rounds;
+        }
+        lx *= 8;
+        return lx <= 0x7fffffff && ly <= 65535;
+    };
+    int64_t lx = 0, ly = 0;
+    if (gd_takes(c, epi, nbatch)) {
+        const void * tiles = nullptr;
+        const float * scales = nullptr;
+        const int64_t MV = c.w2 ? 2 * (int64_t) c.mat[0].M : c.mat[0].M;
+        if (share((MV + GD_ROWS - 1) / GD_ROWS, (c.N + GD_TOKS - 1) / GD_TOKS, (double) MV * c.K * 2, 2, lx, ly) &&
+            vx_qt_kept_tiles(c.mat[0].w, c.w2, c.K, c.mat[0].M, c.mat[0].nb01, st, &tiles, &scales)) {
+            a.wt = (const half8_t *) tiles; a.wdt = scales; a.n_rt = (int) ((MV + 15) / 16);
+            const dim3 grid((unsigned) lx, (unsigned) ly, (unsigned) nbatch);
+            if (epi == GM_SWIGLU) vx_launch(gd_kernel<GM_SWIGLU>, grid, dim3(256), (size_t) GD_LDS, st, a);
+            else                  vx_launch(gd_kernel<GM_PLAIN>, grid, dim3(256), (size_t) GD_LDS, st, a);
+            return VX_OK;
+        }
+    }
+    // the tile whose work-groups finish first by the measured costs
     int best = -1;
     float best_us = 0.0f;
     for (int t = 0; t < GM_N_TILES; ++t) {
@@ -616,19 +883,7 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
     if (epi == GM_SWIGLU) gx = (2 * (int64_t) c.mat[0].M + g.rows - 1) / g.rows;
     else for (int i = 0; i < c.nmat; ++i) { a.mat[i].wg0 = (int) gx; gx += (c.mat[i].M + g.rows - 1) / g.rows; }
     const int64_t gy = (c.N + g.toks - 1) / g.toks;
-    // Which tiles an XCD takes: 1, 2, 4 or all 8 of them share out the row tiles, the rest the token tiles.  What the eight L2s
-    // bring in is every weight once per group of token tiles and every activation once per group of row tiles.
-    const double wbytes = (double) gx * g.rows * (c.K / 32) * (c.wtype == VX_GM_Q8 ? 34 : 64), xbytes = (double) c.N * c.K * 2;
-    double least = 0.0;
-    int64_t lx = 0, ly = 0, fill = 0;
-    for (int r = 3; r >= 0; --r) {
-        const int64_t nx = (gx + (1 << r) - 1) >> r, ny = (gy + (8 >> r) - 1) / (8 >> r), rounds = (nx * ny * nbatch + 31) / 32;
-        const double bytes = wbytes * (8 >> r) + xbytes * (1 << r);
-        if (lx && (rounds > fill || (rounds == fill && bytes >= least))) continue;
-        a.xr = r; least = bytes; lx = nx; ly = ny; fill = rounds;
-    }
-    gx = 8 * lx;
-    if (gx > 0x7fffffff || ly > 65535) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
-    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) gx, (int) ly, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) gx, (int) ly, nbatch, st);
+    if (!share(gx, gy, (double) gx * g.rows * (c.K / 32) * (c.wtype == VX_GM_Q8 ? 34 : 64), 1, lx, ly)) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
+    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) lx, (int) ly, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) lx, (int) ly, nbatch, st);
     return ok ? VX_OK : vx_fail(VX_ERR_HIP, "mul_mat: the kernel could not be given its LDS");
 }

@@ -49,5 +49,8 @@ bool vx_gm_on(int64_t N); // and whether the environment leaves it in place
 static inline bool vx_gm_region(int wtype, int64_t K, int64_t N, int64_t nbatch, int64_t M) { return vx_gm_shape(wtype, K, N, nbatch, M) && vx_gm_on(N); }
 // region, and operands on the boundaries its loads need (dst only needs 4-byte aligned values)
 bool vx_gm_takes(const vx_gm_call & c);
+// Weights as mul_mat.hip's weight pass lays them out for the pre-tiled kernel (f16 integers in operand tiles, the block scales apart;
+// a pair's 16-row tiles alternate), kept for pinned weights: false where there is no such copy to be had.
+bool vx_qt_kept_tiles(const char * w, const char * w2, int64_t K, int64_t M, uint64_t nb01, hipStream_t st, const void ** tiles, const float ** scales);
 size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch); // f16 activation tiles of a product
 vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st);

@@ -2312,6 +2312,11 @@ bool gemm_q8t_takes(const mm_args & a, int nbatch, bool dual) {
            a.K < (1ll << 24) && nbatch <= 65535;
 }
 
+size_t qt_tiles_bytes(const qt_args & q) { return (size_t) q.n_kb * q.n_rt * 1024; }
+size_t qt_scales_bytes(const qt_args & q) { // (+ a scale row's worth: the last stage's 1 KB load of a ragged row tile count stays inside)
+    return ((size_t) q.n_kb * ((q.n_rt + 3) & ~3) * 16 * 4 + 1023) / 1024 * 1024 + 1024;
+}
+
 template <bool DUAL>
 bool launch_gemm_q8t(const mm_args & a, int nbatch, hipStream_t st, bool fold) {
     qt_args q = {};
@@ -2343,7 +2348,7 @@ bool launch_gemm_q8t(const mm_args & a, int nbatch, hipStream_t st, bool fold) {
         q.nseg = a.nseg;
         if (at != a.M) return false;
     }
-    const size_t wt_bytes = (size_t) q.n_kb * q.n_rt * 1024, wd_bytes = ((size_t) q.n_kb * ((q.n_rt + 3) & ~3) * 16 * 4 + 1023) / 1024 * 1024 + 1024; // (+ a scale row's worth: the last stage's 1 KB load of a ragged row tile count stays inside)
+    const size_t wt_bytes = qt_tiles_bytes(q), wd_bytes = qt_scales_bytes(q);
     const size_t xt_bytes = a.tile_in ? 0 : (size_t) nbatch * q.n_kb * q.n_tt * 1024;
     static bool raised = false;
     if (!raised) {
@@ -2369,7 +2374,7 @@ bool launch_gemm_q8t(const mm_args & a, int nbatch, hipStream_t st, bool fold) {
     // the weights' tiles: kept from call to call when the caller has pinned the weights, else made in the workspace
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void) hipGetLastError(); return false; }
-    const vx_derived_key key = { dev, fold ? 2 : 1, a.w, DUAL ? a.w2 : nullptr, a.K, a.M, a.nb01 };
+    const vx_derived_key key = { dev, fold ? 2 : 1, a.w, DUAL ? a.w2 : nullptr, a.K, a.M, a.nb01 }; // (vx_qt_kept_tiles: the same copies)
     bool fresh = false;
     char * kept = segs ? nullptr : (char *) vx_derived_get(key, wt_bytes + wd_bytes, st, &fresh); // (three matrices: tiles made per call)
     void * ws = nullptr;
@@ -2569,6 +2574,28 @@ void launch(const mm_args & a, int nbatch, hipStream_t st) {
 }
 
 } // namespace
+
+bool vx_qt_kept_tiles(const char * w, const char * w2, int64_t K, int64_t M, uint64_t nb01, hipStream_t st, const void ** tiles, const float ** scales) {
+    qt_args q = {};
+    q.w = w; q.w2 = w2; q.K = K; q.M = M; q.nb01 = nb01;
+    q.w_al4 = (((uintptr_t) w | (uintptr_t) w2 | nb01) % 4) == 0;
+    q.n_rt = (int) (((w2 ? 2 * M : M) + 15) / 16); q.n_kb = (int) (K / 32);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) { (void) hipGetLastError(); return false; }
+    const vx_derived_key key = { dev, 1, w, w2, K, M, nb01 };
+    const int64_t units = (int64_t) q.n_kb * q.n_rt * 64;
+    if ((units + 255) / 256 > 0x7fffffff) return false;
+    bool fresh = false;
+    char * kept = (char *) vx_derived_get(key, qt_tiles_bytes(q) + qt_scales_bytes(q), st, &fresh);
+    if (!kept) return false;
+    q.wt = (half8_t *) kept; q.wdt = (float *) (kept + qt_tiles_bytes(q));
+    if (fresh) {
+        vx_launch(qt_weights_kernel, dim3((unsigned) ((units + 255) / 256)), dim3(256), 0, st, q);
+        vx_derived_filled(key, st);
+    }
+    *tiles = kept; *scales = q.wdt;
+    return true;
+}
 
 extern "C" int vx_supports_mul_mat(const vx_tensor * src0, const vx_tensor * src1, const vx_tensor * dst) {
     if (!src0 || !src1 || !dst) return 0;
