@@ -24,6 +24,7 @@
 // staged K-split variant of the GEMM kernel remains for F32 weights and ragged K.
 //
 // Algorithmic HBM bytes: weights once (34 bytes per 32 weights) + activations + output.
+#include "kvs_common.hpp"
 #include "mm_common.hpp"
 #include "gemm_mid.hpp"
 #include "rope_common.hpp"
@@ -76,6 +77,9 @@ struct mm_args {
     // (x is then the un-normalised tensor): x[t][k] / rms(x[t]) * norm_w[k], rounded after each product
     const float * norm_w;
     float norm_eps;
+    // GEMV behind an attention whose launch wrote the cache slots: the write's wave totals, whose ordering scalar (ADD1) joins every
+    // activation before it is rounded (launch_gemv_dma only); null otherwise
+    const double * add_totals; float add_scale, add_bias;
     // GEMV prologue helpers, filled in by launch_gemv: everything a wave needs before it can request its weights is
     // kept free of integer divisions (a dependent chain of some thirty instructions each, ahead of the first load)
     int   nbatch;     // ne12 * ne13 of the activations; 1: no batch index arithmetic at all
@@ -633,7 +637,7 @@ __device__ __forceinline__ void gv_dma16(const char * g, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(base) : "memory");
 }
 
-enum gv_epilogue : int { GV_PLAIN = 0, GV_RES = 1, GV_SWIGLU = 2 };
+enum gv_epilogue : int { GV_PLAIN = 0, GV_RES = 1, GV_SWIGLU = 2, GV_RES_ADD1 = 3 }; // GV_RES_ADD1: GV_RES, a cache write's scalar added to every activation
 
 // Four k blocks of one wave from the LDS images: blocks kb, kb + NW, kb + 2 NW, kb + 3 NW sit at compile-time distances, and
 // with an even wave count they share their parity, so a round is straight-line code over three addresses: all reads first,
@@ -738,6 +742,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_dma_kernel(const mm_args a) {
     auto unit_token = [&](int unit) { return (int) (((float) unit + 0.5f) * a.inv_upr); }; // = unit / upr
     const char * xb = a.x + (uint64_t) tok0 * a.nb11;
     float resv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float y = 0.0f; // GV_RES_ADD1: the scalar, by every wave behind its first requests
 
     // ---- activations without a norm: units of 8 values, a thread's units UB at a time (requested together, then staged: a
     // round trip per unit would be paid a dozen times with sixteen tokens).  With many units the waves that fetch the weights
@@ -752,6 +757,10 @@ __global__ __launch_bounds__(64 * NW) void gemv_dma_kernel(const mm_args a) {
         float v[8];
 #pragma unroll
         for (int i = 0; i < 4; ++i) { v[i] = v0[i]; v[4 + i] = v1[i]; }
+        if constexpr (EPI == GV_RES_ADD1) { // the ADD1 node
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] += y;
+        }
         half8_t h;
         if constexpr (ACT_Q8) { // 4 consecutive units = one 32-wide block
             float amax = 0.0f;
@@ -861,7 +870,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_dma_kernel(const mm_args a) {
             for (int u = lane; u < units_row; u += 64, g += 1024, dst += 1024) gv_dma16(g, dst);
         }
         __builtin_amdgcn_s_setprio(0);
-        if constexpr (EPI == GV_RES) { // the residual values the storing wave will need: in flight with the weights
+        if constexpr (EPI == GV_RES || EPI == GV_RES_ADD1) { // the residual values the storing wave will need: in flight with the weights
             int          row_c, pair_c;
             bool         ok_c;
             const char * wrow_c;
@@ -891,6 +900,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_dma_kernel(const mm_args a) {
         if constexpr (NORM) { // (requested behind the weights, these rows arrive behind them)
             if (2 * NA + wid < N) norm_pair(2 * NA + wid, NWD);
         }
+        if constexpr (EPI == GV_RES_ADD1) y = kvs_scalar_of_16(a.add_totals, lane, a.add_scale, a.add_bias);
         if constexpr (SHARE) stage_rest(64 * NA + tid);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this wave's direct loads have landed (they are not known to the compiler)
     } else {
@@ -926,6 +936,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_dma_kernel(const mm_args a) {
             }
             for (int t = 2 * NW + awid; t < N; t += 2 * NA) norm_pair(t, NA); // (more than 2 NW tokens: four-wave work-groups only)
         } else {
+            if constexpr (EPI == GV_RES_ADD1) y = kvs_scalar_of_16(a.add_totals, lane, a.add_scale, a.add_bias);
 #pragma unroll
             for (int i = 0; i < UB; ++i) {
                 const int unit = atid + i * USTRIDE;
@@ -1005,7 +1016,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_dma_kernel(const mm_args a) {
             acc[r] = (acc[r] / (1.0f + expf(-acc[r]))) * up;
         }
     }
-    if constexpr (EPI == GV_RES) {
+    if constexpr (EPI == GV_RES || EPI == GV_RES_ADD1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = scaled_residual(acc[r], a.res_scale, resv[r]);
     }
@@ -1128,6 +1139,10 @@ bool launch_gemv_dma(mm_args & a, int nbatch, int nw, dim3 grid, hipStream_t st)
     do { if (nw == 4) VX_DMA_GO(4, SEG_, NORM_, EPI_); else if (nw == 8) VX_DMA_GO(8, SEG_, NORM_, EPI_); else VX_DMA_GO(16, SEG_, NORM_, EPI_); } while (0)
     const bool norm = a.norm_w != nullptr;
     const bool many = (a.N < 16 ? a.N : 16) * (a.K / 8) > 64 * (nw - nw / 2); // an activation thread stages more than one unit
+    if (a.add_totals) { // (K of 513 to 1024 and more than 16 tokens: stream_first's shapes)
+        if constexpr (!ACT_Q8) { if (nw == 4 && many && a.res && !norm && !a.nseg && !a.w2) VX_DMA_GO(4, false, false, GV_RES_ADD1); }
+        return false;
+    }
     if (a.nseg > 0) { if (norm) VX_DMA_NW(true, true, GV_PLAIN); else VX_DMA_NW(true, false, GV_PLAIN); }
     if (a.w2)       { if (norm) VX_DMA_NW(false, true, GV_SWIGLU); else VX_DMA_NW(false, false, GV_SWIGLU); }
     if (a.res)      { if (norm) return false; VX_DMA_NW(false, false, GV_RES); }
@@ -1212,6 +1227,7 @@ bool launch_gemv(const mm_args & a0, int nbatch, hipStream_t st) {
     const dim3 grid((unsigned) nwg, (unsigned) nchunk, (unsigned) nbatch);
     const dim3 block((unsigned) (64 * nw));
     if constexpr (WT == WT_Q8) { if (launch_gemv_dma<ACT_Q8>(a, nbatch, nw, grid, st)) return true; }
+    if (a.add_totals) return false;
     // above 64 KiB of LDS a kernel has to be told once that it may be given that much
 #define VX_GEMV_GO(...)                                                                                                \
     do {                                                                                                               \
@@ -3117,6 +3133,13 @@ vx_status vx_proj_add_run(const vx_tensor * w, const vx_tensor * x, const vx_ten
     if (!proj_tiles_fill(b, mid, w, x, residual, dst, scale, act_mode) || !mid) return vx_fail(VX_ERR_UNSUPPORTED, "projection with a scalar: a shape outside the kernel");
     if (!w->data || !residual->data || !dst->data || !x->data) return vx_fail(VX_ERR_INVALID, "projection with a scalar: null data");
     b.ws_offset = ws_offset;
+    // few tokens: the streaming kernel adds the scalar as it stages the rows, and needs no activation pass in front.  (In a prompt of 45
+    // tokens 5.4 us where the pass and gemm_mid.hip's kernel take 3.2 and 6.5; the line is stream_first's, both sides there.)
+    if (stream_first(b, 1, WT_Q8)) {
+        mm_args s = b;
+        s.add_totals = totals; s.add_scale = sync_scale; s.add_bias = sync_bias;
+        if (launch_gemv<WT_Q8, false>(s, 1, st)) { VX_LAUNCH_CHECK(); return VX_OK; }
+    }
     if (!mid_fill(c, b, 1, WT_Q8)) return vx_fail(VX_ERR_UNSUPPORTED, "projection with a scalar: a shape outside the kernel");
     c.add_totals = totals; c.add_scale = sync_scale; c.add_bias = sync_bias;
     const vx_status rc = vx_gm_run(c, st);
