@@ -67,6 +67,14 @@ template <int N> __device__ __forceinline__ void gm_dma_tiles(uint32_t off, cons
 
 template <int N> __device__ __forceinline__ void gm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
 
+// a stage of L loads has landed once only those of the stages behind it, at most MOST of them, are outstanding
+template <int L, int MOST> __device__ __forceinline__ void gm_wait_younger(int younger) {
+    if constexpr (MOST > 0) {
+        if (younger < MOST) { gm_wait_younger<L, MOST - 1>(younger); return; }
+    }
+    gm_wait<L * MOST>();
+}
+
 constexpr int KG = 4; // waves of a row group, over the k blocks: the streaming kernel's four waves
 
 template <int WT, int MT, int NT, int RW, int CH, int S>
@@ -88,7 +96,6 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
     using sh = gm_shape<WT, MT, NT, RW, CH, S>;
     static_assert((CH == 1 || CH == 2) && 4 * CH % KG == 0, "stages of 128 or 256 k, whole steps");
     static_assert(EPI == GM_PLAIN || MT == 2, "pairs of row tiles inside a wave");
-    static_assert(S == 3, "what the waits below count");
     extern __shared__ __align__(1024) char gm_smem[];
     typedef __attribute__((address_space(3))) char lds_char;
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
@@ -150,9 +157,7 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
             for (int s = 0; s < S; ++s) if (s < nst) issue(s, s);
             int buf = S - 1; // where the stage before last lies (st = 0: unused)
             for (int st = 0; st < nst; ++st) {
-                const int younger = min(st == 0 ? S - 1 : S - 2, nst - 1 - st);
-                if (younger >= S - 2) gm_wait<L * (S - 2)>();
-                else gm_wait<0>();
+                gm_wait_younger<L, S - 2>(nst - 1 - st);
                 __builtin_amdgcn_s_barrier();
                 if (st > 0 && st - 1 + S < nst) issue(st - 1 + S, buf);
                 buf = buf + 1 == S ? 0 : buf + 1;
@@ -176,9 +181,7 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
             for (int s = 0; s < S; ++s) if (s < nst) issue(s, s);
             int buf = S - 1;
             for (int st = 0; st < nst; ++st) {
-                const int younger = min(st == 0 ? S - 1 : S - 2, nst - 1 - st);
-                if (younger >= S - 2) gm_wait<L * (S - 2)>();
-                else gm_wait<0>();
+                gm_wait_younger<L, S - 2>(nst - 1 - st);
                 __builtin_amdgcn_s_barrier();
                 if (st > 0 && st - 1 + S < nst) issue(st - 1 + S, buf);
                 buf = buf + 1 == S ? 0 : buf + 1;
@@ -676,13 +679,14 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
 }
 
 // ---- tile choice -----------------------------------------------------------------------------------------------------
-// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages); what a work-group costs, measured with Q8_0 weights:
+// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages: four or five where two work-groups still share a compute
+// unit's LDS -- with three the down projection of 45 tokens takes 9.3 us, with five 8.3, and six no less); what a work-group costs, measured with Q8_0 weights:
 // microseconds per 128 of K and fixed
 #define GM_TILES(X) \
-    X(0, 1, 1, 1, 2, 3, 0.127f, 0.95f) \
-    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f) \
-    X(2, 2, 2, 1, 2, 3, 0.190f, 1.40f) \
-    X(3, 2, 4, 1, 1, 3, 0.276f, 1.30f) \
+    X(0, 1, 1, 1, 2, 5, 0.127f, 0.95f) \
+    X(1, 1, 2, 1, 2, 5, 0.135f, 1.10f) \
+    X(2, 2, 2, 1, 2, 4, 0.190f, 1.40f) \
+    X(3, 2, 4, 1, 1, 5, 0.276f, 1.30f) \
     X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
     X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f)
 constexpr int GM_N_TILES = 6;
