@@ -54,12 +54,15 @@ enum { GM_PLAIN = 0, GM_SWIGLU = 1, GM_SEGS = 2 };
 // N consecutive 1 KB tiles from global memory (uniform base + lane offset) into LDS at lds + 16 lane: one statement, since the
 // compiler may write M0 between two
 template <int N> __device__ __forceinline__ void gm_dma_tiles(uint32_t off, const char * base, uint32_t lds) {
-    static_assert(N == 1 || N == 2 || N == 4, "instances of gm_kernel");
+    static_assert(N >= 1 && N <= 4, "one statement's loads");
     if constexpr (N == 1)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
     else if constexpr (N == 2)
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(off), "s"(base), "s"(lds)
                      : "memory");
+    else if constexpr (N == 3)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(off), "s"(base), "s"(lds) : "memory");
     else
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024\n\t"
                      "global_load_lds_dwordx4 %0, %1 offset:2048\n\tglobal_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(off), "s"(base), "s"(lds) : "memory");
@@ -171,8 +174,9 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
                 for (int kb = 0; kb < 4 * CH; ++kb) { // NT consecutive tiles of a k block (past the last token tile: the next block's, dropped at the store)
                     const char * p = xsrc + (int64_t) (st * 4 * CH + kb) * a.n_tt * 1024;
 #pragma unroll
-                    for (int t0 = 0; t0 < NT; t0 += 4)
-                        gm_dma_tiles<(NT < 4 ? NT : 4)>(loff, p + t0 * 1024, base + (uint32_t) (kb * NT + t0) * 1024);
+                    for (int t0 = 0; t0 + 4 <= NT; t0 += 4) gm_dma_tiles<4>(loff, p + t0 * 1024, base + (uint32_t) (kb * NT + t0) * 1024);
+                    constexpr int rest = NT & 3;
+                    if constexpr (rest) gm_dma_tiles<rest>(loff, p + (NT - rest) * 1024, base + (uint32_t) (kb * NT + NT - rest) * 1024);
                 }
             };
             constexpr int L = sh::XINST;
@@ -617,7 +621,7 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
     if ((int) blockIdx.x >= a.row_blocks) { // the angle table: (cos, sin) of (token, pair), a chain of multiplications and two trigonometric evaluations each
         const int idx = ((int) blockIdx.x - a.row_blocks) * 256 + (int) threadIdx.x;
-        if (idx >= a.N * 32 || blockIdx.y) return;
+        if (idx >= a.N * 32 || blockIdx.y || blockIdx.z) return;
         const int tok = idx >> 5, ip = idx & 31;
         float c, sn;
         rope_cos_sin(a.rp, (float) a.pos[tok % a.rope_T], ip, a.ff ? a.ff[ip] : 1.0f, c, sn);
@@ -633,7 +637,7 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
         *(half4_t *) (out + (int64_t) (iv >> 3) * a.n_tt * 1024 + ((iv >> 1) & 3) * 256 + (iv & 1) * 8) = h;
     };
     if (tok >= a.N) { // (uniform) the last tile's missing tokens
-        for (int iv = lane; iv < nvec; iv += 64) put(iv, half4_t{0, 0, 0, 0});
+        for (int iv = 256 * (int) blockIdx.z + lane; iv < min(nvec, 256 * ((int) blockIdx.z + 1)); iv += 64) put(iv, half4_t{0, 0, 0, 0});
         return;
     }
     const float * row = (const float *) (a.x + (uint64_t) i12 * a.nb12 + (uint64_t) i13 * a.nb13 + (uint64_t) tok * a.nb11);
@@ -656,19 +660,22 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
             put(lane + 64 * cc, h);
         }
     } else {
+        // (blockIdx.z: 1024 columns of the row.  As one wave a row, four trips one after the other, the pass made products of K 4096 over 203 tokens
+        // 14.5 us, 13.1 now; 337 tokens 17.5 / 16.6)
         float y = 0.0f;
-        for (int iv0 = lane; iv0 < nvec; iv0 += 64 * 4) { // (nvec is a multiple of 64: whole waves)
+        const int end = min(nvec, 256 * ((int) blockIdx.z + 1));
+        for (int iv0 = 256 * (int) blockIdx.z + lane; iv0 < end; iv0 += 64 * 4) { // (nvec is a multiple of 64: whole waves)
             float4_t v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = ((const float4_t *) row)[min(iv0 + 64 * u, nvec - 1)];
             if (a.totals) { // (uniform) the ADD1 node
-                if (iv0 == lane) y = kvs_scalar_of_16(a.totals, lane, a.sync_scale, a.sync_bias);
+                if (iv0 < 256 * (int) blockIdx.z + 64) y = kvs_scalar_of_16(a.totals, lane, a.sync_scale, a.sync_bias);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) v[u] += y;
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                if (iv0 + 64 * u >= nvec) break;
+                if (iv0 + 64 * u >= end) break;
                 half4_t h;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) h[i] = (_Float16) v[u][i];
@@ -682,14 +689,17 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
 // (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages: four or five where two work-groups still share a compute
 // unit's LDS -- with three the down projection of 45 tokens takes 9.3 us, with five 8.3, and six no less); what a work-group costs, measured with Q8_0 weights:
 // microseconds per 128 of K and fixed
+// (96 and 112 tokens: 4096 x 1024 x 337 tokens with F16 weights 13.2 us on 192 work-groups of 128 tokens, 12.0 on 256 of 96)
 #define GM_TILES(X) \
     X(0, 1, 1, 1, 2, 5, 0.127f, 0.95f) \
     X(1, 1, 2, 1, 2, 5, 0.135f, 1.10f) \
     X(2, 2, 2, 1, 2, 4, 0.190f, 1.40f) \
     X(3, 2, 4, 1, 1, 5, 0.276f, 1.30f) \
     X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
-    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f)
-constexpr int GM_N_TILES = 6;
+    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f) \
+    X(6, 2, 6, 2, 1, 3, 0.430f, 2.50f) \
+    X(7, 2, 7, 2, 1, 3, 0.468f, 2.68f)
+constexpr int GM_N_TILES = 8;
 // lone: a compute unit's LDS holds one work-group (F16 rows are twice the bytes: more of the tiles)
 struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2]; };
 const gm_tile gm_tiles[GM_N_TILES] = {
@@ -832,8 +842,8 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
             a.rope_tab = p.tab;
             blocks += (a.N * 32 + 255) / 256;
         }
-        if (c.norm_w) vx_launch(gm_acts_kernel<true>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p);
-        else          vx_launch(gm_acts_kernel<false>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p);
+        if (c.norm_w) vx_launch(gm_acts_kernel<true>, dim3((unsigned) blocks, (unsigned) nbatch), dim3(256), 0, st, p); // (K of at most 1024)
+        else          vx_launch(gm_acts_kernel<false>, dim3((unsigned) blocks, (unsigned) nbatch, (unsigned) ((c.K + 1023) / 1024)), dim3(256), 0, st, p);
     }
     const int epi = c.w2 ? GM_SWIGLU : c.nmat > 1 ? GM_SEGS : GM_PLAIN;
     // Which tiles an XCD takes: 1, 2, 4 or all 8 of them share out the row tiles, the rest the token tiles.  What the eight L2s

@@ -77,9 +77,6 @@ struct mm_args {
     // (x is then the un-normalised tensor): x[t][k] / rms(x[t]) * norm_w[k], rounded after each product
     const float * norm_w;
     float norm_eps;
-    // GEMV behind an attention whose launch wrote the cache slots: the write's wave totals, whose ordering scalar (ADD1) joins every
-    // activation before it is rounded (launch_gemv_dma only); null otherwise
-    const double * add_totals; float add_scale, add_bias;
     // GEMV prologue helpers, filled in by launch_gemv: everything a wave needs before it can request its weights is
     // kept free of integer divisions (a dependent chain of some thirty instructions each, ahead of the first load)
     int   nbatch;     // ne12 * ne13 of the activations; 1: no batch index arithmetic at all
@@ -89,6 +86,9 @@ struct mm_args {
     // gemv_dma_kernel: the weight rows of a work-group as an image in LDS
     int   w_lds_off;  // byte offset of the image in the work-group's dynamic LDS (a multiple of 16)
     int   w_slot;     // bytes between the images of consecutive MFMA columns: the row's bytes plus padding
+    // GEMV behind an attention whose launch wrote the cache slots: the write's wave totals, whose ordering scalar (ADD1) joins every
+    // activation before it is rounded (launch_gemv_dma only); null otherwise
+    const double * add_totals; float add_scale, add_bias;
 };
 
 constexpr int WT_Q8 = 0, WT_F16 = 1, WT_F32 = 2;
@@ -1139,15 +1139,15 @@ bool launch_gemv_dma(mm_args & a, int nbatch, int nw, dim3 grid, hipStream_t st)
     do { if (nw == 4) VX_DMA_GO(4, SEG_, NORM_, EPI_); else if (nw == 8) VX_DMA_GO(8, SEG_, NORM_, EPI_); else VX_DMA_GO(16, SEG_, NORM_, EPI_); } while (0)
     const bool norm = a.norm_w != nullptr;
     const bool many = (a.N < 16 ? a.N : 16) * (a.K / 8) > 64 * (nw - nw / 2); // an activation thread stages more than one unit
-    if (a.add_totals) { // (K of 513 to 1024 and more than 16 tokens: stream_first's shapes)
-        if constexpr (!ACT_Q8) { if (nw == 4 && many && a.res && !norm && !a.nseg && !a.w2) VX_DMA_GO(4, false, false, GV_RES_ADD1); }
-        return false;
+    if (!a.add_totals) {
+        if (a.nseg > 0) { if (norm) VX_DMA_NW(true, true, GV_PLAIN); else VX_DMA_NW(true, false, GV_PLAIN); }
+        if (a.w2)       { if (norm) VX_DMA_NW(false, true, GV_SWIGLU); else VX_DMA_NW(false, false, GV_SWIGLU); }
+        if (a.res)      { if (norm) return false; VX_DMA_NW(false, false, GV_RES); }
+        if (norm) VX_DMA_NW(false, true, GV_PLAIN);
+        VX_DMA_NW(false, false, GV_PLAIN);
     }
-    if (a.nseg > 0) { if (norm) VX_DMA_NW(true, true, GV_PLAIN); else VX_DMA_NW(true, false, GV_PLAIN); }
-    if (a.w2)       { if (norm) VX_DMA_NW(false, true, GV_SWIGLU); else VX_DMA_NW(false, false, GV_SWIGLU); }
-    if (a.res)      { if (norm) return false; VX_DMA_NW(false, false, GV_RES); }
-    if (norm) VX_DMA_NW(false, true, GV_PLAIN);
-    VX_DMA_NW(false, false, GV_PLAIN);
+    // (last: a decode step's kernels keep their places in the code object.  K of 513 to 1024, more than 16 tokens: stream_first's shapes)
+    if constexpr (!ACT_Q8) { if (nw == 4 && many && a.res && !norm && !a.nseg && !a.w2) VX_DMA_GO(4, false, false, GV_RES_ADD1); }
 #undef VX_DMA_NW
 #undef VX_DMA_GO
     return false;
