@@ -808,6 +808,8 @@ static bool gd_takes(const vx_gm_call & c, int epi, int nbatch) {
     return (MV + GD_ROWS - 1) / GD_ROWS * ((c.N + GD_TOKS - 1) / GD_TOKS) * nbatch >= (c.w2 ? 160 : 192);
 }
 
+static void gd_launch(int epi, dim3 grid, const gm_args & a, hipStream_t st);
+
 vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
     const int nbatch = c.ne12 * c.ne13;
     gm_args a = {};
@@ -871,8 +873,7 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
             vx_qt_kept_tiles(c.mat[0].w, c.w2, c.K, c.mat[0].M, c.mat[0].nb01, st, &tiles, &scales)) {
             a.wt = (const half8_t *) tiles; a.wdt = scales; a.n_rt = (int) ((MV + 15) / 16);
             const dim3 grid((unsigned) lx, (unsigned) ly, (unsigned) nbatch);
-            if (epi == GM_SWIGLU) vx_launch(gd_kernel<GM_SWIGLU>, grid, dim3(256), (size_t) GD_LDS, st, a);
-            else                  vx_launch(gd_kernel<GM_PLAIN>, grid, dim3(256), (size_t) GD_LDS, st, a);
+            gd_launch(epi, grid, a, st);
             return VX_OK;
         }
     }
@@ -900,4 +901,10 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
     if (!share(gx, gy, (double) gx * g.rows * (c.K / 32) * (c.wtype == VX_GM_Q8 ? 34 : 64), 1, lx, ly)) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
     const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) lx, (int) ly, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) lx, (int) ly, nbatch, st);
     return ok ? VX_OK : vx_fail(VX_ERR_HIP, "mul_mat: the kernel could not be given its LDS");
+}
+
+// (last: gm_kernel's instances keep their places in the code object)
+static void gd_launch(int epi, dim3 grid, const gm_args & a, hipStream_t st) {
+    if (epi == GM_SWIGLU) vx_launch(gd_kernel<GM_SWIGLU>, grid, dim3(256), (size_t) GD_LDS, st, a);
+    else                  vx_launch(gd_kernel<GM_PLAIN>, grid, dim3(256), (size_t) GD_LDS, st, a);
 }

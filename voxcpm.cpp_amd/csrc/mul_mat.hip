@@ -1109,16 +1109,22 @@ size_t gemv_dma_lds(const mm_args & a, bool act_q8, int nw, int rows_wg) {
     return (gemv_smem(a, act_q8, nw, true) + 15) / 16 * 16 + (size_t) rows_wg * gemv_dma_slot(a.K);
 }
 
-// Launches gemv_dma_kernel if the call is one it takes (a: as launch_gemv has prepared it, rows_wg and the prologue
+// The kernel's own arguments (a: as gemv_fill has prepared it); its LDS, or 0 where it does not take the call
+size_t gemv_dma_fill(mm_args & a, bool act_q8, int nbatch, int nw) {
+    if (!gemv_dma_takes(a, nbatch, nw)) return 0;
+    a.w_slot    = gemv_dma_slot(a.K);
+    a.w_lds_off = (int) ((gemv_smem(a, act_q8, nw, true) + 15) / 16 * 16);
+    a.exact = (a.K / 32) % (4 * nw) == 0; // whole four-block rounds for every wave
+    const size_t smem = (size_t) a.w_lds_off + (size_t) a.rows_wg * a.w_slot;
+    return smem > GV_MAX_LDS ? 0 : smem;
+}
+
+// Launches gemv_dma_kernel if the call is one it takes (a: as gemv_fill has prepared it, rows_wg and the prologue
 // helpers included; nw: the wave count every kernel uses for this shape).
 template <bool ACT_Q8>
 bool launch_gemv_dma(mm_args & a, int nbatch, int nw, dim3 grid, hipStream_t st) {
-    if (!gemv_dma_takes(a, nbatch, nw)) return false;
-    a.w_slot    = gemv_dma_slot(a.K);
-    a.w_lds_off = (int) ((gemv_smem(a, ACT_Q8, nw, true) + 15) / 16 * 16);
-    const size_t smem = (size_t) a.w_lds_off + (size_t) a.rows_wg * a.w_slot;
-    if (smem > GV_MAX_LDS) return false;
-    a.exact = (a.K / 32) % (4 * nw) == 0; // whole four-block rounds for every wave
+    const size_t smem = gemv_dma_fill(a, ACT_Q8, nbatch, nw);
+    if (!smem) return false;
     const dim3 block((unsigned) (64 * nw));
 #define VX_DMA_GO(NW_, SEG_, NORM_, EPI_)                                                                              \
     do {                                                                                                               \
@@ -1139,15 +1145,11 @@ bool launch_gemv_dma(mm_args & a, int nbatch, int nw, dim3 grid, hipStream_t st)
     do { if (nw == 4) VX_DMA_GO(4, SEG_, NORM_, EPI_); else if (nw == 8) VX_DMA_GO(8, SEG_, NORM_, EPI_); else VX_DMA_GO(16, SEG_, NORM_, EPI_); } while (0)
     const bool norm = a.norm_w != nullptr;
     const bool many = (a.N < 16 ? a.N : 16) * (a.K / 8) > 64 * (nw - nw / 2); // an activation thread stages more than one unit
-    if (!a.add_totals) {
-        if (a.nseg > 0) { if (norm) VX_DMA_NW(true, true, GV_PLAIN); else VX_DMA_NW(true, false, GV_PLAIN); }
-        if (a.w2)       { if (norm) VX_DMA_NW(false, true, GV_SWIGLU); else VX_DMA_NW(false, false, GV_SWIGLU); }
-        if (a.res)      { if (norm) return false; VX_DMA_NW(false, false, GV_RES); }
-        if (norm) VX_DMA_NW(false, true, GV_PLAIN);
-        VX_DMA_NW(false, false, GV_PLAIN);
-    }
-    // (last: a decode step's kernels keep their places in the code object.  K of 513 to 1024, more than 16 tokens: stream_first's shapes)
-    if constexpr (!ACT_Q8) { if (nw == 4 && many && a.res && !norm && !a.nseg && !a.w2) VX_DMA_GO(4, false, false, GV_RES_ADD1); }
+    if (a.nseg > 0) { if (norm) VX_DMA_NW(true, true, GV_PLAIN); else VX_DMA_NW(true, false, GV_PLAIN); }
+    if (a.w2)       { if (norm) VX_DMA_NW(false, true, GV_SWIGLU); else VX_DMA_NW(false, false, GV_SWIGLU); }
+    if (a.res)      { if (norm) return false; VX_DMA_NW(false, false, GV_RES); }
+    if (norm) VX_DMA_NW(false, true, GV_PLAIN);
+    VX_DMA_NW(false, false, GV_PLAIN);
 #undef VX_DMA_NW
 #undef VX_DMA_GO
     return false;
@@ -1184,9 +1186,9 @@ int gemv_waves(const mm_args & a, int nbatch) {
     return nw;
 }
 
+// What both streaming kernels need of a call: work-groups, waves, the prologue's helpers.  False where it is not their shape.
 template <int WT, bool ACT_Q8>
-bool launch_gemv(const mm_args & a0, int nbatch, hipStream_t st) {
-    mm_args a = a0;
+bool gemv_fill(mm_args & a, int nbatch, int & nw, dim3 & grid) {
     {
         // (several matrices in one launch: wherever each of them alone is this kernel's shape -- the launch then sums every
         // product as its own call would)
@@ -1211,10 +1213,8 @@ bool launch_gemv(const mm_args & a0, int nbatch, hipStream_t st) {
     };
     const int64_t nchunk = (a.N + 15) / 16;
     while (a.rows_wg > 4 && groups(a.rows_wg) * nbatch * nchunk < 128) a.rows_wg /= 2;
-    const int nw = gemv_waves(a, nbatch);
-    if (nw < 0) return false;
-    const size_t smem = gemv_smem(a, ACT_Q8, nw);
-    if (smem > GV_MAX_LDS) return false;
+    nw = gemv_waves(a, nbatch);
+    if (nw < 0 || gemv_smem(a, ACT_Q8, nw) > GV_MAX_LDS) return false;
     if constexpr (WT == WT_Q8) { // the kernel that keeps a work-group's rows in LDS: fewer rows each when they would not fit
         if (gemv_dma_takes(a, nbatch, nw))
             while (a.rows_wg > 4 && gemv_dma_lds(a, ACT_Q8, nw, a.rows_wg) > GV_MAX_LDS) a.rows_wg /= 2;
@@ -1224,10 +1224,19 @@ bool launch_gemv(const mm_args & a0, int nbatch, hipStream_t st) {
         int wg0 = 0;
         for (int i = 0; i < a.nseg; ++i) { a.seg[i].wg0 = wg0; wg0 += (int) ((a.seg[i].M + a.rows_wg - 1) / a.rows_wg); }
     }
-    const dim3 grid((unsigned) nwg, (unsigned) nchunk, (unsigned) nbatch);
+    grid = dim3((unsigned) nwg, (unsigned) nchunk, (unsigned) nbatch);
+    return true;
+}
+
+template <int WT, bool ACT_Q8>
+bool launch_gemv(const mm_args & a0, int nbatch, hipStream_t st) {
+    mm_args a = a0;
+    int  nw;
+    dim3 grid;
+    if (!gemv_fill<WT, ACT_Q8>(a, nbatch, nw, grid)) return false;
+    const size_t smem = gemv_smem(a, ACT_Q8, nw);
     const dim3 block((unsigned) (64 * nw));
     if constexpr (WT == WT_Q8) { if (launch_gemv_dma<ACT_Q8>(a, nbatch, nw, grid, st)) return true; }
-    if (a.add_totals) return false;
     // above 64 KiB of LDS a kernel has to be told once that it may be given that much
 #define VX_GEMV_GO(...)                                                                                                \
     do {                                                                                                               \
@@ -3125,6 +3134,20 @@ bool vx_proj_add_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor * 
 
 size_t vx_proj_add_bytes(const vx_tensor * w, const vx_tensor * x) { return vx_gm_tile_bytes(w->ne[0], x->ne[1], 1); }
 
+// The streaming kernel with a cache write's scalar added to every activation (K of 513 to 1024 and more than 16 tokens: four waves).  Here and
+// not in launch_gemv_dma, so that the instance lies behind the decode step's kernels in the code object: among them, a step of batch 16
+// took 0.8 % longer with the same instructions in every kernel.
+static bool launch_gemv_add1(const mm_args & b, hipStream_t st) {
+    mm_args a = b;
+    int  nw;
+    dim3 grid;
+    if (!gemv_fill<WT_Q8, false>(a, 1, nw, grid) || nw != 4 || a.norm_w || a.nseg || a.w2 || !a.res || 16 * (a.K / 8) <= 64 * (nw - nw / 2)) return false;
+    const size_t smem = gemv_dma_fill(a, false, 1, nw);
+    if (!smem || smem > 64 * 1024) return false; // (16 rows of 1024 as f16 and as many weight rows: 51 KB)
+    vx_launch(gemv_dma_kernel<false, 4, false, false, GV_RES_ADD1, true>, grid, dim3(64 * 4), smem, st, a);
+    return true;
+}
+
 vx_status vx_proj_add_run(const vx_tensor * w, const vx_tensor * x, const vx_tensor * residual, const vx_tensor * dst, float scale, int act_mode,
                           const double * totals, float sync_scale, float sync_bias, size_t ws_offset, hipStream_t st) {
     mm_args b;
@@ -3138,7 +3161,7 @@ vx_status vx_proj_add_run(const vx_tensor * w, const vx_tensor * x, const vx_ten
     if (stream_first(b, 1, WT_Q8)) {
         mm_args s = b;
         s.add_totals = totals; s.add_scale = sync_scale; s.add_bias = sync_bias;
-        if (launch_gemv<WT_Q8, false>(s, 1, st)) { VX_LAUNCH_CHECK(); return VX_OK; }
+        if (launch_gemv_add1(s, st)) { VX_LAUNCH_CHECK(); return VX_OK; }
     }
     if (!mid_fill(c, b, 1, WT_Q8)) return vx_fail(VX_ERR_UNSUPPORTED, "projection with a scalar: a shape outside the kernel");
     c.add_totals = totals; c.add_scale = sync_scale; c.add_bias = sync_bias;
