@@ -687,12 +687,13 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
 
 // ---- tile choice -----------------------------------------------------------------------------------------------------
 // (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages: four or five where two work-groups still share a compute
-// unit's LDS -- with three the down projection of 45 tokens takes 9.3 us, with five 8.3, and six no less); what a work-group costs, measured with Q8_0 weights:
-// microseconds per 128 of K and fixed
+// unit's LDS and more than three gain -- the down projection of 45 tokens 9.3 us with three, 8.3 with five, no less with six; tile 1 over
+// K 4096 x 128 tokens 12.3 with three, 12.6 with five); what a work-group costs, measured with Q8_0 weights: microseconds per 128 of K
+// and fixed
 // (96 and 112 tokens: 4096 x 1024 x 337 tokens with F16 weights 13.2 us on 192 work-groups of 128 tokens, 12.0 on 256 of 96)
 #define GM_TILES(X) \
     X(0, 1, 1, 1, 2, 5, 0.127f, 0.95f) \
-    X(1, 1, 2, 1, 2, 5, 0.135f, 1.10f) \
+    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f) \
     X(2, 2, 2, 1, 2, 4, 0.190f, 1.40f) \
     X(3, 2, 4, 1, 1, 5, 0.276f, 1.30f) \
     X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
