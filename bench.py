@@ -675,7 +675,7 @@ PROFILE_RUNS = [
     ("step_1_kv37", "step_b1_kv37_f32", "A decode step of one sequence behind 37 keys through 24 layers (resident stack), Q8_0 weights, F32 KV cache, replayed from a HIP graph",
      [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "stack"),
     ("prompt_1x45", "prompt_1x45_f32", "A prompt of 45 tokens through 24 layers, Q8_0 weights, F32 KV cache", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "gm_|fattn"),
-    ("prompt_2x512", "prompt_2x512_f16", "Two prompts of 512 tokens through 24 layers, Q8_0 weights, f16 KV cache", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "gm_|pf_"),
+    ("prompt_2x512", "prompt_2x512_f16", "Two prompts of 512 tokens through 24 layers, Q8_0 weights, f16 KV cache", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)], "gm_|gd_|pf_"),
     ("locdit_8_requests", "locdit_r8_l7", "One LocDiT estimator pass of eight concurrent requests, 4 layers, replayed from a HIP graph", [("sq1", SQ_SET_1), ("sq2", SQ_SET_2)],
      "gm_|gemv|fattn"),
     ("cfm_solve_cfg3", "cfm", "One UnifiedCFM solve of one request (10 Euler steps, CFG pair as one 14-token sequence, 4 LocDiT layers; BASELINE config 3)", [], ""),
