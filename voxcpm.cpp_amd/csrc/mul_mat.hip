@@ -1913,13 +1913,16 @@ __global__ __launch_bounds__(64) void qt_rope_table_kernel(const int32_t * __res
     tab[gid] = make_float2(c, sn);
 }
 
-// one thread = 8 quants of a block: (virtual row, block, j)
+// A wave takes a 16-row tile of QT_W_UNROLL consecutive blocks, all their loads in flight together (a row's blocks share cache lines);
+// one thread = 8 quants of a row in each.  The four waves of a work-group are the row tiles of one 64-row group, whose scales
+// interleave in memory.  Memory bounds it, the tiles written (2 bytes a weight) before the rows read: 8192 x 1024 weights 12.3 us (2.1 TB/s),
+// 14.4 with one block a wave and its place by 64-bit divisions; no less with a row group's blocks on one XCD (13.7).
+constexpr int QT_W_UNROLL = 4;
 __global__ __launch_bounds__(256) void qt_weights_kernel(const qt_args a) {
-    const int64_t idx = (int64_t) blockIdx.x * 256 + threadIdx.x;
-    const int     slot = (int) (idx & 63), c = slot & 15, j = slot >> 4;
-    const int64_t t = idx >> 6;
-    const int64_t kb = t % a.n_kb; // (neighbouring waves: neighbouring blocks of the same 16 rows, which share cache lines)
-    const int64_t rt = t / a.n_kb;
+    const uint32_t n_kg = (uint32_t) (a.n_kb + QT_W_UNROLL - 1) / QT_W_UNROLL, group = blockIdx.x / n_kg;
+    const int     slot = threadIdx.x & 63, c = slot & 15, j = slot >> 4;
+    const int     kb0 = (int) (blockIdx.x - group * n_kg) * QT_W_UNROLL;
+    const int64_t rt = 4 * (int64_t) group + __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6));
     if (rt >= a.n_rt) return;
     const bool    dual = a.w2 != nullptr;
     int64_t       row  = dual ? 16 * (int64_t) (rt >> 1) + c : 16 * (int64_t) rt + c; // of its own matrix
@@ -1931,23 +1934,35 @@ __global__ __launch_bounds__(256) void qt_weights_kernel(const qt_args a) {
         wsel = a.seg_w[sg]; nb01 = a.seg_nb01[sg]; rows = a.seg_row[sg + 1] - a.seg_row[sg];
         row -= a.seg_row[sg];
     }
-    half8_t h = {0, 0, 0, 0, 0, 0, 0, 0};
-    float   d = 0.0f;
-    if (row < rows) {
-        const char * wrow = wsel + (uint64_t) row * nb01;
-        h = q8_unpack(q8_load(wrow, kb, j, a.w_al4 != 0), kb, a.w_al4 != 0);
-        const _Float16 dh = *(const _Float16 *) (wrow + kb * VX_Q8_BLOCK);
-        d = (float) dh;
+    const bool   live = row < rows;
+    const char * wrow = wsel + (uint64_t) (live ? row : 0) * nb01;
+    const bool   al4 = a.w_al4 != 0;
+    decltype(q8_load(wrow, 0, j, al4)) raw[QT_W_UNROLL];
+    _Float16 dh[QT_W_UNROLL];
+#pragma unroll
+    for (int u = 0; u < QT_W_UNROLL; ++u) { // (past the last block: that one again)
+        const int kb = min(kb0 + u, a.n_kb - 1);
+        raw[u] = q8_load(wrow, kb, j, al4);
+        dh[u] = *(const _Float16 *) (wrow + (uint64_t) kb * VX_Q8_BLOCK);
+    }
+#pragma unroll
+    for (int u = 0; u < QT_W_UNROLL; ++u) {
+        const int64_t kb = kb0 + u;
+        if (kb >= a.n_kb) break;
+        half8_t h = q8_unpack(raw[u], kb, al4);
         if (a.fold) { // q * d rounded once to f16, as gemm_lds_kernel's FOLD form parks it
 #pragma unroll
-            for (int i = 0; i < 8; ++i) h[i] *= dh;
+            for (int i = 0; i < 8; ++i) h[i] *= dh[u];
         }
+        a.wt[(kb * a.n_rt + rt) * 64 + slot] = live ? h : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        // (scales: within every 64 rows, row 16 t + c sits at 4 c + t, so that a lane of the product kernel reads the scales of
+        // its row c in the wave's four row tiles with one 16-byte load)
+        if (j == 0) a.wdt[kb * ((int64_t) ((a.n_rt + 3) & ~3) * 16) + 64 * (rt >> 2) + 4 * c + (rt & 3)] = live ? (float) dh[u] : 0.0f; // (a row of whole groups of 64)
     }
-    a.wt[(kb * a.n_rt + rt) * 64 + slot] = h;
-    // (scales: within every 64 rows, row 16 t + c sits at 4 c + t, so that a lane of the product kernel reads the scales of
-    // its row c in the wave's four row tiles with one 16-byte load)
-    if (j == 0) a.wdt[kb * ((int64_t) ((a.n_rt + 3) & ~3) * 16) + 64 * (rt >> 2) + 4 * c + (rt & 3)] = d; // (a row of whole groups of 64)
 }
+
+// its work-groups, one for QT_W_UNROLL blocks of 64 rows
+int64_t qt_weights_groups(const qt_args & q) { return (int64_t) ((q.n_rt + 3) / 4) * ((q.n_kb + QT_W_UNROLL - 1) / QT_W_UNROLL); }
 
 // one thread = 8 consecutive k of a token in each of QT_ACT_UNROLL k blocks: (token, group of blocks, j); blockIdx.y =
 // batch entry.  A wave reads 16 tokens x 128 bytes per block, all blocks' loads in flight together, and writes one 1 KB
@@ -2388,8 +2403,8 @@ bool launch_gemm_q8t(const mm_args & a, int nbatch, hipStream_t st, bool fold) {
         }
         raised = true;
     }
-    const int64_t wunits = (int64_t) q.n_kb * q.n_rt * 64, xunits = (int64_t) ((q.n_kb + QT_ACT_UNROLL - 1) / QT_ACT_UNROLL) * q.n_tt * 64;
-    if ((wunits + 255) / 256 > 0x7fffffff || (xunits + 255) / 256 > 0x7fffffff) return false;
+    const int64_t xunits = (int64_t) ((q.n_kb + QT_ACT_UNROLL - 1) / QT_ACT_UNROLL) * q.n_tt * 64;
+    if (qt_weights_groups(q) > 0x7fffffff || (xunits + 255) / 256 > 0x7fffffff) return false;
     const int gx = (q.n_rt + 15) / 16, gy = (q.n_tt + 7) / 8, Gx = (gx + 3) / 4, Gy = (gy + 7) / 8;
     if (segs && a.M > QT_SEG_ROWS) return false;
     // groups of 32 work-groups, dealt to the XCDs in turn: 4 row tiles x 8 token tiles, or (segments) all gx row tiles x 32 / gx token tiles
@@ -2417,7 +2432,7 @@ bool launch_gemm_q8t(const mm_args & a, int nbatch, hipStream_t st, bool fold) {
     if (kept) { q.wt = (half8_t *) kept; q.wdt = (float *) (kept + wt_bytes); q.xt = (half8_t *) base; }
     else      { q.wt = (half8_t *) base; q.wdt = (float *) (base + wt_bytes); q.xt = (half8_t *) (base + wt_bytes + wd_bytes); }
     if (a.tile_in) q.xt = (half8_t *) const_cast<void *>(a.tile_in);
-    if (!kept || fresh) vx_launch(qt_weights_kernel, dim3((unsigned) ((wunits + 255) / 256)), dim3(256), 0, st, q);
+    if (!kept || fresh) vx_launch(qt_weights_kernel, dim3((unsigned) qt_weights_groups(q)), dim3(256), 0, st, q);
     if (fresh) vx_derived_filled(key, st);
     q.norm_w = a.norm_w; q.norm_eps = a.norm_eps;
     if (a.tile_in) {} // (the activations are the tiles the product before left)
@@ -2608,14 +2623,13 @@ bool vx_qt_kept_tiles(const char * w, const char * w2, int64_t K, int64_t M, uin
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) { (void) hipGetLastError(); return false; }
     const vx_derived_key key = { dev, 1, w, w2, K, M, nb01 };
-    const int64_t units = (int64_t) q.n_kb * q.n_rt * 64;
-    if ((units + 255) / 256 > 0x7fffffff) return false;
+    if (qt_weights_groups(q) > 0x7fffffff) return false;
     bool fresh = false;
     char * kept = (char *) vx_derived_get(key, qt_tiles_bytes(q) + qt_scales_bytes(q), st, &fresh);
     if (!kept) return false;
     q.wt = (half8_t *) kept; q.wdt = (float *) (kept + qt_tiles_bytes(q));
     if (fresh) {
-        vx_launch(qt_weights_kernel, dim3((unsigned) ((units + 255) / 256)), dim3(256), 0, st, q);
+        vx_launch(qt_weights_kernel, dim3((unsigned) qt_weights_groups(q)), dim3(256), 0, st, q);
         vx_derived_filled(key, st);
     }
     *tiles = kept; *scales = q.wdt;
