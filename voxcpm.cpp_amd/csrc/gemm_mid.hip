@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t smem0 = (uint32_t) (uintptr_t) (lds_char *) gm_smem, loff = (uint32_t) lane * 16;
 
     // The k blocks in the order of the sums: in steps of four, from a group's last block to the next group's first (behind the last
-    // group blocks 4, 8 ... again: fetched for nothing).
+    // group blocks 4 and 8 again: one stage, requested for nothing).
     const int n4 = nkb / 4;
     // ---- a stage: wave w brings token tiles 2 (w mod 2), + 1 of block w / 2, and its own rows' scales of both blocks
     // (past the last token tile: that one again, dropped at the store)
@@ -472,10 +472,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __builtin_amdgcn_sched_barrier(0);
 
     // A block: its operands (set P of the weights and scales, the tokens) are in registers; row by row its products are issued, their
-    // scaled additions two products behind, and what the row leaves free takes the next blocks' bytes.
-    auto block = [&](auto SET, auto LAST) {
+    // scaled additions two products behind, and what the row leaves free takes the next blocks' bytes.  The last turn's four blocks
+    // (ENDING) bring in nothing: every weight they need is in registers or on its way there, the last stage is requested.
+    auto block = [&](auto SET, auto ENDING) {
         constexpr int Q = decltype(SET)::value, P = Q & 1, T = 4 * GD_CT, LAG = 2;
-        constexpr bool more = !decltype(LAST)::value;
+        constexpr bool ending = decltype(ENDING)::value, more = !(ending && Q == 3);
         const uint32_t nbuf = rbuf + GD_STAGE == GD_ST * GD_STAGE ? 0 : rbuf + GD_STAGE;
         const lds_char * nx = (const lds_char *) gm_smem + (P ? nbuf : rbuf + GD_BLOCK) + loff;
         const lds_char * nd = (const lds_char *) gm_smem + (P ? nbuf : rbuf + 256) + dof;
@@ -489,15 +490,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 if constexpr (more) {
                     if (P == 1 && i == GD_CT - 1) {
                         // The next stage has landed once at most these are outstanding: younger than stage 1 are 19 loads, than stage 2 the
-                        // 15 of blocks 0 to 2, later 16.  Behind the barrier every wave has this stage's operands in registers: its
-                        // buffer takes the stage after next.
-                        stage_wait(std::integral_constant<int, 15>{});
+                        // 15 of blocks 0 to 2, later 16.  In the last turn 12: behind the last stage's third load the turn before fetched nine
+                        // tiles and requested three loads (with 8 allowed, four of the nine may go or move).  Behind the barrier every wave has
+                        // this stage's operands in registers: its buffer takes the stage after next.
+                        stage_wait(std::integral_constant<int, ending ? 8 : 15>{});
                         barrier();
                     }
-                    if (P == 1 && i > GD_CT && i % GD_CT == 1) request(rt - 1);
+                    if (!ending && P == 1 && i > GD_CT && i % GD_CT == 1) request(rt - 1);
                     if (rt == 3) x[n] = *(lds_half8 *) (nx + n * 1024);
                     if (rt == 2 && n == GD_CT - 1) d[1 - P] = *(lds_float4 *) nd;
-                    if (n == GD_CT - 1) fetch(Q, rt);
+                    if (!ending && n == GD_CT - 1) fetch(Q, rt);
                 }
             }
             if (i >= LAG) {
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     using set1 = std::integral_constant<int, 1>;
     using set2 = std::integral_constant<int, 2>;
     using set3 = std::integral_constant<int, 3>;
-    auto four = [&](auto LAST) { block(set0{}, std::false_type{}); block(set1{}, std::false_type{}); block(set2{}, std::false_type{}); block(set3{}, LAST); };
+    auto four = [&](auto ENDING) { block(set0{}, ENDING); block(set1{}, ENDING); block(set2{}, ENDING); block(set3{}, ENDING); };
     const int turns = nkb / 16; // of a group
     for (int g = 0; g < 3; ++g) {
         for (int s = 0; s < turns; ++s) four(std::false_type{});
