@@ -90,8 +90,9 @@ VX_API vx_status    vx_workspace_info(vx_stream stream, void ** ptr, size_t * by
 /* Constant weights.  ggml marks the buffers that hold a model's weights (ggml_backend_buffer_set_usage(...,
  * GGML_BACKEND_BUFFER_USAGE_WEIGHTS), the reference's src/weight-store.cpp:86 and src/minicpm.cpp:472); this is the same
  * statement for the C ABI.  For a tensor that lies wholly inside a pinned range an operator may keep a re-laid-out copy
- * between calls instead of producing it on every call (today: the tiles of the Q8_0 weights of products with 1024 tokens
- * or more, 2.1 bytes per weight, at most VX_DERIVED_WEIGHTS_MB megabytes per process, default 8192).  Results do not
+ * between calls instead of producing it on every call (today: the tiles of the Q8_0 weights of products that fill enough
+ * tiles of 256 rows x 64 tokens -- a pair of 4096 rows from 257 tokens on --, 2.1 bytes per weight, at most
+ * VX_DERIVED_WEIGHTS_MB megabytes of copies per process, default 8192, several to an allocation).  Results do not
  * depend on it.  The owner of the memory calls vx_weights_changed for every range it writes to afterwards (copies derived
  * from those bytes are dropped), and vx_weights_unpin(base) before it frees or reuses the memory.  Ranges are per device
  * (the current one); the calls are thread-safe.  vx_weights_info reports the ranges pinned and the copies held. */

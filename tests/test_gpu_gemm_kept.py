@@ -77,3 +77,72 @@ def test_mlp_from_kept_tiles(pkg, gpu, T):
     finally:
         for t in (pair, down):
             L.vx_weights_unpin(t.data_ptr())
+
+
+def test_copies_share_allocations(pkg, gpu):
+    """The first product over each of many pinned matrices does not allocate by itself; rewriting one of them again and again, its neighbours'
+    copies in use, takes no more and more memory, and all of it goes back when the range is unpinned."""
+    import torch
+    say("kept tiles: several copies to an allocation")
+    L, d = pkg.lib(), pkg.desc
+    M, K, N, W = 4096, 1024, 768, 9
+    g = rng("kept-blocks")
+    pool = torch.stack([q8_dev((0.05 * g.standard_normal((M, K))).astype(np.float32))[0] for _ in range(W)]).contiguous()
+    spare = torch.stack([pool[1].clone(), pool[2].clone()])
+    x = dev(g.standard_normal((N, K)).astype(np.float32))
+    out = torch.empty((N, M), dtype=torch.float32, device="cuda")
+
+    def product(w):
+        ok(pkg, L.vx_mul_mat(pkg.desc_q8(w, K), d(x), d(out), pkg.ACT_FLOAT, None), "mul_mat")
+        torch.cuda.synchronize()
+        return out
+
+    free = lambda: torch.cuda.mem_get_info()[0]
+    want = [product(w).clone() for w in pool]
+    start, copies = free(), kept_bytes(L)[1]
+    pkg.check(L.vx_weights_pin(pool.data_ptr(), pool.numel()), "pin")
+    try:
+        seen = set()
+        for w, r in zip(pool, want):
+            assert same_bits(product(w), r)
+            seen.add(free())
+        assert kept_bytes(L)[1] == copies + W
+        assert len(seen) <= 2 and start - min(seen) <= 300 << 20
+        for turn in range(100):   # 100 more copies of 9 MB
+            pool[0].copy_(spare[turn % 2])
+            pkg.check(L.vx_weights_changed(pool[0].data_ptr(), pool[0].numel()), "changed")
+            assert same_bits(product(pool[0]), want[1 + turn % 2]) and same_bits(product(pool[5]), want[5])
+        assert kept_bytes(L)[1] == copies + W and start - free() <= 600 << 20
+    finally:
+        L.vx_weights_unpin(pool.data_ptr())
+    assert kept_bytes(L)[1] == copies and free() >= start
+
+
+def test_copy_filled_on_one_stream_read_on_another(pkg, gpu):
+    import torch
+    say("kept tiles: filled on one stream, read on another at once")
+    L, d = pkg.lib(), pkg.desc
+    M, K, N, W = 4096, 1024, 768, 6
+    g = rng("kept-streams")
+    pool = torch.stack([q8_dev((0.05 * g.standard_normal((M, K))).astype(np.float32))[0] for _ in range(W)]).contiguous()
+    x = dev(g.standard_normal((N, K)).astype(np.float32))
+    outs = torch.empty((3, W, N, M), dtype=torch.float32, device="cuda")
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def product(i, w, stream):
+        pkg.check(L.vx_mul_mat(pkg.desc_q8(pool[w], K), d(x), d(outs[i, w]), pkg.ACT_FLOAT, stream), "mul_mat")
+
+    for s in streams:
+        product(0, 0, s.cuda_stream)   # (the streams' workspaces)
+    for w in range(W):
+        product(0, w, None)
+    torch.cuda.synchronize()
+    pkg.check(L.vx_weights_pin(pool.data_ptr(), pool.numel()), "pin")
+    try:
+        for w in range(W):
+            product(1, w, streams[w % 2].cuda_stream)
+            product(2, w, streams[1 - w % 2].cuda_stream)
+        torch.cuda.synchronize()
+        assert same_bits(outs[0], outs[1]) and same_bits(outs[0], outs[2])
+    finally:
+        L.vx_weights_unpin(pool.data_ptr())
