@@ -1,0 +1,58 @@
+"""CPU: the tile rules of the mid-size products (csrc/gm_tiles.hpp)."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+Q8, F16 = 0, 1
+PLAIN, SWIGLU, SEGS = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("gm_tiles") / "gm_tiles_check.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(ROOT, "tests", "gm_tiles_check.cpp")])
+    return C.CDLL(so)
+
+
+def choice(rules, wtype, epi, rows, K, N, nb=1):
+    out = (C.c_int64 * 8)()
+    m = (C.c_int64 * len(rows))(*rows)
+    rules.gm_choice(wtype, epi, m, len(rows), C.c_int64(K), C.c_int64(N), C.c_int64(nb), out)
+    return dict(zip(("tile", "rows", "toks", "lone", "xr", "nx", "ny", "rounds"), out))
+
+
+SHAPES = [(PLAIN, [m], k) for m, k in ((16, 1024), (128, 1024), (520, 2304), (1000, 4096), (1024, 1024), (1536, 3072), (4096, 1024), (6144, 768))] + \
+         [(SWIGLU, [m], 1024) for m in (512, 2816, 4096, 5504)] + [(SEGS, [1024, 128, 128], 1024), (SEGS, [2048, 512, 512], 1024)]
+
+
+@pytest.mark.parametrize("wtype", [Q8, F16])
+@pytest.mark.parametrize("epi,rows,K", SHAPES)
+def test_work_groups_cover_every_tile_once_and_rounds_are_an_xcds(rules, wtype, epi, rows, K):
+    """gm_kernel's mapping of work-groups to tiles, written out: every tile once, and no XCD with more rounds than the choice counted."""
+    for N in (17, 45, 100, 203, 337, 416, 448, 777, 1152, 3072):
+        for nb in (1, 3):
+            c = choice(rules, wtype, epi, rows, K, N, nb)
+            mul = 2 if epi == SWIGLU else 1
+            gx, gy = sum(-(-mul * m // c["rows"]) for m in rows), -(-N // c["toks"])
+            seen, load = set(), [0] * 8
+            for y in range(c["ny"]):
+                for x in range(8 * c["nx"]):
+                    xcd = x & 7
+                    tx, ty = ((x >> 3) << c["xr"]) + (xcd & ((1 << c["xr"]) - 1)), (y << (3 - c["xr"])) + (xcd >> c["xr"])
+                    load[xcd] += 1
+                    if tx < gx and ty < gy:
+                        assert (tx, ty) not in seen
+                        seen.add((tx, ty))
+            assert len(seen) == gx * gy, (N, c)
+            assert -(-max(load) * nb // 32) == c["rounds"], (N, c)
+
+
+@pytest.mark.parametrize("wtype", [Q8, F16])
+@pytest.mark.parametrize("M,K,N", [(520, 2304, 416), (520, 2304, 448), (520, 2304, 480), (520, 2304, 850), (520, 2304, 950)])
+def test_an_odd_number_of_row_tiles_does_not_take_a_second_round(rules, wtype, M, K, N):
+    """Just under 256 work-groups of a tile that has a compute unit to itself, of which an XCD's share is more than its 32 units."""
+    c = choice(rules, wtype, PLAIN, [M], K, N)
+    assert c["rounds"] == 1 or not c["lone"], c

@@ -49,8 +49,6 @@ struct gm_args {
     const float2 * rope_tab;       // [token][32] cos, sin
 };
 
-enum { GM_PLAIN = 0, GM_SWIGLU = 1, GM_SEGS = 2 };
-
 // N consecutive 1 KB tiles from global memory (uniform base + lane offset) into LDS at lds + 16 lane: one statement, since the
 // compiler may write M0 between two
 template <int N> __device__ __forceinline__ void gm_dma_tiles(uint32_t off, const char * base, uint32_t lds) {
@@ -78,21 +76,7 @@ template <int L, int MOST> __device__ __forceinline__ void gm_wait_younger(int y
     gm_wait<L * MOST>();
 }
 
-constexpr int KG = 4; // waves of a row group, over the k blocks: the streaming kernel's four waves
-
-template <int WT, int MT, int NT, int RW, int CH, int S>
-struct gm_shape {
-    static constexpr int NC = KG * RW, NWAVES = NC + 2;       // compute waves; one wave brings the weights, one the activations
-    static constexpr int ROWS = 16 * MT * RW, TOKS = 16 * NT;
-    static constexpr int PIECES = WT == VX_GM_Q8 ? (CH == 1 ? 9 : 17) : 16 * CH; // 16-byte pieces of a row per stage
-    static constexpr int PITCH = PIECES * 16;
-    static constexpr int WINST = (ROWS * PIECES + 63) / 64, XINST = 4 * CH * NT;
-    static constexpr int WBYTES = WINST * 1024, XBYTES = XINST * 1024, STAGE = WBYTES + XBYTES;
-    static constexpr int STEPS = 4 * CH / KG;                 // k blocks of a stage per compute wave
-    static constexpr int NP = NT < 4 ? NT : 4;                // token tiles per pass of the final sum
-    static constexpr int RED = KG * RW * MT * NP * 1024;
-    static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
-};
+constexpr int KG = GM_KG;
 
 template <int WT, int MT, int NT, int RW, int CH, int S, int EPI>
 __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a) {
@@ -381,7 +365,7 @@ __global__ __launch_bounds__(64 * (KG * RW + 2)) void gm_kernel(const gm_args a)
 // two work-groups a compute unit.  In a layer of 1024 tokens the pair of 4096 rows takes 28 us, 42.5 on gm_kernel; 24 layers 2769 -> 2481.
 // The k blocks are walked group by group (0, 4, 8 ..., then 1, 5, ...) and a group's sum is added to the total before the next
 // begins: gm_kernel's order of every sum, so which of the two runs does not show in the result.
-constexpr int GD_CT = 4, GD_ST = 3, GD_ROWS = 256, GD_TOKS = 16 * GD_CT;
+constexpr int GD_ST = 3;
 constexpr int GD_BLOCK = GD_CT * 1024, GD_STAGE = 2 * GD_BLOCK + 4 * 1024; // two blocks of token tiles, 1 KB of scales per wave (512 bytes of it read)
 constexpr int GD_LDS = GD_ST * GD_STAGE;
 
@@ -687,32 +671,6 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
     }
 }
 
-// ---- tile choice -----------------------------------------------------------------------------------------------------
-// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages: four or five where two work-groups still share a compute
-// unit's LDS and more than three gain -- the down projection of 45 tokens 9.3 us with three, 8.3 with five, no less with six; tile 1 over
-// K 4096 x 128 tokens 12.3 with three, 12.6 with five); what a work-group costs, measured with Q8_0 weights: microseconds per 128 of K
-// and fixed
-// (96 and 112 tokens: 4096 x 1024 x 337 tokens with F16 weights 13.2 us on 192 work-groups of 128 tokens, 12.0 on 256 of 96)
-#define GM_TILES(X) \
-    X(0, 1, 1, 1, 2, 5, 0.127f, 0.95f) \
-    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f) \
-    X(2, 2, 2, 1, 2, 4, 0.190f, 1.40f) \
-    X(3, 2, 4, 1, 1, 5, 0.276f, 1.30f) \
-    X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
-    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f) \
-    X(6, 2, 6, 2, 1, 3, 0.430f, 2.50f) \
-    X(7, 2, 7, 2, 1, 3, 0.468f, 2.68f)
-constexpr int GM_N_TILES = 8;
-// lone: a compute unit's LDS holds one work-group (F16 rows are twice the bytes: more of the tiles)
-struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2]; };
-const gm_tile gm_tiles[GM_N_TILES] = {
-#define X(I, MT, NT, RW, CH, S, A_, B_)                                                          \
-    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, CH, S>::LDS > 160 * 1024, \
-                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, CH, S>::LDS > 160 * 1024 } },
-    GM_TILES(X)
-#undef X
-};
-
 template <int WT, int MT, int NT, int RW, int CH, int S, int EPI>
 bool gm_launch(const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
     using sh = gm_shape<WT, MT, NT, RW, CH, S>;
@@ -800,17 +758,6 @@ size_t vx_gm_tile_bytes(int64_t K, int64_t N, int64_t nbatch) {
     return (size_t) nbatch * (size_t) (K / 32) * (size_t) ((N + 15) / 16) * 1024 + 8192;
 }
 
-// Single products and pairs that gd_kernel takes where the weights' tiles are kept: from the number of its 256 x 64 tiles on at which
-// it beats gm_kernel's smaller ones.  gm_kernel / here, microseconds, activation pass included: 4096 x 1024 x 768 tokens (192 tiles)
-// 21.9 / 21.2, x 512 (128) 15.0 / 19.6, x 2048 42 / 32; 1024 x 4096 x 3000 (188) 64.9 / 58.8, x 2048 (128) 41 / 54.  A pair of 4096 rows
-// with its down projection behind it, by the token count: 256 (128 tiles) 27.2 / 31.0, 300 (160) 36.5 / 32.4, 512 38.7 / 34.7, 1024 62.8 / 49.5.
-static bool gd_takes(const vx_gm_call & c, int epi, int nbatch) {
-    if (c.wtype != VX_GM_Q8 || epi == GM_SEGS || c.K % 512) return false; // (a group's k blocks in whole fours)
-    const int64_t MV = c.w2 ? 2 * (int64_t) c.mat[0].M : c.mat[0].M;
-    if ((c.w2 && c.mat[0].M % 32) || (MV + 15) / 16 * (c.K / 32) >= (1 << 22)) return false;
-    return (MV + GD_ROWS - 1) / GD_ROWS * ((c.N + GD_TOKS - 1) / GD_TOKS) * nbatch >= (c.w2 ? 160 : 192);
-}
-
 static void gd_launch(int epi, dim3 grid, const gm_args & a, hipStream_t st);
 
 vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
@@ -851,58 +798,27 @@ vx_status vx_gm_run(const vx_gm_call & c, hipStream_t st) {
         else          vx_launch(gm_acts_kernel<false>, dim3((unsigned) blocks, (unsigned) nbatch, (unsigned) ((c.K + 1023) / 1024)), dim3(256), 0, st, p);
     }
     const int epi = c.w2 ? GM_SWIGLU : c.nmat > 1 ? GM_SEGS : GM_PLAIN;
-    // Which tiles an XCD takes: 1, 2, 4 or all 8 of them share out the row tiles, the rest the token tiles.  What the eight L2s
-    // bring in is every weight once per group of token tiles and every activation once per group of row tiles.
-    auto share = [&](int64_t gx, int64_t gy, double wbytes, int per_cu, int64_t & lx, int64_t & ly) {
-        const double xbytes = (double) c.N * c.K * 2;
-        double least = 0.0;
-        int64_t fill = 0;
-        lx = ly = 0;
-        for (int r = 3; r >= 0; --r) {
-            const int64_t nx = (gx + (1 << r) - 1) >> r, ny = (gy + (8 >> r) - 1) / (8 >> r), rounds = (nx * ny * nbatch + 32 * per_cu - 1) / (32 * per_cu);
-            const double bytes = wbytes * (8 >> r) + xbytes * (1 << r);
-            if (lx && (rounds > fill || (rounds == fill && bytes >= least))) continue;
-            a.xr = r; least = bytes; lx = nx; ly = ny; fill = rounds;
-        }
-        lx *= 8;
-        return lx <= 0x7fffffff && ly <= 65535;
-    };
-    int64_t lx = 0, ly = 0;
-    if (gd_takes(c, epi, nbatch)) {
+    gm_product shape = { c.wtype, epi, c.nmat, {}, c.K, c.N, nbatch };
+    for (int i = 0; i < c.nmat; ++i) shape.M[i] = c.mat[i].M;
+    auto fits = [](const gm_share & s) { return 8 * s.nx <= 0x7fffffff && s.ny <= 65535; };
+    if (gd_takes(shape)) {
         const void * tiles = nullptr;
         const float * scales = nullptr;
         const int64_t MV = c.w2 ? 2 * (int64_t) c.mat[0].M : c.mat[0].M;
-        if (share((MV + GD_ROWS - 1) / GD_ROWS, (c.N + GD_TOKS - 1) / GD_TOKS, (double) MV * c.K * 2, 2, lx, ly) &&
-            vx_qt_kept_tiles(c.mat[0].w, c.w2, c.K, c.mat[0].M, c.mat[0].nb01, st, &tiles, &scales)) {
-            a.wt = (const half8_t *) tiles; a.wdt = scales; a.n_rt = (int) ((MV + 15) / 16);
-            const dim3 grid((unsigned) lx, (unsigned) ly, (unsigned) nbatch);
-            gd_launch(epi, grid, a, st);
+        const gm_share s = gm_share_out((MV + GD_ROWS - 1) / GD_ROWS, (c.N + GD_TOKS - 1) / GD_TOKS, nbatch, (double) MV * c.K * 2, (double) c.N * c.K * 2, GD_PER_CU);
+        if (fits(s) && vx_qt_kept_tiles(c.mat[0].w, c.w2, c.K, c.mat[0].M, c.mat[0].nb01, st, &tiles, &scales)) {
+            a.wt = (const half8_t *) tiles; a.wdt = scales; a.n_rt = (int) ((MV + 15) / 16); a.xr = s.xr;
+            gd_launch(epi, dim3((unsigned) (8 * s.nx), (unsigned) s.ny, (unsigned) nbatch), a, st);
             return VX_OK;
         }
     }
-    // the tile whose work-groups finish first by the measured costs
-    int best = -1;
-    float best_us = 0.0f;
-    for (int t = 0; t < GM_N_TILES; ++t) {
-        const gm_tile & g = gm_tiles[t];
-        if (epi != GM_PLAIN && g.mt % 2) continue;
-        int64_t wx = 0;
-        if (epi == GM_SWIGLU) wx = (2 * (int64_t) c.mat[0].M + g.rows - 1) / g.rows;
-        else for (int i = 0; i < c.nmat; ++i) wx += (c.mat[i].M + g.rows - 1) / g.rows;
-        const int64_t wgs = wx * ((c.N + g.toks - 1) / g.toks) * nbatch;
-        const float one = g.fixed + g.per_step * (float) (c.K / 128);
-        // (work-groups that share a compute unit share its vector units: the fixed part of one hides behind the other's products)
-        const float per_cu = (float) ((wgs + 255) / 256);
-        const float us = per_cu <= 1.0f ? one : g.lone[c.wtype] ? per_cu * one : one + (per_cu - 1.0f) * (g.per_step * (float) (c.K / 128) + 0.3f * g.fixed);
-        if (best < 0 || us < best_us) { best = t; best_us = us; }
-    }
-    const gm_tile & g = gm_tiles[best];
-    int64_t gx = 0;
-    if (epi == GM_SWIGLU) gx = (2 * (int64_t) c.mat[0].M + g.rows - 1) / g.rows;
-    else for (int i = 0; i < c.nmat; ++i) { a.mat[i].wg0 = (int) gx; gx += (c.mat[i].M + g.rows - 1) / g.rows; }
-    const int64_t gy = (c.N + g.toks - 1) / g.toks;
-    if (!share(gx, gy, (double) gx * g.rows * (c.K / 32) * (c.wtype == VX_GM_Q8 ? 34 : 64), 1, lx, ly)) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
-    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(best, epi, a, (int) lx, (int) ly, nbatch, st) : gm_go<VX_GM_F16>(best, epi, a, (int) lx, (int) ly, nbatch, st);
+    gm_share s = {};
+    const int tile = gm_tile_choice(shape, s);
+    if (!fits(s)) return vx_fail(VX_ERR_UNSUPPORTED, "mul_mat: launch too large");
+    a.xr = s.xr;
+    if (epi != GM_SWIGLU) for (int i = 0, wg = 0; i < c.nmat; ++i) { a.mat[i].wg0 = wg; wg += (c.mat[i].M + gm_tiles[tile].rows - 1) / gm_tiles[tile].rows; }
+    const int gx = (int) (8 * s.nx), gy = (int) s.ny;
+    const bool ok = c.wtype == VX_GM_Q8 ? gm_go<VX_GM_Q8>(tile, epi, a, gx, gy, nbatch, st) : gm_go<VX_GM_F16>(tile, epi, a, gx, gy, nbatch, st);
     return ok ? VX_OK : vx_fail(VX_ERR_HIP, "mul_mat: the kernel could not be given its LDS");
 }
 

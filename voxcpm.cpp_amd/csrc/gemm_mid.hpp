@@ -1,9 +1,8 @@
 // gemm_mid.hpp -- the product kernel for some tens to a few thousand tokens (gemm_mid.hip), as mul_mat.hip calls it.
 #pragma once
 #include "vx_common.hpp"
+#include "gm_tiles.hpp"
 #include "rope_common.hpp"
-
-enum { VX_GM_Q8 = 0, VX_GM_F16 = 1 };
 
 struct vx_gm_mat {        // one weight matrix of a launch and where its product goes
     const char * w;

@@ -1,0 +1,112 @@
+// gm_tiles.hpp -- which tile of gm_kernel (or gd_kernel's) a product of gemm_mid.hip runs on, and which XCD takes which of its tiles.
+// Free of HIP calls, so that the rules can be asked on a host without a device.
+#pragma once
+
+#include <cstdint>
+
+enum { VX_GM_Q8 = 0, VX_GM_F16 = 1 };
+enum { GM_PLAIN = 0, GM_SWIGLU = 1, GM_SEGS = 2 };
+
+constexpr int GM_KG = 4; // waves of a row group, over the k blocks: the streaming kernel's four waves
+
+// gm_kernel's tile: row tiles of 16 a wave, token tiles of 16, row groups, 128-k chunks a stage, stages
+template <int WT, int MT, int NT, int RW, int CH, int S>
+struct gm_shape {
+    static constexpr int NC = GM_KG * RW, NWAVES = NC + 2;    // compute waves; one wave brings the weights, one the activations
+    static constexpr int ROWS = 16 * MT * RW, TOKS = 16 * NT;
+    static constexpr int PIECES = WT == VX_GM_Q8 ? (CH == 1 ? 9 : 17) : 16 * CH; // 16-byte pieces of a row per stage
+    static constexpr int PITCH = PIECES * 16;
+    static constexpr int WINST = (ROWS * PIECES + 63) / 64, XINST = 4 * CH * NT;
+    static constexpr int WBYTES = WINST * 1024, XBYTES = XINST * 1024, STAGE = WBYTES + XBYTES;
+    static constexpr int STEPS = 4 * CH / GM_KG;              // k blocks of a stage per compute wave
+    static constexpr int NP = NT < 4 ? NT : 4;                // token tiles per pass of the final sum
+    static constexpr int RED = GM_KG * RW * MT * NP * 1024;
+    static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
+};
+
+// ---- tile choice -----------------------------------------------------------------------------------------------------
+// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages: four or five where two work-groups still share a compute
+// unit's LDS and more than three gain -- the down projection of 45 tokens 9.3 us with three, 8.3 with five, no less with six; tile 1 over
+// K 4096 x 128 tokens 12.3 with three, 12.6 with five); what a work-group costs, measured with Q8_0 weights: microseconds per 128 of K
+// and fixed
+// (96 and 112 tokens: 4096 x 1024 x 337 tokens with F16 weights 13.2 us on 192 work-groups of 128 tokens, 12.0 on 256 of 96)
+#define GM_TILES(X) \
+    X(0, 1, 1, 1, 2, 5, 0.127f, 0.95f) \
+    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f) \
+    X(2, 2, 2, 1, 2, 4, 0.190f, 1.40f) \
+    X(3, 2, 4, 1, 1, 5, 0.276f, 1.30f) \
+    X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
+    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f) \
+    X(6, 2, 6, 2, 1, 3, 0.430f, 2.50f) \
+    X(7, 2, 7, 2, 1, 3, 0.468f, 2.68f)
+constexpr int GM_N_TILES = 8;
+// lone: a compute unit's LDS holds one work-group (F16 rows are twice the bytes: more of the tiles)
+struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2]; };
+constexpr gm_tile gm_tiles[GM_N_TILES] = {
+#define X(I, MT, NT, RW, CH, S, A_, B_)                                                          \
+    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, CH, S>::LDS > 160 * 1024, \
+                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, CH, S>::LDS > 160 * 1024 } },
+    GM_TILES(X)
+#undef X
+};
+
+// gd_kernel's tile, and the work-groups that share a compute unit
+constexpr int GD_CT = 4, GD_ROWS = 256, GD_TOKS = 16 * GD_CT, GD_PER_CU = 2;
+
+struct gm_product { int wtype, epi, nmat; int64_t M[3], K, N, nbatch; }; // (a pair: M[0] rows of each matrix)
+
+// Which tiles an XCD takes: 1, 2, 4 or all 8 of them (2^xr) share out the gx row tiles, the rest the gy token tiles -- nx by ny tiles an
+// XCD and batch entry.  What the eight L2s bring in is every weight once per group of token tiles and every activation once per group of
+// row tiles: the fewest bytes of those divisions that leave the fullest XCD (32 compute units, per_cu work-groups each at a time) the
+// fewest rounds.
+struct gm_share { int xr; int64_t nx, ny, rounds, tiles; }; // tiles: of the whole product
+static inline gm_share gm_share_out(int64_t gx, int64_t gy, int64_t nbatch, double wbytes, double xbytes, int per_cu) {
+    gm_share s = { 0, 0, 0, 0, gx * gy * nbatch };
+    double least = 0.0;
+    for (int r = 3; r >= 0; --r) {
+        const int64_t nx = (gx + (1 << r) - 1) >> r, ny = (gy + (8 >> r) - 1) / (8 >> r), rounds = (nx * ny * nbatch + 32 * per_cu - 1) / (32 * per_cu);
+        const double bytes = wbytes * (8 >> r) + xbytes * (1 << r);
+        if (s.nx && (rounds > s.rounds || (rounds == s.rounds && bytes >= least))) continue;
+        s = { r, nx, ny, rounds, s.tiles };
+        least = bytes;
+    }
+    return s;
+}
+
+static inline gm_share gm_tile_share(const gm_product & p, int tile) {
+    const gm_tile & g = gm_tiles[tile];
+    int64_t gx = 0;
+    if (p.epi == GM_SWIGLU) gx = (2 * p.M[0] + g.rows - 1) / g.rows;
+    else for (int i = 0; i < p.nmat; ++i) gx += (p.M[i] + g.rows - 1) / g.rows;
+    return gm_share_out(gx, (p.N + g.toks - 1) / g.toks, p.nbatch, (double) gx * g.rows * (double) (p.K / 32) * (p.wtype == VX_GM_Q8 ? 34 : 64), (double) p.N * p.K * 2, 1);
+}
+
+// The tile whose work-groups finish first by the costs.  One that has a compute unit to itself: on the XCD that has most of them.  (Counted
+// over the chip, 238 work-groups of 520 rows x 448 tokens of K 2304 seemed one round of 256; at least 34 are an XCD's, which has 32 compute
+// units: 16.0 us where another tile takes 12.7.)  Where two share one, an XCD's last few join others and cost far less than a round: over the chip.
+static inline int gm_tile_choice(const gm_product & p, gm_share & share) {
+    int best = -1;
+    float best_us = 0.0f;
+    for (int t = 0; t < GM_N_TILES; ++t) {
+        const gm_tile & g = gm_tiles[t];
+        if (p.epi != GM_PLAIN && g.mt % 2) continue;
+        const gm_share s = gm_tile_share(p, t);
+        const float steps = g.per_step * (float) (p.K / 128), one = g.fixed + steps, rounds = (float) (g.lone[p.wtype] ? s.rounds : (s.tiles + 255) / 256);
+        // (work-groups that share a compute unit share its vector units: the fixed part of one hides behind the other's products)
+        const float us = g.lone[p.wtype] ? rounds * one : one + (rounds - 1.0f) * (steps + 0.3f * g.fixed);
+        if (best < 0 || us < best_us) { best = t; best_us = us; share = s; }
+    }
+    return best;
+}
+
+// Single products and pairs that gd_kernel takes where the weights' tiles are kept: from the number of its 256 x 64 tiles on at which
+// it beats gm_kernel's smaller ones.  gm_kernel / here, microseconds, activation pass included: 4096 x 1024 x 768 tokens (192 tiles)
+// 21.9 / 21.2, x 512 (128) 15.0 / 19.6, x 2048 42 / 32; 1024 x 4096 x 3000 (188) 64.9 / 58.8, x 2048 (128) 41 / 54.  A pair of 4096 rows
+// with its down projection behind it, by the token count: 256 (128 tiles) 27.2 / 31.0, 300 (160) 36.5 / 32.4, 512 38.7 / 34.7, 1024 62.8 / 49.5.
+static inline bool gd_takes(const gm_product & p) {
+    if (p.wtype != VX_GM_Q8 || p.epi == GM_SEGS || p.K % 512) return false; // (a group's k blocks in whole fours)
+    const bool pair = p.epi == GM_SWIGLU;
+    const int64_t MV = pair ? 2 * p.M[0] : p.M[0];
+    if ((pair && p.M[0] % 32) || (MV + 15) / 16 * (p.K / 32) >= (1 << 22)) return false;
+    return (MV + GD_ROWS - 1) / GD_ROWS * ((p.N + GD_TOKS - 1) / GD_TOKS) * p.nbatch >= (pair ? 160 : 192);
+}
