@@ -56,3 +56,10 @@ def test_an_odd_number_of_row_tiles_does_not_take_a_second_round(rules, wtype, M
     """Just under 256 work-groups of a tile that has a compute unit to itself, of which an XCD's share is more than its 32 units."""
     c = choice(rules, wtype, PLAIN, [M], K, N)
     assert c["rounds"] == 1 or not c["lone"], c
+
+
+@pytest.mark.parametrize("epi,rows,K,N", [(SWIGLU, [5504], 1024, 24), (SWIGLU, [5504], 1024, 32), (PLAIN, [3072], 768, 160)])
+def test_small_tiles_share_a_compute_unit(rules, epi, rows, K, N):
+    """Q8_0, a little more than a work-group for each compute unit: the 32 x 32 tiles that run there leave room for a second one."""
+    c = choice(rules, Q8, epi, rows, K, N)
+    assert c["rows"] == c["toks"] == 32 and not c["lone"], c

@@ -687,14 +687,18 @@ bool gm_launch(const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
 template <int WT>
 bool gm_go(int tile, int epi, const gm_args & a, int gx, int gy, int nbatch, hipStream_t st) {
     switch (tile) {
-#define X(I, MT, NT, RW, CH, S, A_, B_)                                                                                   \
-        case I:                                                                                                         \
-            if (epi == GM_PLAIN) return gm_launch<WT, MT, NT, RW, CH, S, GM_PLAIN>(a, gx, gy, nbatch, st);              \
-            if constexpr (MT % 2 == 0) {                                                                                \
-                if (epi == GM_SWIGLU) return gm_launch<WT, MT, NT, RW, CH, S, GM_SWIGLU>(a, gx, gy, nbatch, st);        \
-                return gm_launch<WT, MT, NT, RW, CH, S, GM_SEGS>(a, gx, gy, nbatch, st);                                \
+#define X(I, MT, NT, RW, CH, SQ, SF, A_, B_)                                                                            \
+        case I: {                                                                                                       \
+            constexpr int S = WT == VX_GM_Q8 ? SQ : SF;                                                                 \
+            if constexpr (S > 0) {                                                                                      \
+                if (epi == GM_PLAIN) return gm_launch<WT, MT, NT, RW, CH, S, GM_PLAIN>(a, gx, gy, nbatch, st);          \
+                if constexpr (MT % 2 == 0) {                                                                            \
+                    if (epi == GM_SWIGLU) return gm_launch<WT, MT, NT, RW, CH, S, GM_SWIGLU>(a, gx, gy, nbatch, st);    \
+                    return gm_launch<WT, MT, NT, RW, CH, S, GM_SEGS>(a, gx, gy, nbatch, st);                            \
+                }                                                                                                       \
             }                                                                                                           \
-            return false;
+            return false;                                                                                               \
+        }
         GM_TILES(X)
 #undef X
     }

@@ -25,30 +25,43 @@ struct gm_shape {
 };
 
 // ---- tile choice -----------------------------------------------------------------------------------------------------
-// (row tiles per wave, token tiles, row groups, 128-k chunks a stage, stages: four or five where two work-groups still share a compute
-// unit's LDS and more than three gain -- the down projection of 45 tokens 9.3 us with three, 8.3 with five, no less with six; tile 1 over
-// K 4096 x 128 tokens 12.3 with three, 12.6 with five); what a work-group costs, measured with Q8_0 weights: microseconds per 128 of K
-// and fixed
-// (96 and 112 tokens: 4096 x 1024 x 337 tokens with F16 weights 13.2 us on 192 work-groups of 128 tokens, 12.0 on 256 of 96)
+// (row tiles per wave, token tiles, row groups, 128-k chunks a stage; stages with Q8_0 and with F16 weights, 0: not built; what a
+// work-group costs beside the other tiles': microseconds per 128 of K and fixed)
+//   Stages.  Three, or more where that gains within one round of work-groups; measured as kernels of 256 and 512 work-groups (K 1024 /
+// 4352) and as whole products (1024 x 4096), microseconds with three and with these:
+//   * 16 x 16, five: two share a unit's LDS with either type; 256: Q8_0 K 4352 7.4 / 7.1, F16 7.4 / 6.7; 45 tokens: 9.4 / 9.3, F16 9.3 / 8.8;
+//   * 32 x 32, four: alone on a unit; 256: Q8_0 5.6 / 5.8 and 11.7 / 10.4, F16 5.1 / 5.0 and 12.8 / 12.5; 203 tokens: 13.9 / 13.5, F16 13.1 / 12.7.
+//     F16 does not share with three either.  Q8_0 does: a tile of its own (8) for more work-groups than units, 512: 7.3 / 10.5, pairs of 5504 rows
+//     by 24 tokens 10.2 / 10.8;
+//   * 32 x 64, five: alone on a unit; 256: Q8_0 6.4 / 6.6 and 14.2 / 12.8, F16 6.2 / 5.9 and 16.2 / 15.1; 337 tokens: 17.4 / 17.5, F16 17.6 / 16.5; a
+//     prompt of 45 tokens, whose gate/up pair is one round of it, 974 / 963.  With three two share a unit (512: 8.8 / 11.7), but from there on
+//     the larger tiles are the faster.
+//   Costs.  Those of the tiles up to 64 x 128 come from kernels with Q8_0 weights and three stages, without what every tile pays alike; 96
+// and 112 tokens lie on the line between 64 and 128.  They only serve to compare: over 994 products, pairs and q/k/v groups of 17 to 3072 tokens,
+// both types, the tile chosen takes 0.5 % longer than the fastest one on average, more than 3 % in 66 of them, at most 14 (520 rows x 416 tokens of
+// K 2304); no other pair of values for 96 or 112 tokens does better by more than 0.03 %.
 #define GM_TILES(X) \
-    X(0, 1, 1, 1, 2, 5, 0.127f, 0.95f) \
-    X(1, 1, 2, 1, 2, 3, 0.135f, 1.10f) \
-    X(2, 2, 2, 1, 2, 4, 0.190f, 1.40f) \
-    X(3, 2, 4, 1, 1, 5, 0.276f, 1.30f) \
-    X(4, 2, 4, 2, 1, 3, 0.355f, 2.15f) \
-    X(5, 2, 8, 2, 1, 3, 0.505f, 2.85f) \
-    X(6, 2, 6, 2, 1, 3, 0.430f, 2.50f) \
-    X(7, 2, 7, 2, 1, 3, 0.468f, 2.68f)
-constexpr int GM_N_TILES = 8;
+    X(0, 1, 1, 1, 2, 5, 5, 0.127f, 0.95f) \
+    X(1, 1, 2, 1, 2, 3, 3, 0.135f, 1.10f) \
+    X(2, 2, 2, 1, 2, 4, 4, 0.190f, 1.40f) \
+    X(3, 2, 4, 1, 1, 5, 5, 0.276f, 1.30f) \
+    X(4, 2, 4, 2, 1, 3, 3, 0.355f, 2.15f) \
+    X(5, 2, 8, 2, 1, 3, 3, 0.505f, 2.85f) \
+    X(6, 2, 6, 2, 1, 3, 3, 0.430f, 2.50f) \
+    X(7, 2, 7, 2, 1, 3, 3, 0.468f, 2.68f) \
+    X(8, 2, 2, 1, 2, 3, 0, 0.190f, 1.40f)
+constexpr int GM_N_TILES = 9;
 // lone: a compute unit's LDS holds one work-group (F16 rows are twice the bytes: more of the tiles)
-struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2]; };
+struct gm_tile { int rows, toks, mt; float per_step, fixed; bool lone[2], built[2]; };
 constexpr gm_tile gm_tiles[GM_N_TILES] = {
-#define X(I, MT, NT, RW, CH, S, A_, B_)                                                          \
-    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, CH, S>::LDS > 160 * 1024, \
-                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, CH, S>::LDS > 160 * 1024 } },
+#define X(I, MT, NT, RW, CH, SQ, SF, A_, B_)                                                          \
+    { 16 * MT * RW, 16 * NT, MT, A_, B_, { 2 * gm_shape<VX_GM_Q8, MT, NT, RW, CH, SQ>::LDS > 160 * 1024, \
+                                           2 * gm_shape<VX_GM_F16, MT, NT, RW, CH, SF>::LDS > 160 * 1024 }, { SQ > 0, SF > 0 } },
     GM_TILES(X)
 #undef X
 };
+static_assert(!gm_tiles[0].lone[VX_GM_Q8] && !gm_tiles[0].lone[VX_GM_F16] && !gm_tiles[1].lone[VX_GM_Q8] && !gm_tiles[1].lone[VX_GM_F16] &&
+              !gm_tiles[8].lone[VX_GM_Q8], "two of these share a compute unit: more stages would end that");
 
 // gd_kernel's tile, and the work-groups that share a compute unit
 constexpr int GD_CT = 4, GD_ROWS = 256, GD_TOKS = 16 * GD_CT, GD_PER_CU = 2;
@@ -89,7 +102,7 @@ static inline int gm_tile_choice(const gm_product & p, gm_share & share) {
     float best_us = 0.0f;
     for (int t = 0; t < GM_N_TILES; ++t) {
         const gm_tile & g = gm_tiles[t];
-        if (p.epi != GM_PLAIN && g.mt % 2) continue;
+        if (!g.built[p.wtype] || (p.epi != GM_PLAIN && g.mt % 2)) continue;
         const gm_share s = gm_tile_share(p, t);
         const float steps = g.per_step * (float) (p.K / 128), one = g.fixed + steps, rounds = (float) (g.lone[p.wtype] ? s.rounds : (s.tiles + 255) / 256);
         // (work-groups that share a compute unit share its vector units: the fixed part of one hides behind the other's products)
