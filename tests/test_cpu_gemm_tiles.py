@@ -63,3 +63,13 @@ def test_small_tiles_share_a_compute_unit(rules, epi, rows, K, N):
     """Q8_0, a little more than a work-group for each compute unit: the 32 x 32 tiles that run there leave room for a second one."""
     c = choice(rules, Q8, epi, rows, K, N)
     assert c["rows"] == c["toks"] == 32 and not c["lone"], c
+
+
+@pytest.mark.parametrize("epi,M,K,N,nb,kept", [
+    (PLAIN, 4096, 1024, 700, 1, 0), (PLAIN, 4096, 1024, 768, 1, 1), (PLAIN, 4096, 768, 1000, 1, 0), (SWIGLU, 4096, 1024, 256, 1, 0), (SWIGLU, 4096, 1024, 257, 1, 1),
+    (SWIGLU, 2800, 1024, 3000, 1, 0), (SWIGLU, 2784, 1024, 3000, 1, 1), (PLAIN, 1024, 4096, 3072, 1, 0), (PLAIN, 2048, 4096, 1536, 1, 0), (SWIGLU, 1024, 4096, 1400, 1, 0),
+    (PLAIN, 2048, 4096, 1856, 1, 1), (PLAIN, 1536, 4096, 2560, 1, 1), (PLAIN, 1536, 4096, 2688, 1, 0), (PLAIN, 2048, 4096, 2304, 1, 0), (PLAIN, 2048, 4096, 2432, 1, 1),
+    (PLAIN, 2048, 16384, 1792, 1, 0), (PLAIN, 2048, 16384, 1856, 1, 1), (SWIGLU, 2048, 2560, 400, 3, 1), (SWIGLU, 768, 3072, 896, 3, 0)])
+def test_products_from_kept_tiles(rules, epi, M, K, N, nb, kept):
+    """Where gd_kernel was measured to be the faster kernel it is taken, elsewhere not."""
+    assert rules.gm_kept(Q8, epi, C.c_int64(M), C.c_int64(K), C.c_int64(N), C.c_int64(nb)) == kept

@@ -112,14 +112,27 @@ static inline int gm_tile_choice(const gm_product & p, gm_share & share) {
     return best;
 }
 
-// Single products and pairs that gd_kernel takes where the weights' tiles are kept: from the number of its 256 x 64 tiles on at which
-// it beats gm_kernel's smaller ones.  gm_kernel / here, microseconds, activation pass included: 4096 x 1024 x 768 tokens (192 tiles)
-// 21.9 / 21.2, x 512 (128) 15.0 / 19.6, x 2048 42 / 32; 1024 x 4096 x 3000 (188) 64.9 / 58.8, x 2048 (128) 41 / 54.  A pair of 4096 rows
-// with its down projection behind it, by the token count: 256 (128 tiles) 27.2 / 31.0, 300 (160) 36.5 / 32.4, 512 38.7 / 34.7, 1024 62.8 / 49.5.
+// Single products and pairs that gd_kernel takes where the weights' tiles are kept: from the number of its 256 x 64 tiles on at which it
+// beats gm_kernel.  gm_kernel / here, microseconds, activation pass included, by the tokens (tiles):
+//   * K 1024, single: 4096 rows 512 (128) 15.1 / 19.8, 768 (192) 21.4 / 21.6, 1024 (256) 24.4 / 24.0, 1088 (272) 30.1 / 27.9, 2048 (512) 45.9 / 33.6; 6144
+//     rows 512 (192) 21.9 / 22.1, 640 (240) 24.8 / 23.5; 2048 rows 1536 (192) 22.4 / 21.9;
+//   * K 1024, a pair with its down projection behind it: 4096 rows 256 (128) 27.9 / 31.9, 300 (160) 37.0 / 35.4, 512 (256) 41.7 / 36.7, 576 (288) 50.6 /
+//     47.7, 1024 (512) 66.4 / 54.6, 1280 (640) 83.2 / 69.8, 3072 (1536) 179 / 133;
+//   * a long K, on which few work-groups take longer: K 4096, 1024 rows 3072 (192) 61.4 / 65.5, 1536 rows 2240 (210) 60.4 / 62.3, 2304 (216) 64.9 / 62.8,
+//     2048 rows 1664 (208) 59.9 / 58.7, 2048 (256) 66.4 / 63.0, 4096 rows 2048 (512) 119 / 100; K 16384, 2048 rows 1792 (224) 206 / 225, 1856 (232) 225 / 226;
+//   * and just over a work-group for each of an XCD's compute units there: K 4096, 1536 rows 2688 (252, no XCD fewer than 33) 70.7 / 81.2, 2048 rows
+//     2304 (288, 36) 80.4 / 80.5, 2432 (304, 38) 87.3 / 81.4.
 static inline bool gd_takes(const gm_product & p) {
     if (p.wtype != VX_GM_Q8 || p.epi == GM_SEGS || p.K % 512) return false; // (a group's k blocks in whole fours)
     const bool pair = p.epi == GM_SWIGLU;
-    const int64_t MV = pair ? 2 * p.M[0] : p.M[0];
+    const int64_t MV = pair ? 2 * p.M[0] : p.M[0], gx = (MV + GD_ROWS - 1) / GD_ROWS, gy = (p.N + GD_TOKS - 1) / GD_TOKS, tiles = gx * gy * p.nbatch;
     if ((pair && p.M[0] % 32) || (MV + 15) / 16 * (p.K / 32) >= (1 << 22)) return false;
-    return (MV + GD_ROWS - 1) / GD_ROWS * ((p.N + GD_TOKS - 1) / GD_TOKS) * p.nbatch >= (pair ? 160 : 192);
+    if (p.K <= 1024) return tiles >= (pair ? 160 : 192);
+    if (tiles < (p.K > 8192 ? 232 : 216)) return false;
+    int64_t fullest = INT64_MAX; // XCD's work-groups, of the most even division
+    for (int r = 0; r < 4; ++r) {
+        const int64_t n = ((gx + (1 << r) - 1) >> r) * ((gy + (8 >> r) - 1) / (8 >> r)) * p.nbatch;
+        fullest = n < fullest ? n : fullest;
+    }
+    return fullest <= 32 || fullest > 36;
 }
