@@ -73,3 +73,23 @@ def test_small_tiles_share_a_compute_unit(rules, epi, rows, K, N):
 def test_products_from_kept_tiles(rules, epi, M, K, N, nb, kept):
     """Where gd_kernel was measured to be the faster kernel it is taken, elsewhere not."""
     assert rules.gm_kept(Q8, epi, C.c_int64(M), C.c_int64(K), C.c_int64(N), C.c_int64(nb)) == kept
+
+
+def test_the_gpu_cases_run_on_the_tiles_they_name(rules):
+    """tests/test_gpu_gemm_tiles.py: 96 and 112 tokens in every form, the 32 x 32 tile that shares a compute unit."""
+    import test_gpu_gemm_tiles as cases
+    types = {"q8": Q8, "f16": F16}
+
+    def tile(wtype, epi, rows, K, N):
+        c = choice(rules, wtype, epi, rows, K, N)
+        return c["rows"], c["toks"], bool(c["lone"])
+
+    for wtype in (Q8, F16):
+        at = {(m, k, n): tile(wtype, PLAIN, [m], k, n) for m, k, n in cases.PRODUCTS}
+        assert [at[c][1] for c in cases.PRODUCTS[:6]] == [96, 96, 96, 112, 112, 112]
+        if wtype == Q8:
+            assert [at[c] for c in cases.PRODUCTS[6:8]] == [(32, 32, False)] * 2
+        assert {at[c][1] for c in cases.PRODUCTS[8:10]} == {64}
+    pairs = [tile(types[w], SWIGLU, [m], 1024, n) for m, n, w in cases.PAIRS]
+    assert [t[1] for t in pairs] == [96, 96, 112, 112, 112, 112, 32, 32] and not pairs[6][2] and not pairs[7][2]
+    assert [tile(types[w], SEGS, [1024, 128, 128], 1024, t * b)[1] for t, b, w in cases.GROUPS] == [96, 96, 112, 112]
