@@ -93,3 +93,15 @@ def test_the_gpu_cases_run_on_the_tiles_they_name(rules):
     pairs = [tile(types[w], SWIGLU, [m], 1024, n) for m, n, w in cases.PAIRS]
     assert [t[1] for t in pairs] == [96, 96, 112, 112, 112, 112, 32, 32] and not pairs[6][2] and not pairs[7][2]
     assert [tile(types[w], SEGS, [1024, 128, 128], 1024, t * b)[1] for t, b, w in cases.GROUPS] == [96, 96, 112, 112]
+
+
+def test_the_gpu_cases_of_kept_tiles_run_on_gd_kernel(rules):
+    """tests/test_gpu_gemm_kept.py says which of its products and pairs do."""
+    import test_gpu_gemm_kept as cases
+    kept = lambda *a: bool(rules.gm_kept(Q8, a[0], *(C.c_int64(v) for v in a[1:])))
+    for M, K, N, nb, single, pair in cases.PRODUCTS:
+        assert (kept(PLAIN, M, K, N, nb), kept(SWIGLU, M, K, N, nb)) == (single, pair), (M, K, N, nb)
+    for T, M, copies in cases.MLPS:
+        assert kept(SWIGLU, 4096, 1024, T, 1) + kept(PLAIN, M, 4096, T, 1) == copies, (T, M)
+    assert any(copies == 2 for _, _, copies in cases.MLPS)
+    assert any(pair and 2 * M % 256 for M, _, _, _, _, pair in cases.PRODUCTS) and any(single and M % 256 for M, _, _, _, single, _ in cases.PRODUCTS)

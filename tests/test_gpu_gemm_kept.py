@@ -17,9 +17,15 @@ def kept_bytes(L):
     return [t.value for t in v]
 
 
-@pytest.mark.parametrize("M,K,N,nb", [(4096, 1024, 768, 1), (4096, 1024, 1024, 1), (4064, 768, 1001, 1), (6144, 1024, 513, 1), (1000, 1024, 3071, 1),
-                                      (1024, 4096, 3072, 1), (2080, 2304, 450, 3), (4096, 1024, 65, 6)])
-def test_products_from_kept_tiles(pkg, gpu, M, K, N, nb):
+# rows (of each matrix), K, tokens, batch; whether the single product and the pair run on gd_kernel (tests/test_cpu_gemm_tiles.py holds this
+# against the rule): whole and ragged 256-row tiles of both, the shortest K and long ones, batches
+PRODUCTS = [(4096, 1024, 768, 1, True, True), (4096, 1024, 1024, 1, True, True), (4064, 1024, 1001, 1, True, True), (6144, 1024, 513, 1, True, True),
+            (1000, 1024, 3071, 1, True, False), (2784, 1024, 513, 1, False, True), (2048, 4096, 1857, 1, True, True), (2080, 2560, 450, 3, True, True),
+            (4096, 1024, 65, 6, True, True), (1536, 8192, 2310, 1, True, True), (1024, 4096, 3072, 1, False, True), (4096, 768, 1001, 1, False, False)]
+
+
+@pytest.mark.parametrize("M,K,N,nb,single,pair", PRODUCTS)
+def test_products_from_kept_tiles(pkg, gpu, M, K, N, nb, single, pair):
     import torch
     say(f"products from kept tiles M={M} K={K} N={N} batch={nb}")
     L, d = pkg.lib(), pkg.desc
@@ -29,51 +35,67 @@ def test_products_from_kept_tiles(pkg, gpu, M, K, N, nb):
     wd, wd2 = pkg.desc_q8(pool[0], K), pkg.desc_q8(pool[1], K)
     x, res = dev(g.standard_normal((nb, N, K)).astype(np.float32)), dev(g.standard_normal((nb, N, M)).astype(np.float32))
     v = (lambda t: t.unsqueeze(1)) if nb > 1 else (lambda t: t[0])
+    calls = [lambda o: L.vx_mul_mat(wd, d(v(x)), d(v(o)), pkg.ACT_FLOAT, None),
+             lambda o: L.vx_mul_mat_scale_add(wd, d(v(x)), d(v(res)), d(v(o)), 0.7, pkg.ACT_FLOAT, None)]
+    if L.vx_supports_mul_mat_swiglu_tiled(wd, wd2, d(v(x)), d(v(res)), pkg.ACT_FLOAT):
+        calls.append(lambda o: L.vx_mul_mat_swiglu(wd, wd2, d(v(x)), d(v(o)), pkg.ACT_FLOAT, None))
+    assert len(calls) == 3 or not pair
 
-    def all_three():
-        outs = [torch.full((nb, N, M), 7.0, dtype=torch.float32, device="cuda") for _ in range(3)]
-        ok(pkg, L.vx_mul_mat(wd, d(v(x)), d(v(outs[0])), pkg.ACT_FLOAT, None), "mul_mat")
-        ok(pkg, L.vx_mul_mat_scale_add(wd, d(v(x)), d(v(res)), d(v(outs[1])), 0.7, pkg.ACT_FLOAT, None), "mul_mat_scale_add")
-        if L.vx_supports_mul_mat_swiglu_tiled(wd, wd2, d(v(x)), d(v(outs[2])), pkg.ACT_FLOAT):
-            ok(pkg, L.vx_mul_mat_swiglu(wd, wd2, d(v(x)), d(v(outs[2])), pkg.ACT_FLOAT, None), "mul_mat_swiglu")
+    def run(call):
+        out = torch.full((nb, N, M), 7.0, dtype=torch.float32, device="cuda")
+        ok(pkg, call(out), "product")
         torch.cuda.synchronize()
-        return outs
+        return out
 
-    want = all_three()
-    base = kept_bytes(L)
+    want = [run(c) for c in calls]
     pkg.check(L.vx_weights_pin(pool.data_ptr(), pool.numel()), "pin")
     try:
+        base = held = kept_bytes(L)[1:]
         for turn in range(2):   # the copies are made, then used again
-            assert all(same_bits(a, b) for a, b in zip(want, all_three())), turn
-        assert kept_bytes(L) != base
+            for c, w, copies in zip(calls, want, (single, single, single + pair)):
+                assert same_bits(w, run(c)), turn
+                before, held = held, kept_bytes(L)[1:]
+                if turn == 0:
+                    assert held[0] == base[0] + copies
+                    assert held == before or held[1] - before[1] >= 2 * M * K * (held[0] - base[0])    # (f16 values; the pair's are two matrices')
+                else:
+                    assert held == before
     finally:
         L.vx_weights_unpin(pool.data_ptr())
+    assert kept_bytes(L)[1:] == base
 
 
-@pytest.mark.parametrize("T", [768, 1000, 1024, 2048])
-def test_mlp_from_kept_tiles(pkg, gpu, T):
+# tokens, rows behind the down projection; copies: the pair's, and down's where that runs on gd_kernel as well, from the tiles that the pair left
+MLPS = [(768, 1024, 1), (1000, 1024, 1), (1024, 1024, 1), (2048, 1024, 1), (3072, 1024, 1), (1801, 2048, 2), (1856, 2040, 2)]
+
+
+@pytest.mark.parametrize("T,M,copies", MLPS)
+def test_mlp_from_kept_tiles(pkg, gpu, T, M, copies):
     """The whole MLP: the pair leaves its result as the down projection's tiles."""
     import torch
-    say(f"MLP from kept tiles T={T}")
+    say(f"MLP from kept tiles T={T} rows={M}")
     L, d = pkg.lib(), pkg.desc
     K, F = 1024, 4096
-    g = rng("kept-mlp", T)
+    g = rng("kept-mlp", T, M)
     mk = lambda m, k: q8_dev((0.05 * g.standard_normal((m, k))).astype(np.float32))[0]
-    pair, down = torch.stack([mk(F, K), mk(F, K)]).contiguous(), mk(K, F)
+    pair, down = torch.stack([mk(F, K), mk(F, K)]).contiguous(), mk(M, F)
     wg, wu, wd = pkg.desc_q8(pair[0], K), pkg.desc_q8(pair[1], K), pkg.desc_q8(down, F)
     x, nw = dev((2 * g.standard_normal((T, K))).astype(np.float32)), dev((1 + 0.1 * g.standard_normal(K)).astype(np.float32))
+    res = dev(g.standard_normal((T, M)).astype(np.float32))
 
     def mlp():
-        out = torch.full((T, K), float("nan"), dtype=torch.float32, device="cuda")
-        ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, wg, wu, wd, d(x), 0.3, d(out), pkg.ACT_FLOAT, None), "mlp_tiled")
+        out = torch.full((T, M), float("nan"), dtype=torch.float32, device="cuda")
+        ok(pkg, L.vx_mlp_tiled(d(x), d(nw), 1e-5, wg, wu, wd, d(res), 0.3, d(out), pkg.ACT_FLOAT, None), "mlp_tiled")
         torch.cuda.synchronize()
         return out
 
     want = mlp()
+    base = kept_bytes(L)[1]
     for t in (pair, down):
         pkg.check(L.vx_weights_pin(t.data_ptr(), t.numel()), "pin")
     try:
-        assert same_bits(want, mlp()) and same_bits(want, mlp())
+        for turn in range(2):
+            assert same_bits(want, mlp()) and kept_bytes(L)[1] == base + copies, turn
     finally:
         for t in (pair, down):
             L.vx_weights_unpin(t.data_ptr())
