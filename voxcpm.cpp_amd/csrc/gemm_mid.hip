@@ -617,13 +617,15 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
     const int tok = (int) blockIdx.x * 4 + wid, batch = blockIdx.y;
     if (tok >= 16 * a.n_tt) return;
     const int i12 = batch % a.ne12, i13 = batch / a.ne12;
-    const int nvec = a.K / 4;
+    const int nvec = a.K / 4, iv0 = 256 * (int) blockIdx.z + lane; // (nvec is a multiple of 64: whole waves)
     char * out = (char *) (a.xt + ((int64_t) batch * a.n_kb * a.n_tt + (tok >> 4)) * 64) + (tok & 15) * 16;
     auto put = [&](int iv, half4_t h) { // columns 4 iv .. + 3: half a piece of k block iv / 8
         *(half4_t *) (out + (int64_t) (iv >> 3) * a.n_tt * 1024 + ((iv >> 1) & 3) * 256 + (iv & 1) * 8) = h;
     };
     if (tok >= a.N) { // (uniform) the last tile's missing tokens
-        for (int iv = 256 * (int) blockIdx.z + lane; iv < min(nvec, 256 * ((int) blockIdx.z + 1)); iv += 64) put(iv, half4_t{0, 0, 0, 0});
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (iv0 + 64 * u < nvec) put(iv0 + 64 * u, half4_t{0, 0, 0, 0});
         return;
     }
     const float * row = (const float *) (a.x + (uint64_t) i12 * a.nb12 + (uint64_t) i13 * a.nb13 + (uint64_t) tok * a.nb11);
@@ -648,25 +650,21 @@ __global__ __launch_bounds__(256) void gm_acts_kernel(const gm_acts a) {
     } else {
         // (blockIdx.z: 1024 columns of the row.  As one wave a row, four trips one after the other, the pass made products of K 4096 over 203 tokens
         // 14.5 us, 13.1 now; 337 tokens 17.5 / 16.6)
-        float y = 0.0f;
-        const int end = min(nvec, 256 * ((int) blockIdx.z + 1));
-        for (int iv0 = 256 * (int) blockIdx.z + lane; iv0 < end; iv0 += 64 * 4) { // (nvec is a multiple of 64: whole waves)
-            float4_t v[4];
+        float4_t v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = ((const float4_t *) row)[min(iv0 + 64 * u, nvec - 1)];
-            if (a.totals) { // (uniform) the ADD1 node
-                if (iv0 < 256 * (int) blockIdx.z + 64) y = kvs_scalar_of_16(a.totals, lane, a.sync_scale, a.sync_bias);
+        for (int u = 0; u < 4; ++u) v[u] = ((const float4_t *) row)[min(iv0 + 64 * u, nvec - 1)];
+        if (a.totals) { // (uniform) the ADD1 node
+            const float y = kvs_scalar_of_16(a.totals, lane, a.sync_scale, a.sync_bias);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] += y;
-            }
+            for (int u = 0; u < 4; ++u) v[u] += y;
+        }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (iv0 + 64 * u >= end) break;
-                half4_t h;
+        for (int u = 0; u < 4; ++u) {
+            if (iv0 + 64 * u >= nvec) break;
+            half4_t h;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) h[i] = (_Float16) v[u][i];
-                put(iv0 + 64 * u, h);
-            }
+            for (int i = 0; i < 4; ++i) h[i] = (_Float16) v[u][i];
+            put(iv0 + 64 * u, h);
         }
     }
 }

@@ -3146,11 +3146,11 @@ bool vx_proj_add_ok(const vx_tensor * w, const vx_tensor * x, const vx_tensor * 
     return proj_tiles_fill(b, mid, w, x, residual, dst, 0.0f, act_mode) && mid;
 }
 
+// (the activation tiles of gemm_mid.hip's kernel; where vx_proj_add_run takes the streaming kernel they stay unused)
 size_t vx_proj_add_bytes(const vx_tensor * w, const vx_tensor * x) { return vx_gm_tile_bytes(w->ne[0], x->ne[1], 1); }
 
-// The streaming kernel with a cache write's scalar added to every activation (K of 513 to 1024 and more than 16 tokens: four waves).  Here and
-// not in launch_gemv_dma, so that the instance lies behind the decode step's kernels in the code object: among them, a step of batch 16
-// took 0.8 % longer with the same instructions in every kernel.
+// The streaming kernel with a cache write's scalar added to every activation (K of 513 to 1024 and more than 16 tokens: four waves).  By itself
+// and not in launch_gemv_dma: one caller, one wave count, one epilogue.
 static bool launch_gemv_add1(const mm_args & b, hipStream_t st) {
     mm_args a = b;
     int  nw;
