@@ -168,3 +168,34 @@ def test_copy_filled_on_one_stream_read_on_another(pkg, gpu):
         assert same_bits(outs[0], outs[1]) and same_bits(outs[0], outs[2])
     finally:
         L.vx_weights_unpin(pool.data_ptr())
+
+
+def test_dropping_one_of_several_copies_waits_for_its_readers(pkg, gpu):
+    """As dropping an allocation of its own does: the caller may write to or free the weights next."""
+    import torch
+    say("kept tiles: a copy dropped with kernels in flight, its neighbour staying")
+    L, d = pkg.lib(), pkg.desc
+    M, K, N = 4096, 1024, 2048
+    g = rng("kept-drop")
+    pool = torch.stack([q8_dev((0.05 * g.standard_normal((M, K))).astype(np.float32))[0] for _ in range(2)]).contiguous()
+    x = dev(g.standard_normal((N, K)).astype(np.float32))
+    outs = torch.empty((2, N, M), dtype=torch.float32, device="cuda")
+    side, done = torch.cuda.Stream(), torch.cuda.Event()
+
+    def product(w):
+        pkg.check(L.vx_mul_mat(pkg.desc_q8(pool[w], K), d(x), d(outs[w]), pkg.ACT_FLOAT, side.cuda_stream), "mul_mat")
+
+    copies = kept_bytes(L)[1]
+    pkg.check(L.vx_weights_pin(pool.data_ptr(), pool.numel()), "pin")
+    try:
+        product(0)
+        product(1)
+        torch.cuda.synchronize()
+        assert kept_bytes(L)[1] == copies + 2
+        for _ in range(400):   # some 13 ms of kernels
+            product(0)
+        done.record(side)
+        pkg.check(L.vx_weights_changed(pool[0].data_ptr(), pool[0].numel()), "changed")
+        assert done.query() and kept_bytes(L)[1] == copies + 1
+    finally:
+        L.vx_weights_unpin(pool.data_ptr())

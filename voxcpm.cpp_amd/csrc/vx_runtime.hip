@@ -110,11 +110,17 @@ void * block_space(int dev, size_t bytes, size_t cap, void ** block) { // (g_pin
     b->live++;
     return at;
 }
-void release_copy(derived_entry & e) { // (g_pin_mutex held) hipFree waits for the kernels still reading
+// (g_pin_mutex held) Waits for the kernels still reading, of the copy or, under its fill, of the weights, which the caller may free next:
+// hipFree does.
+void release_copy(derived_entry & e) {
     if (e.ready) (void) hipEventDestroy(e.ready);
     for (size_t i = 0; i < g_blocks.size(); ++i) {
         derived_block & b = g_blocks[i];
-        if (b.ptr != e.block || --b.live > 0) continue;
+        if (b.ptr != e.block) continue;
+        if (--b.live > 0) {
+            if (hipDeviceSynchronize() != hipSuccess) (void) hipGetLastError();
+            break;
+        }
         (void) hipFree(b.ptr);
         g_block_bytes -= b.bytes;
         g_blocks.erase(g_blocks.begin() + (long) i);
